@@ -818,6 +818,14 @@ template <typename T> int launch_pair(erm_ctx *c, const Params &k, int n, bool b
   return launch_check(c, "k_pair");
 }
 
+// realcal_self of n configurations of k.ns sites into out[n].  A workgroup
+// per configuration: 1024 threads from 64 sites on (2016 pairs, two or more
+// per thread), where a configuration's pairs are the longest chain of the
+// launch, 256 below it.
+void launch_selfreal(erm_ctx *c, const Params &k, int n, const double *spos, const double *q, double *out) {
+  hipLaunchKernelGGL(k_selfreal, dim3(n), dim3(k.ns >= 64 ? SELF_THR : NTHR), 0, c->st, k, spos, q, out);
+}
+
 // Energies of a batch of configurations into d_uv (sorted molecule order);
 // flags select the terms.  Stage events ev[0..6].
 template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
@@ -951,12 +959,9 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
     // particle (engproc.F90:712-730), recomputed per configuration otherwise
     int per_item = (c->P.slttype != 2);
     if (per_item) {
-      for (int b = 0; b < n; ++b)
-        hipLaunchKernelGGL(k_selfreal, dim3(1), dim3(NTHR), 0, c->st, k, dp<double>(c->d_spos), b,
-                           dp<double>(c->d_qslt), dp<double>(c->d_selfreal) + b);
+      launch_selfreal(c, k, n, dp<double>(c->d_spos), dp<double>(c->d_qslt), dp<double>(c->d_selfreal));
     } else if (!c->have_usreal) {
-      hipLaunchKernelGGL(k_selfreal, dim3(1), dim3(NTHR), 0, c->st, k, dp<double>(c->d_spos), 0,
-                         dp<double>(c->d_qslt), dp<double>(c->d_usreal));
+      launch_selfreal(c, k, 1, dp<double>(c->d_spos), dp<double>(c->d_qslt), dp<double>(c->d_usreal));
       c->have_usreal = true;
     }
     TRY(launch_check(c, "k_selfreal"));
@@ -1644,8 +1649,8 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
     km.solute_charge = m->mol_charge[m->slt_template];
     TRY(ensure(m, m->d_usreal, sizeof(double)));
     if (!m->have_usreal) {
-      hipLaunchKernelGGL(k_selfreal, dim3(1), dim3(NTHR), 0, c->st, km, dp<double>(c->d_spos) + (size_t)R[r].site0 * 3,
-                         0, dp<double>(m->d_qslt), dp<double>(m->d_usreal));
+      launch_selfreal(c, km, 1, dp<double>(c->d_spos) + (size_t)R[r].site0 * 3, dp<double>(m->d_qslt),
+                      dp<double>(m->d_usreal));
       TRY(launch_check(c, "k_selfreal"));
       m->have_usreal = true;
     }
@@ -2305,8 +2310,7 @@ int32_t erm_realcal_self(erm_ctx *c, int32_t solute, const double *pos, double *
     if (!pos) return fail(c, ERM_E_ARG, "refs mode needs test-particle coordinates");
     HIPCHK(c, hipMemcpyAsync(c->d_spos.p, pos, sizeof(double) * ns * 3, hipMemcpyHostToDevice, c->st));
   }
-  hipLaunchKernelGGL(k_selfreal, dim3(1), dim3(NTHR), 0, c->st, c->kp, dp<double>(c->d_spos), 0,
-                     dp<double>(c->d_qslt), dp<double>(c->d_selfreal));
+  launch_selfreal(c, c->kp, 1, dp<double>(c->d_spos), dp<double>(c->d_qslt), dp<double>(c->d_selfreal));
   TRY(launch_check(c, "k_selfreal"));
   HIPCHK(c, hipMemcpyAsync(self_real, c->d_selfreal.p, sizeof(double), hipMemcpyDeviceToHost, c->st));
   return sync(c);

@@ -599,11 +599,7 @@ template <typename T> int frame_prep(erm_ctx *c) {
   Params &k = c->kp;
   const int ncell = k.nb[0] * k.nb[1] * k.nb[2];
   const int S = c->slvmax;
-  int nsites = 0;
-  for (int kk = 0; kk < S; ++kk) {
-    int m = c->tagpt[kk];
-    nsites += c->mol_begin[m + 1] - c->mol_begin[m];
-  }
+  const int nsites = c->nsites;
   TRY(ensure(c, c->d_cellid, sizeof(int) * S));
   TRY(ensure(c, c->d_count, sizeof(int) * (ncell + 1)));
   TRY(ensure(c, c->d_cell_start, sizeof(int) * (ncell + 1)));
@@ -614,7 +610,6 @@ template <typename T> int frame_prep(erm_ctx *c) {
   TRY(ensure(c, c->d_mol_first, sizeof(int) * (S + 1)));
   TRY(ensure(c, c->d_mol_q, sizeof(double) * S));
   TRY(ensure(c, c->d_mol_spec, sizeof(int) * S));
-  TRY(ensure(c, c->d_mol_m, sizeof(int) * S));
   TRY(ensure(c, c->d_mol_d1, sizeof(double) * S));
   TRY(ensure(c, c->d_jof, sizeof(int) * S));
   TRY(ensure(c, c->d_sx, sizeof(double) * nsites));
@@ -638,27 +633,26 @@ template <typename T> int frame_prep(erm_ctx *c) {
   TRY(launch_check(c, "k_frame_clear"));
   const int tb = 256, gb = (S + tb - 1) / tb;
   hipLaunchKernelGGL(k_mol_cell, dim3(gb), dim3(tb), 0, c->st, k, dp<double>(c->d_pos), dp<int>(c->d_tagpt),
-                     dp<int>(c->d_mol_begin), dp<int>(c->d_cellid), dp<int>(c->d_count),
-                     dp<unsigned long long>(c->d_rm));
+                     dp<int>(c->d_mol_begin), dp<int>(c->d_cellid), dp<int>(c->d_count));
   TRY(launch_check(c, "k_mol_cell"));
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->st, dp<int>(c->d_count), dp<int>(c->d_cell_start), ncell,
                      dp<int>(c->d_fill), (int *)nullptr, 0, 0);
   TRY(launch_check(c, "k_scan"));
   hipLaunchKernelGGL(k_mol_scatter, dim3(gb), dim3(tb), 0, c->st, k, dp<int>(c->d_cellid), dp<int>(c->d_fill),
-                     dp<int>(c->d_tagpt), dp<int>(c->d_mol_begin), dp<int>(c->d_mol_k), dp<int>(c->d_mol_ns),
-                     dp<int>(c->d_jof));
+                     dp<int>(c->d_tagpt), dp<int>(c->d_mol_begin), dp<double>(c->d_mol_charge), dp<int>(c->d_uvspec),
+                     dp<int>(c->d_mol_k), dp<int>(c->d_mol_ns), dp<int>(c->d_jof), dp<double>(c->d_mol_q),
+                     dp<int>(c->d_mol_spec), dp<double>(c->d_mol_d1));
   TRY(launch_check(c, "k_mol_scatter"));
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->st, dp<int>(c->d_mol_ns), dp<int>(c->d_mol_first), S,
                      (int *)nullptr, (int *)nullptr, 0, 0);
   TRY(launch_check(c, "k_scan"));
-  hipLaunchKernelGGL(k_site_fill<T>, dim3(gb), dim3(tb), 0, c->st, k, dp<double>(c->d_pos), dp<int>(c->d_tagpt),
-                     dp<int>(c->d_mol_begin), dp<double>(c->d_charge), dp<int>(c->d_cvt),
-                     dp<double>(c->d_mol_charge), dp<int>(c->d_uvspec), dp<int>(c->d_mol_k),
+  hipLaunchKernelGGL(k_site_fill<T>, dim3((nsites + SITE_THR - 1) / SITE_THR), dim3(SITE_THR), 0, c->st, k, nsites,
+                     dp<double>(c->d_pos), dp<int>(c->d_site_k), dp<int>(c->d_site_a), dp<int>(c->d_tagpt),
+                     dp<int>(c->d_mol_begin), dp<double>(c->d_charge), dp<int>(c->d_cvt), dp<int>(c->d_jof),
                      dp<int>(c->d_mol_first), dp<double>(c->d_sx), dp<double>(c->d_sy), dp<double>(c->d_sz),
-                     dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sg), dp<T>(c->d_sw), dp<double>(c->d_mol_q),
-                     dp<int>(c->d_mol_spec), dp<int>(c->d_mol_m), dp<double>(c->d_mol_d1));
+                     dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sg), dp<T>(c->d_sw), dp<double>(c->d_mol_d1),
+                     dp<unsigned long long>(c->d_rm));
   TRY(launch_check(c, "k_site_fill"));
-  c->nsites = nsites;
   c->jof_stale = true;
   if (!zsort) return ERM_OK;
   // sites sorted by PME plane g3, dealt over the gather's LDS bank classes
@@ -1969,6 +1963,14 @@ int32_t erm_set_topology(erm_ctx *c, int32_t natom, int32_t nmol, const int32_t 
       cvt[a] = cv[t];
     }
   }
+  // the physical sites in tagpt order: their molecule's tagpt index and atom
+  std::vector<int> site_k, site_a;
+  for (int k = 0; k < c->slvmax; ++k)
+    for (int a = c->mol_begin[c->tagpt[k]]; a < c->mol_begin[c->tagpt[k] + 1]; ++a) {
+      site_k.push_back(k);
+      site_a.push_back(a);
+    }
+  c->nsites = (int)site_k.size();
   c->nvt = (int)c->vtypes.size();
   size_t tbytes = c->fp32 ? 4 : 8;
   if ((size_t)2 * c->ns * c->nvt * tbytes + 4 * (size_t)c->ns * tbytes > 100 * 1024)
@@ -1999,6 +2001,8 @@ int32_t erm_set_topology(erm_ctx *c, int32_t natom, int32_t nmol, const int32_t 
   TRY(upload(c, c->d_charge, charge, natom));
   TRY(upload(c, c->d_tagpt, c->tagpt.data(), c->slvmax));
   TRY(upload(c, c->d_kof, c->kof.data(), c->nmol));
+  TRY(upload(c, c->d_site_k, site_k.data(), site_k.size()));
+  TRY(upload(c, c->d_site_a, site_a.data(), site_a.size()));
   TRY(upload(c, c->d_cvt, cvt.data(), natom));
   TRY(upload(c, c->d_mol_charge, mol_charge, nmol));
   TRY(upload(c, c->d_uvspec, uvspec, nmol));

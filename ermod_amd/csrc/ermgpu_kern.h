@@ -65,31 +65,17 @@ __device__ __forceinline__ int cell_index(const Params &P, const double *w) {
   return c[0] + P.nb[0] * (c[1] + P.nb[1] * c[2]);
 }
 
-// cell of each physical molecule (by its first site) and the largest
-// distance of a site from its molecule's first site
+// cell of each physical molecule (by its first site)
 static __global__ void k_mol_cell(Params P, const double *__restrict__ pos, const int *__restrict__ tagpt,
-                           const int *__restrict__ mol_begin, int *cellid, int *count,
-                           unsigned long long *rm_ord) {
+                           const int *__restrict__ mol_begin, int *cellid, int *count) {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= P.slvmax) return;
-  int m = tagpt[k];
-  int a0 = mol_begin[m], a1 = mol_begin[m + 1];
+  const int a0 = mol_begin[tagpt[k]];
   double w[3];
   for (int d = 0; d < 3; ++d) w[d] = wrap1(pos[3 * a0 + d], P.L[d]);
   int c = P.boxshp ? cell_index(P, w) : 0;
   cellid[k] = c;
   atomicAdd(&count[c], 1);
-  double rm = 0.0;
-  for (int a = a0 + 1; a < a1; ++a) {
-    double s2 = 0.0;
-    for (int d = 0; d < 3; ++d) {
-      double x = pos[3 * a + d] - pos[3 * a0 + d];
-      if (P.boxshp) x -= P.L[d] * rint(x / P.L[d]);
-      s2 += x * x;
-    }
-    rm = fmax(rm, sqrt(s2));
-  }
-  atomicMax(rm_ord, dbl_to_ord(rm));
 }
 
 // Exclusive scan of in[0, n) into out[0, n], out[n] the total (one
@@ -134,12 +120,15 @@ static __global__ void k_frame_clear(int *count, int nc, int *zcount, int nz, un
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nc) count[i] = 0;
   if (i < nz) zcount[i] = 0;
-  if (i == 0) *rm = 0ULL;
+  if (i == 0) *rm = dbl_to_ord(0.0);
 }
 
+// sorted slot of every molecule and its per-molecule data; its reach mol_d1
+// starts at 0 and k_site_fill raises it
 static __global__ void k_mol_scatter(Params P, const int *__restrict__ cellid, int *fill,
                               const int *__restrict__ tagpt, const int *__restrict__ mol_begin,
-                              int *mol_k, int *mol_ns, int *jof) {
+                              const double *__restrict__ mol_charge, const int *__restrict__ uvspec, int *mol_k,
+                              int *mol_ns, int *jof, double *mol_q, int *mol_spec, double *mol_d1) {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= P.slvmax) return;
   int j = atomicAdd(&fill[cellid[k]], 1);
@@ -147,68 +136,79 @@ static __global__ void k_mol_scatter(Params P, const int *__restrict__ cellid, i
   mol_k[j] = k;
   jof[k] = j;
   mol_ns[j] = mol_begin[m + 1] - mol_begin[m];
+  mol_q[j] = mol_charge[m];
+  mol_spec[j] = uvspec[m];
+  mol_d1[j] = 0.0;
 }
 
 // sorted site arrays: wrapped coordinates (realcal.F90:789-885, cuboid),
 // charges, compact LJ types and B-spline weights (calc_spline_molecule,
-// recpcal.F90:408-442)
+// recpcal.F90:408-442), and the reach of every molecule from its first site
+// (mol_d1, and its largest value rm_ord): minimum images in a periodic box,
+// the pair kernels' convention, so no site of the molecule lies farther than
+// mol_d1 from its first.  A thread takes one physical site i (tagpt index
+// site_k[i], atom site_a[i]); its molecule's sorted first site gives its
+// slot.  Bound by the latency of the 3 p weights' FP64 chains: a thread per
+// molecule ran a 300-site solute's sites one after another (20000 waters,
+// order 6: 4.17 ms, now 0.032 ms), a 12-site one's likewise (0.079 -> 0.011 ms).  The
+// reach is a maximum: the order of its atomics does not show.
+constexpr int SITE_THR = 64;  // one wave: SITE_THR sites' chains per SIMD, most CUs busy from 16000 sites on
 template <typename T>
-__global__ void k_site_fill(Params P, const double *__restrict__ pos, const int *__restrict__ tagpt,
-                            const int *__restrict__ mol_begin, const double *__restrict__ charge,
-                            const int *__restrict__ cvt, const double *__restrict__ mol_charge,
-                            const int *__restrict__ uvspec, const int *__restrict__ mol_k,
-                            const int *__restrict__ mol_first, double *sx, double *sy, double *sz,
-                            T *sq, int *sct, int *sg, T *sw, double *mol_q, int *mol_spec,
-                            int *mol_m, double *mol_d1) {
+__global__ __launch_bounds__(SITE_THR) void k_site_fill(Params P, int nsites, const double *__restrict__ pos,
+                            const int *__restrict__ site_k, const int *__restrict__ site_a,
+                            const int *__restrict__ tagpt, const int *__restrict__ mol_begin,
+                            const double *__restrict__ charge, const int *__restrict__ cvt,
+                            const int *__restrict__ jof, const int *__restrict__ mol_first, double *sx, double *sy,
+                            double *sz, T *sq, int *sct, int *sg, T *sw, double *mol_d1,
+                            unsigned long long *rm_ord) {
 #pragma clang fp contract(off)
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= P.slvmax) return;
-  int m = tagpt[mol_k[j]];
-  mol_q[j] = mol_charge[m];
-  mol_spec[j] = uvspec[m];
-  mol_m[j] = m;
-  {
-    // the molecule's reach from its first site (minimum images in a
-    // periodic box, the pair kernels' convention): no site of the molecule
-    // lies farther than mol_d1 from its first
-    const double *x0 = pos + 3 * mol_begin[m];
-    double d1 = 0.0;
-    for (int a = mol_begin[m] + 1; a < mol_begin[m + 1]; ++a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  unsigned long long reach = 0ULL;  // bits of a distance >= 0 order like the distance
+  if (i < nsites) {
+    const int k = site_k[i], a = site_a[i], j = jof[k], a0 = mol_begin[tagpt[k]];
+    const int t = mol_first[j] + (a - a0);
+    const double *x = pos + 3 * a, *x0 = pos + 3 * a0;
+    if (a != a0) {
       double dd = 0.0;
       for (int e = 0; e < 3; ++e) {
-        double d = pos[3 * a + e] - x0[e];
+        double d = x[e] - x0[e];
         if (P.boxshp) d = d - P.L[e] * rint(d / P.L[e]);
         dd = dd + d * d;
       }
-      d1 = fmax(d1, sqrt(dd));
+      const double d1 = sqrt(dd);
+      if (d1 > 0.0) {
+        reach = (unsigned long long)__double_as_longlong(d1);
+        atomicMax(reinterpret_cast<unsigned long long *>(mol_d1 + j), reach);
+      }
     }
-    mol_d1[j] = d1;
-  }
-  int t = mol_first[j];
-  const int Ks[3] = {P.K1, P.K2, P.K3};
-  for (int a = mol_begin[m]; a < mol_begin[m + 1]; ++a, ++t) {
-    const double *x = pos + 3 * a;
     // raw coordinates without a box (realcal_prepare, realcal.F90:137-146)
     sx[t] = P.boxshp ? wrap1(x[0], P.L[0]) : x[0];
     sy[t] = P.boxshp ? wrap1(x[1], P.L[1]) : x[1];
     sz[t] = P.boxshp ? wrap1(x[2], P.L[2]) : x[2];
     sq[t] = (T)charge[a];
     sct[t] = cvt[a];
-    if (P.cltype == 0) continue;  // no reciprocal space
-    int g[3];
-    for (int d = 0; d < 3; ++d) {
-      double f = P.invcl[d] * x[0] + P.invcl[3 + d] * x[1] + P.invcl[6 + d] * x[2];
-      f = f - floor(f);
-      double factor = f * (double)Ks[d];
-      // f - floor(f) may round to 1.0: factor == K gives the weights of
-      // base K, i.e. of base 0 (indices are taken mod K); NaN maps to 0
-      int rci = (factor >= 0.0 && factor <= (double)Ks[d]) ? (int)factor : 0;
-      for (int s = 0; s < P.p; ++s)
-        sw[((size_t)t * 3 + d) * P.p + s] = (T)spline_value_dev(P.coeff, P.p, factor - (double)(rci - s));
-      g[d] = rci % Ks[d];
+    if (P.cltype != 0) {
+      const int Ks[3] = {P.K1, P.K2, P.K3};
+      int g[3];
+      for (int d = 0; d < 3; ++d) {
+        double f = P.invcl[d] * x[0] + P.invcl[3 + d] * x[1] + P.invcl[6 + d] * x[2];
+        f = f - floor(f);
+        double factor = f * (double)Ks[d];
+        // f - floor(f) may round to 1.0: factor == K gives the weights of
+        // base K, i.e. of base 0 (indices are taken mod K); NaN maps to 0
+        int rci = (factor >= 0.0 && factor <= (double)Ks[d]) ? (int)factor : 0;
+        for (int s = 0; s < P.p; ++s)
+          sw[((size_t)t * 3 + d) * P.p + s] = (T)spline_value_dev(P.coeff, P.p, factor - (double)(rci - s));
+        g[d] = rci % Ks[d];
+      }
+      sg[t] = g[0] | (g[1] << 10) | (g[2] << 20);
     }
-    sg[t] = g[0] | (g[1] << 10) | (g[2] << 20);
   }
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long v = __shfl_xor(reach, o, 64);
+    reach = (v > reach) ? v : reach;
+  }
+  if (threadIdx.x == 0 && reach) atomicMax(rm_ord, dbl_to_ord(__longlong_as_double((long long)reach)));
 }
 
 // --------------------------------------------------------------------------

@@ -651,7 +651,7 @@ template <typename T> int frame_prep(erm_ctx *c) {
                      dp<int>(c->d_mol_begin), dp<double>(c->d_charge), dp<int>(c->d_cvt), dp<int>(c->d_jof),
                      dp<int>(c->d_mol_first), dp<double>(c->d_sx), dp<double>(c->d_sy), dp<double>(c->d_sz),
                      dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sg), dp<T>(c->d_sw), dp<double>(c->d_mol_d1),
-                     dp<unsigned long long>(c->d_rm));
+                     c->sltlist.size() == 1 ? c->kof[c->sltlist[0]] : -1, dp<unsigned long long>(c->d_rm));
   TRY(launch_check(c, "k_site_fill"));
   c->jof_stale = true;
   if (!zsort) return ERM_OK;
@@ -760,6 +760,45 @@ inline int pair_splits(int nchunk, int nwave) {
   return std::max(1, std::min(64, (nchunk + per - 1) / per));
 }
 
+// How one launch of the tiled pair kernel divides n configurations with
+// about `cand` candidate molecules each: cm molecules per chunk, nsplit
+// workgroups per configuration and the solute in `parts` of nss sites.
+struct PairShape {
+  int cm, nsplit, parts, nss;
+};
+// Enough waves to fill the chip come first.  Every wave would take
+// PAIR_CHUNKS_PER_WAVE chunks of 64 molecules (the set-up of a workgroup is
+// shared); with fewer than PAIR_WAVES waves in all it takes less, down to
+// PAIR_MIN_MOLS molecules (48 water sites of a tile of 64), and a solute of
+// more than PAIR_PART sites whose configurations still leave half the chip
+// idle goes over in parts of at least PAIR_PART sites.  A rigid test particle
+// stays whole: a group's members sum its sites in one order whatever the
+// batch, and so does the context alone.  PAIR_WAVES = 1024 (4 per CU): with
+// 4096, 256 configurations of a 20-site solute took four workgroups each and
+// their set-up cost more than it gave (12000 sites: division 11.35 against
+// 11.08 ms).  Measured per launch against 4 chunks per wave throughout: one
+// 300-site solute in 20000 waters 3.94 -> 0.099 ms (8 parts), one 12-site
+// solute in 1000 waters 0.076 -> 0.017 ms, 50 insertions of 5 sites
+// 0.047 -> 0.021 ms.
+constexpr int PAIR_WAVES = 1024, PAIR_MIN_MOLS = 16, PAIR_PART = 32, PAIR_MAX_PARTS = 8;
+PairShape pair_shape(int n, double cand, int ns, int nwave, bool whole) {
+  PairShape s;
+  double mpw = cand * n / PAIR_WAVES;  // molecules per wave
+  mpw = std::min(64.0 * PAIR_CHUNKS_PER_WAVE, std::max((double)PAIR_MIN_MOLS, mpw));
+  s.cm = std::min(64, (int)std::ceil(mpw / 16.0) * 16);
+  const int per = s.cm * std::max(1, (int)std::ceil(mpw / s.cm)) * nwave;
+  s.nsplit = std::max(1, (int)std::ceil(cand / per));
+  s.parts = 1;
+  const long waves = (long)n * s.nsplit * nwave;
+  if (!whole && ns > PAIR_PART && waves < PAIR_WAVES)
+    s.parts = std::min({PAIR_MAX_PARTS, ns / PAIR_PART, (int)((2 * PAIR_WAVES + waves - 1) / waves)});
+  s.nss = (ns + s.parts - 1) / s.parts;
+  s.nss = (s.nss + PT_GRP - 1) / PT_GRP * PT_GRP;
+  s.parts = (ns + s.nss - 1) / s.nss;
+  if (s.parts == 1) s.nss = ns;
+  return s;
+}
+
 // real-space pairs of a batch: the tiled kernel with compacted pair lists,
 // or the kernel with one thread per candidate molecule (pair_path 1, or
 // when the tiles' LDS does not fit)
@@ -771,28 +810,32 @@ template <typename T> int launch_pair(erm_ctx *c, const Params &k, int n, bool b
   const int nwave = NTHR / 64;
   const size_t lt = pair_tile_lds<T>(ns, c->nvt, segcap, nwave);
   if (c->pair_path == 0 && lt <= c->lds_cap) {
-    // chunks of 64 candidate molecules, PAIR_CHUNKS_PER_WAVE per wave (the
-    // per-configuration set-up of a workgroup is shared by its chunks)
-    const int nchunk = (int)std::ceil(frac * S / 64.0);
-    const int nsplit = pair_splits(nchunk, nwave);
-    if (bare) {
-      TRY(set_lds(c, (const void *)k_pair_tile<T, true>, lt, "k_pair_tile"));
-      hipLaunchKernelGGL((k_pair_tile<T, true>), dim3(n, nsplit), dim3(NTHR), lt, c->st, k, dp<double>(c->d_spos),
-                         dp<double>(c->d_sref), dp<T>(c->d_qslt_t), dp<T>(c->d_sltlj), dp<int>(c->d_cell_start),
-                         dp<int>(c->d_mol_first), dp<int>(c->d_mol_ns), dp<double>(c->d_sx), dp<double>(c->d_sy),
-                         dp<double>(c->d_sz), dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sltj),
-                         dp<double>(c->d_rm), dp<double>(c->d_sltlj64), dp<double>(c->d_qslt),
-                         dp<double>(c->d_mol_d1), dp<double>(c->d_uv));
-    } else {
-      TRY(set_lds(c, (const void *)k_pair_tile<T, false>, lt, "k_pair_tile"));
-      hipLaunchKernelGGL((k_pair_tile<T, false>), dim3(n, nsplit), dim3(NTHR), lt, c->st, k, dp<double>(c->d_spos),
-                         dp<double>(c->d_sref), dp<T>(c->d_qslt_t), dp<T>(c->d_sltlj), dp<int>(c->d_cell_start),
-                         dp<int>(c->d_mol_first), dp<int>(c->d_mol_ns), dp<double>(c->d_sx), dp<double>(c->d_sy),
-                         dp<double>(c->d_sz), dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sltj),
-                         dp<double>(c->d_rm), dp<double>(c->d_sltlj64), dp<double>(c->d_qslt),
-                         dp<double>(c->d_mol_d1), dp<double>(c->d_uv));
+    const PairShape ps = pair_shape(n, frac * S, ns, nwave, c->P.slttype == 2);
+    const size_t nuv = (size_t)n * (S + 1);
+    double *out = dp<double>(c->d_uv);
+    if (ps.parts > 1) {
+      TRY(ensure(c, c->d_upart, sizeof(double) * nuv * ps.parts));
+      out = dp<double>(c->d_upart);
+      hipLaunchKernelGGL(k_fill<double>, dim3((unsigned)((nuv * ps.parts + NTHR - 1) / NTHR)), dim3(NTHR), 0, c->st, out,
+                         nuv * ps.parts, 0.0);
+      TRY(launch_check(c, "k_fill"));
     }
-    return launch_check(c, "k_pair_tile");
+    const size_t lp = pair_tile_lds<T>(ps.nss, c->nvt, segcap, nwave);
+    auto *f = bare ? k_pair_tile<T, true> : k_pair_tile<T, false>;
+    TRY(set_lds(c, (const void *)f, lp, "k_pair_tile"));
+    hipLaunchKernelGGL(f, dim3(n, ps.nsplit, ps.parts), dim3(NTHR), lp, c->st, k, ps.cm, ps.nss, nuv,
+                       dp<double>(c->d_spos), dp<double>(c->d_sref), dp<T>(c->d_qslt_t), dp<T>(c->d_sltlj),
+                       dp<int>(c->d_cell_start), dp<int>(c->d_mol_first), dp<int>(c->d_mol_ns), dp<double>(c->d_sx),
+                       dp<double>(c->d_sy), dp<double>(c->d_sz), dp<T>(c->d_sq), dp<int>(c->d_sct),
+                       dp<int>(c->d_sltj), dp<double>(c->d_rm), dp<double>(c->d_sltlj64), dp<double>(c->d_qslt),
+                       dp<double>(c->d_mol_d1), out);
+    TRY(launch_check(c, "k_pair_tile"));
+    if (ps.parts > 1) {
+      hipLaunchKernelGGL(k_pair_parts, dim3((unsigned)((nuv + NTHR - 1) / NTHR)), dim3(NTHR), 0, c->st, nuv, ps.parts,
+                         out, dp<double>(c->d_uv));
+      TRY(launch_check(c, "k_pair_parts"));
+    }
+    return ERM_OK;
   }
   const int nsplit = std::max(1, std::min(16, (int)std::ceil(frac * S / (2.0 * NTHR))));
   const size_t lpair = sizeof(T) * ((size_t)7 * ns + (size_t)2 * ns * c->nvt) + sizeof(int) * (2 * MAXSEG + 2) + 64;
@@ -1622,7 +1665,8 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
         Params kr = k;
         kr.ns = R[r].ns;
         const size_t c0 = R[r].cfg0;
-        hipLaunchKernelGGL((k_pair_tile<T, false>), dim3(R[r].ncfg, R[r].nsplit), dim3(NTHR), lt, c->st, kr,
+        hipLaunchKernelGGL((k_pair_tile<T, false>), dim3(R[r].ncfg, R[r].nsplit), dim3(NTHR), lt, c->st, kr, 64,
+                           R[r].ns, (size_t)0,
                            dp<double>(c->d_spos) + (size_t)R[r].site0 * 3, dp<double>(c->d_sref) + 4 * c0,
                            static_cast<const T *>(R[r].q_t), static_cast<const T *>(R[r].lj_t),
                            dp<int>(c->d_cell_start), dp<int>(c->d_mol_first), dp<int>(c->d_mol_ns),

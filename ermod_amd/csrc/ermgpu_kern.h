@@ -151,7 +151,9 @@ static __global__ void k_mol_scatter(Params P, const int *__restrict__ cellid, i
 // slot.  Bound by the latency of the 3 p weights' FP64 chains: a thread per
 // molecule ran a 300-site solute's sites one after another (20000 waters,
 // order 6: 4.17 ms, now 0.032 ms), a 12-site one's likewise (0.079 -> 0.011 ms).  The
-// reach is a maximum: the order of its atomics does not show.
+// reach is a maximum: the order of its atomics does not show.  skip_k: the
+// only solute, which is never its own solvent (-1: none); its extent stays out
+// of rm_ord, which sets the radius of the pair kernels' candidates.
 constexpr int SITE_THR = 64;  // one wave: SITE_THR sites' chains per SIMD, most CUs busy from 16000 sites on
 template <typename T>
 __global__ __launch_bounds__(SITE_THR) void k_site_fill(Params P, int nsites, const double *__restrict__ pos,
@@ -159,7 +161,7 @@ __global__ __launch_bounds__(SITE_THR) void k_site_fill(Params P, int nsites, co
                             const int *__restrict__ tagpt, const int *__restrict__ mol_begin,
                             const double *__restrict__ charge, const int *__restrict__ cvt,
                             const int *__restrict__ jof, const int *__restrict__ mol_first, double *sx, double *sy,
-                            double *sz, T *sq, int *sct, int *sg, T *sw, double *mol_d1,
+                            double *sz, T *sq, int *sct, int *sg, T *sw, double *mol_d1, int skip_k,
                             unsigned long long *rm_ord) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -179,6 +181,7 @@ __global__ __launch_bounds__(SITE_THR) void k_site_fill(Params P, int nsites, co
       if (d1 > 0.0) {
         reach = (unsigned long long)__double_as_longlong(d1);
         atomicMax(reinterpret_cast<unsigned long long *>(mol_d1 + j), reach);
+        if (k == skip_k) reach = 0ULL;
       }
     }
     // raw coordinates without a box (realcal_prepare, realcal.F90:137-146)
@@ -2257,10 +2260,10 @@ __device__ __forceinline__ int lanes_below(unsigned long long m) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
-// Configuration b (ns sites at xs), split `split` of nsplit workgroups;
-// all threads of the workgroup call it
+// Configuration b (ns sites at xs), split `split` of nsplit workgroups, cm
+// <= 64 candidate molecules per chunk; all threads of the workgroup call it
 template <typename T, bool BARE>
-__device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, int split, int nsplit,
+__device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, int split, int nsplit, int cm,
                                                const double *__restrict__ xs, const double *__restrict__ sref,
                                                const T *__restrict__ slt_q, const T *__restrict__ slt_lj,
                                                const int *__restrict__ cell_start,
@@ -2374,12 +2377,12 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
   // evaluation reads and writes a full round of slots without branches
   weq[PT_QCAP + lane] = 0.0;
   for (int k = lane; k < PT_QCAP + 64; k += 64) wq[k] = lane;
-  const int nchunk = (total + 63) >> 6;
+  const int nchunk = (total + cm - 1) / cm;
   for (int c = split * nw + wv; c < nchunk; c += nsplit * nw) {
-    // molecule of this lane: flattened candidate c*64 + lane
-    const int idx = c * 64 + lane;
+    // molecule of this lane: flattened candidate c*cm + lane
+    const int idx = c * cm + lane;
     int j = -1, nsm = 0, first = 0;
-    if (idx < total) {
+    if (lane < cm && idx < total) {
       int lo_s = 0, hi_s = nsg;  // last segment with seg_pre <= idx
       while (hi_s - lo_s > 1) {
         const int mid = (lo_s + hi_s) >> 1;
@@ -2693,8 +2696,13 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
   }
 }
 
+// Grid (configuration, split, part): a workgroup takes the solute sites
+// [part nss, part nss + nss) of its configuration, and the energies of part z
+// go to uv + z stride (uv itself with one part; with several, zeroed buffers
+// that k_pair_parts adds up).
 template <typename T, bool BARE = false>
-__global__ __launch_bounds__(NTHR) void k_pair_tile(Params P, const double *__restrict__ spos,
+__global__ __launch_bounds__(NTHR) void k_pair_tile(Params P, int cm, int nss, size_t stride,
+                                                    const double *__restrict__ spos,
                                                     const double *__restrict__ sref,
                                                     const T *__restrict__ slt_q, const T *__restrict__ slt_lj,
                                                     const int *__restrict__ cell_start,
@@ -2707,10 +2715,20 @@ __global__ __launch_bounds__(NTHR) void k_pair_tile(Params P, const double *__re
                                                     const double *__restrict__ slt_lj64,
                                                     const double *__restrict__ slt_q64,
                                                     const double *__restrict__ mol_d1, double *uv) {
-  const int b = blockIdx.x;
-  pair_tile_body<T, BARE>(P, P.ns, b, blockIdx.y, gridDim.y, spos + (size_t)b * P.ns * 3, sref, slt_q, slt_lj,
-                          cell_start, mol_first, mol_ns, sx, sy, sz, sq, sct, slt_j, rm_ord_p, slt_lj64, slt_q64,
-                          mol_d1, uv);
+  const int b = blockIdx.x, s0 = blockIdx.z * nss, ns = min(nss, P.ns - s0);
+  const size_t row = (size_t)2 * s0 * P.nvt;
+  pair_tile_body<T, BARE>(P, ns, b, blockIdx.y, gridDim.y, cm, spos + ((size_t)b * P.ns + s0) * 3, sref, slt_q + s0,
+                          slt_lj + row, cell_start, mol_first, mol_ns, sx, sy, sz, sq, sct, slt_j, rm_ord_p,
+                          slt_lj64 + row, slt_q64 + s0, mol_d1, uv + blockIdx.z * stride);
+}
+
+// uv[i] += the parts' energies, in part order
+static __global__ void k_pair_parts(size_t n, int np, const double *__restrict__ part, double *uv) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  double e = part[i];
+  for (int k = 1; k < np; ++k) e += part[k * n + i];
+  uv[i] += e;
 }
 
 // real space of a heterogeneous batch as one persistent launch:
@@ -2738,7 +2756,7 @@ __global__ __launch_bounds__(NTHR) void k_pair_tile_runs(Params P, const double 
     const int ns = runs[r].ns, nsplit = runs[r].nsplit, rel = it - runs[r].pitem0;
     const int bl = rel / nsplit, split = rel - bl * nsplit, b = runs[r].cfg0 + bl;
     const double *xs = spos + ((size_t)runs[r].site0 + (size_t)bl * ns) * 3;
-    pair_tile_body<T, BARE>(P, ns, b, split, nsplit, xs, sref, static_cast<const T *>(runs[r].q_t),
+    pair_tile_body<T, BARE>(P, ns, b, split, nsplit, 64, xs, sref, static_cast<const T *>(runs[r].q_t),
                             static_cast<const T *>(runs[r].lj_t), cell_start, mol_first, mol_ns, sx, sy, sz, sq, sct,
                             slt_j, rm_ord_p, runs[r].lj64, runs[r].q64, mol_d1, uv);
   }

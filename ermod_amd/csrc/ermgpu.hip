@@ -2821,39 +2821,18 @@ int32_t erm_engstore(erm_ctx *c) {
   TRY(need(c, false, true));
   if (hipSetDevice(c->P.device) != hipSuccess) return fail(c, ERM_E_DEVICE, "hipSetDevice");
   // single process: edens/engnorm, ecorr/engnorm, eself/engnorm, avslf/engnorm
-  const int E = c->ermax;
-  std::vector<double> sc(8), e(E);
-  HIPCHK(c, hipMemcpyAsync(sc.data(), c->d_scal.p, sizeof(double) * 8, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipMemcpyAsync(e.data(), c->d_edens.p, sizeof(double) * E, hipMemcpyDeviceToHost, c->st));
-  TRY(sync(c));
-  const double en = sc[0];
-  for (double &v : e) v = v / en;
-  TRY(upload(c, c->d_edens, e.data(), E));
-  if (c->P.corrcal) {
-    std::vector<double> m((size_t)E * E);
-    HIPCHK(c, hipMemcpyAsync(m.data(), c->d_ecorr.p, sizeof(double) * m.size(), hipMemcpyDeviceToHost, c->st));
-    TRY(sync(c));
-    for (double &v : m) v = v / en;
-    TRY(upload(c, c->d_ecorr, m.data(), m.size()));
-  }
-  if (c->esmax) {
-    std::vector<double> s(c->esmax);
-    HIPCHK(c, hipMemcpyAsync(s.data(), c->d_eself.p, sizeof(double) * s.size(), hipMemcpyDeviceToHost, c->st));
-    TRY(sync(c));
-    for (double &v : s) v = v / en;
-    TRY(upload(c, c->d_eself, s.data(), s.size()));
-  }
-  sc[2] = sc[2] / en;
-  TRY(upload(c, c->d_scal, sc.data(), 8));
-  if (c->kp.intm) {
-    // edintm / norm_intm (extensions/Intermediate/engproc.F90:656)
-    std::vector<double> ed(E), isc(3);
-    HIPCHK(c, hipMemcpyAsync(ed.data(), c->d_edintm.p, sizeof(double) * E, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(isc.data(), c->d_intm_sc.p, sizeof(double) * 3, hipMemcpyDeviceToHost, c->st));
-    TRY(sync(c));
-    for (double &v : ed) v = v / isc[0];
-    TRY(upload(c, c->d_edintm, ed.data(), E));
-  }
+  const size_t E = c->ermax;
+  auto over = [&](size_t n, const double *norm, double *acc) -> int {
+    hipLaunchKernelGGL(k_engstore, dim3((unsigned)((n + NTHR - 1) / NTHR)), dim3(NTHR), 0, c->st, n, norm, acc);
+    return launch_check(c, "k_engstore");
+  };
+  double *sc = dp<double>(c->d_scal);
+  TRY(over(E, sc, dp<double>(c->d_edens)));
+  if (c->P.corrcal) TRY(over(E * E, sc, dp<double>(c->d_ecorr)));
+  if (c->esmax) TRY(over(c->esmax, sc, dp<double>(c->d_eself)));
+  TRY(over(1, sc, sc + 2));
+  // edintm / norm_intm (extensions/Intermediate/engproc.F90:656)
+  if (c->kp.intm) TRY(over(E, dp<double>(c->d_intm_sc), dp<double>(c->d_edintm)));
   return sync(c);
 }
 

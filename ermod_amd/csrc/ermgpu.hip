@@ -441,6 +441,22 @@ int upload_real(erm_ctx *c, DBuf &b, const std::vector<double> &v) {
   return upload(c, b, v.data(), v.size());
 }
 
+// Configurations per batch when the caller leaves the choice (max_batch = 0):
+// 1024 where the half spectra, per-site sums and energies of so many stay
+// within 4 GiB, else 256.  A launch of the light kernels (poses, solute
+// splines, binning, weights, edens, the correlation matrix) costs 5-30 us
+// however few configurations it holds, and the heavy ones fill the chip's last
+// wave of workgroups once a batch.  Measured, 256 against 1024: 4 frames of
+// 1000 insertions of 20 sites among 4000 waters, 48^3, 11.08 -> 9.60 ms in
+// FP64, 7.97 -> 6.61 ms in FP32 (binning 450 -> 196, poses 304 -> 95, solute
+// splines 264 -> 92 us); 500 insertions at 64^3, order 6, 4.12 -> 3.93 ms.
+int default_batch(const erm_ctx *c) {
+  const size_t vb = c->fp32 ? sizeof(float2) : sizeof(double2);
+  const size_t hk = c->P.cltype == ERM_EL_COULOMB ? 0 : vb * c->kp.H * c->kp.K2 * c->kp.K3;
+  const size_t one = hk + sizeof(double) * ((size_t)c->nsites + c->slvmax + 1);
+  return 1024 * one <= ((size_t)4 << 30) ? 1024 : 256;
+}
+
 // per-solute-type tables: charges and LJ rows against the solvent types
 int solute_tables(erm_ctx *c) {
   int m = c->slt_template;
@@ -1829,7 +1845,7 @@ int32_t erm_create(const erm_params *prm, erm_ctx **out) {
   c->P = P;
   for (int d = 0; d < 3; ++d) c->P.ms[d] = msv[d];
   c->fp32 = (P.precision == ERM_FP32);
-  c->Bmax = P.max_batch > 0 ? P.max_batch : 256;
+  c->Bmax = P.max_batch > 0 ? P.max_batch : 256;  // 0: set with the topology (default_batch)
   {
     // LDS a workgroup may opt into (160 KB per CU on gfx950), with room for
     // the kernels' static arrays
@@ -2015,6 +2031,7 @@ int32_t erm_set_topology(erm_ctx *c, int32_t natom, int32_t nmol, const int32_t 
       site_a.push_back(a);
     }
   c->nsites = (int)site_k.size();
+  if (c->P.max_batch <= 0 && !c->batch_set) c->Bmax = default_batch(c);
   c->nvt = (int)c->vtypes.size();
   size_t tbytes = c->fp32 ? 4 : 8;
   if ((size_t)2 * c->ns * c->nvt * tbytes + 4 * (size_t)c->ns * tbytes > 100 * 1024)
@@ -2931,7 +2948,10 @@ int32_t erm_set_tuning(erm_ctx *c, int32_t max_batch, int32_t pme_path, int32_t 
       (column_threads != 0 && column_threads != 256 && column_threads != 512))
     return fail(c, ERM_E_ARG, "tuning out of range");
   if (column_threads > 0) c->zcol_T = column_threads;
-  if (max_batch > 0) c->Bmax = max_batch;
+  if (max_batch > 0) {
+    c->Bmax = max_batch;
+    c->batch_set = true;
+  }
   if (slab_planes > 0) c->tune_S = slab_planes;
   if (group_planes > 0) c->tune_Q = group_planes;
   if (slab_threads > 0) c->xslab_T = slab_threads;
@@ -3029,6 +3049,7 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
     }
   }
   TRY(apply(bestB, bestP, bestS, bestQ, bestT));
+  c->batch_set = true;
   if (bestP == 3) {  // z-column workgroup size for the chosen shape
     const int z0 = c->zcol_T;
     double ms;

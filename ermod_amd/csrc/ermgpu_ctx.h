@@ -45,6 +45,7 @@ struct erm_ctx {
   double stage_ms[ermh::NSTAGE_OUT] = {};
   bool fp32 = false;
   int Bmax = 256;
+  bool batch_set = false;  // Bmax chosen by erm_set_tuning or the autotuner
   // topology
   bool have_topo = false, have_bins = false, have_frame = false;
   int natom = 0, nmol = 0, ntype = 0;

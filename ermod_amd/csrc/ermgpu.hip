@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "ermgpu_ctx.h"
+#include "ermgpu_fft2.h"
 #include "ermgpu_grad.h"
 #include "ermgpu_traj.h"
 
@@ -521,6 +522,10 @@ bool zcol_fft(const erm_ctx *c, bool regp) { return regp && (c->kp.p == 4 || c->
 // z-column workgroups per configuration
 int zcol_groups(const erm_ctx *c, bool regp, int vb) {
   const int ncol = c->kp.H * c->kp.K2;
+  if (c->two_step) {
+    const int w = (vb == (int)sizeof(double2)) ? z2_cols<double> : z2_cols<float>;
+    return (ncol + w - 1) / w;
+  }
   if (!regp) {
     const int w = zcol_width(c->kp.K3, vb);
     return (ncol + w - 1) / w;
@@ -552,6 +557,69 @@ int launch_mol_sum(erm_ctx *c, const Params &kg, int n, const double *esite, con
                      c->st, kg, c->nsites, n, esite, dp<int>(c->d_zpos), dp<int>(c->d_mol_first),
                      dp<int>(c->d_mol_ns), dp<double>(c->d_mol_q), sltj, uv);
   return launch_check(c, "k_mol_sum");
+}
+
+// Slab shape of the two-step y/x kernel for n configurations: S planes per
+// workgroup, Q planes in LDS at a time (S = 0: none).
+struct Xy2Shape {
+  int S = 0, Q = 0;
+  size_t lds = 0;
+};
+// Two workgroups share a CU where a plane fits half its LDS.  A workgroup
+// transforms S + p - 1 planes for S owned ones: deeper slabs waste fewer halo
+// planes, shallower ones give few configurations more workgroups, so S is the
+// depth of the least work for the busiest CU.
+template <typename T> Xy2Shape xy2_shape(const erm_ctx *c, int n) {
+  const Params &k = c->kp;
+  Xy2Shape best;
+  const size_t cu = c->lds_cap + 10 * 1024;  // LDS of a CU
+  for (int per : {2, 1}) {
+    const size_t cap = std::min(cu / per, c->lds_cap);
+    int Q = 0;
+    while (xy2_lds<T>(Q + 1, k.K1, k.K2, k.H) <= cap) ++Q;
+    if (!Q) continue;
+    double cost = 0.0;
+    for (int S = 1; S <= std::min(k.K3, 32); ++S) {
+      const int nslab = (k.K3 + S - 1) / S;
+      const int planes = S + k.p - 1, ngrp = (planes + Q - 1) / Q;
+      const double t = std::max(1.0, (double)n * nslab / (per * c->ncu)) * (planes + 0.5 * ngrp);
+      if (!best.S || t < cost) {
+        cost = t;
+        best.S = S;
+        best.Q = std::min(Q, planes);
+      }
+    }
+    if (best.S) break;
+  }
+  if (best.S) best.lds = xy2_lds<T>(best.Q, k.K1, k.K2, k.H);
+  return best;
+}
+
+// The two-step PME kernels over n configurations, solute sites from site0 of
+// the batch buffers: z columns into d_Hk, then the y and x transforms and the
+// gather into d_esite.
+template <typename T> int launch_zcol2(erm_ctx *c, const Params &k, int n, int nblk) {
+  using V = typename C2<T>::type;
+  Fft2 f;
+  if (!fft2_split<T>(k.K3, f)) return fail(c, ERM_E_ENG_BUG, "two-step z length");
+  const size_t lds = z2_lds<T>(k.K3, k.p);
+  TRY(set_lds(c, (const void *)k_pme_zcol2<T>, lds, "k_pme_zcol2"));
+  hipLaunchKernelGGL(k_pme_zcol2<T>, dim3(nblk, n), dim3(Z2_THR), lds, c->st, k, f.A, f.B, dp<T>(c->d_engfac),
+                     dp<int>(c->d_sg3), dp<T>(c->d_sw3), dp<T>(c->d_sqv), dp<V>(c->d_w1h), dp<V>(c->d_w2h),
+                     dp<V>(c->d_tw3), dp<V>(c->d_Hk), dp<double>(c->d_selfp));
+  return launch_check(c, "k_pme_zcol2");
+}
+template <typename T> int launch_xyslab(erm_ctx *c, const Params &k, int n) {
+  using V = typename C2<T>::type;
+  Fft2 fy, fx;
+  const Xy2Shape sh = xy2_shape<T>(c, n);
+  if (!fft2_split<T>(k.K2, fy) || !fft2_split<T>(k.K1, fx) || !sh.S) return fail(c, ERM_E_ENG_BUG, "two-step slab");
+  TRY(set_lds(c, (const void *)k_pme_xyslab<T>, sh.lds, "k_pme_xyslab"));
+  const int nslab = (k.K3 + sh.S - 1) / sh.S;
+  hipLaunchKernelGGL(k_pme_xyslab<T>, dim3(nslab, n), dim3(XY2_THR), sh.lds, c->st, k, sh.S, sh.Q, fy, fx, c->nsites, dp<V>(c->d_Hk),
+                     dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<int>(c->d_zstart), dp<int>(c->d_zg), dp<T>(c->d_zq),
+                     dp<T>(c->d_zw), dp<double>(c->d_esite));
+  return launch_check(c, "k_pme_xyslab");
 }
 
 // Slab shape of the fused PME kernels from the frame's z-sorted site counts:
@@ -591,6 +659,9 @@ template <typename T> int choose_slab(erm_ctx *c) {
   }
   if (c->P.pme_path == 3 && !c->xslab_Q)
     return fail(c, ERM_E_UNSUPPORTED, "register-column PME path does not support this grid");
+  Fft2 f;
+  c->two_step = c->P.pme_path == 0 && !c->xslab_Q && fft2_split<T>(k.K1, f) && fft2_split<T>(k.K2, f) &&
+                fft2_split<T>(K3, f) && z2_lds<T>(K3, k.p) <= c->lds_cap && xy2_shape<T>(c, 1).S > 0;
   return ERM_OK;
 }
 
@@ -640,7 +711,7 @@ template <typename T> int frame_prep(erm_ctx *c) {
   const int K3 = k.K3;
   const bool zsort = (c->P.cltype != ERM_EL_COULOMB);
   const int KB = (K3 * ZCLASS <= ZBUCKET_MAX) ? ZCLASS : 1, nbk = K3 * KB;
-  const int rowp = k.K1 + 2;
+  const int rowp = 2 * k.H;  // values of a real row in LDS
   if (zsort) TRY(ensure(c, c->d_zcount, sizeof(int) * (nbk + 1)));
   const int nclr = std::max(ncell + 1, zsort ? nbk + 1 : 0);
   hipLaunchKernelGGL(k_frame_clear, dim3((nclr + 255) / 256), dim3(256), 0, c->st, dp<int>(c->d_count), ncell + 1,
@@ -941,6 +1012,16 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
     ERM_KSWITCH(K1, (rc = launch_xslab<T, KK>(c, k, n, lx)));
     TRY(rc);
     TRY(launch_check(c, "k_pme_xslab"));
+    TRY(mark(c, 4));
+    Params kg = k;
+    if (!(flags & DO_RESIDUAL)) kg.solute_charge = 0.0;
+    TRY(launch_mol_sum(c, kg, n, dp<double>(c->d_esite), dp<int>(c->d_sltj), dp<double>(c->d_uv)));
+  } else if ((flags & DO_RECIP) && c->two_step) {
+    TRY(launch_zcol2<T>(c, k, n, nzg));
+    TRY(mark(c, 2));
+    TRY(mark(c, 3));
+    TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
+    TRY(launch_xyslab<T>(c, k, n));
     TRY(mark(c, 4));
     Params kg = k;
     if (!(flags & DO_RESIDUAL)) kg.solute_charge = 0.0;
@@ -2995,6 +3076,7 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
   const bool had_usreal = c->have_usreal;
   const int flags = DO_RECIP | DO_REAL | DO_RESIDUAL | DO_SELF;  // accumulators untouched
   std::vector<int> paths;
+  if (c->two_step) paths.push_back(0);
   if (c->xslab_Q) paths.push_back(3);
   if (c->slab_S) paths.push_back(1);
   paths.push_back(2);
@@ -3028,7 +3110,7 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
         for (int Qc : {16, 9, 8, 5, 4, 3}) {
           for (int Tc : {256, 512}) {
             if (pp != 3 && (Qc != 8 || Tc != 256)) continue;
-            if (pp == 2 && Sc != 16) continue;
+            if ((pp == 2 || pp == 0) && Sc != 16) continue;
             if (apply(B, pp, Sc, Qc, Tc) != ERM_OK) {
               c->err.clear();
               continue;

@@ -99,6 +99,7 @@ struct erm_ctx {
   uint64_t alloc_gen = 0;          // bumped by every device (re)allocation
   int ggrid_excl = -2;
   int xslab_Q = 0;            // planes per x-c2r group of the register path
+  bool two_step = false;      // the frame's grid goes through the two-step kernels (ermgpu_fft2.h)
   int tune_S = 16, tune_Q = 8;  // caps on slab depth and planes per group (autotuned)
   int xslab_T = erm::NTHR;           // threads per x-slab workgroup, 256 or 512 (autotuned)
   int zcol_T = erm::NTHR;            // threads per z-column workgroup, 256 or 512 (autotuned)

@@ -1,0 +1,547 @@
+// ermgpu_fft2.h -- PME kernels for grid lengths K = A B transformed in two
+// steps: an A-point DFT of x[n1 + B n2] over n2, the twiddle w_K^(n1 k2), a
+// B-point DFT over n1.  Both steps run in registers (A, B <= 16 values) with
+// one exchange through LDS between them, so a length needs no kernel of its
+// own: the radices are launch arguments.  fft2_split() lists the lengths.
+#pragma once
+
+#include "ermgpu_kern.h"
+
+namespace erm {
+
+struct Fft2 {
+  int A, B;
+};
+
+// K = A B with A <= B, both with a case in ERM_RADIX_A / _B below (T in
+// scope): in FP64 B stops at 12, where a step's values still fit 128
+// registers beside their addresses
+template <typename T> inline bool fft2_split(int K, Fft2 &f) {
+  static const int tab[][3] = {{16, 4, 4},  {18, 3, 6},  {20, 4, 5},   {24, 4, 6},   {25, 5, 5},   {27, 3, 9},
+                               {30, 5, 6},  {32, 4, 8},  {36, 6, 6},   {40, 5, 8},   {45, 5, 9},   {48, 6, 8},
+                               {50, 5, 10}, {54, 6, 9},  {60, 6, 10},  {64, 8, 8},   {72, 8, 9},   {75, 5, 15},
+                               {80, 8, 10}, {81, 9, 9},  {90, 9, 10},  {96, 8, 12},  {100, 10, 10}, {108, 9, 12},
+                               {120, 10, 12}, {128, 8, 16}};
+  for (const auto &t : tab)
+    if (t[0] == K && (sizeof(T) == 4 || t[2] <= 12)) {
+      f.A = t[1];
+      f.B = t[2];
+      return true;
+    }
+  return false;
+}
+
+#define ERM_RADIX_A(A, CALL)                          \
+  switch (A) {                                        \
+    case 3: { constexpr int RR = 3; CALL; } break;    \
+    case 4: { constexpr int RR = 4; CALL; } break;    \
+    case 5: { constexpr int RR = 5; CALL; } break;    \
+    case 6: { constexpr int RR = 6; CALL; } break;    \
+    case 8: { constexpr int RR = 8; CALL; } break;    \
+    case 9: { constexpr int RR = 9; CALL; } break;    \
+    case 10: { constexpr int RR = 10; CALL; } break;  \
+    default: break;                                   \
+  }
+#define ERM_RADIX_B(B, CALL)                          \
+  switch (B) {                                        \
+    case 4: { constexpr int RR = 4; CALL; } break;    \
+    case 5: { constexpr int RR = 5; CALL; } break;    \
+    case 6: { constexpr int RR = 6; CALL; } break;    \
+    case 8: { constexpr int RR = 8; CALL; } break;    \
+    case 9: { constexpr int RR = 9; CALL; } break;    \
+    case 10: { constexpr int RR = 10; CALL; } break;  \
+    case 12: { constexpr int RR = 12; CALL; } break;  \
+    case 15: if constexpr (sizeof(T) == 4) { constexpr int RR = 15; CALL; } break; \
+    case 16: if constexpr (sizeof(T) == 4) { constexpr int RR = 16; CALL; } break; \
+    default: break;                                   \
+  }
+
+// a times the conjugate of w (the twiddle tables hold e^{-2 pi i j / K})
+template <typename V> __device__ __forceinline__ V cmulc(V a, V w) {
+  V r;
+  r.x = a.x * w.x + a.y * w.y;
+  r.y = a.y * w.x - a.x * w.y;
+  return r;
+}
+
+// --------------------------------------------------------------------------
+// z columns.  A workgroup takes C consecutive columns (m1, m2) of one
+// configuration: the solute's sites, in chunks of Z2_SCH sorted by plane, are
+// added to the columns in LDS (buf[z][column], each plane over the sites
+// whose p planes hold it), transformed forward, multiplied by the Green's
+// function (self energy on the way, recpcal.F90:385-394), transformed back
+// and written to Hk.  The Green's function meets the second forward step's
+// registers, and the first inverse step runs on the same registers, so the
+// column makes six trips through LDS and none through memory but its write.
+// Bound by those trips and the spread.  500 FP64 columns sets of 40 x 40 x 80
+// with 20 solute sites: 0.38 ms, where the stages of 2 to 5 points through LDS
+// (k_pme_zcol) took 2.38 ms; 701 FP32 sets of 45 x 60 x 75 with 33 sites
+// 0.85 against 6.14 ms.
+// --------------------------------------------------------------------------
+constexpr int Z2_SCH = 32;   // solute sites per chunk
+constexpr int Z2_THR = 256;
+template <typename T> constexpr int z2_cols = sizeof(T) == 8 ? 32 : 64;  // columns per workgroup
+
+template <typename T> __host__ __device__ inline size_t z2_lds(int K3, int p) {
+  constexpr int C = z2_cols<T>;
+  return sizeof(T) * 2 * ((size_t)K3 * C + (size_t)Z2_SCH * C + K3) + sizeof(T) * (size_t)Z2_SCH * p +
+         sizeof(int) * (Z2_SCH * 2 + (size_t)K3 + 1) + sizeof(double) * Z2_THR + 32;
+}
+
+// first forward step of (n1, column): in place
+template <typename T, int A>
+__device__ __forceinline__ void z2_first(typename C2<T>::type *col, int B, int n1,
+                                         const typename C2<T>::type *__restrict__ tw) {
+  using V = typename C2<T>::type;
+  constexpr int C = z2_cols<T>;
+  V x[A];
+#pragma unroll
+  for (int i = 0; i < A; ++i) x[i] = col[(n1 + B * i) * C];
+  reg_fft<A, -1>(x);
+  col[n1 * C] = x[0];
+#pragma unroll
+  for (int k = 1; k < A; ++k) col[(n1 + B * k) * C] = cmul(x[k], tw[n1 * k]);
+}
+
+// second forward step of (k2, column), Green's function, first inverse step:
+// in place; returns the column's share of the self energy (weight 1)
+template <typename T, int B>
+__device__ __forceinline__ double z2_mid(typename C2<T>::type *col, int A, int k2, const T *__restrict__ g,
+                                         size_t gstr, const typename C2<T>::type *__restrict__ tw) {
+  using V = typename C2<T>::type;
+  constexpr int C = z2_cols<T>;
+  T gv[B];
+#pragma unroll
+  for (int k = 0; k < B; ++k) gv[k] = g[(size_t)(k2 + A * k) * gstr];
+  V x[B];
+#pragma unroll
+  for (int n = 0; n < B; ++n) x[n] = col[(B * k2 + n) * C];
+  reg_fft<B, -1>(x);
+  double self = 0.0;
+#pragma unroll
+  for (int k = 0; k < B; ++k) {
+    self += (double)gv[k] * ((double)x[k].x * (double)x[k].x + (double)x[k].y * (double)x[k].y);
+    x[k].x *= gv[k];
+    x[k].y *= gv[k];
+  }
+  reg_fft<B, +1>(x);
+  col[(B * k2) * C] = x[0];
+#pragma unroll
+  for (int n = 1; n < B; ++n) col[(B * k2 + n) * C] = cmulc(x[n], tw[k2 * n]);
+  return self;
+}
+
+// last inverse step of (n1, column), into Hk
+template <typename T, int A>
+__device__ __forceinline__ void z2_last(const typename C2<T>::type *col, int B, int n1, typename C2<T>::type *out,
+                                        size_t ostr) {
+  using V = typename C2<T>::type;
+  constexpr int C = z2_cols<T>;
+  V x[A];
+#pragma unroll
+  for (int k = 0; k < A; ++k) x[k] = col[(n1 + B * k) * C];
+  reg_fft<A, +1>(x);
+#pragma unroll
+  for (int i = 0; i < A; ++i) out[(size_t)(n1 + B * i) * ostr] = x[i];
+}
+
+template <typename T>
+__global__ __launch_bounds__(Z2_THR) void k_pme_zcol2(Params P, int A, int B, const T *__restrict__ engfac,
+                                                      const int *__restrict__ sg3, const T *__restrict__ sw3,
+                                                      const T *__restrict__ sqv,
+                                                      const typename C2<T>::type *__restrict__ w1h,
+                                                      const typename C2<T>::type *__restrict__ w2h,
+                                                      const typename C2<T>::type *__restrict__ tw3,
+                                                      typename C2<T>::type *Hk, double *selfp) {
+  using V = typename C2<T>::type;
+  constexpr int C = z2_cols<T>;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int b = blockIdx.y, ns = P.ns, p = P.p, K2 = P.K2, K3 = P.K3, H = P.H;
+  V *buf = reinterpret_cast<V *>(lds_raw);       // [K3][C]
+  V *amp = buf + (size_t)K3 * C;                 // [Z2_SCH][C] q what1 what2 of the chunk's sites
+  V *tw = amp + (size_t)Z2_SCH * C;              // [K3]
+  double *red = reinterpret_cast<double *>(tw + K3);  // [Z2_THR]
+  T *wz = reinterpret_cast<T *>(red + Z2_THR);   // [Z2_SCH][p] z weights in plane order
+  int *gz = reinterpret_cast<int *>(wz + (size_t)Z2_SCH * p);  // [Z2_SCH] planes g3, sorted
+  int *ord = gz + Z2_SCH;                        // [Z2_SCH] site of each sorted place
+  int *first = ord + Z2_SCH;                     // [K3 + 1] first sorted place with g3 >= z
+  const int cl = threadIdx.x % C, sub = threadIdx.x / C;
+  constexpr int NSUB = Z2_THR / C;
+  const int ncol = H * K2, c = blockIdx.x * C + cl;
+  const bool on = c < ncol;
+  const int m2 = on ? c / H : 0, m1 = on ? c - m2 * H : 0;
+  for (int t = threadIdx.x; t < K3; t += Z2_THR) tw[t] = tw3[t];
+  for (int s0 = 0; s0 < ns; s0 += Z2_SCH) {
+    const int nc = min(Z2_SCH, ns - s0);
+    const size_t bs = (size_t)b * ns + s0;
+    __syncthreads();  // the previous chunk's sites are used up
+    if (threadIdx.x < (unsigned)nc) {
+      const int g = sg3[bs + threadIdx.x];
+      int rank = 0;
+      for (int j = 0; j < nc; ++j) {
+        const int gj = sg3[bs + j];
+        rank += (gj < g || (gj == g && j < (int)threadIdx.x)) ? 1 : 0;
+      }
+      gz[rank] = g;
+      ord[rank] = threadIdx.x;
+    }
+    __syncthreads();
+    for (int z = threadIdx.x; z <= K3; z += Z2_THR) {
+      int n = 0;
+      for (int j = 0; j < nc; ++j) n += (gz[j] < z) ? 1 : 0;
+      first[z] = n;
+    }
+    for (int t = threadIdx.x; t < nc * p; t += Z2_THR) {
+      const int j = t / p;
+      wz[t] = sw3[(bs + ord[j]) * p + (t - j * p)];
+    }
+    for (int j = sub; j < nc; j += NSUB) {
+      const size_t s = bs + ord[j];
+      V a;
+      a.x = 0;
+      a.y = 0;
+      if (on) {
+        a = cmul(w1h[s * H + m1], w2h[s * K2 + m2]);
+        const T q = sqv[s];
+        a.x *= q;
+        a.y *= q;
+      }
+      amp[j * C + cl] = a;
+    }
+    __syncthreads();
+    // plane z holds the sites with g3 - z in [0, p) (mod K3)
+    for (int z = sub; z < K3; z += NSUB) {
+      V acc;
+      acc.x = 0;
+      acc.y = 0;
+      if (s0) acc = buf[z * C + cl];
+      for (int j = first[z]; j < first[min(z + p, K3)]; ++j) {
+        const V a = amp[j * C + cl];
+        const T w = wz[j * p + gz[j] - z];
+        acc.x += a.x * w;
+        acc.y += a.y * w;
+      }
+      if (z + p > K3)  // planes wrapped past the top
+        for (int j = 0; j < first[z + p - K3]; ++j) {
+          const V a = amp[j * C + cl];
+          const T w = wz[j * p + gz[j] + K3 - z];
+          acc.x += a.x * w;
+          acc.y += a.y * w;
+        }
+      buf[z * C + cl] = acc;
+    }
+  }
+  __syncthreads();
+  for (int n1 = sub; n1 < B; n1 += NSUB) {
+    asm volatile("" : "+v"(n1));  // no radix's addresses are hoisted out of the loop
+    ERM_RADIX_A(A, (z2_first<T, RR>(buf + cl, B, n1, tw)))
+  }
+  __syncthreads();
+  double self = 0.0;
+  const T *g = engfac + (size_t)m2 * H + m1;
+  for (int k2 = sub; k2 < A; k2 += NSUB) {
+    asm volatile("" : "+v"(k2));  // no radix's addresses are hoisted out of the loop
+    ERM_RADIX_B(B, (self += z2_mid<T, RR>(buf + cl, A, k2, g, (size_t)ncol, tw)))
+  }
+  red[threadIdx.x] = on ? ((m1 == 0 || 2 * m1 == P.K1) ? 0.5 : 1.0) * self : 0.0;
+  __syncthreads();
+  if (on) {
+    V *out = Hk + (size_t)b * K3 * ncol + c;
+    for (int n1 = sub; n1 < B; n1 += NSUB) {
+    asm volatile("" : "+v"(n1));  // no radix's addresses are hoisted out of the loop
+      ERM_RADIX_A(A, (z2_last<T, RR>(buf + cl, B, n1, out, (size_t)ncol)))
+    }
+  }
+  for (int s = Z2_THR / 2; s > 0; s >>= 1) {
+    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) selfp[(size_t)b * gridDim.x + blockIdx.x] = red[0];
+}
+
+// --------------------------------------------------------------------------
+// y and x transforms of a slab of z planes, and the gather (the owned planes
+// [zb, zb + S) and their p - 1 halo planes, Q planes in LDS at a time; the
+// sites of the slab are summed as in k_pme_xslab).  A wave owns whole
+// columns (y) and whole row pairs (x), several at once over its lanes: both
+// steps of a transform and their exchange stay within the wave (LDS
+// operations of a wave complete in order), so a group of planes passes
+// three barriers.  The y transform's first step reads Hk straight into
+// registers; the x transform takes two Hermitian rows as one complex row of
+// length K1 (even or odd), and its real rows end in natural order with x[0]
+// repeated at K1 for the gather.  Bound by LDS: the transforms pass each
+// value through it nine times, the gather reads p^3 values per site.  The
+// configurations above: 0.42 ms against 2.71 ms (k_pme_slab), FP32 0.54
+// against 3.62 ms.
+// --------------------------------------------------------------------------
+template <typename T, int A>
+__device__ __forceinline__ void xy2_yfirst(bool on, const typename C2<T>::type *__restrict__ src, size_t sstr,
+                                           typename C2<T>::type *dst, int dstr, int n1,
+                                           const typename C2<T>::type *tw) {
+  using V = typename C2<T>::type;
+  if (!on) return;
+  V x[A];
+#pragma unroll
+  for (int i = 0; i < A; ++i) x[i] = src[(size_t)i * sstr];
+  reg_fft<A, +1>(x);
+  dst[0] = x[0];
+#pragma unroll
+  for (int k = 1; k < A; ++k) dst[k * dstr] = cmulc(x[k], tw[n1 * k]);
+}
+template <typename T, int B>
+__device__ __forceinline__ void xy2_ysecond(bool on, typename C2<T>::type *col, int H, int A, int k2) {
+  using V = typename C2<T>::type;
+  V x[B];
+#pragma unroll
+  for (int n = 0; n < B; ++n) x[n] = on ? col[(k2 * B + n) * H] : V{0, 0};
+  wave_lds_sync();
+  reg_fft<B, +1>(x);
+  if (!on) return;
+#pragma unroll
+  for (int k = 0; k < B; ++k) col[(k2 + A * k) * H] = x[k];
+}
+template <typename T, int A>
+__device__ __forceinline__ void xy2_xfirst(bool on, bool two, typename C2<T>::type *pr, int H, int K1, int B, int n1,
+                                           const typename C2<T>::type *tw) {
+  using V = typename C2<T>::type;
+  V x[A];
+#pragma unroll
+  for (int i = 0; i < A; ++i) {
+    const int n = n1 + B * i;
+    const bool up = n >= H;
+    const int k = up ? K1 - n : n;
+    V a{0, 0}, c{0, 0};
+    if (on) a = pr[k];
+    if (on && two) c = pr[H + k];
+    const bool re = n == 0 || 2 * n == K1;  // real by symmetry: the imaginary part is not read
+    a.y = re ? (T)0 : up ? -a.y : a.y;
+    c.y = re ? (T)0 : up ? -c.y : c.y;
+    x[i].x = a.x - c.y;
+    x[i].y = a.y + c.x;
+  }
+  wave_lds_sync();
+  reg_fft<A, +1>(x);
+  if (!on) return;
+  pr[n1] = x[0];
+#pragma unroll
+  for (int k = 1; k < A; ++k) pr[B * k + n1] = cmulc(x[k], tw[n1 * k]);
+}
+template <typename T, int B>
+__device__ __forceinline__ void xy2_xsecond(bool on, bool two, typename C2<T>::type *pr, int H, int K1, int A,
+                                            int k2) {
+  using V = typename C2<T>::type;
+  V x[B];
+#pragma unroll
+  for (int n = 0; n < B; ++n) x[n] = on ? pr[k2 * B + n] : V{0, 0};
+  wave_lds_sync();
+  reg_fft<B, +1>(x);
+  if (!on) return;
+  T *r0 = reinterpret_cast<T *>(pr), *r1 = r0 + 2 * H;
+#pragma unroll
+  for (int k = 0; k < B; ++k) {
+    r0[k2 + A * k] = x[k].x;
+    if (two) r1[k2 + A * k] = x[k].y;
+  }
+  if (k2 == 0) {
+    r0[K1] = x[0].x;
+    if (two) r1[K1] = x[0].y;
+  }
+}
+
+
+// complex values of a plane in LDS: its rows, an even number of them, padded
+// to whole turns of the 32 LDS banks (the site sort's bank classes then hold
+// for every plane)
+__host__ __device__ inline int xy2_plane(int K2, int H) { return ((K2 + (K2 & 1)) * H + 15) & ~15; }
+template <typename T> __host__ __device__ inline size_t xy2_lds(int Q, int K1, int K2, int H) {
+  return 2 * sizeof(T) * ((size_t)Q * xy2_plane(K2, H) + K1 + K2);
+}
+
+constexpr int XY2_THR = 512;
+// Gather of a group of nq real planes in LDS (first plane zz0) into the
+// per-site sums: the sites whose p planes meet the group are one run
+// [lo, hi) of the z order, dealt over the threads.  A site's first group
+// (first: g3 - p + 1 >= zz0 or the slab's first group) stores its sum, a later
+// one adds to it; the barrier between groups orders the two.
+template <typename T, int PP>
+__device__ __forceinline__ void xy2_gather(const Params &P, const T *real, const int rstr, const int pstr, int zz0,
+                                           int nq, int lo, int hi, const int *__restrict__ zg,
+                                           const T *__restrict__ zq, const T *__restrict__ zw, double *es) {
+  const int K1 = P.K1, K2 = P.K2, p = PP ? PP : P.p;
+  for (int idx = lo + (int)threadIdx.x; idx < hi; idx += XY2_THR) {
+    const int gp = zg[idx];
+    const T qv = zq[idx];
+    const int g1 = gp & 1023, g2 = (gp >> 10) & 1023, g3 = (gp >> 20) & 1023;
+    const int clo = max(0, g3 - (zz0 + nq - 1)), chi = min(p - 1, g3 - zz0);
+    const bool add = g3 - p + 1 < zz0;
+    double acc = add ? es[idx] : 0.0;
+    if constexpr (PP == 4) {
+      // four sites' worth of latency is covered by the other waves; the pairs
+      // of adjacent x values as in xslab_gather4
+      const T *wz = static_cast<const T *>(__builtin_assume_aligned(zw + (size_t)idx * 12, 16));
+      T w[12];
+#pragma unroll
+      for (int k = 0; k < 12; ++k) w[k] = wz[k];
+      const int xa = g1 - 3 + ((g1 < 3) ? K1 : 0);
+      const int xb = g1 - 1 + ((g1 < 1) ? K1 : 0);
+      int ro[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int y = g2 - k;
+        ro[k] = (y + ((y < 0) ? K2 : 0)) * rstr;
+      }
+      const T *ph0 = real + (g3 - zz0) * pstr;
+#pragma unroll
+      for (int c3 = 0; c3 < 4; ++c3) {
+        if (c3 < clo || c3 > chi) continue;
+        const T *ph = ph0 - c3 * pstr;
+        T sum = 0;
+#pragma unroll
+        for (int c2 = 0; c2 < 4; ++c2) {
+          const T *a = ph + ro[c2] + xa, *bb = ph + ro[c2] + xb;
+          const T a0 = a[0], a1 = a[1], b0 = bb[0], b1 = bb[1];
+          T rs = 0;
+          rs += w[0] * b1;
+          rs += w[1] * b0;
+          rs += w[2] * a1;
+          rs += w[3] * a0;
+          sum += w[4 + c2] * rs;
+        }
+        acc += (double)(qv * w[8 + c3] * sum);
+      }
+    } else {
+      const T *wz = zw + (size_t)idx * 3 * p;  // [3][p]
+      if constexpr (PP > 0) {
+        T w1[PP], w2[PP];
+        int xo[PP], yo[PP];
+#pragma unroll
+        for (int k = 0; k < PP; ++k) {
+          w1[k] = wz[k];
+          w2[k] = wz[PP + k];
+          const int x = g1 - k, y = g2 - k;
+          xo[k] = x + ((x < 0) ? K1 : 0);
+          yo[k] = (y + ((y < 0) ? K2 : 0)) * rstr;
+        }
+        for (int c3 = clo; c3 <= chi; ++c3) {
+          const T *ph = real + (g3 - c3 - zz0) * pstr;
+          T sum = 0;
+#pragma unroll
+          for (int c2 = 0; c2 < PP; ++c2) {
+            const T *row = ph + yo[c2];
+            T rs = 0;
+#pragma unroll
+            for (int c1 = 0; c1 < PP; ++c1) rs += w1[c1] * row[xo[c1]];
+            sum += w2[c2] * rs;
+          }
+          acc += (double)(qv * wz[2 * PP + c3] * sum);
+        }
+      } else {
+        for (int c3 = clo; c3 <= chi; ++c3) {
+          const T *ph = real + (g3 - c3 - zz0) * pstr;
+          T sum = 0;
+          for (int c2 = 0; c2 < p; ++c2) {
+            int y = g2 - c2;
+            y += (y < 0) ? K2 : 0;
+            const T *row = ph + y * rstr;
+            T rs = 0;
+            for (int c1 = 0; c1 < p; ++c1) {
+              int x = g1 - c1;
+              x += (x < 0) ? K1 : 0;
+              rs += wz[c1] * row[x];
+            }
+            sum += wz[p + c2] * rs;
+          }
+          acc += (double)(qv * wz[2 * p + c3] * sum);
+        }
+      }
+    }
+    es[idx] = acc;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) void k_pme_xyslab(Params P, int S, int Q, Fft2 fy, Fft2 fx, int nsites,
+                                                        const typename C2<T>::type *__restrict__ Hk,
+                                                        const typename C2<T>::type *__restrict__ tw1,
+                                                        const typename C2<T>::type *__restrict__ tw2,
+                                                        const int *__restrict__ z_start, const int *__restrict__ zg,
+                                                        const T *__restrict__ zq, const T *__restrict__ zw,
+                                                        double *e_site) {
+  using V = typename C2<T>::type;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int K1 = P.K1, K2 = P.K2, K3 = P.K3, H = P.H, p = P.p;
+  const int plane = xy2_plane(K2, H);
+  V *stage = reinterpret_cast<V *>(lds_raw);   // [Q][plane]
+  V *twy = stage + (size_t)Q * plane;          // [K2]
+  V *twx = twy + K2;                           // [K1]
+  for (int t = threadIdx.x; t < K2; t += XY2_THR) twy[t] = tw2[t];
+  for (int t = threadIdx.x; t < K1; t += XY2_THR) twx[t] = tw1[t];
+  // XCD-aware order, as in k_pme_xslab
+  const int nwg = gridDim.x * gridDim.y;
+  int L = blockIdx.y * gridDim.x + blockIdx.x;
+  if (nwg % 8 == 0) L = (L % 8) * (nwg / 8) + L / 8;
+  const int b = L / gridDim.x;
+  const int zb = (L - b * gridDim.x) * S, ze = min(zb + S, K3);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  constexpr int NW = XY2_THR / 64;
+  // columns of a wave's round: lane = n1 Gy + column in the first step,
+  // k2 Gy + column in the second
+  const int Gy = 64 / fy.B;
+  // row pairs of a round: lane = pair B + n1, then pair A + k2
+  const int Gx = 64 / fx.B;
+  const int npair = (K2 + 1) / 2;
+  double *es = e_site + (size_t)b * nsites;
+  __syncthreads();
+  for (int zz0 = zb - p + 1; zz0 < ze; zz0 += Q) {
+    const int nq = min(Q, ze - zz0), ncol = nq * H;
+    for (int c0 = wv * Gy; c0 < ncol; c0 += NW * Gy) {
+      int ly = lane / Gy;
+      asm volatile("" : "+v"(ly));  // no radix's addresses are hoisted out of the loop
+      const int lg = lane - ly * Gy, cid = c0 + lg;
+      const bool in = lg < Gy && cid < ncol;  // lanes past B Gy have ly = B
+      const int q = in ? cid / H : 0, m1 = in ? cid - q * H : 0;
+      const int z = (((zz0 + q) % K3) + K3) % K3;
+      V *col = stage + (size_t)q * plane + m1;
+      const V *src = Hk + (((size_t)b * K3 + z) * K2 + ly) * H + m1;
+      ERM_RADIX_A(fy.A, (xy2_yfirst<T, RR>(in && ly < fy.B, src, (size_t)fy.B * H, col + ly * H, fy.B * H, ly, twy)))
+      wave_lds_sync();
+      ERM_RADIX_B(fy.B, (xy2_ysecond<T, RR>(in && ly < fy.A, col, H, fy.A, ly)))
+    }
+    __syncthreads();
+    const int nrow = nq * npair;
+    for (int p0 = wv * Gx; p0 < nrow; p0 += NW * Gx) {
+      {
+        int xg1 = lane / fx.B;
+        asm volatile("" : "+v"(xg1));
+        const int xn1 = lane - xg1 * fx.B, pid = p0 + xg1;
+        const bool in = xg1 < Gx && pid < nrow;
+        const int q = in ? pid / npair : 0, pr = in ? pid - q * npair : 0;
+        V *row = stage + (size_t)q * plane + (size_t)2 * pr * H;
+        ERM_RADIX_A(fx.A, (xy2_xfirst<T, RR>(in, 2 * pr + 1 < K2, row, H, K1, fx.B, xn1, twx)))
+      }
+      wave_lds_sync();
+      {
+        int xg2 = lane / fx.A;
+        asm volatile("" : "+v"(xg2));
+        const int xk2 = lane - xg2 * fx.A, pid = p0 + xg2;
+        const bool in = xg2 < Gx && pid < nrow;
+        const int q = in ? pid / npair : 0, pr = in ? pid - q * npair : 0;
+        V *row = stage + (size_t)q * plane + (size_t)2 * pr * H;
+        ERM_RADIX_B(fx.B, (xy2_xsecond<T, RR>(in, 2 * pr + 1 < K2, row, H, K1, fx.A, xk2)))
+      }
+      wave_lds_sync();
+    }
+    __syncthreads();
+    const T *real = reinterpret_cast<const T *>(stage);
+    const int lo = z_start[max(zb, zz0)], hi = z_start[min(ze, zz0 + nq + p - 1)];
+    if (p == 4)
+      xy2_gather<T, 4>(P, real, 2 * H, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
+    else if (p == 6)
+      xy2_gather<T, 6>(P, real, 2 * H, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
+    else
+      xy2_gather<T, 0>(P, real, 2 * H, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
+    __syncthreads();
+  }
+}
+
+}  // namespace erm

@@ -1388,17 +1388,16 @@ __global__ __launch_bounds__(NTHR) void k_pme_ycol_reg(Params P, const typename 
 // complex row's bytes), and repeats x[0], x[1] in the row's two spare values
 // K1, K1 + 1.  Each thread then adds the planes' contributions to its MAXR
 // owned sites (FP64 sums).
-// gather of one group of nq real planes (first plane zz0, rows of K1 + 2)
-// into the per-site sums acc[] of the sites a thread owns.  PP: the spline
-// order at compile time (weights, row offsets and the p^3 products in
-// registers, loads independent); PP = 0 takes it from P.p.
-template <typename T, int K1, int MAXR, int PP, int XT>
-__device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int zz0, int nq, int s_beg,
+// gather of one group of nq real planes (first plane zz0, `plane` reals
+// each, rows of K1P reals) into the per-site sums acc[] of the sites a thread
+// owns.  PP: the spline order at compile time (weights, row offsets and the
+// p^3 products in registers, loads independent); PP = 0 takes it from P.p.
+template <typename T, int MAXR, int PP, int XT>
+__device__ __forceinline__ void xslab_gather(const Params &P, const T *real, const int K1, const int K1P,
+                                             const int plane, int zz0, int nq, int s_beg,
                                              const int *gz, const int *__restrict__ zg, const T *__restrict__ zq,
                                              const T *__restrict__ zw, double *acc) {
-  constexpr int K1P = K1 + 2;
   const int K2 = P.K2, p = PP ? PP : P.p;
-  const size_t plane = (size_t)K2 * (K1 / 2 + 1) * 2;  // reals per plane
 #pragma unroll
   for (int r = 0; r < MAXR; ++r) {
     const int g3 = gz[r];
@@ -1425,7 +1424,7 @@ __device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int
         yo[k] = (y + ((y < 0) ? K2 : 0)) * K1P;
       }
       for (int c3 = clo; c3 <= chi; ++c3) {
-        const T *ph = real + (size_t)(g3 - c3 - zz0) * plane;
+        const T *ph = real + (ptrdiff_t)(g3 - c3 - zz0) * plane;
         T sum = 0;
 #pragma unroll
         for (int c2 = 0; c2 < PP; ++c2) {
@@ -1444,7 +1443,7 @@ __device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int
         w2[k] = wz[p + k];
       }
       for (int c3 = clo; c3 <= chi; ++c3) {
-        const T *ph = real + (size_t)(g3 - c3 - zz0) * plane;
+        const T *ph = real + (ptrdiff_t)(g3 - c3 - zz0) * plane;
         T sum = 0;
         for (int c2 = 0; c2 < p; ++c2) {
           int y = g2 - c2;
@@ -1474,13 +1473,12 @@ __device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int
 // end is such a pair (g1 = 0: (K1-3, K1-2), (K1-1, K1); g1 = 1: (K1-2, K1-1),
 // (0, 1); g1 = 2: (K1-1, K1), (1, 2)).  Products and sums are formed in the
 // order of xslab_gather, so both give the same values.
-template <typename T, int K1, int MAXR, int XT>
-__device__ __forceinline__ void xslab_gather4(const Params &P, const T *real, int zz0, int nq, int s_beg,
+template <typename T, int MAXR, int XT>
+__device__ __forceinline__ void xslab_gather4(const Params &P, const T *real, const int K1, const int K1P,
+                                              const int plane, int zz0, int nq, int s_beg,
                                               size_t np, const int *gz, const int *__restrict__ zg,
                                               const T *__restrict__ zq, const T *__restrict__ zw, double *acc) {
-  constexpr int K1P = K1 + 2;
   const int K2 = P.K2;
-  const ptrdiff_t plane = (ptrdiff_t)K2 * (K1 / 2 + 1) * 2;  // reals per plane
   constexpr int RB = MAXR < 4 ? MAXR : 4;  // sites whose loads fly together
 #pragma unroll
   for (int r0 = 0; r0 < MAXR; r0 += RB) {
@@ -1645,12 +1643,13 @@ __global__ __launch_bounds__(XT) void k_pme_xslab(Params P, int S, int Q, int ns
     T *real = xslab_stage<T, K1, YF>(Hk, stage, b, zz0, nq, K2, K3);
     // gather: owned sites whose support g3 - c3 meets planes [zz0, zz0 + nq);
     // the common spline orders get fully unrolled register code
+    const int plane = K2 * (K1 + 2);  // reals
     if (p == 4)
-      xslab_gather4<T, K1, MAXR, XT>(P, real, zz0, nq, s_beg, np, gz, zg, zq, zw, acc);
+      xslab_gather4<T, MAXR, XT>(P, real, K1, K1 + 2, plane, zz0, nq, s_beg, np, gz, zg, zq, zw, acc);
     else if (p == 6)
-      xslab_gather<T, K1, MAXR, 6, XT>(P, real, zz0, nq, s_beg, gz, zg, zq, zw, acc);
+      xslab_gather<T, MAXR, 6, XT>(P, real, K1, K1 + 2, plane, zz0, nq, s_beg, gz, zg, zq, zw, acc);
     else
-      xslab_gather<T, K1, MAXR, 0, XT>(P, real, zz0, nq, s_beg, gz, zg, zq, zw, acc);
+      xslab_gather<T, MAXR, 0, XT>(P, real, K1, K1 + 2, plane, zz0, nq, s_beg, gz, zg, zq, zw, acc);
     __syncthreads();
   }
 #pragma unroll

@@ -576,10 +576,10 @@ template <typename T> Xy2Shape xy2_shape(const erm_ctx *c, int n) {
   for (int per : {2, 1}) {
     const size_t cap = std::min(cu / per, c->lds_cap);
     int Q = 0;
-    while (xy2_lds<T>(Q + 1, k.K1, k.K2, k.H) <= cap) ++Q;
+    while (xy2_lds<T>(Q + 1, k.K1, k.K2, k.p) <= cap) ++Q;
     if (!Q) continue;
     double cost = 0.0;
-    for (int S = 1; S <= std::min(k.K3, 32); ++S) {
+    for (int S = 1; S <= k.K3; ++S) {
       const int nslab = (k.K3 + S - 1) / S;
       const int planes = S + k.p - 1, ngrp = (planes + Q - 1) / Q;
       const double t = std::max(1.0, (double)n * nslab / (per * c->ncu)) * (planes + 0.5 * ngrp);
@@ -591,7 +591,7 @@ template <typename T> Xy2Shape xy2_shape(const erm_ctx *c, int n) {
     }
     if (best.S) break;
   }
-  if (best.S) best.lds = xy2_lds<T>(best.Q, k.K1, k.K2, k.H);
+  if (best.S) best.lds = xy2_lds<T>(best.Q, k.K1, k.K2, k.p);
   return best;
 }
 
@@ -711,7 +711,10 @@ template <typename T> int frame_prep(erm_ctx *c) {
   const int K3 = k.K3;
   const bool zsort = (c->P.cltype != ERM_EL_COULOMB);
   const int KB = (K3 * ZCLASS <= ZBUCKET_MAX) ? ZCLASS : 1, nbk = K3 * KB;
-  const int rowp = 2 * k.H;  // values of a real row in LDS
+  // values of a real row in LDS, in the kernel the grid will take
+  Fft2 f2;
+  const bool xy = (c->P.pme_path == 0 || c->P.pme_path == 3) && fft2_split<T>(k.K1, f2) && fft2_split<T>(k.K2, f2);
+  const int rowp = 2 * (xy ? xy2_row(k.K1, k.p) : k.H);
   if (zsort) TRY(ensure(c, c->d_zcount, sizeof(int) * (nbk + 1)));
   const int nclr = std::max(ncell + 1, zsort ? nbk + 1 : 0);
   hipLaunchKernelGGL(k_frame_clear, dim3((nclr + 255) / 256), dim3(256), 0, c->st, dp<int>(c->d_count), ncell + 1,
@@ -1001,17 +1004,9 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
     TRY(rz);
     TRY(launch_check(c, zfft ? "k_pme_zcol_fft" : "k_pme_zcol_reg"));
     TRY(mark(c, 2));
-    if (!xslab_folds_y(c)) {
-      ERM_KSWITCH(K2, (launch_ycol_reg<T, KK>(c, k, n)));
-      TRY(launch_check(c, "y columns"));
-    }
-    TRY(mark(c, 3));
     TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
-    const size_t lx = 2 * sizeof(T) * (size_t)c->xslab_Q * H * K2;
-    int rc = ERM_E_UNSUPPORTED;
-    ERM_KSWITCH(K1, (rc = launch_xslab<T, KK>(c, k, n, lx)));
-    TRY(rc);
-    TRY(launch_check(c, "k_pme_xslab"));
+    TRY(mark(c, 3));
+    TRY(launch_xyslab<T>(c, k, n));
     TRY(mark(c, 4));
     Params kg = k;
     if (!(flags & DO_RESIDUAL)) kg.solute_charge = 0.0;
@@ -1713,18 +1708,8 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
     }
   }
   TRY(mark(c, 2));
-  if (!xslab_folds_y(c)) {
-    ERM_KSWITCH(K2, (launch_ycol_reg<T, KK>(c, k, n)));
-    TRY(launch_check(c, "y columns"));
-  }
   TRY(mark(c, 3));
-  {
-    const size_t lx = 2 * sizeof(T) * (size_t)c->xslab_Q * H * K2;
-    int rc = ERM_E_UNSUPPORTED;
-    ERM_KSWITCH(k.K1, (rc = launch_xslab<T, KK>(c, k, n, lx)));
-    TRY(rc);
-    TRY(launch_check(c, "k_pme_xslab"));
-  }
+  TRY(launch_xyslab<T>(c, k, n));
   TRY(mark(c, 4));
   for (int r = 0; r < nrun; ++r) {
     erm_ctx *m = g->ctx[R[r].member];
@@ -3081,7 +3066,7 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
   if (c->slab_S) paths.push_back(1);
   paths.push_back(2);
   double best = 1e300;
-  int bestB = c->Bmax, bestP = c->P.pme_path, bestS = c->tune_S, bestQ = c->tune_Q, bestT = c->xslab_T, bestZ = 0;
+  int bestB = c->Bmax, bestP = c->P.pme_path, bestS = c->tune_S, bestZ = 0;
   auto timed = [&](double *ms) -> int {
     Batch bt{n_trial, 0, nullptr, nullptr, nullptr, true, seed, 0};
     TRY(process(c, bt, flags, nullptr));  // warm-up (allocations, first launches)
@@ -3095,42 +3080,35 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
     return ERM_OK;
   };
   c->use_graph = false;
-  auto apply = [&](int B, int pp, int Sc, int Qc, int Tc) -> int {
+  auto apply = [&](int B, int pp, int Sc) -> int {
     c->Bmax = B;
     c->P.pme_path = pp;
     c->tune_S = Sc;
-    c->tune_Q = Qc;
-    c->xslab_T = Tc;
     return c->fp32 ? choose_slab<float>(c) : choose_slab<double>(c);
   };
+  const int S0 = c->tune_S;
   for (int B : {128, 256, 512, 1024}) {
     if (B > 4 * n_trial && B > 128) break;
     for (int pp : paths) {
       for (int Sc : {16, 8, 6, 5, 4, 3}) {
-        for (int Qc : {16, 9, 8, 5, 4, 3}) {
-          for (int Tc : {256, 512}) {
-            if (pp != 3 && (Qc != 8 || Tc != 256)) continue;
-            if ((pp == 2 || pp == 0) && Sc != 16) continue;
-            if (apply(B, pp, Sc, Qc, Tc) != ERM_OK) {
-              c->err.clear();
-              continue;
-            }
-            double ms;
-            TRY(timed(&ms));
-            if (ms < best) {
-              best = ms;
-              bestB = B;
-              bestP = pp;
-              bestS = Sc;
-              bestQ = Qc;
-              bestT = Tc;
-            }
-          }
+        // the slab depth shapes the fused LDS path alone
+        if (pp != 1 && Sc != 16) continue;
+        if (apply(B, pp, pp == 1 ? Sc : S0) != ERM_OK) {
+          c->err.clear();
+          continue;
+        }
+        double ms;
+        TRY(timed(&ms));
+        if (ms < best) {
+          best = ms;
+          bestB = B;
+          bestP = pp;
+          bestS = pp == 1 ? Sc : S0;
         }
       }
     }
   }
-  TRY(apply(bestB, bestP, bestS, bestQ, bestT));
+  TRY(apply(bestB, bestP, bestS));
   c->batch_set = true;
   if (bestP == 3) {  // z-column workgroup size for the chosen shape
     const int z0 = c->zcol_T;
@@ -3144,20 +3122,6 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
       }
     }
     c->zcol_T = bestZ ? bestZ : z0;
-    // inverse y transform inside the x slab, or its own kernel
-    if (c->xslab_T == 512 && c->kp.K2 == c->kp.K1) {
-      const bool y0 = c->xslab_yf;
-      int besty = -1;
-      for (int yf : {0, 1}) {
-        c->xslab_yf = (yf == 1);
-        TRY(timed(&ms));
-        if (ms < best) {
-          best = ms;
-          besty = yf;
-        }
-      }
-      c->xslab_yf = (besty >= 0) ? (besty == 1) : y0;
-    }
   }
   // real-space kernel: compacted tiles or one thread per candidate molecule
   {

@@ -261,8 +261,6 @@ template <typename T, int K>
 int launch_zcol_fft(erm_ctx *c, const Params &k, int n, int nblk, size_t site0 = 0, size_t cfg0 = 0);
 template <typename T, int K>
 int launch_zcol_fft_runs(erm_ctx *c, const Params &k, int nblk, const GRun *runs, int nrun, int nitem, int *counter);
-template <typename T, int K> void launch_ycol_reg(erm_ctx *c, const Params &k, int n);
-template <typename T, int K> int launch_xslab(erm_ctx *c, const Params &k, int n, size_t lds);
 template <typename T, int K> void launch_xr2c(erm_ctx *c, const Params &k);
 template <typename T, int K> void launch_xc2r(erm_ctx *c, const Params &k);
 template <typename T, int K, int SIGN> void launch_ydense(erm_ctx *c, const Params &k);

@@ -292,16 +292,8 @@ template <typename V> __host__ __device__ __forceinline__ V cadd_h(V a, V b) {
   return r;
 }
 
-// output q of an R-point DFT: sum_s v[s] w_R^(s q)
-template <int R, int SIGN, int Q, typename V, int... S>
-__host__ __device__ __forceinline__ V dft_out(const V (&v)[R], std::integer_sequence<int, S...>) {
-  V acc = v[0];
-  ((acc = (S == 0) ? acc : cadd_h(acc, rot<SIGN, (S * Q) % R, R>(v[S]))), ...);
-  return acc;
-}
-
-template <int R, int SIGN, typename V, int... Q>
-__host__ __device__ __forceinline__ void small_dft(const V (&v)[R], V (&o)[R], std::integer_sequence<int, Q...>) {
+// R-point DFT, R = 2, 3, 4, 5
+template <int R, int SIGN, typename V> __host__ __device__ __forceinline__ void small_dft(const V (&v)[R], V (&o)[R]) {
   if constexpr (R == 4) {
     const V s0 = cadd_h(v[0], v[2]), s1 = cadd_h(v[1], v[3]);
     V d0, d1;
@@ -320,8 +312,50 @@ __host__ __device__ __forceinline__ void small_dft(const V (&v)[R], V (&o)[R], s
     o[0] = cadd_h(v[0], v[1]);
     o[1].x = v[0].x - v[1].x;
     o[1].y = v[0].y - v[1].y;
+  } else if constexpr (R == 3) {
+    // v1 w + v2 w^2 = -(v1 + v2) / 2 + SIGN i sin(2 pi / 3) (v1 - v2)
+    using S = decltype(v[0].x);
+    constexpr S s1 = (S)taylor_cos(kTwoPiOver4 / 3.0);
+    const V t = cadd_h(v[1], v[2]);
+    V d, m, a;
+    d.x = v[1].x - v[2].x;
+    d.y = v[1].y - v[2].y;
+    m.x = v[0].x - (S)0.5 * t.x;
+    m.y = v[0].y - (S)0.5 * t.y;
+    a.x = -SIGN * s1 * d.y;
+    a.y = SIGN * s1 * d.x;
+    o[0] = cadd_h(v[0], t);
+    o[1] = cadd_h(m, a);
+    o[2].x = m.x - a.x;
+    o[2].y = m.y - a.y;
   } else {
-    ((o[Q] = dft_out<R, SIGN, Q>(v, std::make_integer_sequence<int, R>{})), ...);
+    // the symmetric and antisymmetric pairs (v1, v4), (v2, v3) of R = 5
+    static_assert(R == 5);
+    using S = decltype(v[0].x);
+    constexpr S c1 = (S)taylor_sin(kTwoPiOver4 / 5.0), c2 = -(S)taylor_cos(kTwoPiOver4 * 2.0 / 5.0);
+    constexpr S s1 = (S)taylor_cos(kTwoPiOver4 / 5.0), s2 = (S)taylor_sin(kTwoPiOver4 * 2.0 / 5.0);
+    const V t1 = cadd_h(v[1], v[4]), t2 = cadd_h(v[2], v[3]);
+    V d1, d2, a1, a2, b1, b2;
+    d1.x = v[1].x - v[4].x;
+    d1.y = v[1].y - v[4].y;
+    d2.x = v[2].x - v[3].x;
+    d2.y = v[2].y - v[3].y;
+    a1.x = v[0].x + c1 * t1.x + c2 * t2.x;
+    a1.y = v[0].y + c1 * t1.y + c2 * t2.y;
+    a2.x = v[0].x + c2 * t1.x + c1 * t2.x;
+    a2.y = v[0].y + c2 * t1.y + c1 * t2.y;
+    b1.x = -SIGN * (s1 * d1.y + s2 * d2.y);
+    b1.y = SIGN * (s1 * d1.x + s2 * d2.x);
+    b2.x = -SIGN * (s2 * d1.y - s1 * d2.y);
+    b2.y = SIGN * (s2 * d1.x - s1 * d2.x);
+    o[0].x = v[0].x + t1.x + t2.x;
+    o[0].y = v[0].y + t1.y + t2.y;
+    o[1] = cadd_h(a1, b1);
+    o[4].x = a1.x - b1.x;
+    o[4].y = a1.y - b1.y;
+    o[2] = cadd_h(a2, b2);
+    o[3].x = a2.x - b2.x;
+    o[3].y = a2.y - b2.y;
   }
 }
 
@@ -334,7 +368,7 @@ __host__ __device__ __forceinline__ void dif_col(V (&x)[TOT], std::integer_seque
   constexpr int R = sizeof...(K), M = N / R;
   const V v[R] = {x[BASE + N1 + M * K]...};
   V o[R];
-  small_dft<R, SIGN>(v, o, std::make_integer_sequence<int, R>{});
+  small_dft<R, SIGN>(v, o);
   ((x[BASE + N1 + M * K] = rot<SIGN, N1 * K, N>(o[K])), ...);
 }
 
@@ -374,38 +408,6 @@ template <int N, int SIGN, typename V> __host__ __device__ __forceinline__ void 
   static_assert(Fact<N>::valid(), "FFT length must factor into 2, 3, 4, 5");
   dif<N, N, 0, SIGN>(x);
   dif_unscramble<N>(x, std::make_integer_sequence<int, N>{});
-}
-
-// Inverse real transform of one Hermitian row through a half-length complex
-// FFT: for k < M = N/2 with X[0] and X[M] taken as real,
-//   E[k] = X[k] + conj X[M-k],  O[k] = (X[k] - conj X[M-k]) e^{+2 pi i k/N},
-//   z = IFFT_M(E + i O)  gives  x[2m] = Re z[m], x[2m+1] = Im z[m]
-// (unnormalised, e^{+i}), i.e. x[n] = sum_{k<N} X[k] e^{2 pi i k n / N}.
-template <typename V> __host__ __device__ __forceinline__ V c2r_one(V a, V b, V w) {
-  V e, d, z;
-  e.x = a.x + b.x;
-  e.y = a.y - b.y;
-  d.x = a.x - b.x;
-  d.y = a.y + b.y;
-  const V o = cmul_h(d, w);
-  z.x = e.x - o.y;
-  z.y = e.y + o.x;
-  return z;
-}
-
-template <int N, typename V, int... K>
-__host__ __device__ __forceinline__ void c2r_pack(const V *__restrict__ X, V (&Z)[N / 2],
-                                                  std::integer_sequence<int, K...>) {
-  constexpr int M = N / 2;
-  V x0 = X[0], xm = X[M];
-  x0.y = 0;
-  xm.y = 0;
-  ((Z[K] = c2r_one(K == 0 ? x0 : X[K], K == 0 ? xm : X[M - K], root_v<V, +1, K, N>())), ...);
-}
-
-template <int N, typename V> __host__ __device__ __forceinline__ void c2r_half(const V *__restrict__ X, V (&Z)[N / 2]) {
-  c2r_pack<N>(X, Z, std::make_integer_sequence<int, N / 2>{});
-  reg_fft<N / 2, +1>(Z);
 }
 
 // the same with the (unused) twiddle table of the axis, for the kernels that

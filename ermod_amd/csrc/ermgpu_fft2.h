@@ -268,54 +268,73 @@ __global__ __launch_bounds__(Z2_THR) void k_pme_zcol2(Params P, int A, int B, co
 // operations of a wave complete in order), so a group of planes passes
 // three barriers.  The y transform's first step reads Hk straight into
 // registers; the x transform takes two Hermitian rows as one complex row of
-// length K1 (even or odd), and its real rows end in natural order with x[0]
-// repeated at K1 for the gather.  Bound by LDS: the transforms pass each
+// length K1 (even or odd), and its real rows end in natural order behind
+// a copy of their last p - 1 values for the gather.  Bound by LDS: the transforms pass each
 // value through it nine times, the gather reads p^3 values per site.  The
 // configurations above: 0.42 ms against 2.71 ms (k_pme_slab), FP32 0.54
 // against 3.62 ms.
 // --------------------------------------------------------------------------
+// (off lanes, on = false, read where they may and write nothing)
 template <typename T, int A>
-__device__ __forceinline__ void xy2_yfirst(bool on, const typename C2<T>::type *__restrict__ src, size_t sstr,
-                                           typename C2<T>::type *dst, int dstr, int n1,
+__device__ __forceinline__ void xy2_yfirst(bool on, const typename C2<T>::type *__restrict__ src, unsigned off,
+                                           unsigned sstr, typename C2<T>::type *dst, int dstr, int n1,
                                            const typename C2<T>::type *tw) {
   using V = typename C2<T>::type;
-  if (!on) return;
   V x[A];
 #pragma unroll
-  for (int i = 0; i < A; ++i) x[i] = src[(size_t)i * sstr];
+  for (int i = 0; i < A; ++i) x[i] = src[off + i * sstr];
   reg_fft<A, +1>(x);
+  if (!on) return;
   dst[0] = x[0];
 #pragma unroll
   for (int k = 1; k < A; ++k) dst[k * dstr] = cmulc(x[k], tw[n1 * k]);
 }
 template <typename T, int B>
-__device__ __forceinline__ void xy2_ysecond(bool on, typename C2<T>::type *col, int H, int A, int k2) {
+__device__ __forceinline__ void xy2_ysecond(bool on, typename C2<T>::type *col, int rs, int A, int k2) {
   using V = typename C2<T>::type;
   V x[B];
 #pragma unroll
-  for (int n = 0; n < B; ++n) x[n] = on ? col[(k2 * B + n) * H] : V{0, 0};
+  for (int n = 0; n < B; ++n) x[n] = col[(k2 * B + n) * rs];
   wave_lds_sync();
   reg_fft<B, +1>(x);
   if (!on) return;
 #pragma unroll
-  for (int k = 0; k < B; ++k) col[(k2 + A * k) * H] = x[k];
+  for (int k = 0; k < B; ++k) col[(k2 + A * k) * rs] = x[k];
 }
+// o2: offset of the pair's second row, 0 for a last row without a partner
+// (its values then end in the imaginary parts too).  n = n1 + B i lies in the
+// upper half, X[n] = conj X[K1 - n], for every i > A / 2 and for i = A / 2
+// beyond K1 / 2; X[0] and X[K1 / 2] are real and their imaginary parts are
+// not read, i = 0 and i = A / 2 again.
 template <typename T, int A>
-__device__ __forceinline__ void xy2_xfirst(bool on, bool two, typename C2<T>::type *pr, int H, int K1, int B, int n1,
+__device__ __forceinline__ void xy2_xfirst(bool on, int o2, typename C2<T>::type *pr, int K1, int B, int n1,
                                            const typename C2<T>::type *tw) {
   using V = typename C2<T>::type;
   V x[A];
 #pragma unroll
   for (int i = 0; i < A; ++i) {
     const int n = n1 + B * i;
-    const bool up = n >= H;
-    const int k = up ? K1 - n : n;
-    V a{0, 0}, c{0, 0};
-    if (on) a = pr[k];
-    if (on && two) c = pr[H + k];
-    const bool re = n == 0 || 2 * n == K1;  // real by symmetry: the imaginary part is not read
-    a.y = re ? (T)0 : up ? -a.y : a.y;
-    c.y = re ? (T)0 : up ? -c.y : c.y;
+    V a, c;
+    if (i < A / 2) {
+      a = pr[n];
+      c = pr[o2 + n];
+      if (i == 0) {
+        a.y = (n1 == 0) ? (T)0 : a.y;
+        c.y = (n1 == 0) ? (T)0 : c.y;
+      }
+    } else if (i > A / 2) {
+      a = pr[K1 - n];
+      c = pr[o2 + K1 - n];
+      a.y = -a.y;
+      c.y = -c.y;
+    } else {
+      const int t = 2 * n - K1, k = (t > 0) ? K1 - n : n;
+      a = pr[k];
+      c = pr[o2 + k];
+      const T sg = (T)((t < 0) - (t > 0));
+      a.y = sg * a.y;
+      c.y = sg * c.y;
+    }
     x[i].x = a.x - c.y;
     x[i].y = a.y + c.x;
   }
@@ -326,133 +345,115 @@ __device__ __forceinline__ void xy2_xfirst(bool on, bool two, typename C2<T>::ty
 #pragma unroll
   for (int k = 1; k < A; ++k) pr[B * k + n1] = cmulc(x[k], tw[n1 * k]);
 }
+// the real rows, x[n] at n + h, with x[K1 - h + i] again at i < h (the
+// gather's wrap, h = p - 1)
 template <typename T, int B>
-__device__ __forceinline__ void xy2_xsecond(bool on, bool two, typename C2<T>::type *pr, int H, int K1, int A,
+__device__ __forceinline__ void xy2_xsecond(bool on, bool two, typename C2<T>::type *pr, int rs, int K1, int A, int h,
                                             int k2) {
   using V = typename C2<T>::type;
   V x[B];
 #pragma unroll
-  for (int n = 0; n < B; ++n) x[n] = on ? pr[k2 * B + n] : V{0, 0};
+  for (int n = 0; n < B; ++n) x[n] = pr[k2 * B + n];
   wave_lds_sync();
   reg_fft<B, +1>(x);
   if (!on) return;
-  T *r0 = reinterpret_cast<T *>(pr), *r1 = r0 + 2 * H;
+  T *r0 = reinterpret_cast<T *>(pr) + h + k2, *r1 = r0 + 2 * rs;
 #pragma unroll
-  for (int k = 0; k < B; ++k) {
-    r0[k2 + A * k] = x[k].x;
-    if (two) r1[k2 + A * k] = x[k].y;
+  for (int k = 0; k < B; ++k) r0[A * k] = x[k].x;
+  if (two) {
+#pragma unroll
+    for (int k = 0; k < B; ++k) r1[A * k] = x[k].y;
   }
-  if (k2 == 0) {
-    r0[K1] = x[0].x;
-    if (two) r1[K1] = x[0].y;
+#pragma unroll
+  for (int k = B - 1; k >= 0; --k) {
+    if (A * (k + 1) <= K1 - h) break;  // uniform: no lane's value lies in the wrap
+    if (k2 + A * k >= K1 - h) {
+      r0[A * k - K1] = x[k].x;
+      if (two) r1[A * k - K1] = x[k].y;
+    }
   }
 }
+// v / d for 0 <= v < 2^20 from f = 1 / d: (v + 1/2) f lies at least 1 / 2d
+// from an integer, far above the rounding of the product
+__device__ __forceinline__ int div_by(int v, float f) { return (int)(((float)v + 0.5f) * f); }
 
-
-// complex values of a plane in LDS: its rows, an even number of them, padded
-// to whole turns of the 32 LDS banks (the site sort's bank classes then hold
-// for every plane)
-__host__ __device__ inline int xy2_plane(int K2, int H) { return ((K2 + (K2 & 1)) * H + 15) & ~15; }
-template <typename T> __host__ __device__ inline size_t xy2_lds(int Q, int K1, int K2, int H) {
-  return 2 * sizeof(T) * ((size_t)Q * xy2_plane(K2, H) + K1 + K2);
+// complex values of a row in LDS: the half spectrum, then the real row with
+// its p - 1 repeated values
+__host__ __device__ inline int xy2_row(int K1, int p) {
+  const int H = K1 / 2 + 1, r = (K1 + p) / 2;
+  return r > H ? r : H;
+}
+// complex values of a plane: its rows, an even number of them, padded to
+// whole turns of the 32 LDS banks (the site sort's bank classes then hold for
+// every plane)
+__host__ __device__ inline int xy2_plane(int K2, int rs) { return ((K2 + (K2 & 1)) * rs + 15) & ~15; }
+template <typename T> __host__ __device__ inline size_t xy2_lds(int Q, int K1, int K2, int p) {
+  return 2 * sizeof(T) * ((size_t)Q * xy2_plane(K2, xy2_row(K1, p)) + K1 + K2);
 }
 
 constexpr int XY2_THR = 512;
 // Gather of a group of nq real planes in LDS (first plane zz0) into the
 // per-site sums: the sites whose p planes meet the group are one run
 // [lo, hi) of the z order, dealt over the threads.  A site's first group
-// (first: g3 - p + 1 >= zz0 or the slab's first group) stores its sum, a later
-// one adds to it; the barrier between groups orders the two.
+// (first: g3 - p + 1 >= zz0) stores its sum, a later one adds to it; the
+// barrier between groups orders the two.  The planes are added in ascending
+// order, so a sum does not depend on where the groups or slabs end (one
+// configuration in any batch gives the same bits).
+// A site's x values g1 - p + 1 .. g1 lie at g1 .. g1 + p - 1 of a row.
 template <typename T, int PP>
 __device__ __forceinline__ void xy2_gather(const Params &P, const T *real, const int rstr, const int pstr, int zz0,
                                            int nq, int lo, int hi, const int *__restrict__ zg,
                                            const T *__restrict__ zq, const T *__restrict__ zw, double *es) {
-  const int K1 = P.K1, K2 = P.K2, p = PP ? PP : P.p;
+  const int K2 = P.K2, p = PP ? PP : P.p;
   for (int idx = lo + (int)threadIdx.x; idx < hi; idx += XY2_THR) {
     const int gp = zg[idx];
     const T qv = zq[idx];
+    const T *wz = zw + (size_t)idx * 3 * p;  // [3][p]
     const int g1 = gp & 1023, g2 = (gp >> 10) & 1023, g3 = (gp >> 20) & 1023;
     const int clo = max(0, g3 - (zz0 + nq - 1)), chi = min(p - 1, g3 - zz0);
     const bool add = g3 - p + 1 < zz0;
     double acc = add ? es[idx] : 0.0;
-    if constexpr (PP == 4) {
-      // four sites' worth of latency is covered by the other waves; the pairs
-      // of adjacent x values as in xslab_gather4
-      const T *wz = static_cast<const T *>(__builtin_assume_aligned(zw + (size_t)idx * 12, 16));
-      T w[12];
+    // rstr, pstr < 2^24
+    const T *ph0 = real + __mul24(g3 - zz0, pstr) + g1;  // plane c3 = 0
+    if constexpr (PP > 0) {
+      T w[3 * PP];
+      if constexpr (PP == 4) wz = static_cast<const T *>(__builtin_assume_aligned(wz, 16));
 #pragma unroll
-      for (int k = 0; k < 12; ++k) w[k] = wz[k];
-      const int xa = g1 - 3 + ((g1 < 3) ? K1 : 0);
-      const int xb = g1 - 1 + ((g1 < 1) ? K1 : 0);
-      int ro[4];
+      for (int k = 0; k < 3 * PP; ++k) w[k] = wz[k];
+      int ro[PP];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < PP; ++k) {
         const int y = g2 - k;
-        ro[k] = (y + ((y < 0) ? K2 : 0)) * rstr;
+        ro[k] = __mul24(y + ((y < 0) ? K2 : 0), rstr);
       }
-      const T *ph0 = real + (g3 - zz0) * pstr;
 #pragma unroll
-      for (int c3 = 0; c3 < 4; ++c3) {
+      for (int c3 = PP - 1; c3 >= 0; --c3) {
         if (c3 < clo || c3 > chi) continue;
         const T *ph = ph0 - c3 * pstr;
         T sum = 0;
 #pragma unroll
-        for (int c2 = 0; c2 < 4; ++c2) {
-          const T *a = ph + ro[c2] + xa, *bb = ph + ro[c2] + xb;
-          const T a0 = a[0], a1 = a[1], b0 = bb[0], b1 = bb[1];
+        for (int c2 = 0; c2 < PP; ++c2) {
+          const T *row = ph + ro[c2];
           T rs = 0;
-          rs += w[0] * b1;
-          rs += w[1] * b0;
-          rs += w[2] * a1;
-          rs += w[3] * a0;
-          sum += w[4 + c2] * rs;
+#pragma unroll
+          for (int c1 = 0; c1 < PP; ++c1) rs += w[c1] * row[PP - 1 - c1];
+          sum += w[PP + c2] * rs;
         }
-        acc += (double)(qv * w[8 + c3] * sum);
+        acc += (double)(qv * w[2 * PP + c3] * sum);
       }
     } else {
-      const T *wz = zw + (size_t)idx * 3 * p;  // [3][p]
-      if constexpr (PP > 0) {
-        T w1[PP], w2[PP];
-        int xo[PP], yo[PP];
-#pragma unroll
-        for (int k = 0; k < PP; ++k) {
-          w1[k] = wz[k];
-          w2[k] = wz[PP + k];
-          const int x = g1 - k, y = g2 - k;
-          xo[k] = x + ((x < 0) ? K1 : 0);
-          yo[k] = (y + ((y < 0) ? K2 : 0)) * rstr;
+      for (int c3 = chi; c3 >= clo; --c3) {
+        const T *ph = ph0 - c3 * pstr;
+        T sum = 0;
+        for (int c2 = 0; c2 < p; ++c2) {
+          int y = g2 - c2;
+          y += (y < 0) ? K2 : 0;
+          const T *row = ph + y * rstr;
+          T rs = 0;
+          for (int c1 = 0; c1 < p; ++c1) rs += wz[c1] * row[p - 1 - c1];
+          sum += wz[p + c2] * rs;
         }
-        for (int c3 = clo; c3 <= chi; ++c3) {
-          const T *ph = real + (g3 - c3 - zz0) * pstr;
-          T sum = 0;
-#pragma unroll
-          for (int c2 = 0; c2 < PP; ++c2) {
-            const T *row = ph + yo[c2];
-            T rs = 0;
-#pragma unroll
-            for (int c1 = 0; c1 < PP; ++c1) rs += w1[c1] * row[xo[c1]];
-            sum += w2[c2] * rs;
-          }
-          acc += (double)(qv * wz[2 * PP + c3] * sum);
-        }
-      } else {
-        for (int c3 = clo; c3 <= chi; ++c3) {
-          const T *ph = real + (g3 - c3 - zz0) * pstr;
-          T sum = 0;
-          for (int c2 = 0; c2 < p; ++c2) {
-            int y = g2 - c2;
-            y += (y < 0) ? K2 : 0;
-            const T *row = ph + y * rstr;
-            T rs = 0;
-            for (int c1 = 0; c1 < p; ++c1) {
-              int x = g1 - c1;
-              x += (x < 0) ? K1 : 0;
-              rs += wz[c1] * row[x];
-            }
-            sum += wz[p + c2] * rs;
-          }
-          acc += (double)(qv * wz[2 * p + c3] * sum);
-        }
+        acc += (double)(qv * wz[2 * p + c3] * sum);
       }
     }
     es[idx] = acc;
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
   using V = typename C2<T>::type;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int K1 = P.K1, K2 = P.K2, K3 = P.K3, H = P.H, p = P.p;
-  const int plane = xy2_plane(K2, H);
+  const int rs = xy2_row(K1, p), plane = xy2_plane(K2, rs);
   V *stage = reinterpret_cast<V *>(lds_raw);   // [Q][plane]
   V *twy = stage + (size_t)Q * plane;          // [K2]
   V *twx = twy + K2;                           // [K1]
@@ -486,48 +487,49 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
   constexpr int NW = XY2_THR / 64;
   // columns of a wave's round: lane = n1 Gy + column in the first step,
   // k2 Gy + column in the second
-  const int Gy = 64 / fy.B;
+  const int Gy = 64 / fy.B, ly0 = lane / Gy, lg = lane - ly0 * Gy;
   // row pairs of a round: lane = pair B + n1, then pair A + k2
   const int Gx = 64 / fx.B;
+  const int xg1 = lane / fx.B, xn0 = lane - xg1 * fx.B, xg2 = lane / fx.A, xk0 = lane - xg2 * fx.A;
   const int npair = (K2 + 1) / 2;
+  const float fH = 1.0f / (float)H, fpair = 1.0f / (float)npair;
   double *es = e_site + (size_t)b * nsites;
+  const V *src = Hk + (size_t)b * K3 * K2 * H;  // K1 K2 K3 < 2^29 values
   __syncthreads();
   for (int zz0 = zb - p + 1; zz0 < ze; zz0 += Q) {
     const int nq = min(Q, ze - zz0), ncol = nq * H;
     for (int c0 = wv * Gy; c0 < ncol; c0 += NW * Gy) {
-      int ly = lane / Gy;
+      int ly = ly0;
       asm volatile("" : "+v"(ly));  // no radix's addresses are hoisted out of the loop
-      const int lg = lane - ly * Gy, cid = c0 + lg;
-      const bool in = lg < Gy && cid < ncol;  // lanes past B Gy have ly = B
-      const int q = in ? cid / H : 0, m1 = in ? cid - q * H : 0;
-      const int z = (((zz0 + q) % K3) + K3) % K3;
-      V *col = stage + (size_t)q * plane + m1;
-      const V *src = Hk + (((size_t)b * K3 + z) * K2 + ly) * H + m1;
-      ERM_RADIX_A(fy.A, (xy2_yfirst<T, RR>(in && ly < fy.B, src, (size_t)fy.B * H, col + ly * H, fy.B * H, ly, twy)))
+      const bool in = lg < Gy && c0 + lg < ncol;  // lanes past B Gy have ly >= B
+      const int cid = in ? c0 + lg : c0, q = div_by(cid, fH), m1 = cid - q * H;
+      const int z = zz0 + q + ((zz0 + q < 0) ? K3 : 0);
+      V *col = stage + q * plane + m1;
+      const int l1 = min(ly, fy.B - 1), l2 = min(ly, fy.A - 1);
+      ERM_RADIX_A(fy.A, (xy2_yfirst<T, RR>(in && ly < fy.B, src, (unsigned)((z * K2 + l1) * H + m1),
+                                           (unsigned)(fy.B * H), col + l1 * rs, fy.B * rs, l1, twy)))
       wave_lds_sync();
-      ERM_RADIX_B(fy.B, (xy2_ysecond<T, RR>(in && ly < fy.A, col, H, fy.A, ly)))
+      ERM_RADIX_B(fy.B, (xy2_ysecond<T, RR>(in && ly < fy.A, col, rs, fy.A, l2)))
     }
     __syncthreads();
     const int nrow = nq * npair;
     for (int p0 = wv * Gx; p0 < nrow; p0 += NW * Gx) {
       {
-        int xg1 = lane / fx.B;
-        asm volatile("" : "+v"(xg1));
-        const int xn1 = lane - xg1 * fx.B, pid = p0 + xg1;
-        const bool in = xg1 < Gx && pid < nrow;
-        const int q = in ? pid / npair : 0, pr = in ? pid - q * npair : 0;
-        V *row = stage + (size_t)q * plane + (size_t)2 * pr * H;
-        ERM_RADIX_A(fx.A, (xy2_xfirst<T, RR>(in, 2 * pr + 1 < K2, row, H, K1, fx.B, xn1, twx)))
+        int xn1 = xn0;
+        asm volatile("" : "+v"(xn1));
+        const bool in = xg1 < Gx && p0 + xg1 < nrow;
+        const int pid = in ? p0 + xg1 : p0, q = div_by(pid, fpair), pr = pid - q * npair;
+        V *row = stage + q * plane + 2 * pr * rs;
+        ERM_RADIX_A(fx.A, (xy2_xfirst<T, RR>(in, (2 * pr + 1 < K2) ? rs : 0, row, K1, fx.B, xn1, twx)))
       }
       wave_lds_sync();
       {
-        int xg2 = lane / fx.A;
-        asm volatile("" : "+v"(xg2));
-        const int xk2 = lane - xg2 * fx.A, pid = p0 + xg2;
-        const bool in = xg2 < Gx && pid < nrow;
-        const int q = in ? pid / npair : 0, pr = in ? pid - q * npair : 0;
-        V *row = stage + (size_t)q * plane + (size_t)2 * pr * H;
-        ERM_RADIX_B(fx.B, (xy2_xsecond<T, RR>(in, 2 * pr + 1 < K2, row, H, K1, fx.A, xk2)))
+        int xk2 = xk0;
+        asm volatile("" : "+v"(xk2));
+        const bool in = xg2 < Gx && p0 + xg2 < nrow;
+        const int pid = in ? p0 + xg2 : p0, q = div_by(pid, fpair), pr = pid - q * npair;
+        V *row = stage + q * plane + 2 * pr * rs;
+        ERM_RADIX_B(fx.B, (xy2_xsecond<T, RR>(in, 2 * pr + 1 < K2, row, rs, K1, fx.A, p - 1, xk2)))
       }
       wave_lds_sync();
     }
@@ -535,11 +537,11 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
     const T *real = reinterpret_cast<const T *>(stage);
     const int lo = z_start[max(zb, zz0)], hi = z_start[min(ze, zz0 + nq + p - 1)];
     if (p == 4)
-      xy2_gather<T, 4>(P, real, 2 * H, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
+      xy2_gather<T, 4>(P, real, 2 * rs, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
     else if (p == 6)
-      xy2_gather<T, 6>(P, real, 2 * H, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
+      xy2_gather<T, 6>(P, real, 2 * rs, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
     else
-      xy2_gather<T, 0>(P, real, 2 * H, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
+      xy2_gather<T, 0>(P, real, 2 * rs, 2 * plane, zz0, nq, lo, hi, zg, zq, zw, es);
     __syncthreads();
   }
 }

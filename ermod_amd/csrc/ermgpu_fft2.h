@@ -262,17 +262,23 @@ __global__ __launch_bounds__(Z2_THR) void k_pme_zcol2(Params P, int A, int B, co
 // --------------------------------------------------------------------------
 // y and x transforms of a slab of z planes, and the gather (the owned planes
 // [zb, zb + S) and their p - 1 halo planes, Q planes in LDS at a time; the
-// sites of the slab are summed as in k_pme_xslab).  A wave owns whole
+// sites of the slab summed in the z order).  A wave owns whole
 // columns (y) and whole row pairs (x), several at once over its lanes: both
 // steps of a transform and their exchange stay within the wave (LDS
 // operations of a wave complete in order), so a group of planes passes
 // three barriers.  The y transform's first step reads Hk straight into
 // registers; the x transform takes two Hermitian rows as one complex row of
 // length K1 (even or odd), and its real rows end in natural order behind
-// a copy of their last p - 1 values for the gather.  Bound by LDS: the transforms pass each
-// value through it nine times, the gather reads p^3 values per site.  The
-// configurations above: 0.42 ms against 2.71 ms (k_pme_slab), FP32 0.54
-// against 3.62 ms.
+// a copy of their last p - 1 values for the gather.  Bound by VALU issue (63%
+// busy) and LDS (28% of its cycles are bank conflicts) in turn, a group's
+// phases overlapping with the other workgroup of the CU.  Measured: 500 FP64
+// configurations of 40 x 40 x 80, 12000 sites, 0.32 ms (k_pme_slab 2.71); 701
+// FP32 ones of 45 x 60 x 75, 18000 sites, 0.52 ms (3.62).  Against a register
+// FFT per row with the planes staged in LDS and y columns transformed in HBM
+// (the register lengths until then): 1000 configurations of 48^3, 12000 sites,
+// FP64 1.24 -> 0.53 ms, FP32 0.75 -> 0.29; 500 of 64^3, order 6, 21000 sites,
+// FP64 2.23 -> 0.93; 5000 of 64^3, 29200 sites, FP32 with the y columns in
+// LDS, 4.03 -> 3.23 ms.
 // --------------------------------------------------------------------------
 // (off lanes, on = false, read where they may and write nothing)
 template <typename T, int A>
@@ -477,7 +483,9 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
   V *twx = twy + K2;                           // [K1]
   for (int t = threadIdx.x; t < K2; t += XY2_THR) twy[t] = tw2[t];
   for (int t = threadIdx.x; t < K1; t += XY2_THR) twx[t] = tw1[t];
-  // XCD-aware order, as in k_pme_xslab
+  // XCD-aware order: workgroups go to the 8 XCDs round-robin by linear index,
+  // so XCD x takes the x-th contiguous share of the (configuration, slab)
+  // items and finds the halo planes of consecutive slabs in its L2
   const int nwg = gridDim.x * gridDim.y;
   int L = blockIdx.y * gridDim.x + blockIdx.x;
   if (nwg % 8 == 0) L = (L % 8) * (nwg / 8) + L / 8;

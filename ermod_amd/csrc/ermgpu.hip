@@ -842,6 +842,13 @@ int stage_configs(erm_ctx *c, const Batch &bt, const Params &k) {
   return ERM_OK;
 }
 
+// sites per workgroup of k_solute_prep: two workgroups per CU, of at least 8
+// sites each
+int prep_sites(int n, int ns) {
+  const int nblk = std::max(1, std::min((ns + 7) / 8, 512 / std::max(n, 1)));
+  return (ns + nblk - 1) / nblk;
+}
+
 // workgroups per configuration of the tiled pair kernel: nchunk chunks of 64
 // candidate molecules over nwave waves, PAIR_CHUNKS_PER_WAVE chunks each
 constexpr int PAIR_CHUNKS_PER_WAVE = 4;
@@ -988,7 +995,9 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
   if (flags & DO_RECIP) TRY(ensure(c, c->d_Hk, vb * (size_t)n * K3 * K2 * H));
   TRY(mark(c, 0));
   TRY(stage_configs(c, bt, k));
-  hipLaunchKernelGGL(k_solute_prep<T>, dim3(n), dim3(128), 0, c->st, k, dp<double>(c->d_spos),
+  const int spb = prep_sites(n, ns);
+  hipLaunchKernelGGL(k_solute_prep<T>, dim3(n, (ns + spb - 1) / spb), dim3(PREP_THR), sizeof(int) * ns, c->st, k, spb,
+                     dp<double>(c->d_spos),
                      dp<double>(c->d_qslt), dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<V>(c->d_tw3),
                      dp<double>(c->d_sref), dp<int>(c->d_sg3), dp<T>(c->d_sw3), dp<T>(c->d_sqv),
                      dp<V>(c->d_w1h), dp<V>(c->d_w2h), (regp && !zfft) ? dp<V>(c->d_w3h) : (V *)nullptr);
@@ -1495,7 +1504,9 @@ template <typename T> int gradient_batch(erm_ctx *c, const Batch &bt, const Grad
   TRY(ensure(c, c->d_w2h, sizeof(V) * (size_t)n * ns * k.K2));
   TRY(ensure(c, c->d_sltj, sizeof(int) * n));
   TRY(stage_configs(c, bt, k));
-  hipLaunchKernelGGL(k_solute_prep<T>, dim3(n), dim3(128), 0, c->st, k, dp<double>(c->d_spos),
+  const int spb = prep_sites(n, ns);
+  hipLaunchKernelGGL(k_solute_prep<T>, dim3(n, (ns + spb - 1) / spb), dim3(PREP_THR), sizeof(int) * ns, c->st, k, spb,
+                     dp<double>(c->d_spos),
                      dp<double>(c->d_qslt), dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<V>(c->d_tw3),
                      dp<double>(c->d_sref), dp<int>(c->d_sg3), dp<T>(c->d_sw3), dp<T>(c->d_sqv),
                      dp<V>(c->d_w1h), dp<V>(c->d_w2h), (V *)nullptr);
@@ -1681,7 +1692,9 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
                        offset[r], dp<double>(m->d_bf), 0, dp<double>(m->d_sitemass) + m->mol_begin[m->slt_template],
                        dp<double>(m->d_cellm), dp<double>(m->d_aggcen), dp<double>(c->d_spos) + so * 3);
     TRY(launch_check(c, "k_pose"));
-    hipLaunchKernelGGL(k_solute_prep<T>, dim3(R[r].ncfg), dim3(128), 0, c->st, km, dp<double>(c->d_spos) + so * 3,
+    const int spb = prep_sites(R[r].ncfg, m->ns);
+    hipLaunchKernelGGL(k_solute_prep<T>, dim3(R[r].ncfg, (m->ns + spb - 1) / spb), dim3(PREP_THR), sizeof(int) * m->ns,
+                       c->st, km, spb, dp<double>(c->d_spos) + so * 3,
                        dp<double>(m->d_qslt), dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<V>(c->d_tw3),
                        dp<double>(c->d_sref) + 4 * (size_t)R[r].cfg0, dp<int>(c->d_sg3) + so, dp<T>(c->d_sw3) + so * p,
                        dp<T>(c->d_sqv) + so, dp<V>(c->d_w1h) + so * H, dp<V>(c->d_w2h) + so * K2, (V *)nullptr);

@@ -66,7 +66,7 @@ template <typename V> __device__ __forceinline__ V cmulc(V a, V w) {
 
 // --------------------------------------------------------------------------
 // z columns.  A workgroup takes C consecutive columns (m1, m2) of one
-// configuration: the solute's sites, in chunks of Z2_SCH sorted by plane, are
+// configuration: the solute's sites, in chunks of Z2_SCH in plane order, are
 // added to the columns in LDS (buf[z][column], each plane over the sites
 // whose p planes hold it), transformed forward, multiplied by the Green's
 // function (self energy on the way, recpcal.F90:385-394), transformed back
@@ -80,12 +80,12 @@ template <typename V> __device__ __forceinline__ V cmulc(V a, V w) {
 // --------------------------------------------------------------------------
 constexpr int Z2_SCH = 32;   // solute sites per chunk
 constexpr int Z2_THR = 256;
-template <typename T> constexpr int z2_cols = sizeof(T) == 8 ? 32 : 64;  // columns per workgroup
+template <typename T> constexpr int z2_cols = sizeof(T) == 8 ? 16 : 32;  // columns per workgroup
 
 template <typename T> __host__ __device__ inline size_t z2_lds(int K3, int p) {
   constexpr int C = z2_cols<T>;
   return sizeof(T) * 2 * ((size_t)K3 * C + (size_t)Z2_SCH * C + K3) + sizeof(T) * (size_t)Z2_SCH * p +
-         sizeof(int) * (Z2_SCH * 2 + (size_t)K3 + 1) + sizeof(double) * Z2_THR + 32;
+         sizeof(int) * (Z2_SCH + (size_t)K3 + 1) + sizeof(double) * Z2_THR + 32;
 }
 
 // first forward step of (n1, column): in place
@@ -161,10 +161,9 @@ __global__ __launch_bounds__(Z2_THR) void k_pme_zcol2(Params P, int A, int B, co
   V *amp = buf + (size_t)K3 * C;                 // [Z2_SCH][C] q what1 what2 of the chunk's sites
   V *tw = amp + (size_t)Z2_SCH * C;              // [K3]
   double *red = reinterpret_cast<double *>(tw + K3);  // [Z2_THR]
-  T *wz = reinterpret_cast<T *>(red + Z2_THR);   // [Z2_SCH][p] z weights in plane order
-  int *gz = reinterpret_cast<int *>(wz + (size_t)Z2_SCH * p);  // [Z2_SCH] planes g3, sorted
-  int *ord = gz + Z2_SCH;                        // [Z2_SCH] site of each sorted place
-  int *first = ord + Z2_SCH;                     // [K3 + 1] first sorted place with g3 >= z
+  T *wz = reinterpret_cast<T *>(red + Z2_THR);   // [Z2_SCH][p] z weights
+  int *gz = reinterpret_cast<int *>(wz + (size_t)Z2_SCH * p);  // [Z2_SCH] planes g3, ascending
+  int *first = gz + Z2_SCH;                      // [K3 + 1] first site of the chunk with g3 >= z
   const int cl = threadIdx.x % C, sub = threadIdx.x / C;
   constexpr int NSUB = Z2_THR / C;
   const int ncol = H * K2, c = blockIdx.x * C + cl;
@@ -175,28 +174,18 @@ __global__ __launch_bounds__(Z2_THR) void k_pme_zcol2(Params P, int A, int B, co
     const int nc = min(Z2_SCH, ns - s0);
     const size_t bs = (size_t)b * ns + s0;
     __syncthreads();  // the previous chunk's sites are used up
+    // site j opens the planes (g3 of j - 1, g3 of j], the last site also
+    // those above it
     if (threadIdx.x < (unsigned)nc) {
-      const int g = sg3[bs + threadIdx.x];
-      int rank = 0;
-      for (int j = 0; j < nc; ++j) {
-        const int gj = sg3[bs + j];
-        rank += (gj < g || (gj == g && j < (int)threadIdx.x)) ? 1 : 0;
-      }
-      gz[rank] = g;
-      ord[rank] = threadIdx.x;
+      const int j = threadIdx.x, g = sg3[bs + j], g0 = j ? sg3[bs + j - 1] : -1;
+      gz[j] = g;
+      for (int z = g0 + 1; z <= g; ++z) first[z] = j;
+      if (j == nc - 1)
+        for (int z = g + 1; z <= K3; ++z) first[z] = nc;
     }
-    __syncthreads();
-    for (int z = threadIdx.x; z <= K3; z += Z2_THR) {
-      int n = 0;
-      for (int j = 0; j < nc; ++j) n += (gz[j] < z) ? 1 : 0;
-      first[z] = n;
-    }
-    for (int t = threadIdx.x; t < nc * p; t += Z2_THR) {
-      const int j = t / p;
-      wz[t] = sw3[(bs + ord[j]) * p + (t - j * p)];
-    }
+    for (int t = threadIdx.x; t < nc * p; t += Z2_THR) wz[t] = sw3[bs * p + t];
     for (int j = sub; j < nc; j += NSUB) {
-      const size_t s = bs + ord[j];
+      const size_t s = bs + j;
       V a;
       a.x = 0;
       a.y = 0;

@@ -423,8 +423,20 @@ static __global__ __launch_bounds__(64) void k_pose(Params P, int n, const uint6
     for (int i = ln; i < 3 * ns; i += nl) out[i] = x[i];
 }
 
+// Solute configurations for the PME kernels: the reference point (sref), and
+// per site its z plane, z weights, charge and the spectra of its weights
+// along x and y (z too when w3h is given).  The sites are written in the order
+// of (z plane, index), which is how the z-column kernels read them: they
+// ranked every chunk again in each of their workgroups before (5000 FP32
+// configurations of 5 to 150 sites at 64^3: z columns 2.93 -> 2.37 ms).
+// Grid (configuration, block of spb sites): one block per configuration of a
+// full batch, up to one per 8 sites where a few configurations would leave
+// the chip idle (one solute of 300 sites, 96^3: 0.34 -> 0.03 ms).  Bound by the spectra
+// (p twiddle loads per value) and their writes.
+constexpr int PREP_THR = 128;
+constexpr int PREP_SITES = 64;  // sites per chunk through LDS
 template <typename T>
-__global__ __launch_bounds__(128) void k_solute_prep(Params P, const double *__restrict__ spos,
+__global__ __launch_bounds__(PREP_THR) void k_solute_prep(Params P, int spb, const double *__restrict__ spos,
                                                      const double *__restrict__ qsolute,
                                                      const typename C2<T>::type *__restrict__ tw1,
                                                      const typename C2<T>::type *__restrict__ tw2,
@@ -435,77 +447,95 @@ __global__ __launch_bounds__(128) void k_solute_prep(Params P, const double *__r
                                                      typename C2<T>::type *w3h) {
 #pragma clang fp contract(off)
   using V = typename C2<T>::type;
+  extern __shared__ int prep_g3[];  // [ns] z planes of every site
   const int b = blockIdx.x, ns = P.ns, p = P.p;
   const double *x = spos + (size_t)b * ns * 3;
-  __shared__ double red[128 * 3];
-  __shared__ int gsh[3 * 64];
-  __shared__ double wsh[3 * MAXP * 64];
-  // reference point
-  double s0 = 0, s1 = 0, s2 = 0;
-  for (int s = threadIdx.x; s < ns; s += blockDim.x) {
-    s0 += x[3 * s];
-    s1 += x[3 * s + 1];
-    s2 += x[3 * s + 2];
-  }
-  red[threadIdx.x * 3] = s0;
-  red[threadIdx.x * 3 + 1] = s1;
-  red[threadIdx.x * 3 + 2] = s2;
-  __syncthreads();
-  __shared__ double cpt[4];
-  if (threadIdx.x == 0) {
-    double a = 0, bb = 0, c = 0;
-    for (int i = 0; i < (int)blockDim.x; ++i) {
-      a += red[3 * i];
-      bb += red[3 * i + 1];
-      c += red[3 * i + 2];
+  __shared__ double red[PREP_THR * 3];
+  __shared__ int gsh[3 * PREP_SITES], place[PREP_SITES];
+  __shared__ double wsh[3 * MAXP * PREP_SITES];
+  if (blockIdx.y == 0) {
+    // reference point: the sites' centre and their largest distance from it
+    double s0 = 0, s1 = 0, s2 = 0;
+    for (int s = threadIdx.x; s < ns; s += PREP_THR) {
+      s0 += x[3 * s];
+      s1 += x[3 * s + 1];
+      s2 += x[3 * s + 2];
     }
-    cpt[0] = a / ns;
-    cpt[1] = bb / ns;
-    cpt[2] = c / ns;
-  }
-  __syncthreads();
-  double rmax = 0.0;
-  for (int s = threadIdx.x; s < ns; s += blockDim.x) {
-    double d0 = x[3 * s] - cpt[0], d1 = x[3 * s + 1] - cpt[1], d2 = x[3 * s + 2] - cpt[2];
-    rmax = fmax(rmax, sqrt(d0 * d0 + d1 * d1 + d2 * d2));
-  }
-  red[threadIdx.x] = rmax;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double r = 0;
-    for (int i = 0; i < (int)blockDim.x; ++i) r = fmax(r, red[i]);
-    sref[4 * b + 0] = cpt[0];
-    sref[4 * b + 1] = cpt[1];
-    sref[4 * b + 2] = cpt[2];
-    sref[4 * b + 3] = r;
+    red[threadIdx.x * 3] = s0;
+    red[threadIdx.x * 3 + 1] = s1;
+    red[threadIdx.x * 3 + 2] = s2;
+    for (int h = PREP_THR / 2; h > 0; h >>= 1) {
+      __syncthreads();
+      if ((int)threadIdx.x < h)
+        for (int d = 0; d < 3; ++d) red[threadIdx.x * 3 + d] += red[(threadIdx.x + h) * 3 + d];
+    }
+    __syncthreads();
+    const double c0 = red[0] / ns, c1 = red[1] / ns, c2 = red[2] / ns;
+    __syncthreads();
+    double rmax = 0.0;
+    for (int s = threadIdx.x; s < ns; s += PREP_THR) {
+      double d0 = x[3 * s] - c0, d1 = x[3 * s + 1] - c1, d2 = x[3 * s + 2] - c2;
+      rmax = fmax(rmax, sqrt(d0 * d0 + d1 * d1 + d2 * d2));
+    }
+    red[threadIdx.x] = rmax;
+    for (int h = PREP_THR / 2; h > 0; h >>= 1) {
+      __syncthreads();
+      if ((int)threadIdx.x < h) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + h]);
+    }
+    if (threadIdx.x == 0) {
+      sref[4 * b + 0] = c0;
+      sref[4 * b + 1] = c1;
+      sref[4 * b + 2] = c2;
+      sref[4 * b + 3] = red[0];
+    }
   }
   if (P.cltype == 0) return;  // bare Coulomb: no reciprocal space
-  // splines, in chunks of 64 sites through LDS
   const int Ks[3] = {P.K1, P.K2, P.K3};
-  for (int s0c = 0; s0c < ns; s0c += 64) {
-    int nc = min(64, ns - s0c);
+  // grid coordinate of site s along d, its base (an index in [0, K])
+  auto grid = [&](int s, int d, double &factor) {
+    const double *xs = x + 3 * s;
+    double f = P.invcl[d] * xs[0] + P.invcl[3 + d] * xs[1] + P.invcl[6 + d] * xs[2];
+    f = f - floor(f);
+    factor = f * (double)Ks[d];
+    return (factor >= 0.0 && factor <= (double)Ks[d]) ? (int)factor : 0;
+  };
+  for (int s = threadIdx.x; s < ns; s += PREP_THR) {
+    double factor;
+    prep_g3[s] = grid(s, 2, factor) % Ks[2];
+  }
+  // splines and spectra of the block's sites, in chunks through LDS
+  const int beg = blockIdx.y * spb, end = min(ns, beg + spb);
+  for (int s0c = beg; s0c < end; s0c += PREP_SITES) {
+    const int nc = min(PREP_SITES, end - s0c);
     __syncthreads();
-    for (int t = threadIdx.x; t < nc * 3; t += blockDim.x) {
-      int s = s0c + t / 3, d = t % 3;
-      const double *xs = x + 3 * s;
-      double f = P.invcl[d] * xs[0] + P.invcl[3 + d] * xs[1] + P.invcl[6 + d] * xs[2];
-      f = f - floor(f);
-      double factor = f * (double)Ks[d];
-      int rci = (factor >= 0.0 && factor <= (double)Ks[d]) ? (int)factor : 0;
+    for (int t = threadIdx.x; t < nc * 3; t += PREP_THR) {
+      const int s = s0c + t / 3, d = t % 3;
+      double factor;
+      const int rci = grid(s, d, factor);
       for (int k = 0; k < p; ++k)
         wsh[((t / 3) * 3 + d) * MAXP + k] = spline_value_dev(P.coeff, p, factor - (double)(rci - k));
       gsh[(t / 3) * 3 + d] = rci % Ks[d];
     }
+    // the site's place in the order of (plane, index)
+    for (int t = threadIdx.x; t < nc; t += PREP_THR) {
+      const int s = s0c + t, g = prep_g3[s];
+      int r = 0;
+      for (int u = 0; u < ns; ++u) {
+        const int gu = prep_g3[u];
+        r += (gu < g || (gu == g && u < s)) ? 1 : 0;
+      }
+      place[t] = r;
+    }
     __syncthreads();
-    for (int t = threadIdx.x; t < nc; t += blockDim.x) {
-      int s = s0c + t;
-      sg3[(size_t)b * ns + s] = gsh[t * 3 + 2];
-      sqv[(size_t)b * ns + s] = (T)qsolute[s];
-      for (int k = 0; k < p; ++k) sw3[((size_t)b * ns + s) * p + k] = (T)wsh[(t * 3 + 2) * MAXP + k];
+    for (int t = threadIdx.x; t < nc; t += PREP_THR) {
+      const size_t s = (size_t)b * ns + place[t];
+      sg3[s] = gsh[t * 3 + 2];
+      sqv[s] = (T)qsolute[s0c + t];
+      for (int k = 0; k < p; ++k) sw3[s * p + k] = (T)wsh[(t * 3 + 2) * MAXP + k];
     }
     // spectra along the three axes (axis 3 only when w3h is requested)
     int nm = P.H + P.K2 + (w3h ? P.K3 : 0);
-    for (int t = threadIdx.x; t < nc * nm; t += blockDim.x) {
+    for (int t = threadIdx.x; t < nc * nm; t += PREP_THR) {
       int sl = t / nm, mm = t - sl * nm;
       int d = (mm < P.H) ? 0 : (mm < P.H + P.K2) ? 1 : 2;
       int m = (d == 0) ? mm : (d == 1) ? mm - P.H : mm - P.H - P.K2;
@@ -526,13 +556,13 @@ __global__ __launch_bounds__(128) void k_solute_prep(Params P, const double *__r
         acc.x += wt * w.x;
         acc.y += wt * w.y;
       }
-      int s = s0c + sl;
+      const size_t s = (size_t)b * ns + place[sl];
       if (d == 0)
-        w1h[((size_t)b * ns + s) * P.H + m] = acc;
+        w1h[s * P.H + m] = acc;
       else if (d == 1)
-        w2h[((size_t)b * ns + s) * P.K2 + m] = acc;
+        w2h[s * P.K2 + m] = acc;
       else
-        w3h[((size_t)b * ns + s) * P.K3 + m] = acc;
+        w3h[s * P.K3 + m] = acc;
     }
   }
 }
@@ -972,8 +1002,8 @@ __device__ __forceinline__ void zspread_half(V (&Y)[K3 / 2], const V a, const T 
   }
 }
 
-// k_pme_zcol_fft stages its sites in chunks of zfft_sch<T>, sorted by z
-// plane (128 in FP32: the 150-site solutes take two chunks, and three
+// k_pme_zcol_fft stages its sites in chunks of zfft_sch<T>, in z plane order
+// (128 in FP32: the 150-site solutes take two chunks, and three
 // 256-thread workgroups still fit a CU's LDS)
 template <typename T> constexpr int zfft_sch = sizeof(T) == 4 ? 128 : 64;
 constexpr int ZFFT_KMAX = 96;  // largest z grid length of the register kernels
@@ -990,19 +1020,18 @@ __host__ __device__ inline int zcol_fft_rows(int H, int K2, int XT, int L = 2) {
 
 // dynamic LDS of k_pme_zcol_fft with XT threads and L lanes per column:
 // zfft_sch<T> sites x (H + the block's m2 rows) spectra, charge-scaled z
-// weights, planes and ranks, the bucket starts, and the self-energy
-// reduction
+// weights, the bucket starts, and the self-energy reduction
 template <typename T>
 __host__ __device__ inline size_t zcol_fft_lds(int H, int K2, int XT = NTHR, int L = 2) {
   const size_t spec = (size_t)zfft_sch<T> * (H + zcol_fft_rows(H, K2, XT, L)) * 2 * sizeof(T);
-  const size_t small = (size_t)zfft_sch<T> * (sizeof(T) * MAXP + 2 * sizeof(int)) + (ZFFT_KMAX + 1) * sizeof(int);
+  const size_t small = (size_t)zfft_sch<T> * sizeof(T) * MAXP + (ZFFT_KMAX + 1) * sizeof(int);
   return ((spec + small + 15) & ~(size_t)15) + XT * sizeof(double);
 }
 
-// Site chunk of the z-column kernels in LDS: ranks by (plane, index), the
-// bucket starts per plane, the sorted spectra what1 (all m1) and what2 (the
-// block's nm2 rows from m2lo) and the charge-scaled z weights.  All threads
-// call it; the caller's barrier precedes the next chunk's call.
+// Site chunk of the z-column kernels in LDS (the sites come in plane order,
+// k_solute_prep): the bucket starts per plane, the spectra what1 (all m1) and
+// what2 (the block's nm2 rows from m2lo) and the charge-scaled z weights.
+// All threads call it; the caller's barrier precedes the next chunk's call.
 template <typename T, int PP>
 __device__ __forceinline__ void zcol_stage_chunk(int s0, int nc, int K3, int H, int K2, int m2lo, int nm2,
                                                  const T *__restrict__ sqv,
@@ -1010,41 +1039,24 @@ __device__ __forceinline__ void zcol_stage_chunk(int s0, int nc, int K3, int H, 
                                                  const typename C2<T>::type *__restrict__ w2h,
                                                  const int *__restrict__ sg3, const T *__restrict__ sw3,
                                                  typename C2<T>::type *l1, typename C2<T>::type *l2, T *lw,
-                                                 int *lg, int *lr, int *lst) {
+                                                 int *lst) {
   __syncthreads();  // the previous chunk is consumed
-  for (int t = threadIdx.x; t < nc; t += blockDim.x) lg[t] = sg3[(size_t)s0 + t];
-  __syncthreads();
-  // rank by (plane, index); bucket starts = sites on lower planes (a plane
-  // outside [0, K3) falls in no bucket)
+  // bucket starts: site t opens the planes (g3 of t - 1, g3 of t], the last
+  // site also those above it
   for (int t = threadIdx.x; t < nc; t += blockDim.x) {
-    const int g = lg[t];
-    int r = 0;
-    for (int u = 0; u < nc; ++u) {
-      const int gu = lg[u];
-      r += (gu < g) || (gu == g && u < t);
-    }
-    lr[t] = r;
+    const int g = sg3[(size_t)s0 + t], g0 = t ? sg3[(size_t)s0 + t - 1] : -1;
+    for (int z = g0 + 1; z <= g; ++z) lst[z] = t;
+    if (t == nc - 1)
+      for (int z = g + 1; z <= K3; ++z) lst[z] = nc;
   }
-  for (int t = threadIdx.x; t <= K3; t += blockDim.x) {
-    int r = 0;
-    for (int u = 0; u < nc; ++u) r += lg[u] < t;
-    lst[t] = r;
+  const typename C2<T>::type *r1 = w1h + (size_t)s0 * H;
+  for (int t = threadIdx.x; t < nc * H; t += blockDim.x) l1[t] = r1[t];
+  for (int t = threadIdx.x; t < nc * nm2; t += blockDim.x) {
+    const int sl = t / nm2, m = t - sl * nm2;
+    l2[t] = w2h[((size_t)s0 + sl) * K2 + m2lo + m];
   }
-  __syncthreads();
-  const int nsp = H + nm2;
-  for (int t = threadIdx.x; t < nc * nsp; t += blockDim.x) {
-    const int sl = t / nsp, m = t - sl * nsp;
-    const size_t bs = (size_t)s0 + sl;
-    const int r = lr[sl];
-    if (m < H)
-      l1[r * H + m] = w1h[bs * H + m];
-    else
-      l2[r * nm2 + (m - H)] = w2h[bs * K2 + m2lo + (m - H)];
-  }
-  for (int t = threadIdx.x; t < nc * PP; t += blockDim.x) {
-    const int sl = t / PP, k = t - sl * PP;
-    lw[lr[sl] * PP + k] = sqv[(size_t)s0 + sl] * sw3[(size_t)s0 * PP + t];
-  }
+  for (int t = threadIdx.x; t < nc * PP; t += blockDim.x)
+    lw[t] = sqv[(size_t)s0 + t / PP] * sw3[(size_t)s0 * PP + t];
   __syncthreads();
 }
 
@@ -1068,9 +1080,7 @@ __device__ __forceinline__ void zcol_fft_body1(const Params &P, int ns, int blk,
   V *l1 = reinterpret_cast<V *>(lds_raw);
   V *l2 = l1 + zfft_sch<T> * H;
   T *lw = reinterpret_cast<T *>(l2 + zfft_sch<T> * rows);
-  int *lg = reinterpret_cast<int *>(lw + zfft_sch<T> * MAXP);
-  int *lr = lg + zfft_sch<T>;
-  int *lst = lr + zfft_sch<T>;
+  int *lst = reinterpret_cast<int *>(lw + zfft_sch<T> * MAXP);
   double *red = reinterpret_cast<double *>(lds_raw + zcol_fft_lds<T>(H, K2, XT, 1) - XT * sizeof(double));
   const int ncol = H * K2;
   const int c = blk * XT + (int)threadIdx.x;
@@ -1106,7 +1116,7 @@ __device__ __forceinline__ void zcol_fft_body1(const Params &P, int ns, int blk,
   };
   for (int s0 = 0; s0 < ns; s0 += zfft_sch<T>) {
     const int nc = min(zfft_sch<T>, ns - s0);
-    zcol_stage_chunk<T, PP>(s0, nc, K3, H, K2, m2lo, nm2, sqv, w1h, w2h, sg3, sw3, l1, l2, lw, lg, lr, lst);
+    zcol_stage_chunk<T, PP>(s0, nc, K3, H, K2, m2lo, nm2, sqv, w1h, w2h, sg3, sw3, l1, l2, lw, lst);
     lsa = lst[lane];
     if constexpr (K3 >= 64) lsb = lst[64 + lane < ZFFT_KMAX + 1 ? 64 + lane : ZFFT_KMAX];
     [&]<int... Gs>(std::integer_sequence<int, Gs...>) {
@@ -1177,9 +1187,7 @@ __device__ __forceinline__ void zcol_fft_body(const Params &P, int ns, int blk, 
   V *l1 = reinterpret_cast<V *>(lds_raw);           // [zfft_sch<T>][H], sorted order
   V *l2 = l1 + zfft_sch<T> * H;                        // [zfft_sch<T>][nm2] the block's m2 rows
   T *lw = reinterpret_cast<T *>(l2 + zfft_sch<T> * rows);  // [zfft_sch<T>][PP] z weights x charge
-  int *lg = reinterpret_cast<int *>(lw + zfft_sch<T> * MAXP);  // [zfft_sch<T>] planes, chunk order
-  int *lr = lg + zfft_sch<T>;                          // [zfft_sch<T>] rank of each site by plane
-  int *lst = lr + zfft_sch<T>;                         // [K3 + 1] first sorted site of each plane
+  int *lst = reinterpret_cast<int *>(lw + zfft_sch<T> * MAXP);  // [K3 + 1] first sorted site of each plane
   double *red = reinterpret_cast<double *>(lds_raw + zcol_fft_lds<T>(H, K2, XT) - XT * sizeof(double));
   const int ncol = H * K2;
   const int h = threadIdx.x & 1;
@@ -1218,7 +1226,7 @@ __device__ __forceinline__ void zcol_fft_body(const Params &P, int ns, int blk, 
   };
   for (int s0 = 0; s0 < ns; s0 += zfft_sch<T>) {
     const int nc = min(zfft_sch<T>, ns - s0);
-    zcol_stage_chunk<T, PP>(s0, nc, K3, H, K2, m2lo, nm2, sqv, w1h, w2h, sg3, sw3, l1, l2, lw, lg, lr, lst);
+    zcol_stage_chunk<T, PP>(s0, nc, K3, H, K2, m2lo, nm2, sqv, w1h, w2h, sg3, sw3, l1, l2, lw, lst);
     lsa = lst[lane];
     if constexpr (K3 >= 64) lsb = lst[64 + lane < ZFFT_KMAX + 1 ? 64 + lane : ZFFT_KMAX];
     [&]<int... Gs>(std::integer_sequence<int, Gs...>) {

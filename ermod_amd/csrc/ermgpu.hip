@@ -516,24 +516,64 @@ template <typename T> bool reg_path_ok(const erm_ctx *c) {
   return reg_len<T>(k.K1) && reg_len<T>(k.K2) && reg_len<T>(k.K3) && (k.K1 % 2 == 0);
 }
 
-// the register path's z columns go through the z FFT for spline orders 4
-// and 6 (two lanes per column), else they sum the solute's z spectra
-bool zcol_fft(const erm_ctx *c, bool regp) { return regp && (c->kp.p == 4 || c->kp.p == 6); }
+// FP32 grid lengths compiled for their z columns alone
+#define ERM_ZSWITCH(K, CALL)                   \
+  switch (K) {                                 \
+    case 18: { constexpr int KK = 18; CALL; } break; \
+    case 20: { constexpr int KK = 20; CALL; } break; \
+    case 25: { constexpr int KK = 25; CALL; } break; \
+    case 27: { constexpr int KK = 27; CALL; } break; \
+    case 30: { constexpr int KK = 30; CALL; } break; \
+    case 36: { constexpr int KK = 36; CALL; } break; \
+    case 40: { constexpr int KK = 40; CALL; } break; \
+    case 45: { constexpr int KK = 45; CALL; } break; \
+    case 50: { constexpr int KK = 50; CALL; } break; \
+    case 54: { constexpr int KK = 54; CALL; } break; \
+    case 60: { constexpr int KK = 60; CALL; } break; \
+    case 72: { constexpr int KK = 72; CALL; } break; \
+    case 75: { constexpr int KK = 75; CALL; } break; \
+    case 80: { constexpr int KK = 80; CALL; } break; \
+    case 81: { constexpr int KK = 81; CALL; } break; \
+    case 90: { constexpr int KK = 90; CALL; } break; \
+    case 100: { constexpr int KK = 100; CALL; } break; \
+    default: break;                            \
+  }
+
+// Kernel of the z columns.  Z_SPEC sums the solute's z spectra (register
+// lengths, spline orders without a z FFT kernel), Z_FFT and Z_FFT256 spread
+// and transform a column in registers (orders 4 and 6; the tuned workgroup
+// size, or 256 threads for the lengths with z columns alone), Z_TWO is the
+// two-step kernel, Z_LDS the general one.  The registers win where a column
+// leaves room for two waves per SIMD: 1000 FP32 configurations of 48^3 0.138
+// against 0.250 ms in two steps, FP64 0.335 against 0.416; a 64-point FP64
+// column does not (500 configurations of 64^3, order 6: 0.751 against 0.475).
+// 701 FP32 configurations of 45 x 60 x 75: 0.236 in registers, 0.618 in two
+// steps.
+enum ZKernel { Z_SPEC, Z_FFT, Z_FFT256, Z_TWO, Z_LDS };
+ZKernel z_kernel(const erm_ctx *c, bool regp) {
+  const int K3 = c->kp.K3;
+  const bool p46 = c->kp.p == 4 || c->kp.p == 6;
+  const bool reg = p46 && (c->fp32 ? reg_len<float>(K3) : reg_len<double>(K3) && K3 < 64);
+  if (regp) return !p46 ? Z_SPEC : reg ? Z_FFT : Z_TWO;
+  if (!c->two_step) return Z_LDS;
+  if (reg) return Z_FFT;
+  bool z32 = false;
+  if (c->fp32 && p46) ERM_ZSWITCH(K3, z32 = KK > 0)
+  return z32 ? Z_FFT256 : Z_TWO;
+}
 // z-column workgroups per configuration
 int zcol_groups(const erm_ctx *c, bool regp, int vb) {
   const int ncol = c->kp.H * c->kp.K2;
-  if (c->two_step) {
-    const int w = (vb == (int)sizeof(double2)) ? z2_cols<double> : z2_cols<float>;
-    return (ncol + w - 1) / w;
-  }
-  if (!regp) {
+  const ZKernel zk = z_kernel(c, regp);
+  if (zk == Z_TWO) return (ncol + Z2_COLS - 1) / Z2_COLS;
+  if (zk == Z_LDS) {
     const int w = zcol_width(c->kp.K3, vb);
     return (ncol + w - 1) / w;
   }
-  const int zt = (c->zcol_T == 512) ? 512 : NTHR;
+  const int zt = (c->zcol_T == 512 && zk != Z_FFT256) ? 512 : NTHR;
   // lanes per column: the spectral form one, the spread-and-FFT form
   // zfft_lanes (vb = 2 sizeof(T))
-  const int L = zcol_fft(c, regp) ? zfft_lanes(vb / 2, c->kp.K3) : 1;
+  const int L = zk == Z_SPEC ? 1 : zfft_lanes(vb / 2, c->kp.K3);
   return (L * ncol + zt - 1) / zt;
 }
 
@@ -598,15 +638,18 @@ template <typename T> Xy2Shape xy2_shape(const erm_ctx *c, int n) {
 // The two-step PME kernels over n configurations, solute sites from site0 of
 // the batch buffers: z columns into d_Hk, then the y and x transforms and the
 // gather into d_esite.
-template <typename T> int launch_zcol2(erm_ctx *c, const Params &k, int n, int nblk) {
+template <typename T>
+int launch_zcol2(erm_ctx *c, const Params &k, int n, int nblk, size_t site0 = 0, size_t cfg0 = 0) {
   using V = typename C2<T>::type;
   Fft2 f;
   if (!fft2_split<T>(k.K3, f)) return fail(c, ERM_E_ENG_BUG, "two-step z length");
   const size_t lds = z2_lds<T>(k.K3, k.p);
-  TRY(set_lds(c, (const void *)k_pme_zcol2<T>, lds, "k_pme_zcol2"));
-  hipLaunchKernelGGL(k_pme_zcol2<T>, dim3(nblk, n), dim3(Z2_THR), lds, c->st, k, f.A, f.B, dp<T>(c->d_engfac),
-                     dp<int>(c->d_sg3), dp<T>(c->d_sw3), dp<T>(c->d_sqv), dp<V>(c->d_w1h), dp<V>(c->d_w2h),
-                     dp<V>(c->d_tw3), dp<V>(c->d_Hk), dp<double>(c->d_selfp));
+  auto *kz = f.B <= 10 ? k_pme_zcol2<T, 10> : k_pme_zcol2<T, fft2_bmax<T>>;
+  TRY(set_lds(c, (const void *)kz, lds, "k_pme_zcol2"));
+  hipLaunchKernelGGL(kz, dim3(nblk, n), dim3(z2_threads(f.B)), lds, c->st, k, f.A, f.B, dp<T>(c->d_engfac),
+                     dp<int>(c->d_sg3) + site0, dp<T>(c->d_sw3) + site0 * k.p, dp<T>(c->d_sqv) + site0,
+                     dp<V>(c->d_w1h) + site0 * k.H, dp<V>(c->d_w2h) + site0 * k.K2, dp<V>(c->d_tw3),
+                     dp<V>(c->d_Hk) + cfg0 * k.K3 * (size_t)k.K2 * k.H, dp<double>(c->d_selfp) + cfg0 * nblk);
   return launch_check(c, "k_pme_zcol2");
 }
 template <typename T> int launch_xyslab(erm_ctx *c, const Params &k, int n) {
@@ -982,8 +1025,9 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
   TRY(ensure(c, c->d_w1h, sizeof(V) * (size_t)n * ns * H));
   TRY(ensure(c, c->d_w2h, sizeof(V) * (size_t)n * ns * K2));
   const bool regp = (flags & DO_RECIP) && c->xslab_Q > 0 && (c->P.pme_path == 0 || c->P.pme_path == 3);
-  const bool zfft = zcol_fft(c, regp);  // else the preparation writes the z spectra
-  if (regp && !zfft) TRY(ensure(c, c->d_w3h, sizeof(V) * (size_t)n * ns * K3));
+  const ZKernel zk = z_kernel(c, regp);
+  const bool zspec = (flags & DO_RECIP) && zk == Z_SPEC;  // the preparation writes the z spectra
+  if (zspec) TRY(ensure(c, c->d_w3h, sizeof(V) * (size_t)n * ns * K3));
   TRY(ensure(c, c->d_uv, sizeof(double) * (size_t)n * (S + 1)));
   TRY(ensure(c, c->d_sltj, sizeof(int) * n));
   TRY(ensure(c, c->d_selfreal, sizeof(double) * n));
@@ -1000,31 +1044,25 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
                      dp<double>(c->d_spos),
                      dp<double>(c->d_qslt), dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<V>(c->d_tw3),
                      dp<double>(c->d_sref), dp<int>(c->d_sg3), dp<T>(c->d_sw3), dp<T>(c->d_sqv),
-                     dp<V>(c->d_w1h), dp<V>(c->d_w2h), (regp && !zfft) ? dp<V>(c->d_w3h) : (V *)nullptr);
+                     dp<V>(c->d_w1h), dp<V>(c->d_w2h), zspec ? dp<V>(c->d_w3h) : (V *)nullptr);
   TRY(launch_check(c, "k_solute_prep"));
   TRY(mark(c, 1));
-  if (regp) {
+  if ((flags & DO_RECIP) && zk != Z_LDS) {
     int rz = ERM_E_UNSUPPORTED;
-    if (zfft) {
-      ERM_KSWITCH(K3, (rz = launch_zcol_fft<T, KK>(c, k, n, nzg)));
-    } else {
+    if (zk == Z_TWO) {
+      rz = launch_zcol2<T>(c, k, n, nzg);
+    } else if (zk == Z_SPEC) {
       ERM_KSWITCH(K3, (rz = launch_zcol_reg<T, KK>(c, k, n, nzg)));
+    } else if (zk == Z_FFT) {
+      ERM_KSWITCH(K3, (rz = launch_zcol_fft<T, KK>(c, k, n, nzg)));
+    } else if constexpr (sizeof(T) == 4) {
+      ERM_ZSWITCH(K3, (rz = launch_zcol_fft256<T, KK>(c, k, n, nzg)));
     }
     TRY(rz);
-    TRY(launch_check(c, zfft ? "k_pme_zcol_fft" : "k_pme_zcol_reg"));
+    TRY(launch_check(c, "z columns"));
     TRY(mark(c, 2));
     TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
     TRY(mark(c, 3));
-    TRY(launch_xyslab<T>(c, k, n));
-    TRY(mark(c, 4));
-    Params kg = k;
-    if (!(flags & DO_RESIDUAL)) kg.solute_charge = 0.0;
-    TRY(launch_mol_sum(c, kg, n, dp<double>(c->d_esite), dp<int>(c->d_sltj), dp<double>(c->d_uv)));
-  } else if ((flags & DO_RECIP) && c->two_step) {
-    TRY(launch_zcol2<T>(c, k, n, nzg));
-    TRY(mark(c, 2));
-    TRY(mark(c, 3));
-    TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
     TRY(launch_xyslab<T>(c, k, n));
     TRY(mark(c, 4));
     Params kg = k;
@@ -1705,7 +1743,8 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
   hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(32), 0, c->st, dp<int>(g->d_counter), (size_t)4, 0);
   TRY(launch_check(c, "k_fill"));
   // z columns over every run: one persistent launch, or one launch per run
-  if (g->persistent & 1) {
+  const ZKernel zk = z_kernel(c, true);
+  if (zk == Z_FFT && (g->persistent & 1)) {
     int rz = ERM_E_UNSUPPORTED;
     ERM_KSWITCH(K3, (rz = launch_zcol_fft_runs<T, KK>(c, k, nzg, d_runs, nrun, nitem_z, dp<int>(g->d_counter))));
     TRY(rz);
@@ -1715,9 +1754,13 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
       Params kr = k;
       kr.ns = R[r].ns;
       int rz = ERM_E_UNSUPPORTED;
-      ERM_KSWITCH(K3, (rz = launch_zcol_fft<T, KK>(c, kr, R[r].ncfg, nzg, (size_t)R[r].site0, (size_t)R[r].cfg0)));
+      if (zk == Z_TWO) {
+        rz = launch_zcol2<T>(c, kr, R[r].ncfg, nzg, (size_t)R[r].site0, (size_t)R[r].cfg0);
+      } else {
+        ERM_KSWITCH(K3, (rz = launch_zcol_fft<T, KK>(c, kr, R[r].ncfg, nzg, (size_t)R[r].site0, (size_t)R[r].cfg0)));
+      }
       TRY(rz);
-      TRY(launch_check(c, "k_pme_zcol_fft"));
+      TRY(launch_check(c, "z columns"));
     }
   }
   TRY(mark(c, 2));
@@ -2625,7 +2668,7 @@ int32_t erm_group_insert_random(erm_group *g, const int32_t *n, const uint64_t *
     return gfail(g, ERM_E_ARG, "erm_group_set_frame has not been called for the current frame");
   for (int i = 0; i < nm; ++i)
     if (n[i] < 0) return gfail(g, ERM_E_ARG, "negative count for member %d", i);
-  const bool ok_path = (c->fp32 ? reg_path_ok<float>(c) : reg_path_ok<double>(c)) && zcol_fft(c, true) &&
+  const bool ok_path = (c->fp32 ? reg_path_ok<float>(c) : reg_path_ok<double>(c)) && (c->kp.p == 4 || c->kp.p == 6) &&
                        c->xslab_Q > 0 && (c->P.pme_path == 0 || c->P.pme_path == 3);
   if (!ok_path) return gfail(g, ERM_E_UNSUPPORTED, "groups need the register PME path with spline order 4 or 6");
   for (int i = 0; i < NSTAGE_OUT; ++i) g->stage_ms[i] = 0;

@@ -13,9 +13,12 @@ struct Fft2 {
   int A, B;
 };
 
-// K = A B with A <= B, both with a case in ERM_RADIX_A / _B below (T in
-// scope): in FP64 B stops at 12, where a step's values still fit 128
-// registers beside their addresses
+// the largest B: in FP64 12, where a step's values still fit 128 registers
+// beside their addresses
+template <typename T> constexpr int fft2_bmax = sizeof(T) == 4 ? 16 : 12;
+
+// K = A B with A <= B, both with a case in ERM_RADIX_A / _B below (B <= BMAX,
+// a constant in scope)
 template <typename T> inline bool fft2_split(int K, Fft2 &f) {
   static const int tab[][3] = {{16, 4, 4},  {18, 3, 6},  {20, 4, 5},   {24, 4, 6},   {25, 5, 5},   {27, 3, 9},
                                {30, 5, 6},  {32, 4, 8},  {36, 6, 6},   {40, 5, 8},   {45, 5, 9},   {48, 6, 8},
@@ -23,7 +26,7 @@ template <typename T> inline bool fft2_split(int K, Fft2 &f) {
                                {80, 8, 10}, {81, 9, 9},  {90, 9, 10},  {96, 8, 12},  {100, 10, 10}, {108, 9, 12},
                                {120, 10, 12}, {128, 8, 16}};
   for (const auto &t : tab)
-    if (t[0] == K && (sizeof(T) == 4 || t[2] <= 12)) {
+    if (t[0] == K && t[2] <= fft2_bmax<T>) {
       f.A = t[1];
       f.B = t[2];
       return true;
@@ -50,9 +53,9 @@ template <typename T> inline bool fft2_split(int K, Fft2 &f) {
     case 8: { constexpr int RR = 8; CALL; } break;    \
     case 9: { constexpr int RR = 9; CALL; } break;    \
     case 10: { constexpr int RR = 10; CALL; } break;  \
-    case 12: { constexpr int RR = 12; CALL; } break;  \
-    case 15: if constexpr (sizeof(T) == 4) { constexpr int RR = 15; CALL; } break; \
-    case 16: if constexpr (sizeof(T) == 4) { constexpr int RR = 16; CALL; } break; \
+    case 12: if constexpr (BMAX >= 12) { constexpr int RR = 12; CALL; } break; \
+    case 15: if constexpr (BMAX >= 15) { constexpr int RR = 15; CALL; } break; \
+    case 16: if constexpr (BMAX >= 16) { constexpr int RR = 16; CALL; } break; \
     default: break;                                   \
   }
 
@@ -67,49 +70,123 @@ template <typename V> __device__ __forceinline__ V cmulc(V a, V w) {
 // --------------------------------------------------------------------------
 // z columns.  A workgroup takes C consecutive columns (m1, m2) of one
 // configuration: the solute's sites, in chunks of Z2_SCH in plane order, are
-// added to the columns in LDS (buf[z][column], each plane over the sites
-// whose p planes hold it), transformed forward, multiplied by the Green's
-// function (self energy on the way, recpcal.F90:385-394), transformed back
-// and written to Hk.  The Green's function meets the second forward step's
-// registers, and the first inverse step runs on the same registers, so the
-// column makes six trips through LDS and none through memory but its write.
-// Bound by those trips and the spread.  500 FP64 columns sets of 40 x 40 x 80
-// with 20 solute sites: 0.38 ms, where the stages of 2 to 5 points through LDS
-// (k_pme_zcol) took 2.38 ms; 701 FP32 sets of 45 x 60 x 75 with 33 sites
-// 0.85 against 6.14 ms.
+// added to the columns (each plane over the sites whose p planes hold it),
+// transformed forward, multiplied by the Green's function (self energy on the
+// way, recpcal.F90:385-394), transformed back and written to Hk.  The spread
+// leaves the values in the registers of the first forward step, and the
+// Green's function meets those of the second, which run the first inverse
+// step as well: a column makes four trips through LDS and none through memory
+// but its write.
+// Bound by the latency of its four phases and the spread; a workgroup's threads
+// take one first step each.  500 FP64 configurations of 40 x 40 x 80 with 20
+// solute sites: 0.25 ms (2.2 TB/s of spectrum written), where the stages of 2
+// to 5 points through LDS (k_pme_zcol) took 2.38 ms and 32 columns spread in
+// LDS 0.35; one of 96^3 with 300 sites, order 6: 0.26 -> 0.053 ms.
 // --------------------------------------------------------------------------
-constexpr int Z2_SCH = 32;   // solute sites per chunk
-constexpr int Z2_THR = 256;
-template <typename T> constexpr int z2_cols = sizeof(T) == 8 ? 16 : 32;  // columns per workgroup
+constexpr int Z2_SCH = 64;   // solute sites per chunk
+constexpr int Z2_COLS = 16;  // columns per workgroup: 128 or 256 contiguous bytes of a plane
+// threads: one per column and value of n1 (whole waves), so every thread
+// takes one first step and those with k2 < A one second step
+inline int z2_threads(int B) { return (Z2_COLS * B + 63) & ~63; }
+constexpr int Z2_MAXT = 256;
 
+// (the columns take the place of the last chunk's amplitudes)
 template <typename T> __host__ __device__ inline size_t z2_lds(int K3, int p) {
-  constexpr int C = z2_cols<T>;
-  return sizeof(T) * 2 * ((size_t)K3 * C + (size_t)Z2_SCH * C + K3) + sizeof(T) * (size_t)Z2_SCH * p +
-         sizeof(int) * (Z2_SCH + (size_t)K3 + 1) + sizeof(double) * Z2_THR + 32;
+  const size_t buf = 2 * sizeof(T) * (size_t)K3 * Z2_COLS;
+  const size_t chunk = 2 * sizeof(T) * (size_t)Z2_SCH * Z2_COLS + sizeof(T) * (size_t)Z2_SCH * p +
+                       sizeof(int) * (Z2_SCH + (size_t)K3 + 1);
+  return (((buf > chunk ? buf : chunk) + 15) & ~(size_t)15) + 2 * sizeof(T) * K3 + sizeof(double) * (Z2_MAXT / 64);
 }
 
-// first forward step of (n1, column): in place
+struct Z2Args {
+  int ns, p, K2, K3, H, m1, m2, cl, sub, nsub;
+  bool on;
+};
+
+// Spread and first forward step of (n1 = sub, column): the thread's A planes
+// n1 + B i are summed over the sites whose p planes hold them, chunk by
+// chunk, in registers, transformed and written to the column.
 template <typename T, int A>
-__device__ __forceinline__ void z2_first(typename C2<T>::type *col, int B, int n1,
-                                         const typename C2<T>::type *__restrict__ tw) {
+__device__ __forceinline__ void z2_front(const Z2Args &q, int B, unsigned char *lds,
+                                         const typename C2<T>::type *tw, const int *__restrict__ sg3,
+                                         const T *__restrict__ sw3, const T *__restrict__ sqv,
+                                         const typename C2<T>::type *__restrict__ w1h,
+                                         const typename C2<T>::type *__restrict__ w2h) {
   using V = typename C2<T>::type;
-  constexpr int C = z2_cols<T>;
+  constexpr int C = Z2_COLS;
+  const int p = q.p, K3 = q.K3;
+  V *amp = reinterpret_cast<V *>(lds);                       // [Z2_SCH][C] q what1 what2 of the chunk's sites
+  T *wz = reinterpret_cast<T *>(amp + (size_t)Z2_SCH * C);   // [Z2_SCH][p] z weights
+  int *gz = reinterpret_cast<int *>(wz + (size_t)Z2_SCH * p);  // [Z2_SCH] planes g3, ascending
+  int *first = gz + Z2_SCH;                                  // [K3 + 1] first site of the chunk with g3 >= z
   V x[A];
 #pragma unroll
-  for (int i = 0; i < A; ++i) x[i] = col[(n1 + B * i) * C];
-  reg_fft<A, -1>(x);
-  col[n1 * C] = x[0];
+  for (int i = 0; i < A; ++i) {
+    x[i].x = 0;
+    x[i].y = 0;
+  }
+  for (int s0 = 0; s0 < q.ns; s0 += Z2_SCH) {
+    const int nc = min(Z2_SCH, q.ns - s0);
+    if (s0) __syncthreads();  // the previous chunk's sites are used up
+    // site j opens the planes (g3 of j - 1, g3 of j], the last site also
+    // those above it
+    if (threadIdx.x < (unsigned)nc) {
+      const int j = threadIdx.x, g = sg3[s0 + j], g0 = j ? sg3[s0 + j - 1] : -1;
+      gz[j] = g;
+      for (int z = g0 + 1; z <= g; ++z) first[z] = j;
+      if (j == nc - 1)
+        for (int z = g + 1; z <= K3; ++z) first[z] = nc;
+    }
+    for (int t = threadIdx.x; t < nc * p; t += blockDim.x) wz[t] = sw3[(size_t)s0 * p + t];
+    for (int j = q.sub; j < nc; j += q.nsub) {
+      const size_t s = (size_t)s0 + j;
+      V a = cmul(w1h[s * q.H + q.m1], w2h[s * q.K2 + q.m2]);
+      const T c = q.on ? sqv[s] : (T)0;
+      a.x *= c;
+      a.y *= c;
+      amp[j * C + q.cl] = a;
+    }
+    __syncthreads();
+    if (q.sub < B) {
 #pragma unroll
-  for (int k = 1; k < A; ++k) col[(n1 + B * k) * C] = cmul(x[k], tw[n1 * k]);
+      for (int i = 0; i < A; ++i) {
+        // plane z holds the sites with g3 - z in [0, p) (mod K3)
+        int z = q.sub + B * i;
+        asm volatile("" : "+v"(z));  // the planes' addresses are formed one plane at a time
+        const int zt = z + p;
+        for (int j = first[z]; j < first[min(zt, K3)]; ++j) {
+          const V a = amp[j * C + q.cl];
+          const T w = wz[j * p + gz[j] - z];
+          x[i].x += a.x * w;
+          x[i].y += a.y * w;
+        }
+        if (zt > K3)  // planes wrapped past the top
+          for (int j = 0; j < first[zt - K3]; ++j) {
+            const V a = amp[j * C + q.cl];
+            const T w = wz[j * p + gz[j] + K3 - z];
+            x[i].x += a.x * w;
+            x[i].y += a.y * w;
+          }
+      }
+    }
+  }
+  __syncthreads();
+  if (q.sub < B) {
+    V *col = reinterpret_cast<V *>(lds) + q.cl;
+    reg_fft<A, -1>(x);
+    col[q.sub * C] = x[0];
+#pragma unroll
+    for (int k = 1; k < A; ++k) col[(q.sub + B * k) * C] = cmul(x[k], tw[q.sub * k]);
+  }
 }
 
 // second forward step of (k2, column), Green's function, first inverse step:
 // in place; returns the column's share of the self energy (weight 1)
 template <typename T, int B>
 __device__ __forceinline__ double z2_mid(typename C2<T>::type *col, int A, int k2, const T *__restrict__ g,
-                                         size_t gstr, const typename C2<T>::type *__restrict__ tw) {
+                                         size_t gstr, const typename C2<T>::type *tw) {
   using V = typename C2<T>::type;
-  constexpr int C = z2_cols<T>;
+  constexpr int C = Z2_COLS;
   T gv[B];
 #pragma unroll
   for (int k = 0; k < B; ++k) gv[k] = g[(size_t)(k2 + A * k) * gstr];
@@ -136,7 +213,7 @@ template <typename T, int A>
 __device__ __forceinline__ void z2_last(const typename C2<T>::type *col, int B, int n1, typename C2<T>::type *out,
                                         size_t ostr) {
   using V = typename C2<T>::type;
-  constexpr int C = z2_cols<T>;
+  constexpr int C = Z2_COLS;
   V x[A];
 #pragma unroll
   for (int k = 0; k < A; ++k) x[k] = col[(n1 + B * k) * C];
@@ -145,107 +222,57 @@ __device__ __forceinline__ void z2_last(const typename C2<T>::type *col, int B, 
   for (int i = 0; i < A; ++i) out[(size_t)(n1 + B * i) * ostr] = x[i];
 }
 
-template <typename T>
-__global__ __launch_bounds__(Z2_THR) void k_pme_zcol2(Params P, int A, int B, const T *__restrict__ engfac,
-                                                      const int *__restrict__ sg3, const T *__restrict__ sw3,
-                                                      const T *__restrict__ sqv,
-                                                      const typename C2<T>::type *__restrict__ w1h,
-                                                      const typename C2<T>::type *__restrict__ w2h,
-                                                      const typename C2<T>::type *__restrict__ tw3,
-                                                      typename C2<T>::type *Hk, double *selfp) {
+template <typename T, int BMAX>
+__global__ __launch_bounds__(Z2_MAXT) void k_pme_zcol2(Params P, int A, int B, const T *__restrict__ engfac,
+                                                       const int *__restrict__ sg3, const T *__restrict__ sw3,
+                                                       const T *__restrict__ sqv,
+                                                       const typename C2<T>::type *__restrict__ w1h,
+                                                       const typename C2<T>::type *__restrict__ w2h,
+                                                       const typename C2<T>::type *__restrict__ tw3,
+                                                       typename C2<T>::type *Hk, double *selfp) {
   using V = typename C2<T>::type;
-  constexpr int C = z2_cols<T>;
+  constexpr int C = Z2_COLS;
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  const int b = blockIdx.y, ns = P.ns, p = P.p, K2 = P.K2, K3 = P.K3, H = P.H;
-  V *buf = reinterpret_cast<V *>(lds_raw);       // [K3][C]
-  V *amp = buf + (size_t)K3 * C;                 // [Z2_SCH][C] q what1 what2 of the chunk's sites
-  V *tw = amp + (size_t)Z2_SCH * C;              // [K3]
-  double *red = reinterpret_cast<double *>(tw + K3);  // [Z2_THR]
-  T *wz = reinterpret_cast<T *>(red + Z2_THR);   // [Z2_SCH][p] z weights
-  int *gz = reinterpret_cast<int *>(wz + (size_t)Z2_SCH * p);  // [Z2_SCH] planes g3, ascending
-  int *first = gz + Z2_SCH;                      // [K3 + 1] first site of the chunk with g3 >= z
-  const int cl = threadIdx.x % C, sub = threadIdx.x / C;
-  constexpr int NSUB = Z2_THR / C;
-  const int ncol = H * K2, c = blockIdx.x * C + cl;
-  const bool on = c < ncol;
-  const int m2 = on ? c / H : 0, m1 = on ? c - m2 * H : 0;
-  for (int t = threadIdx.x; t < K3; t += Z2_THR) tw[t] = tw3[t];
-  for (int s0 = 0; s0 < ns; s0 += Z2_SCH) {
-    const int nc = min(Z2_SCH, ns - s0);
-    const size_t bs = (size_t)b * ns + s0;
-    __syncthreads();  // the previous chunk's sites are used up
-    // site j opens the planes (g3 of j - 1, g3 of j], the last site also
-    // those above it
-    if (threadIdx.x < (unsigned)nc) {
-      const int j = threadIdx.x, g = sg3[bs + j], g0 = j ? sg3[bs + j - 1] : -1;
-      gz[j] = g;
-      for (int z = g0 + 1; z <= g; ++z) first[z] = j;
-      if (j == nc - 1)
-        for (int z = g + 1; z <= K3; ++z) first[z] = nc;
-    }
-    for (int t = threadIdx.x; t < nc * p; t += Z2_THR) wz[t] = sw3[bs * p + t];
-    for (int j = sub; j < nc; j += NSUB) {
-      const size_t s = bs + j;
-      V a;
-      a.x = 0;
-      a.y = 0;
-      if (on) {
-        a = cmul(w1h[s * H + m1], w2h[s * K2 + m2]);
-        const T q = sqv[s];
-        a.x *= q;
-        a.y *= q;
-      }
-      amp[j * C + cl] = a;
-    }
-    __syncthreads();
-    // plane z holds the sites with g3 - z in [0, p) (mod K3)
-    for (int z = sub; z < K3; z += NSUB) {
-      V acc;
-      acc.x = 0;
-      acc.y = 0;
-      if (s0) acc = buf[z * C + cl];
-      for (int j = first[z]; j < first[min(z + p, K3)]; ++j) {
-        const V a = amp[j * C + cl];
-        const T w = wz[j * p + gz[j] - z];
-        acc.x += a.x * w;
-        acc.y += a.y * w;
-      }
-      if (z + p > K3)  // planes wrapped past the top
-        for (int j = 0; j < first[z + p - K3]; ++j) {
-          const V a = amp[j * C + cl];
-          const T w = wz[j * p + gz[j] + K3 - z];
-          acc.x += a.x * w;
-          acc.y += a.y * w;
-        }
-      buf[z * C + cl] = acc;
-    }
-  }
-  __syncthreads();
-  for (int n1 = sub; n1 < B; n1 += NSUB) {
-    asm volatile("" : "+v"(n1));  // no radix's addresses are hoisted out of the loop
-    ERM_RADIX_A(A, (z2_first<T, RR>(buf + cl, B, n1, tw)))
-  }
+  const int b = blockIdx.y, K3 = P.K3;
+  V *buf = reinterpret_cast<V *>(lds_raw);       // [K3][C], after the last chunk
+  double *red = reinterpret_cast<double *>(lds_raw + z2_lds<T>(K3, P.p) - sizeof(double) * (Z2_MAXT / 64));
+  V *tw = reinterpret_cast<V *>(red) - K3;       // [K3]
+  Z2Args q;
+  q.ns = P.ns;
+  q.p = P.p;
+  q.K2 = P.K2;
+  q.K3 = K3;
+  q.H = P.H;
+  q.cl = threadIdx.x % C;
+  q.sub = threadIdx.x / C;
+  q.nsub = blockDim.x / C;
+  const int ncol = P.H * P.K2, c = blockIdx.x * C + q.cl;
+  q.on = c < ncol;
+  q.m2 = q.on ? c / P.H : 0;
+  q.m1 = q.on ? c - q.m2 * P.H : 0;
+  for (int t = threadIdx.x; t < K3; t += blockDim.x) tw[t] = tw3[t];
+  const size_t bs = (size_t)b * q.ns;
+  ERM_RADIX_A(A, (z2_front<T, RR>(q, B, lds_raw, tw, sg3 + bs, sw3 + bs * q.p, sqv + bs, w1h + bs * q.H,
+                                  w2h + bs * q.K2)))
   __syncthreads();
   double self = 0.0;
-  const T *g = engfac + (size_t)m2 * H + m1;
-  for (int k2 = sub; k2 < A; k2 += NSUB) {
-    asm volatile("" : "+v"(k2));  // no radix's addresses are hoisted out of the loop
-    ERM_RADIX_B(B, (self += z2_mid<T, RR>(buf + cl, A, k2, g, (size_t)ncol, tw)))
+  if (q.sub < A) {
+    const T *g = engfac + (size_t)q.m2 * q.H + q.m1;
+    ERM_RADIX_B(B, (self = z2_mid<T, RR>(buf + q.cl, A, q.sub, g, (size_t)ncol, tw)))
   }
-  red[threadIdx.x] = on ? ((m1 == 0 || 2 * m1 == P.K1) ? 0.5 : 1.0) * self : 0.0;
+  self = q.on ? ((q.m1 == 0 || 2 * q.m1 == P.K1) ? 0.5 : 1.0) * self : 0.0;
+  for (int o = 32; o > 0; o >>= 1) self += __shfl_xor(self, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = self;
   __syncthreads();
-  if (on) {
+  if (threadIdx.x == 0) {
+    double sum = red[0];
+    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) sum += red[w];
+    selfp[(size_t)b * gridDim.x + blockIdx.x] = sum;
+  }
+  if (q.on && q.sub < B) {
     V *out = Hk + (size_t)b * K3 * ncol + c;
-    for (int n1 = sub; n1 < B; n1 += NSUB) {
-    asm volatile("" : "+v"(n1));  // no radix's addresses are hoisted out of the loop
-      ERM_RADIX_A(A, (z2_last<T, RR>(buf + cl, B, n1, out, (size_t)ncol)))
-    }
+    ERM_RADIX_A(A, (z2_last<T, RR>(buf + q.cl, B, q.sub, out, (size_t)ncol)))
   }
-  for (int s = Z2_THR / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) selfp[(size_t)b * gridDim.x + blockIdx.x] = red[0];
 }
 
 // --------------------------------------------------------------------------
@@ -467,6 +494,7 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int K1 = P.K1, K2 = P.K2, K3 = P.K3, H = P.H, p = P.p;
   const int rs = xy2_row(K1, p), plane = xy2_plane(K2, rs);
+  constexpr int BMAX = fft2_bmax<T>;
   V *stage = reinterpret_cast<V *>(lds_raw);   // [Q][plane]
   V *twy = stage + (size_t)Q * plane;          // [K2]
   V *twx = twy + K2;                           // [K1]

@@ -1006,11 +1006,12 @@ __device__ __forceinline__ void zspread_half(V (&Y)[K3 / 2], const V a, const T 
 // (128 in FP32: the 150-site solutes take two chunks, and three
 // 256-thread workgroups still fit a CU's LDS)
 template <typename T> constexpr int zfft_sch = sizeof(T) == 4 ? 128 : 64;
-constexpr int ZFFT_KMAX = 96;  // largest z grid length of the register kernels
+constexpr int ZFFT_KMAX = 100;  // largest z grid length of the register kernels
 
-// lanes per z column in k_pme_zcol_fft: one in FP32 up to K3 = 64 (the
-// whole column, 2 K3 floats, in one lane's registers), else a lane pair
-__host__ __device__ constexpr int zfft_lanes(int tbytes, int K3) { return (tbytes == 4 && K3 <= 64) ? 1 : 2; }
+// lanes per z column in k_pme_zcol_fft: one in FP32 up to K3 = 81 (the
+// whole column, 2 K3 floats, in one lane's registers; 238 of them at 81), else
+// a lane pair
+__host__ __device__ constexpr int zfft_lanes(int tbytes, int K3) { return (tbytes == 4 && K3 <= 81) ? 1 : 2; }
 
 // m2 rows a workgroup of XT threads (XT / L columns, m1 fastest) touches
 __host__ __device__ inline int zcol_fft_rows(int H, int K2, int XT, int L = 2) {
@@ -1060,7 +1061,7 @@ __device__ __forceinline__ void zcol_stage_chunk(int s0, int nc, int K3, int H, 
   __syncthreads();
 }
 
-// One lane per column (m1, m2) (FP32, K3 <= 64): the same spread, Green's
+// One lane per column (m1, m2) (FP32, K3 <= 81): the same spread, Green's
 // function and transforms as the lane-pair form below, with the whole column
 // in one lane's registers in plane order.  Every site adds to its PP planes
 // directly (no lane masks), the forward and inverse z FFTs are one K3-point
@@ -1168,17 +1169,12 @@ __device__ __forceinline__ void zcol_fft_body1(const Params &P, int ns, int blk,
 // the configuration's first site, Hk at its spectrum); the block's
 // self-energy sum goes to *self_out.  All threads of the workgroup call it.
 template <typename T, int K3, int PP, int XT>
-__device__ __forceinline__ void zcol_fft_body(const Params &P, int ns, int blk, const T *__restrict__ engfac,
-                                              const T *__restrict__ sqv,
-                                              const typename C2<T>::type *__restrict__ w1h,
-                                              const typename C2<T>::type *__restrict__ w2h,
-                                              const int *__restrict__ sg3, const T *__restrict__ sw3,
-                                              typename C2<T>::type *Hk, double *self_out) {
-  static_assert(K3 <= ZFFT_KMAX, "z grid length");
-  if constexpr (zfft_lanes(sizeof(T), K3) == 1) {
-    zcol_fft_body1<T, K3, PP, XT>(P, ns, blk, engfac, sqv, w1h, w2h, sg3, sw3, Hk, self_out);
-    return;
-  }
+__device__ __forceinline__ void zcol_fft_body2(const Params &P, int ns, int blk, const T *__restrict__ engfac,
+                                               const T *__restrict__ sqv,
+                                               const typename C2<T>::type *__restrict__ w1h,
+                                               const typename C2<T>::type *__restrict__ w2h,
+                                               const int *__restrict__ sg3, const T *__restrict__ sw3,
+                                               typename C2<T>::type *Hk, double *self_out) {
   using V = typename C2<T>::type;
   constexpr int HK = K3 / 2;
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -1277,8 +1273,23 @@ __device__ __forceinline__ void zcol_fft_body(const Params &P, int ns, int blk, 
   }
 }
 
+template <typename T, int K3, int PP, int XT>
+__device__ __forceinline__ void zcol_fft_body(const Params &P, int ns, int blk, const T *__restrict__ engfac,
+                                              const T *__restrict__ sqv,
+                                              const typename C2<T>::type *__restrict__ w1h,
+                                              const typename C2<T>::type *__restrict__ w2h,
+                                              const int *__restrict__ sg3, const T *__restrict__ sw3,
+                                              typename C2<T>::type *Hk, double *self_out) {
+  static_assert(K3 <= ZFFT_KMAX, "z grid length");
+  if constexpr (zfft_lanes(sizeof(T), K3) == 1)
+    zcol_fft_body1<T, K3, PP, XT>(P, ns, blk, engfac, sqv, w1h, w2h, sg3, sw3, Hk, self_out);
+  else
+    zcol_fft_body2<T, K3, PP, XT>(P, ns, blk, engfac, sqv, w1h, w2h, sg3, sw3, Hk, self_out);
+}
+
+// (two waves per SIMD: 256 registers)
 template <typename T, int K3, int PP, int XT = NTHR>
-__global__ __launch_bounds__(XT) void k_pme_zcol_fft(Params P, const T *__restrict__ engfac,
+__global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(2))) void k_pme_zcol_fft(Params P, const T *__restrict__ engfac,
                                                        const T *__restrict__ sqv,
                                                        const typename C2<T>::type *__restrict__ w1h,
                                                        const typename C2<T>::type *__restrict__ w2h,

@@ -961,7 +961,8 @@ template <typename T> int launch_pair(erm_ctx *c, const Params &k, int n, bool b
       TRY(launch_check(c, "k_fill"));
     }
     const size_t lp = pair_tile_lds<T>(ps.nss, c->nvt, segcap, nwave);
-    auto *f = bare ? k_pair_tile<T, true> : k_pair_tile<T, false>;
+    auto *f = bare ? k_pair_tile<T, true, false>
+                   : k.ljswitch == 0 ? k_pair_tile<T, false, true> : k_pair_tile<T, false, false>;
     TRY(set_lds(c, (const void *)f, lp, "k_pair_tile"));
     hipLaunchKernelGGL(f, dim3(n, ps.nsplit, ps.parts), dim3(NTHR), lp, c->st, k, ps.cm, ps.nss, nuv,
                        dp<double>(c->d_spos), dp<double>(c->d_sref), dp<T>(c->d_qslt_t), dp<T>(c->d_sltlj),
@@ -1783,7 +1784,8 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
     const size_t lt = pair_tile_lds<T>(nsmax, c->nvt, segcap, NTHR / 64);
     if (lt > c->lds_cap) return fail(c, ERM_E_UNSUPPORTED, "solute too large for the pair kernel's LDS");
     if (g->persistent & 2) {
-      const void *f = (const void *)k_pair_tile_runs<T, false>;
+      auto *kr = k.ljswitch == 0 ? k_pair_tile_runs<T, false, true> : k_pair_tile_runs<T, false, false>;
+      const void *f = (const void *)kr;
       TRY(set_lds(c, f, lt, "k_pair_tile_runs"));
       int occ = 0;
       if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, f, NTHR, lt) != hipSuccess || occ < 1) {
@@ -1791,19 +1793,20 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
         occ = 1;
       }
       const int grid = std::min(nitem_p, std::max(1, occ * c->ncu));
-      hipLaunchKernelGGL((k_pair_tile_runs<T, false>), dim3(grid), dim3(NTHR), lt, c->st, k, dp<double>(c->d_spos),
+      hipLaunchKernelGGL(kr, dim3(grid), dim3(NTHR), lt, c->st, k, dp<double>(c->d_spos),
                          dp<double>(c->d_sref), dp<int>(c->d_cell_start), dp<int>(c->d_mol_first),
                          dp<int>(c->d_mol_ns), dp<double>(c->d_sx), dp<double>(c->d_sy), dp<double>(c->d_sz),
                          dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sltj), dp<double>(c->d_rm), d_runs, nrun,
                          nitem_p, dp<int>(g->d_counter) + 1, dp<double>(c->d_mol_d1), dp<double>(c->d_uv));
       TRY(launch_check(c, "k_pair_tile_runs"));
     } else {
-      TRY(set_lds(c, (const void *)k_pair_tile<T, false>, lt, "k_pair_tile"));
+      auto *f = k.ljswitch == 0 ? k_pair_tile<T, false, true> : k_pair_tile<T, false, false>;
+      TRY(set_lds(c, (const void *)f, lt, "k_pair_tile"));
       for (int r = 0; r < nrun; ++r) {
         Params kr = k;
         kr.ns = R[r].ns;
         const size_t c0 = R[r].cfg0;
-        hipLaunchKernelGGL((k_pair_tile<T, false>), dim3(R[r].ncfg, R[r].nsplit), dim3(NTHR), lt, c->st, kr, 64,
+        hipLaunchKernelGGL(f, dim3(R[r].ncfg, R[r].nsplit), dim3(NTHR), lt, c->st, kr, 64,
                            R[r].ns, (size_t)0,
                            dp<double>(c->d_spos) + (size_t)R[r].site0 * 3, dp<double>(c->d_sref) + 4 * c0,
                            static_cast<const T *>(R[r].q_t), static_cast<const T *>(R[r].lj_t),

@@ -1938,24 +1938,26 @@ template <typename T> struct V4T;
 template <> struct V4T<float> { using type = float4; };
 template <> struct V4T<double> { using type = double4; };
 
-// LDS of k_pair_tile.  Head: the solute's sites as (x, y, z, q), their low
-// parts and their test rows (-2x, -2y, -2z, threshold) (T4 each, ns rounded
-// up to whole groups of PT_GRP: the slots past ns hold sentinels that fail
-// every test), the LJ rows
-// [ns][nvt] (eps, sig2), the pillar segments
-// (segcap = 2 nb1 nb2 slots).  Per wave: the tile's sites (x, y, z, q) and
-// (low parts, LJ type), molecule offsets [65] and first sites [64], the queue
-// [PT_QCAP + 64] (int) and its energies [PT_QCAP + 64] (f64; the last 64 are
-// the lanes' spare slots, energy 0), the per-site sums [64] (f64), the slots
-// of the queued pairs evaluated in FP64 [PT_QCAP] (int).
+// LDS of k_pair_tile.  Head: the solute's sites as (x, y, z, q), in FP32
+// their low parts, and their test rows (-2x, -2y, -2z, threshold) (T4 each, ns
+// rounded up to whole groups of PT_GRP: the slots past ns hold sentinels that
+// fail every test), the LJ rows [ns][nvt] (eps, sig2), the pillar segments
+// (segcap = 2 nb1 nb2 slots).  Per wave: the tile's sites (x, y, z, q) (and
+// low parts with the LJ type in FP32; the types alone in FP64), the queue's
+// energies [PT_QCAP + 64] (f64; the last 64 are the lanes' spare slots,
+// energy 0), the per-site sums [64] (f64), molecule offsets [65] and first
+// sites [64], the queue [PT_QCAP + 64] (16 bits: site of the group << 6 | tile
+// lane) and in FP32 the slots of the queued pairs evaluated in FP64 [PT_QCAP].
+// Three workgroups of four waves fit a CU with a solute of a few dozen sites.
 template <typename T> __host__ __device__ inline size_t pair_tile_wave_lds() {
-  return ((size_t)2 * 64 * 4 * sizeof(T) + 65 * 4 + 64 * 4 + (size_t)PT_QCAP * (4 + 8 + 4) + 64 * (4 + 8) + 64 * 8 +
-          16 + 15) &
-         ~(size_t)15;
+  const size_t tile = sizeof(T) == 4 ? (size_t)2 * 64 * 4 * sizeof(T) : (size_t)64 * (4 * sizeof(T) + 4);
+  const size_t hot = sizeof(T) == 4 ? (size_t)PT_QCAP * 2 : 0;
+  return (tile + (PT_QCAP + 64 + 64) * 8 + (65 + 64) * 4 + (size_t)(PT_QCAP + 64) * 2 + hot + 15) & ~(size_t)15;
 }
 template <typename T> __host__ __device__ inline size_t pair_tile_head(int ns, int nvt, int segcap) {
   const size_t nsp = (size_t)(ns + PT_GRP - 1) / PT_GRP * PT_GRP;
-  const size_t a = sizeof(T) * ((size_t)12 * nsp + (size_t)2 * ns * nvt) + sizeof(int) * (2 * (size_t)segcap + 2) + 64;
+  const size_t rows = sizeof(T) == 4 ? 12 : 8;
+  const size_t a = sizeof(T) * (rows * nsp + (size_t)2 * ns * nvt) + sizeof(int) * (2 * (size_t)segcap + 2) + 64;
   return (a + 15) & ~(size_t)15;
 }
 template <typename T> __host__ __device__ inline size_t pair_tile_lds(int ns, int nvt, int segcap, int nwave) {
@@ -1973,7 +1975,9 @@ __device__ __forceinline__ int lanes_below(unsigned long long m) {
 
 // Configuration b (ns sites at xs), split `split` of nsplit workgroups, cm
 // <= 64 candidate molecules per chunk; all threads of the workgroup call it
-template <typename T, bool BARE>
+// SW0: the CHARMM potential switch (ljswitch 0, the default) alone, which
+// leaves the other switches' constants out of the registers
+template <typename T, bool BARE, bool SW0>
 __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, int split, int nsplit, int cm,
                                                const double *__restrict__ xs, const double *__restrict__ sref,
                                                const T *__restrict__ slt_q, const T *__restrict__ slt_lj,
@@ -1994,9 +1998,9 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
   const int nvt = P.nvt;
   const int nsp = (ns + PT_GRP - 1) / PT_GRP * PT_GRP;
   T4 *us4 = reinterpret_cast<T4 *>(lds_raw);  // [nsp] (x, y, z, q) offsets from the centre
-  T4 *ul4 = us4 + nsp;                        // [nsp] low parts (x, y, z, 0)
-  T4 *ut4 = ul4 + nsp;                        // [nsp] test rows (-2x, -2y, -2z, threshold)
-  T2 *ulj = reinterpret_cast<T2 *>(ut4 + nsp); // [ns][nvt] (eps, sig2)
+  T4 *ut4 = us4 + nsp;                        // [nsp] test rows (-2x, -2y, -2z, threshold)
+  T4 *ul4 = F32 ? ut4 + nsp : ut4;            // FP32: [nsp] low parts (x, y, z, 0)
+  T2 *ulj = reinterpret_cast<T2 *>(ul4 + nsp);  // [ns][nvt] (eps, sig2)
   const int segcap = 2 * P.nb[1] * P.nb[2];
   int *seg_beg = reinterpret_cast<int *>(ulj + ns * nvt);
   int *seg_pre = seg_beg + segcap;
@@ -2004,16 +2008,16 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
   unsigned char *wl = lds_raw + base + (size_t)wv * pair_tile_wave_lds<T>();
   T4 *tu4 = reinterpret_cast<T4 *>(wl);   // [64] (x, y, z, q) of the tile's sites
-  T4 *tl4 = tu4 + 64;                     // [64] (low x, low y, low z, LJ type bits)
-  int *woff = reinterpret_cast<int *>(tl4 + 64);  // [65] first chunk site of molecule lane
-  int *wfirst = woff + 65;                // [64] first sorted site of molecule lane
-  int *wq = wfirst + 64;                  // [PT_QCAP + 64] queued pairs: solute site << 6 | tile lane
-  // (a byte offset from wl, rounded down to 8 over the spare slot of wq, so
-  // the pointers stay LDS pointers for the compiler)
-  double *weq = reinterpret_cast<double *>(
-      wl + (((size_t)128 * sizeof(T4) + (size_t)(65 + 64 + PT_QCAP + 64 + 1) * sizeof(int)) & ~(size_t)7));
+  T4 *tl4 = tu4 + 64;                     // FP32: [64] (low x, low y, low z, LJ type bits)
+  int *tty = reinterpret_cast<int *>(tl4);  // FP64: [64] LJ types
+  // (byte offsets from wl, so the pointers stay LDS pointers for the compiler)
+  constexpr size_t tile = F32 ? 128 * sizeof(T4) : 64 * (sizeof(T4) + 4);
+  double *weq = reinterpret_cast<double *>(wl + tile);  // [PT_QCAP + 64] energies of the queued pairs
   double *wes = weq + PT_QCAP + 64;       // [64] per-site sums of a tile
-  int *whq = reinterpret_cast<int *>(wes + 64);  // [PT_QCAP] queue slots of the pairs evaluated in FP64
+  int *woff = reinterpret_cast<int *>(wes + 64);  // [65] first chunk site of molecule lane
+  int *wfirst = woff + 65;                // [64] first sorted site of molecule lane
+  unsigned short *wq = reinterpret_cast<unsigned short *>(wfirst + 64);  // [PT_QCAP + 64] queued pairs
+  unsigned short *whq = wq + PT_QCAP + 64;  // FP32: [PT_QCAP] queue slots of the pairs evaluated in FP64
 
   const double C0 = sref[4 * b], C1 = sref[4 * b + 1], C2v = sref[4 * b + 2];
   const double Rs = sref[4 * b + 3];
@@ -2056,7 +2060,7 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
       u.y = u.z = u.w = 0;
     }
     us4[s] = u;
-    ul4[s] = l;
+    if constexpr (F32) ul4[s] = l;
     ut4[s] = t;
   }
   for (int t = threadIdx.x; t < ns * nvt; t += blockDim.x) {
@@ -2087,7 +2091,7 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
   // there); every queue slot holds a valid entry (solute site 0), so the
   // evaluation reads and writes a full round of slots without branches
   weq[PT_QCAP + lane] = 0.0;
-  for (int k = lane; k < PT_QCAP + 64; k += 64) wq[k] = lane;
+  for (int k = lane; k < PT_QCAP + 64; k += 64) wq[k] = (unsigned short)lane;
   const int nchunk = (total + cm - 1) / cm;
   for (int c = split * nw + wv; c < nchunk; c += nsplit * nw) {
     // molecule of this lane: flattened candidate c*cm + lane
@@ -2177,15 +2181,16 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
           tl.y = (T)(dy - (double)tu.y);
           tl.z = (T)(dz - (double)tu.z);
           tl.w = __int_as_float(pc);
-        } else {
-          tl.w = __longlong_as_double((long long)pc);
         }
       }
       // a lane without an active site takes a sentinel displacement, so the
       // distance compare alone decides every pair below
       if (!act) tu.x = (T)PT_FAR;
       tu4[lane] = tu;
-      tl4[lane] = tl;
+      if constexpr (F32)
+        tl4[lane] = tl;
+      else
+        tty[lane] = act ? pc : 0;
       if (t0 + 64 < tot_sites) fetch(t0 + 64);
       const T t2 = tu.x * tu.x + tu.y * tu.y + tu.z * tu.z;  // PT_FAR^2 for an inactive lane
       double e = 0.0;  // this site's energy, in solute-site order
@@ -2204,7 +2209,7 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
           int slot;
           asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(slot) : "v"(PT_QCAP + lane), "v"(pos), "s"(m));
           pend[g] = slot;
-          wq[slot] = ((s0 + g) << 6) | lane;
+          wq[slot] = (unsigned short)((g << 6) | lane);
           qn += (int)__popcll(m);
         };
         // the group's solute rows, all read before the queue writes below
@@ -2246,15 +2251,18 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
           const int qi = q0 + lane;
           const bool valid = qi < qn;
           const int ent = wq[qi];
-          const int i = ent & 63, s = ent >> 6;
-          const T4 v = tu4[i], vl = tl4[i], us = us4[s];
+          const int i = ent & 63, s = s0 + (ent >> 6);
+          const T4 v = tu4[i], us = us4[s];
           T ax, ay, az;
+          int cvi;
           if constexpr (F32) {
-            const T4 ls = ul4[s];
+            const T4 ls = ul4[s], vl = tl4[i];
+            cvi = __float_as_int(vl.w);
             ax = ((v.x - us.x) + vl.x) - ls.x;
             ay = ((v.y - us.y) + vl.y) - ls.y;
             az = ((v.z - us.z) + vl.z) - ls.z;
           } else {
+            cvi = tty[i];
             ax = v.x - us.x;
             ay = v.y - us.y;
             az = v.z - us.z;
@@ -2269,22 +2277,17 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
           }
           const T r2 = ax * ax + ay * ay + az * az;
           const T qsv = v.w;
-          int cvi;
-          if constexpr (F32)
-            cvi = __float_as_int(vl.w);
-          else
-            cvi = (int)__double_as_longlong(vl.w);
           const T2 lj = ulj[__umul24(s, nvt) + cvi];  // s < 4096, nvt < 12800
           const T eps = lj.x, sig2 = lj.y;
           const bool inr = valid && r2 <= cut2;
           bool hot = false;
           if constexpr (F32) hot = inr & hot_pair<T>(eps, sig2, us.w * qsv, r2);  // both evaluated
           const unsigned long long mh = __ballot(hot);
-          if (hot) whq[nh + lanes_below(mh)] = qi;
+          if (hot) whq[nh + lanes_below(mh)] = (unsigned short)qi;
           nh += (int)__popcll(mh);
           T ep = 0;
           if constexpr (F32 && !BARE) {
-            if (P.ljswitch == 0) {
+            if constexpr (SW0) {
               // every lane computes, one select keeps the pairs inside the
               // cutoff: one hardware reciprocal square root (1 ulp) per pair
               // in place of the divisions and the rounded square root (the
@@ -2325,7 +2328,7 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
               ep = lj_bare_t<T>(P, eps, sig2, r2, rst);
               if (rst < (T)P.elecut) ep += us.w * qsv / rst;
             } else {
-              if (P.ljswitch == 0) {
+              if constexpr (SW0) {
                 const T invr2 = sig2 / r2;
                 const T invr6 = invr2 * invr2 * invr2;
                 const T elo = (T)4 * eps * invr6 * (invr6 - (T)1);
@@ -2354,7 +2357,7 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
               if (hi < nh) {
                 const int qi = whq[hi];
                 const int ent = wq[qi];
-                const int i = ent & 63, s = ent >> 6;
+                const int i = ent & 63, s = s0 + (ent >> 6);
                 const T4 v = tu4[i], vl = tl4[i], us = us4[s], ls = ul4[s];
                 const int cvi = __float_as_int(vl.w);
                 const T qsv = v.w;
@@ -2377,7 +2380,12 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
                   epd = lj_bare_t<double>(P, e64, s64, r2d, rd);
                   if (rd < P.elecut) epd += slt_q64[s] * (double)qsv / rd;
                 } else {
-                  if (r2d <= P.lw2)
+                  if constexpr (SW0) {
+                    const double i2 = s64 / r2d, i6 = i2 * i2 * i2, d = r2d - P.up2, w = P.up2 - P.lw2;
+                    const double elo = 4.0 * e64 * i6 * (i6 - 1.0);
+                    const double esw = elo * ((2.0 * r2d + P.up2 - 3.0 * P.lw2) * (d * d)) / (w * w * w);
+                    epd = (r2d <= P.lw2) ? elo : (r2d <= P.up2) ? esw : 0.0;
+                  } else if (r2d <= P.lw2)
                     epd = lj_low_t<double>(P, e64, s64, r2d);
                   else if (r2d <= P.up2)
                     epd = lj_switch_t<double>(P, e64, s64, r2d);
@@ -2411,8 +2419,8 @@ __device__ __forceinline__ void pair_tile_body(const Params &P, int ns, int b, i
 // [part nss, part nss + nss) of its configuration, and the energies of part z
 // go to uv + z stride (uv itself with one part; with several, zeroed buffers
 // that k_pair_parts adds up).
-template <typename T, bool BARE = false>
-__global__ __launch_bounds__(NTHR) void k_pair_tile(Params P, int cm, int nss, size_t stride,
+template <typename T, bool BARE, bool SW0>
+__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(3))) void k_pair_tile(Params P, int cm, int nss, size_t stride,
                                                     const double *__restrict__ spos,
                                                     const double *__restrict__ sref,
                                                     const T *__restrict__ slt_q, const T *__restrict__ slt_lj,
@@ -2428,7 +2436,7 @@ __global__ __launch_bounds__(NTHR) void k_pair_tile(Params P, int cm, int nss, s
                                                     const double *__restrict__ mol_d1, double *uv) {
   const int b = blockIdx.x, s0 = blockIdx.z * nss, ns = min(nss, P.ns - s0);
   const size_t row = (size_t)2 * s0 * P.nvt;
-  pair_tile_body<T, BARE>(P, ns, b, blockIdx.y, gridDim.y, cm, spos + ((size_t)b * P.ns + s0) * 3, sref, slt_q + s0,
+  pair_tile_body<T, BARE, SW0>(P, ns, b, blockIdx.y, gridDim.y, cm, spos + ((size_t)b * P.ns + s0) * 3, sref, slt_q + s0,
                           slt_lj + row, cell_start, mol_first, mol_ns, sx, sy, sz, sq, sct, slt_j, rm_ord_p,
                           slt_lj64 + row, slt_q64 + s0, mol_d1, uv + blockIdx.z * stride);
 }
@@ -2445,8 +2453,8 @@ static __global__ void k_pair_parts(size_t n, int np, const double *__restrict__
 // real space of a heterogeneous batch as one persistent launch:
 // workgroups pull (configuration, split) items, the runs in the order given
 // (largest solutes first), each with its solute type's tables
-template <typename T, bool BARE = false>
-__global__ __launch_bounds__(NTHR) void k_pair_tile_runs(Params P, const double *__restrict__ spos,
+template <typename T, bool BARE, bool SW0>
+__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(3))) void k_pair_tile_runs(Params P, const double *__restrict__ spos,
                                                          const double *__restrict__ sref,
                                                          const int *__restrict__ cell_start,
                                                          const int *__restrict__ mol_first,
@@ -2467,7 +2475,7 @@ __global__ __launch_bounds__(NTHR) void k_pair_tile_runs(Params P, const double 
     const int ns = runs[r].ns, nsplit = runs[r].nsplit, rel = it - runs[r].pitem0;
     const int bl = rel / nsplit, split = rel - bl * nsplit, b = runs[r].cfg0 + bl;
     const double *xs = spos + ((size_t)runs[r].site0 + (size_t)bl * ns) * 3;
-    pair_tile_body<T, BARE>(P, ns, b, split, nsplit, 64, xs, sref, static_cast<const T *>(runs[r].q_t),
+    pair_tile_body<T, BARE, SW0>(P, ns, b, split, nsplit, 64, xs, sref, static_cast<const T *>(runs[r].q_t),
                             static_cast<const T *>(runs[r].lj_t), cell_start, mol_first, mol_ns, sx, sy, sz, sq, sct,
                             slt_j, rm_ord_p, runs[r].lj64, runs[r].q64, mol_d1, uv);
   }

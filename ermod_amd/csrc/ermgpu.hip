@@ -900,6 +900,26 @@ inline int pair_splits(int nchunk, int nwave) {
   return std::max(1, std::min(64, (nchunk + per - 1) / per));
 }
 
+// Waves per workgroup of the persistent pair grid: the fewest (4, 8 or 12)
+// with which the CU holds the most waves, up to the 12 their registers allow.
+// The solute's sites and LJ rows are in LDS once per workgroup, so a large
+// solute's grid wants many waves in one workgroup (150 sites against 14
+// solvent types: 28 KB, with 4 waves 8 per CU, with 12 in one
+// workgroup 12: 5000 FP32 configurations of 5 to 150 sites 3.61 -> 3.08 ms).
+template <typename T> int pair_runs_waves(const erm_ctx *c, int ns) {
+  int best = 4, most = 0;
+  for (int w : {4, 8, 12}) {
+    const size_t lds = pair_tile_lds<T>(ns, c->nvt, 2 * c->kp.nb[1] * c->kp.nb[2], w);
+    if (lds > c->lds_cap) break;
+    const int waves = std::min(12, w * (int)((c->lds_cap + 10 * 1024) / (lds + PAIR_MAXT * sizeof(int))));
+    if (waves > most) {
+      most = waves;
+      best = w;
+    }
+  }
+  return best;
+}
+
 // How one launch of the tiled pair kernel divides n configurations with
 // about `cand` candidate molecules each: cm molecules per chunk, nsplit
 // workgroups per configuration and the solute in `parts` of nss sites.
@@ -1781,19 +1801,20 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
     int nsmax = 0;
     for (int r = 0; r < nrun; ++r) nsmax = std::max(nsmax, R[r].ns);
     const int segcap = 2 * k.nb[1] * k.nb[2];
-    const size_t lt = pair_tile_lds<T>(nsmax, c->nvt, segcap, NTHR / 64);
+    const int nwave = pair_runs_waves<T>(c, nsmax);
+    const size_t lt = pair_tile_lds<T>(nsmax, c->nvt, segcap, nwave);
     if (lt > c->lds_cap) return fail(c, ERM_E_UNSUPPORTED, "solute too large for the pair kernel's LDS");
     if (g->persistent & 2) {
       auto *kr = k.ljswitch == 0 ? k_pair_tile_runs<T, false, true> : k_pair_tile_runs<T, false, false>;
       const void *f = (const void *)kr;
       TRY(set_lds(c, f, lt, "k_pair_tile_runs"));
       int occ = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, f, NTHR, lt) != hipSuccess || occ < 1) {
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, f, 64 * nwave, lt) != hipSuccess || occ < 1) {
         (void)hipGetLastError();
         occ = 1;
       }
       const int grid = std::min(nitem_p, std::max(1, occ * c->ncu));
-      hipLaunchKernelGGL(kr, dim3(grid), dim3(NTHR), lt, c->st, k, dp<double>(c->d_spos),
+      hipLaunchKernelGGL(kr, dim3(grid), dim3(64 * nwave), lt, c->st, k, dp<double>(c->d_spos),
                          dp<double>(c->d_sref), dp<int>(c->d_cell_start), dp<int>(c->d_mol_first),
                          dp<int>(c->d_mol_ns), dp<double>(c->d_sx), dp<double>(c->d_sy), dp<double>(c->d_sz),
                          dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sltj), dp<double>(c->d_rm), d_runs, nrun,
@@ -2715,6 +2736,9 @@ int32_t erm_group_insert_random(erm_group *g, const int32_t *n, const uint64_t *
   const Params &k = c->kp;
   const int vb = c->fp32 ? (int)sizeof(float2) : (int)sizeof(double2);
   const int nzg = zcol_groups(c, true, vb);
+  const int ns_max = g->ctx[order[0]]->ns;
+  const int nwave_p = !(g->persistent & 2) ? NTHR / 64
+                      : c->fp32 ? pair_runs_waves<float>(c, ns_max) : pair_runs_waves<double>(c, ns_max);
   // the run tables of every batch (host), then the batches' launches
   std::vector<int> nrun_b(nb), ncfg_b(nb), nz_b(nb), np_b(nb);
   std::vector<uint64_t> off_b((size_t)nb * GROUP_MAXRUN, 0);
@@ -2731,7 +2755,7 @@ int32_t erm_group_insert_random(erm_group *g, const int32_t *n, const uint64_t *
       const double Rg = k.rcmax + m->slt_radius + c->mol_radius + 0.5 * (k.hcell[0] + k.hcell[1] + k.hcell[2]) / 3.0;
       const double frac = std::min(1.0, 4.18879 * Rg * Rg * Rg / c->volume);
       const int nchunk = (int)std::ceil(frac * c->slvmax / 64.0);
-      const int nsplit = pair_splits(nchunk, NTHR / 64);
+      const int nsplit = pair_splits(nchunk, nwave_p);
       GRun &r = R[nrun];
       r.cfg0 = cfg;
       r.ncfg = cnt;

@@ -1647,9 +1647,10 @@ __device__ __forceinline__ T lj_bare_t(const Params &P, T eps, T sig2, T dis2, T
   return eplj;
 }
 
-// inclusive prefix sum of a[0..n) in LDS, n <= 8 * blockDim.x; all threads call
+// inclusive prefix sum of a[0..n) in LDS; all threads (at most PAIR_MAXT) call
+constexpr int PAIR_MAXT = 768;
 static __device__ void block_inclusive_scan(int *a, int n) {
-  __shared__ int part[NTHR];
+  __shared__ int part[PAIR_MAXT];
   const int per = (n + blockDim.x - 1) / blockDim.x;
   const int b0 = threadIdx.x * per;
   int s = 0;
@@ -2454,7 +2455,7 @@ static __global__ void k_pair_parts(size_t n, int np, const double *__restrict__
 // workgroups pull (configuration, split) items, the runs in the order given
 // (largest solutes first), each with its solute type's tables
 template <typename T, bool BARE, bool SW0>
-__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(3))) void k_pair_tile_runs(Params P, const double *__restrict__ spos,
+__global__ __launch_bounds__(PAIR_MAXT) __attribute__((amdgpu_waves_per_eu(3))) void k_pair_tile_runs(Params P, const double *__restrict__ spos,
                                                          const double *__restrict__ sref,
                                                          const int *__restrict__ cell_start,
                                                          const int *__restrict__ mol_first,

@@ -1520,12 +1520,11 @@ template <typename T> int solvent_grid(erm_ctx *c, int excl) {
   const size_t nr = (size_t)k.K1 * k.K2 * k.K3, nh = (size_t)k.H * k.K2 * k.K3;
   TRY(ensure(c, c->d_ggrid, sizeof(T) * nr));
   TRY(ensure(c, c->d_gHk, sizeof(V) * nh));
-  hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)((nr + NTHR - 1) / NTHR)), dim3(NTHR), 0, c->st,
-                     dp<T>(c->d_ggrid), nr, (T)0);
-  TRY(launch_check(c, "k_fill"));
-  hipLaunchKernelGGL(k_spread_slv<T>, dim3((c->slvmax + NTHR - 1) / NTHR), dim3(NTHR), 0, c->st, k, excl,
-                     dp<int>(c->d_mol_first), dp<int>(c->d_mol_ns), dp<int>(c->d_sg), dp<T>(c->d_sw),
-                     dp<T>(c->d_sq), dp<T>(c->d_ggrid));
+  const size_t lplane = sizeof(T) * k.K1 * k.K2;
+  TRY(set_lds(c, (const void *)k_spread_slv<T>, lplane, "k_spread_slv"));
+  hipLaunchKernelGGL(k_spread_slv<T>, dim3(k.K3), dim3(SPREAD_THR), lplane, c->st, k, excl, dp<int>(c->d_mol_first),
+                     dp<int>(c->d_zstart), dp<int>(c->d_zsite), dp<int>(c->d_zg), dp<T>(c->d_zw), dp<T>(c->d_zq),
+                     dp<T>(c->d_ggrid));
   TRY(launch_check(c, "k_spread_slv"));
   ERM_KSWITCH(k.K1, (launch_xr2c<T, KK>(c, k)));
   TRY(launch_check(c, "k_xrow_r2c"));
@@ -1547,6 +1546,9 @@ struct GradSetup {
   double qslt = 0.0, rf = 0.0;
   int excl = -1;
 };
+
+// k_pair_grad: workgroups in flight, least sites of one, sites staged at a time
+constexpr int GRAD_WGS = 2048, GRAD_SITES = 128, GRAD_CHUNK = 512;
 
 // one batch of the gradient: adds [sum w, sum w u, sum w grad] into acc
 template <typename T> int gradient_batch(erm_ctx *c, const Batch &bt, const GradSetup &g, double *acc) {
@@ -1571,25 +1573,28 @@ template <typename T> int gradient_batch(erm_ctx *c, const Batch &bt, const Grad
                      dp<V>(c->d_w1h), dp<V>(c->d_w2h), (V *)nullptr);
   TRY(launch_check(c, "k_solute_prep"));
   // real space
-  double Rg = k.rcmax + 8.0;
-  double frac = std::min(1.0, 4.18879 * Rg * Rg * Rg / c->volume);
-  int nsplit = std::max(1, std::min(16, (int)std::ceil(frac * c->slvmax / (2.0 * NTHR))));
+  // workgroups per configuration: GRAD_WGS in all fill the chip, as long as one
+  // has GRAD_SITES of the candidates, estimated from a sphere around the solute
+  const double Rg = k.rcmax + 8.0;
+  const double frac = std::min(1.0, 4.18879 * Rg * Rg * Rg / c->volume);
+  const int nsplit = std::max(1, std::min({64, (GRAD_WGS + n - 1) / n, (int)(frac * c->nsites / GRAD_SITES)}));
   const int nsl = std::max(1, NTHR / ns);
-  size_t lds = sizeof(double) * 4 * (size_t)nsl * ns + sizeof(T) * ((size_t)7 * ns + (size_t)3 * ns * c->nvt) +
-               sizeof(int) * (2 * MAXSEG + 2) + 64;
+  int chunk = GRAD_CHUNK;
+  while (chunk > 64 && grad_lds<T>(ns, c->nvt, nsl, chunk) > c->lds_cap) chunk /= 2;
+  const size_t lds = grad_lds<T>(ns, c->nvt, nsl, chunk);
   if (lds > c->lds_cap) return fail(c, ERM_E_UNSUPPORTED, "solute too large for the gradient kernel's LDS");
   TRY(set_lds(c, (const void *)k_pair_grad<T>, lds, "k_pair_grad"));
   TRY(ensure(c, c->d_gpart, sizeof(double) * (size_t)n * nsplit * 4 * ns));
-  hipLaunchKernelGGL(k_pair_grad<T>, dim3(n, nsplit), dim3(NTHR), lds, c->st, k, dp<double>(c->d_spos),
+  hipLaunchKernelGGL(k_pair_grad<T>, dim3(n, nsplit), dim3(NTHR), lds, c->st, k, nsl, chunk, dp<double>(c->d_spos),
                      dp<double>(c->d_sref), dp<T>(c->d_gq_t), dp<T>(c->d_gtab), dp<int>(c->d_cell_start),
-                     dp<int>(c->d_mol_first), dp<int>(c->d_mol_ns), dp<double>(c->d_sx), dp<double>(c->d_sy),
+                     dp<int>(c->d_mol_first), dp<double>(c->d_sx), dp<double>(c->d_sy),
                      dp<double>(c->d_sz), dp<T>(c->d_sq), dp<int>(c->d_sct), dp<int>(c->d_sltj),
                      dp<double>(c->d_rm), dp<double>(c->d_gpart));
   TRY(launch_check(c, "k_pair_grad"));
   // reciprocal space
   TRY(solvent_grid<T>(c, g.excl));
   TRY(ensure(c, c->d_gphi, sizeof(double) * (size_t)n * ns));
-  hipLaunchKernelGGL(k_grad_recip<T>, dim3((n * ns + NTHR - 1) / NTHR), dim3(NTHR), 0, c->st, k, n,
+  hipLaunchKernelGGL(k_grad_recip<T>, dim3((unsigned)(((size_t)n * ns * RECIP_LANES + NTHR - 1) / NTHR)), dim3(NTHR), 0, c->st, k, n,
                      dp<double>(c->d_spos), dp<T>(c->d_ggrid), dp<double>(c->d_gphi));
   TRY(launch_check(c, "k_grad_recip"));
   // weights and sums
@@ -1599,13 +1604,13 @@ template <typename T> int gradient_batch(erm_ctx *c, const Batch &bt, const Grad
   TRY(ensure(c, c->d_gw, sizeof(double) * n));
   TRY(upload(c, c->d_gw, w.data(), n));
   TRY(ensure(c, c->d_gub, sizeof(double) * n));
-  hipLaunchKernelGGL(k_grad_ub, dim3((n + NTHR - 1) / NTHR), dim3(NTHR), 0, c->st, k, n, nsplit,
+  hipLaunchKernelGGL(k_grad_ub, dim3((n + GRAD_THR / 64 - 1) / (GRAD_THR / 64)), dim3(GRAD_THR), 0, c->st, k, n, nsplit,
                      dp<double>(c->d_gpart), dp<double>(c->d_gphi), dp<double>(c->d_gqd), g.rf, g.qslt,
                      dp<double>(c->d_gub));
   TRY(launch_check(c, "k_grad_ub"));
   const int nout = 2 + 3 * ns;
   TRY(ensure(c, c->d_gout, sizeof(double) * nout));
-  hipLaunchKernelGGL(k_grad_reduce, dim3((nout + NTHR - 1) / NTHR), dim3(NTHR), 0, c->st, k, n, nsplit,
+  hipLaunchKernelGGL(k_grad_reduce, dim3(nout), dim3(GRAD_THR), 0, c->st, k, n, nsplit,
                      dp<double>(c->d_gpart), dp<double>(c->d_gphi), dp<double>(c->d_gub), dp<double>(c->d_gw),
                      dp<double>(c->d_gepsd), g.rf, dp<double>(c->d_gout));
   TRY(launch_check(c, "k_grad_reduce"));

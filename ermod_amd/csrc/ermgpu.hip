@@ -593,8 +593,8 @@ int zcol_groups(const erm_ctx *c, bool regp, int vb) {
 int launch_mol_sum(erm_ctx *c, const Params &kg, int n, const double *esite, const int *sltj, double *uv) {
   if (n <= 0) return ERM_OK;
   const int S = c->slvmax;
-  hipLaunchKernelGGL(k_mol_sum, dim3((S + NTHR - 1) / NTHR, (n + MOLSUM_CFG - 1) / MOLSUM_CFG), dim3(NTHR), 0,
-                     c->st, kg, c->nsites, n, esite, dp<int>(c->d_zpos), dp<int>(c->d_mol_first),
+  hipLaunchKernelGGL(n == 1 ? k_mol_sum<true> : k_mol_sum<false>,
+                     dim3((S + NTHR - 1) / NTHR, (n + MOLSUM_CFG - 1) / MOLSUM_CFG), dim3(NTHR), 0, c->st, kg, c->nsites, n, esite, dp<int>(c->d_zpos), dp<int>(c->d_mol_first),
                      dp<int>(c->d_mol_ns), dp<double>(c->d_mol_q), sltj, uv);
   return launch_check(c, "k_mol_sum");
 }
@@ -768,7 +768,7 @@ template <typename T> int frame_prep(erm_ctx *c) {
   hipLaunchKernelGGL(k_mol_cell, dim3(gb), dim3(tb), 0, c->st, k, dp<double>(c->d_pos), dp<int>(c->d_tagpt),
                      dp<int>(c->d_mol_begin), dp<int>(c->d_cellid), dp<int>(c->d_count));
   TRY(launch_check(c, "k_mol_cell"));
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->st, dp<int>(c->d_count), dp<int>(c->d_cell_start), ncell,
+  hipLaunchKernelGGL(k_scan, dim3(1), dim3(SCAN_THR), 0, c->st, dp<int>(c->d_count), dp<int>(c->d_cell_start), ncell,
                      dp<int>(c->d_fill), (int *)nullptr, 0, 0);
   TRY(launch_check(c, "k_scan"));
   hipLaunchKernelGGL(k_mol_scatter, dim3(gb), dim3(tb), 0, c->st, k, dp<int>(c->d_cellid), dp<int>(c->d_fill),
@@ -776,7 +776,7 @@ template <typename T> int frame_prep(erm_ctx *c) {
                      dp<int>(c->d_mol_k), dp<int>(c->d_mol_ns), dp<int>(c->d_jof), dp<double>(c->d_mol_q),
                      dp<int>(c->d_mol_spec), dp<double>(c->d_mol_d1));
   TRY(launch_check(c, "k_mol_scatter"));
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->st, dp<int>(c->d_mol_ns), dp<int>(c->d_mol_first), S,
+  hipLaunchKernelGGL(k_scan, dim3(1), dim3(SCAN_THR), 0, c->st, dp<int>(c->d_mol_ns), dp<int>(c->d_mol_first), S,
                      (int *)nullptr, (int *)nullptr, 0, 0);
   TRY(launch_check(c, "k_scan"));
   hipLaunchKernelGGL(k_site_fill<T>, dim3((nsites + SITE_THR - 1) / SITE_THR), dim3(SITE_THR), 0, c->st, k, nsites,
@@ -802,7 +802,7 @@ template <typename T> int frame_prep(erm_ctx *c) {
   hipLaunchKernelGGL(k_zcount, dim3(gs), dim3(tb), 0, c->st, nsites, nbk, KB, rowp, dp<int>(c->d_sg),
                      dp<int>(c->d_zcount));
   TRY(launch_check(c, "k_zcount"));
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->st, dp<int>(c->d_zcount), dp<int>(c->d_zfine), nbk,
+  hipLaunchKernelGGL(k_scan, dim3(1), dim3(SCAN_THR), 0, c->st, dp<int>(c->d_zcount), dp<int>(c->d_zfine), nbk,
                      dp<int>(c->d_zfill), dp<int>(c->d_zstart), K3, KB);
   TRY(launch_check(c, "k_scan"));
   hipLaunchKernelGGL(k_zscatter<T>, dim3(gs), dim3(tb), 0, c->st, nsites, nbk, KB, rowp, k.p, dp<int>(c->d_sg),
@@ -1021,7 +1021,7 @@ template <typename T> int launch_pair(erm_ctx *c, const Params &k, int n, bool b
 // per thread), where a configuration's pairs are the longest chain of the
 // launch, 256 below it.
 void launch_selfreal(erm_ctx *c, const Params &k, int n, const double *spos, const double *q, double *out) {
-  hipLaunchKernelGGL(k_selfreal, dim3(n), dim3(k.ns >= 64 ? SELF_THR : NTHR), 0, c->st, k, spos, q, out);
+  hipLaunchKernelGGL(k_selfreal, dim3(n, self_parts(k.ns)), dim3(NTHR), 0, c->st, k, spos, q, out);
 }
 
 // Energies of a batch of configurations into d_uv (sorted molecule order);
@@ -1051,8 +1051,8 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
   if (zspec) TRY(ensure(c, c->d_w3h, sizeof(V) * (size_t)n * ns * K3));
   TRY(ensure(c, c->d_uv, sizeof(double) * (size_t)n * (S + 1)));
   TRY(ensure(c, c->d_sltj, sizeof(int) * n));
-  TRY(ensure(c, c->d_selfreal, sizeof(double) * n));
-  TRY(ensure(c, c->d_usreal, sizeof(double)));
+  TRY(ensure(c, c->d_selfreal, sizeof(double) * n * self_parts(ns)));
+  TRY(ensure(c, c->d_usreal, sizeof(double) * self_parts(ns)));
   const size_t vb = sizeof(V);
   const int ncolwg = zcol_width(K3, vb);
   const int nzg = zcol_groups(c, regp, (int)vb);
@@ -1166,8 +1166,8 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
     if (!(flags & DO_RECIP)) {
       HIPCHK(c, hipMemsetAsync(c->d_selfp.p, 0, sizeof(double) * (size_t)n * nzg, c->st));
     }
-    hipLaunchKernelGGL(k_u0, dim3((n + 63) / 64), dim3(64), 0, c->st, ku, n, nzg, dp<double>(c->d_selfp),
-                       per_item ? dp<double>(c->d_selfreal) : dp<double>(c->d_usreal), per_item,
+    hipLaunchKernelGGL(k_u0, dim3((n + NTHR / 64 - 1) / (NTHR / 64)), dim3(NTHR), 0, c->st, ku, n, nzg, dp<double>(c->d_selfp),
+                       per_item ? dp<double>(c->d_selfreal) : dp<double>(c->d_usreal), per_item, self_parts(ns),
                        dp<double>(c->d_uv));
     TRY(launch_check(c, "k_u0"));
   }
@@ -1218,10 +1218,12 @@ int run_corr_at(erm_ctx *c, int n, const HistBufs &hb) {
 int run_histogram_at(erm_ctx *c, int n, int first, const HistBufs &hb, bool without_corr = false) {
   Params k = c->kp;
   const int E = c->ermax;
-  const size_t lb = (size_t)E * (sizeof(double) + sizeof(int)) + sizeof(double) * (size_t)c->numslv * NTHR;
+  auto bin_lds = [&](int thr) { return (size_t)E * (sizeof(double) + sizeof(int)) + sizeof(double) * (size_t)c->numslv * thr; };
+  const int bthr = (c->slvmax > BIN_MOLS && bin_lds(BIN_THR) <= c->lds_cap) ? BIN_THR : NTHR;
+  const size_t lb = bin_lds(bthr);
   TRY(set_lds(c, (const void *)k_bin, lb, "k_bin"));
   if (!hb.mol_spec) return fail(c, ERM_E_ENG_BUG, "histogram without the frame's molecule species");
-  hipLaunchKernelGGL(k_bin, dim3(n), dim3(NTHR), lb, c->st, k, hb.uv, dp<double>(c->d_edges),
+  hipLaunchKernelGGL(k_bin, dim3(n), dim3(bthr), lb, c->st, k, hb.uv, dp<double>(c->d_edges),
                      dp<int>(c->d_specoff), dp<int>(c->d_uvmax), dp<int>(c->d_uvsoft), hb.mol_spec, hb.sltj, hb.hist,
                      hb.flceng, dp<unsigned long long>(c->d_mnmx), hb.status, first);
   TRY(launch_check(c, "k_bin"));
@@ -1852,7 +1854,7 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
     Params km = m->kp;
     km.ns = m->ns;
     km.solute_charge = m->mol_charge[m->slt_template];
-    TRY(ensure(m, m->d_usreal, sizeof(double)));
+    TRY(ensure(m, m->d_usreal, sizeof(double) * self_parts(m->ns)));
     if (!m->have_usreal) {
       launch_selfreal(c, km, 1, dp<double>(c->d_spos) + (size_t)R[r].site0 * 3, dp<double>(m->d_qslt),
                       dp<double>(m->d_usreal));
@@ -1860,8 +1862,8 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
       m->have_usreal = true;
     }
     const size_t c0 = R[r].cfg0;
-    hipLaunchKernelGGL(k_u0, dim3((R[r].ncfg + 63) / 64), dim3(64), 0, c->st, km, R[r].ncfg, nzg,
-                       dp<double>(c->d_selfp) + c0 * nzg, dp<double>(m->d_usreal), 0,
+    hipLaunchKernelGGL(k_u0, dim3((R[r].ncfg + NTHR / 64 - 1) / (NTHR / 64)), dim3(NTHR), 0, c->st, km, R[r].ncfg, nzg,
+                       dp<double>(c->d_selfp) + c0 * nzg, dp<double>(m->d_usreal), 0, self_parts(m->ns),
                        dp<double>(c->d_uv) + c0 * (S + 1));
     TRY(launch_check(c, "k_u0"));
   }
@@ -2516,7 +2518,8 @@ int32_t erm_realcal_self(erm_ctx *c, int32_t solute, const double *pos, double *
   if (hipSetDevice(c->P.device) != hipSuccess) return fail(c, ERM_E_DEVICE, "hipSetDevice");
   const int ns = c->ns;
   TRY(ensure(c, c->d_spos, sizeof(double) * ns * 3));
-  TRY(ensure(c, c->d_selfreal, sizeof(double)));
+  const int parts = self_parts(ns);
+  TRY(ensure(c, c->d_selfreal, sizeof(double) * parts));
   if (c->P.slttype == 1) {
     int sl = solute;
     TRY(check_solutes(c, 1, &sl, nullptr));
@@ -2528,8 +2531,12 @@ int32_t erm_realcal_self(erm_ctx *c, int32_t solute, const double *pos, double *
   }
   launch_selfreal(c, c->kp, 1, dp<double>(c->d_spos), dp<double>(c->d_qslt), dp<double>(c->d_selfreal));
   TRY(launch_check(c, "k_selfreal"));
-  HIPCHK(c, hipMemcpyAsync(self_real, c->d_selfreal.p, sizeof(double), hipMemcpyDeviceToHost, c->st));
-  return sync(c);
+  std::vector<double> part(parts);
+  HIPCHK(c, hipMemcpyAsync(part.data(), c->d_selfreal.p, sizeof(double) * parts, hipMemcpyDeviceToHost, c->st));
+  TRY(sync(c));
+  *self_real = 0.0;
+  for (double v : part) *self_real += v;
+  return ERM_OK;
 }
 
 int32_t erm_engconst(erm_ctx *c, int32_t n, const int32_t *solutes, const double *solute_pos, const double *weights,

@@ -81,33 +81,68 @@ static __global__ void k_mol_cell(Params P, const double *__restrict__ pos, cons
 // Exclusive scan of in[0, n) into out[0, n], out[n] the total (one
 // workgroup).  copy: a second copy of out[0, n) (the fill cursors of a
 // counting sort), or null; planes: planes[z] = out[z KB] for z <= K3, or
-// null.
-static __global__ __launch_bounds__(1024) void k_scan(const int *__restrict__ in, int *out, int n, int *copy, int *planes,
+// null.  The arrays start on 16 bytes.  Bound by latency: SCAN_ITEMS values per
+// thread and step in 16-byte accesses, wave scans by lane shifts, one barrier
+// per step (a serial chunk per thread and ten
+// barrier pairs: 15 us on average for the three scans of a 60000-site frame,
+// this 5).
+constexpr int SCAN_THR = 1024, SCAN_ITEMS = 8;
+static __global__ __launch_bounds__(SCAN_THR) void k_scan(const int *__restrict__ in, int *out, int n, int *copy, int *planes,
                                                int K3, int KB) {
-  __shared__ int part[1024];
-  const int t = threadIdx.x;
-  const int chunk = (n + 1023) / 1024;
-  const int b0 = t * chunk;
-  int s = 0;
-  for (int i = 0; i < chunk; ++i)
-    if (b0 + i < n) s += in[b0 + i];
-  part[t] = s;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    int v = (t >= off) ? part[t - off] : 0;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
-  }
-  int run = (t == 0) ? 0 : part[t - 1];
-  for (int i = 0; i < chunk; ++i)
-    if (b0 + i < n) {
-      int v = in[b0 + i];
-      out[b0 + i] = run;
-      if (copy) copy[b0 + i] = run;
-      run += v;
+  __shared__ int wsum[2][SCAN_THR / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  int carry = 0;
+  for (int base = 0, k = 0; base < n; base += SCAN_THR * SCAN_ITEMS, k ^= 1) {
+    const int b0 = base + t * SCAN_ITEMS;
+    __align__(16) int v[SCAN_ITEMS];
+    const bool full = b0 + SCAN_ITEMS <= n;
+    if (full) {
+#pragma unroll
+      for (int i = 0; i < SCAN_ITEMS; i += 4)
+        *reinterpret_cast<int4 *>(v + i) = *reinterpret_cast<const int4 *>(in + b0 + i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < SCAN_ITEMS; ++i) v[i] = (b0 + i < n) ? in[b0 + i] : 0;
     }
-  if (t == 1023) out[n] = part[1023];
+    int own = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i) own += v[i];
+    int inc = own;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += u;
+    }
+    if (lane == 63) wsum[k][wv] = inc;
+    __syncthreads();
+    int run = carry + inc - own;
+#pragma unroll
+    for (int w = 0; w < SCAN_THR / 64; ++w) {
+      const int x = wsum[k][w];
+      run += (w < wv) ? x : 0;
+      carry += x;
+    }
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i) {
+      const int x = v[i];
+      v[i] = run;
+      run += x;
+    }
+    if (full) {
+#pragma unroll
+      for (int i = 0; i < SCAN_ITEMS; i += 4) {
+        *reinterpret_cast<int4 *>(out + b0 + i) = *reinterpret_cast<const int4 *>(v + i);
+        if (copy) *reinterpret_cast<int4 *>(copy + b0 + i) = *reinterpret_cast<const int4 *>(v + i);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < SCAN_ITEMS; ++i)
+        if (b0 + i < n) {
+          out[b0 + i] = v[i];
+          if (copy) copy[b0 + i] = v[i];
+        }
+    }
+  }
+  if (t == 0) out[n] = carry;
   if (planes) {
     __syncthreads();
     for (int z = t; z <= K3; z += blockDim.x) planes[z] = out[(size_t)z * KB];
@@ -1380,8 +1415,11 @@ __global__ __launch_bounds__(NTHR) void k_pme_ycol_reg(Params P, const typename 
 // configurations and its sites four at a time: the four zpos reads, then
 // the per-site sums of every configuration, all in flight together (one
 // molecule per thread and configuration was a chain of dependent loads).
+// ONE: a batch of one configuration, where the solute's own molecule, which has
+// no energy with itself, may have the longest chain of sites (300 sites: 46 us,
+// with it left out 4; the test itself costs a large batch a tenth).
 constexpr int MOLSUM_CFG = 4;
-static __global__ void k_mol_sum(Params P, int nsites, int ncfg, const double *__restrict__ e_site,
+template <bool ONE> static __global__ void k_mol_sum(Params P, int nsites, int ncfg, const double *__restrict__ e_site,
                                  const int *__restrict__ zpos, const int *__restrict__ mol_first,
                                  const int *__restrict__ mol_ns, const double *__restrict__ mol_q,
                                  const int *__restrict__ slt_j, double *uv) {
@@ -1396,7 +1434,7 @@ static __global__ void k_mol_sum(Params P, int nsites, int ncfg, const double *_
   if (j >= P.slvmax) return;
   const int b0 = bg * MOLSUM_CFG;
   const int nb = min(MOLSUM_CFG, ncfg - b0);
-  const int t0 = mol_first[j], t1 = t0 + mol_ns[j];
+  const int t0 = mol_first[j], t1 = (ONE && j == slt_j[0]) ? t0 : t0 + mol_ns[j];
   const double *es = e_site + (size_t)b0 * nsites;
   double e[MOLSUM_CFG];
 #pragma unroll
@@ -2560,21 +2598,28 @@ __global__ __launch_bounds__(NTHR) void k_pair_open(Params P, const double *__re
 // 30 sites: 7.3 ms, now 0.03 ms).  Pair p < ns (ns - 1) / 2 is
 // (i, i + d mod ns) with i = p mod ns, d = p / ns + 1, which lists every
 // unordered pair once and gives every thread the same number of pairs, where
-// a thread per row had 0 to ns - 1 of them.
-constexpr int SELF_THR = 1024;  // the largest workgroup
-static __global__ __launch_bounds__(SELF_THR) void k_selfreal(Params P, const double *__restrict__ spos,
+// a thread per row had 0 to ns - 1 of them.  A large solute's pairs are split
+// over self_parts(ns) workgroups, out[b][part], which k_u0 adds in order (300
+// sites in one workgroup of 1024 threads 56 us, in 11 of 256 10).
+constexpr int SELF_PAIRS = 16;  // pairs per thread
+static inline int self_parts(int ns) {
+  const long np = (long)ns * (ns - 1) / 2, per = (long)NTHR * SELF_PAIRS;
+  return (int)std::max(1L, (np + per - 1) / per);
+}
+static __global__ __launch_bounds__(NTHR) void k_selfreal(Params P, const double *__restrict__ spos,
                                                    const double *__restrict__ qsolute, double *out) {
-  __shared__ double red[SELF_THR];
+  __shared__ double red[NTHR];
   const int ns = P.ns;
   const double *x = spos + (size_t)blockIdx.x * ns * 3;
   double e = 0.0;
   const double a = P.screen;
-  for (int i = threadIdx.x; i < ns; i += blockDim.x) {
+  const int t0 = blockIdx.y * blockDim.x + threadIdx.x, nt = gridDim.y * blockDim.x;
+  for (int i = t0; i < ns; i += nt) {
     double qi = qsolute[i];
     e += -qi * qi * a / sqrt(3.1415926535897932);
   }
   const int npair = ns * (ns - 1) / 2;  // ns <= 4096
-  for (int p = threadIdx.x; p < npair; p += blockDim.x) {
+  for (int p = t0; p < npair; p += nt) {
     const int i = p % ns;
     int jj = i + p / ns + 1;
     jj -= (jj >= ns) ? ns : 0;
@@ -2593,21 +2638,31 @@ static __global__ __launch_bounds__(SELF_THR) void k_selfreal(Params P, const do
     if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = red[0];
+  if (threadIdx.x == 0) out[(size_t)blockIdx.x * gridDim.y + blockIdx.y] = red[0];
 }
 
-// uvengy(0) = self_recp + realcal_self + residual_self (engproc.F90:701-732)
-static __global__ void k_u0(Params P, int n, int ngrp, const double *__restrict__ selfp,
-                     const double *__restrict__ selfreal, int per_item, double *uv) {
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
+// sum over the lanes of a wave in a fixed order, in every lane
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// uvengy(0) = self_recp + realcal_self + residual_self (engproc.F90:701-732);
+// a wave per configuration, its lanes over the column groups' partial sums (a
+// thread each: 22 us for the groups of a 96^3 grid, so 4)
+static __global__ __launch_bounds__(NTHR) void k_u0(Params P, int n, int ngrp, const double *__restrict__ selfp,
+                     const double *__restrict__ selfreal, int per_item, int nself, double *uv) {
+  const int b = blockIdx.x * (NTHR / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (b >= n) return;
-  double s = 0.0;
-  for (int g = 0; g < ngrp; ++g) s += selfp[(size_t)b * ngrp + g];
-  double pairep = per_item ? selfreal[b] : selfreal[0];
+  double s = 0.0, pairep = 0.0;
+  for (int g = lane; g < ngrp; g += 64) s += selfp[(size_t)b * ngrp + g];
+  for (int g = lane; g < nself; g += 64) pairep += selfreal[(per_item ? (size_t)b * nself : 0) + g];
+  s = wave_sum(s);
+  pairep = wave_sum(pairep);
   double epcl = 3.1415926535897932 * P.solute_charge * P.solute_charge / P.screen / P.screen / P.volume;
   epcl = epcl / 2.0;
   double res = 0.0 - epcl;
-  uv[(size_t)b * (P.slvmax + 1)] = s + pairep + res;
+  if (lane == 0) uv[(size_t)b * (P.slvmax + 1)] = s + pairep + res;
 }
 
 // --------------------------------------------------------------------------
@@ -2730,7 +2785,14 @@ static __global__ void k_pose_refstr(Params P, int n, const uint64_t *__restrict
   if (P.ins_pos == 6) wsol[b] = weight;
 }
 
-static __global__ __launch_bounds__(NTHR) void k_bin(Params P, const double *__restrict__ uv,
+// A workgroup per configuration, bound by the latency of the binary searches
+// in LDS: a thread runs those of JB molecules together, and where a
+// configuration has more than BIN_MOLS molecules the workgroup has BIN_THR
+// threads (one configuration of 20000 molecules: 99 us, 34 so; 1000 of 4000
+// molecules 118 us, 46, and 46 with 1024 threads; 5000 of 7900 in FP32, four
+// species, 0.50 ms, and 0.54 with 256).
+constexpr int BIN_THR = 1024, BIN_MOLS = 6000;
+static __global__ __launch_bounds__(BIN_THR) void k_bin(Params P, const double *__restrict__ uv,
                                               const double *__restrict__ edges,
                                               const int *__restrict__ spec_off, const int *__restrict__ uvmax,
                                               const int *__restrict__ uvsoft, const int *__restrict__ mol_spec,
@@ -2739,7 +2801,7 @@ static __global__ __launch_bounds__(NTHR) void k_bin(Params P, const double *__r
   extern __shared__ __align__(16) unsigned char lds_raw[];
   double *e = reinterpret_cast<double *>(lds_raw);
   // per-thread, per-species energy sums [numslv][blockDim.x] (each thread
-  // adds only to its own slots; they are summed in thread order below, so
+  // adds only to its own slots; they are summed in a fixed order below, so
   // flceng does not depend on the order the threads run in)
   double *part = e + P.ermax;
   int *h = reinterpret_cast<int *>(part + (size_t)P.numslv * blockDim.x);
@@ -2771,7 +2833,7 @@ static __global__ __launch_bounds__(NTHR) void k_bin(Params P, const double *__r
     }
   };
   // a thread's molecules j = tid, tid + blockDim.x, ... in order, their
-  // energies and species loaded four at a time (all in flight together)
+  // energies and species loaded and their bins searched four at a time
   constexpr int JB = 4;
   for (int j0 = threadIdx.x; j0 < P.slvmax; j0 += JB * (int)blockDim.x) {
     double vb[JB];
@@ -2781,6 +2843,28 @@ static __global__ __launch_bounds__(NTHR) void k_bin(Params P, const double *__r
       const int jk = min(j0 + k * (int)blockDim.x, P.slvmax - 1);
       vb[k] = u[jk];
       sb[k] = mol_spec[jk];
+    }
+    // lo[k]: edges of the species below the energy
+    int lob[JB], hib[JB], ob[JB];
+#pragma unroll
+    for (int k = 0; k < JB; ++k) {
+      const bool ok = sb[k] > 0 && sb[k] <= P.numslv;
+      ob[k] = ok ? spec_off[sb[k] - 1] : 0;
+      hib[k] = ok ? uvmax[sb[k] - 1] : 0;
+      lob[k] = 0;
+    }
+    bool more = true;
+    while (more) {
+      more = false;
+#pragma unroll
+      for (int k = 0; k < JB; ++k) {
+        const bool on = lob[k] < hib[k];
+        const int mid = (lob[k] + hib[k]) >> 1;
+        const bool below = e[ob[k] + (on ? mid : 0)] < vb[k];
+        hib[k] = (on && !below) ? mid : hib[k];
+        lob[k] = (on && below) ? mid + 1 : lob[k];
+        more |= lob[k] < hib[k];
+      }
     }
 #pragma unroll
     for (int k = 0; k < JB; ++k) {
@@ -2793,15 +2877,7 @@ static __global__ __launch_bounds__(NTHR) void k_bin(Params P, const double *__r
         continue;
       }
       double v = vb[k];
-      int off = spec_off[pti - 1], n = uvmax[pti - 1];
-      int lo = 0, hi = n;
-      while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (e[off + mid] < v)
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
+      const int off = ob[k], n = uvmax[pti - 1], lo = lob[k];
       if (lo <= 0) {
         set_error(status, 1, first + b, j, v);
         continue;
@@ -2835,12 +2911,16 @@ static __global__ __launch_bounds__(NTHR) void k_bin(Params P, const double *__r
   flush_spec();
   __syncthreads();
   for (int t = threadIdx.x; t < P.ermax; t += blockDim.x) hist[(size_t)b * P.ermax + t] = (double)h[t];
-  if (threadIdx.x < P.numslv) {
+  // a wave per species adds the threads' sums
+  for (int q = threadIdx.x >> 6; q < P.numslv; q += blockDim.x >> 6) {
     double sum = 0.0;
-    for (int t = 0; t < (int)blockDim.x; ++t) sum += part[(size_t)threadIdx.x * blockDim.x + t];
-    flceng[(size_t)b * MAXSPEC + threadIdx.x] = sum;
-    atomicMin(&mnmx[2 * (threadIdx.x + 1)], mn[threadIdx.x]);
-    atomicMax(&mnmx[2 * (threadIdx.x + 1) + 1], mx[threadIdx.x]);
+    for (int t = threadIdx.x & 63; t < (int)blockDim.x; t += 64) sum += part[(size_t)q * blockDim.x + t];
+    sum = wave_sum(sum);
+    if ((threadIdx.x & 63) == 0) {
+      flceng[(size_t)b * MAXSPEC + q] = sum;
+      atomicMin(&mnmx[2 * (q + 1)], mn[q]);
+      atomicMax(&mnmx[2 * (q + 1) + 1], mx[q]);
+    }
   }
 }
 

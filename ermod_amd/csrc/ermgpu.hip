@@ -753,7 +753,8 @@ template <typename T> int frame_prep(erm_ctx *c) {
   // when they fit the workgroup-local counts, else g3
   const int K3 = k.K3;
   const bool zsort = (c->P.cltype != ERM_EL_COULOMB);
-  const int KB = (K3 * ZCLASS <= ZBUCKET_MAX) ? ZCLASS : 1, nbk = K3 * KB;
+  const int ncls = sizeof(T) == 4 ? ZCLASS : ZCLASS / 2;
+  const int KB = (K3 * ncls <= ZBUCKET_MAX) ? ncls : 1, nbk = K3 * KB;
   // values of a real row in LDS, in the kernel the grid will take
   Fft2 f2;
   const bool xy = (c->P.pme_path == 0 || c->P.pme_path == 3) && fft2_split<T>(k.K1, f2) && fft2_split<T>(k.K2, f2);

@@ -1466,21 +1466,24 @@ template <bool ONE> static __global__ void k_mol_sum(Params P, int nsites, int n
 
 // per-frame sort of the solvent sites by grid base g3 (z-sorted copies of
 // base, charge and B-spline weights, the latter one record [3][p] per site,
-// [nsites][3][p]).  Within a plane (KB = ZCLASS) the sites are dealt over
-// the 32 LDS bank classes (rowp g2 + g1) mod 32 of their gather reads (rowp
-// values per real row; a plane is a multiple of 32 values, so the class does
-// not depend on the plane or on the stencil offsets): round r takes the r-th site of every class that has one, the
-// classes in the order 0, 2, ..., 30, 1, 3, ..., 31.  Any 32 consecutive
-// sites of full rounds then read 32 distinct banks, and any 16 read distinct
-// bank pairs, so a half-wave's gather reads do not conflict.  KB = 1: by
-// plane only.
+// [nsites][3][p]).  Within a plane the sites are dealt over the KB LDS bank
+// classes (rowp g2 + g1) mod KB of their gather reads (rowp values per real
+// row; a plane is a multiple of 32 values, so the class does not depend on the
+// plane or on the stencil offsets): round r takes the r-th site of every class
+// that has one.  FP32: KB = 32, a bank each, the classes in the order 0, 2, ...,
+// 30, 1, 3, ..., 31: any 32 consecutive sites of full rounds read 32 distinct
+// banks, and any 16 read distinct bank pairs.  FP64: KB = 16, a bank pair each,
+// since an LDS pass serves 16 lanes of 8 bytes (with the 32 classes two of any
+// 16 sites met: 1000 configurations on 48^3 508 -> 490 us, 500 on 64^3 of order
+// 6 941 -> 859).  KB = 1: by plane only.
 constexpr int ZBUCKET_MAX = 4096;
 constexpr int ZCLASS = 32;
 // bucket of a site: plane g3, then the dealing position of its class
 __device__ __forceinline__ int zbucket(int g, int KB, int rowp) {
   const int g3 = (g >> 20) & 1023;
   if (KB == 1) return g3;
-  const int c = (rowp * ((g >> 10) & 1023) + (g & 1023)) & (ZCLASS - 1);
+  const int c = (rowp * ((g >> 10) & 1023) + (g & 1023)) & (KB - 1);
+  if (KB == ZCLASS / 2) return g3 * KB + c;
   return g3 * ZCLASS + ((c & 1) ? ZCLASS / 2 + (c >> 1) : (c >> 1));
 }
 

@@ -1220,7 +1220,8 @@ int run_histogram_at(erm_ctx *c, int n, int first, const HistBufs &hb, bool with
   Params k = c->kp;
   const int E = c->ermax;
   auto bin_lds = [&](int thr) { return (size_t)E * (sizeof(double) + sizeof(int)) + sizeof(double) * (size_t)c->numslv * thr; };
-  const int bthr = (c->slvmax > BIN_MOLS && bin_lds(BIN_THR) <= c->lds_cap) ? BIN_THR : NTHR;
+  int bthr = c->slvmax > BIN_MOLS ? BIN_THR : BIN_THR / 2;
+  while (bthr > NTHR && bin_lds(bthr) > c->lds_cap) bthr /= 2;
   const size_t lb = bin_lds(bthr);
   TRY(set_lds(c, (const void *)k_bin, lb, "k_bin"));
   if (!hb.mol_spec) return fail(c, ERM_E_ENG_BUG, "histogram without the frame's molecule species");

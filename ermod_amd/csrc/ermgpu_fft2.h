@@ -285,15 +285,17 @@ __global__ __launch_bounds__(Z2_MAXT) void k_pme_zcol2(Params P, int A, int B, c
 // three barriers.  The y transform's first step reads Hk straight into
 // registers; the x transform takes two Hermitian rows as one complex row of
 // length K1 (even or odd), and its real rows end in natural order behind
-// a copy of their last p - 1 values for the gather.  Bound by VALU issue (63%
-// busy) and LDS (28% of its cycles are bank conflicts) in turn, a group's
-// phases overlapping with the other workgroup of the CU.  Measured: 500 FP64
-// configurations of 40 x 40 x 80, 12000 sites, 0.32 ms (k_pme_slab 2.71); 701
+// a copy of their last p - 1 values for the gather.  Bound in FP32 by VALU issue
+// (66% busy at 48^3) and LDS (59%) in turn, in FP64 by LDS (65%), a group's phases
+// overlapping with the other workgroup of the CU; the gather is 40 to 60% of the
+// time, and half its LDS cycles are bank conflicts between sites of a plane's
+// largest class.  Measured: 500 FP64
+// configurations of 40 x 40 x 80, 12000 sites, 0.29 ms (k_pme_slab 2.71); 701
 // FP32 ones of 45 x 60 x 75, 18000 sites, 0.52 ms (3.62).  Against a register
 // FFT per row with the planes staged in LDS and y columns transformed in HBM
 // (the register lengths until then): 1000 configurations of 48^3, 12000 sites,
-// FP64 1.24 -> 0.53 ms, FP32 0.75 -> 0.29; 500 of 64^3, order 6, 21000 sites,
-// FP64 2.23 -> 0.93; 5000 of 64^3, 29200 sites, FP32 with the y columns in
+// FP64 1.24 -> 0.49 ms, FP32 0.75 -> 0.29; 500 of 64^3, order 6, 21000 sites,
+// FP64 2.23 -> 0.86; 5000 of 64^3, 29200 sites, FP32 with the y columns in
 // LDS, 4.03 -> 3.23 ms.
 // --------------------------------------------------------------------------
 // (off lanes, on = false, read where they may and write nothing)

@@ -2788,12 +2788,13 @@ static __global__ void k_pose_refstr(Params P, int n, const uint64_t *__restrict
   if (P.ins_pos == 6) wsol[b] = weight;
 }
 
-// A workgroup per configuration, bound by the latency of the binary searches
-// in LDS: a thread runs those of JB molecules together, and where a
-// configuration has more than BIN_MOLS molecules the workgroup has BIN_THR
-// threads (one configuration of 20000 molecules: 99 us, 34 so; 1000 of 4000
-// molecules 118 us, 46, and 46 with 1024 threads; 5000 of 7900 in FP32, four
-// species, 0.50 ms, and 0.54 with 256).
+// A workgroup per configuration, bound by the latency of a thread's molecules
+// one after another, so it has BIN_THR threads above BIN_MOLS molecules, half of
+// them below (fewer where their sums do not fit the LDS).  Stage times with 256,
+// 512 and 1024 threads: one configuration of 20000 molecules 107, 64 and 42 us;
+// 1000 of 4000 in FP64 75, 72 and 75; 5000 of 7900, four species, 461, 452 and
+// 450 (548 with 256 threads and every workgroup's atomics on the extrema).  Four
+// searches side by side in a thread changed nothing.
 constexpr int BIN_THR = 1024, BIN_MOLS = 6000;
 static __global__ __launch_bounds__(BIN_THR) void k_bin(Params P, const double *__restrict__ uv,
                                               const double *__restrict__ edges,
@@ -2836,7 +2837,7 @@ static __global__ __launch_bounds__(BIN_THR) void k_bin(Params P, const double *
     }
   };
   // a thread's molecules j = tid, tid + blockDim.x, ... in order, their
-  // energies and species loaded and their bins searched four at a time
+  // energies and species loaded four at a time (all in flight together)
   constexpr int JB = 4;
   for (int j0 = threadIdx.x; j0 < P.slvmax; j0 += JB * (int)blockDim.x) {
     double vb[JB];
@@ -2846,28 +2847,6 @@ static __global__ __launch_bounds__(BIN_THR) void k_bin(Params P, const double *
       const int jk = min(j0 + k * (int)blockDim.x, P.slvmax - 1);
       vb[k] = u[jk];
       sb[k] = mol_spec[jk];
-    }
-    // lo[k]: edges of the species below the energy
-    int lob[JB], hib[JB], ob[JB];
-#pragma unroll
-    for (int k = 0; k < JB; ++k) {
-      const bool ok = sb[k] > 0 && sb[k] <= P.numslv;
-      ob[k] = ok ? spec_off[sb[k] - 1] : 0;
-      hib[k] = ok ? uvmax[sb[k] - 1] : 0;
-      lob[k] = 0;
-    }
-    bool more = true;
-    while (more) {
-      more = false;
-#pragma unroll
-      for (int k = 0; k < JB; ++k) {
-        const bool on = lob[k] < hib[k];
-        const int mid = (lob[k] + hib[k]) >> 1;
-        const bool below = e[ob[k] + (on ? mid : 0)] < vb[k];
-        hib[k] = (on && !below) ? mid : hib[k];
-        lob[k] = (on && below) ? mid + 1 : lob[k];
-        more |= lob[k] < hib[k];
-      }
     }
 #pragma unroll
     for (int k = 0; k < JB; ++k) {
@@ -2880,7 +2859,15 @@ static __global__ __launch_bounds__(BIN_THR) void k_bin(Params P, const double *
         continue;
       }
       double v = vb[k];
-      const int off = ob[k], n = uvmax[pti - 1], lo = lob[k];
+      const int off = spec_off[pti - 1], n = uvmax[pti - 1];
+      int lo = 0, hi = n;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (e[off + mid] < v)
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
       if (lo <= 0) {
         set_error(status, 1, first + b, j, v);
         continue;
@@ -2919,11 +2906,16 @@ static __global__ __launch_bounds__(BIN_THR) void k_bin(Params P, const double *
     double sum = 0.0;
     for (int t = threadIdx.x & 63; t < (int)blockDim.x; t += 64) sum += part[(size_t)q * blockDim.x + t];
     sum = wave_sum(sum);
-    if ((threadIdx.x & 63) == 0) {
-      flceng[(size_t)b * MAXSPEC + q] = sum;
-      atomicMin(&mnmx[2 * (q + 1)], mn[q]);
-      atomicMax(&mnmx[2 * (q + 1) + 1], mx[q]);
-    }
+    if ((threadIdx.x & 63) == 0) flceng[(size_t)b * MAXSPEC + q] = sum;
+  }
+  // the species' extrema by the lanes of one wave, and only where they are new:
+  // every workgroup's atomics meet on these few addresses
+  if (threadIdx.x < P.numslv) {
+    unsigned long long *g = mnmx + 2 * (threadIdx.x + 1);
+    if (mn[threadIdx.x] < __hip_atomic_load(g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin(g, mn[threadIdx.x]);
+    if (mx[threadIdx.x] > __hip_atomic_load(g + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(g + 1, mx[threadIdx.x]);
   }
 }
 

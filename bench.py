@@ -42,8 +42,8 @@ FP64_MFMA_PEAK = 78.6      # TFLOP/s dense FP64 MFMA
 FP64_PEAK = 78.6           # TFLOP/s dense FP64 vector
 FP32_PEAK = 157.3          # TFLOP/s dense FP32 vector
 
-STAGE_KERNELS = {"prep": "k_pose + k_solute_prep", "pme_z": "k_pme_zcol_fft", "pme_y": "k_pme_ycol_reg",
-                 "pme_x": "k_pme_xslab", "mol_sum": "k_mol_sum", "pair": "k_pair_tile", "self": "k_selfreal + k_u0",
+STAGE_KERNELS = {"prep": "k_pose + k_solute_prep", "pme_z": "k_pme_zcol_fft",
+                 "pme_x": "k_pme_xyslab", "mol_sum": "k_mol_sum", "pair": "k_pair_tile", "self": "k_selfreal + k_u0",
                  "bin": "k_bin + k_scalars + k_edens", "corr": "k_corr"}
 
 
@@ -100,11 +100,10 @@ def stage_work(sy, T, slvmax, ermax, npair):
         # spread along z + z FFT + Green's function: the spectrum it writes,
         # the per-site x / y spectra and z weights it reads
         "pme_z": ("hbm", hk + ns * (2 * T * (H + K2) + (T + 4) * p + T), 0),
-        "pme_y": ("hbm", 2 * hk, 0),                   # inverse y transform in place
-        # x transform + gather: the potential grid (T K^3) and the per-site
-        # sums it writes; solvent site data (base, charge, 3p weights, index)
-        # once per launch
-        "pme_x": ("hbm", T * K1 * K2 * K3 + 8 * nv, nv * (8 + T * (3 * p + 1))),
+        # y and x transforms + gather: the half spectrum it reads and the
+        # per-site sums it writes; solvent site data (base, charge, 3p
+        # weights, index) once per launch
+        "pme_x": ("hbm", hk + 8 * nv, nv * (8 + T * (3 * p + 1))),
         "mol_sum": ("hbm", 8 * nv + 8 * (slvmax + 1), 16 * slvmax),
         "pair": ("valu", 40.0 * npair, 0),
         "bin": ("hbm", 8 * (slvmax + 1) + 8 * ermax, 4 * slvmax),
@@ -213,8 +212,7 @@ def mixed_setup(torch, dev, nframes):
 
 # the shape the autotuner settles on for the mixed-solvent workload, used
 # when it is skipped (profiling runs)
-FIXED_TUNING = dict(max_batch=1024, pme_path="register", slab_planes=6, group_planes=9, slab_threads=512,
-                    column_threads=256, fold_y=True)
+FIXED_TUNING = dict(max_batch=1024, pme_path="register", slab_planes=6, column_threads=256)
 
 
 def run_mixed(torch, syss, dpos, prec, steps, warmup, per_frame, tune=True, schedule="group", graph_steps=0):
@@ -261,63 +259,28 @@ def run_mixed(torch, syss, dpos, prec, steps, warmup, per_frame, tune=True, sche
             group = ErmGroup(engines)
             total = sum(share)
             if tune:
-                # the group's y/x transforms and gather run in the slab shape
-                # of its first member, autotuned alone on a quarter of the
-                # insertions: the shapes of the fixed tuning compete with it
-                t0m = engines[0].tuning()
-                own = dict(slab_planes=t0m["slab_cap"], group_planes=t0m["group_cap"],
-                           slab_threads=t0m["slab_threads"], fold_y=t0m["fold_y"])
-                # (slab_planes caps the slab depth: 16 gives 8-plane slabs of
-                # 16 sites per thread on this workload, 8 gives 4-plane slabs)
-                shapes = [own] + [dict(slab_planes=sp, group_planes=gp, slab_threads=512, fold_y=fy)
-                                  for sp, gp, fy in ((16, 8, True), (16, 8, False), (8, 8, True), (6, 9, True))]
-
-                def set_shape(shape):
-                    engines[0].set_tuning(max_batch=0, pme_path=t0m["pme_path"], use_graph=False, **shape)
-
-                def frames_min(fs, measure):
-                    # the smallest of a few frames' measures
+                def frames_min(fs):
+                    # the smallest wall time of a few frames
                     t = None
                     for f in fs:
                         torch.cuda.synchronize()
                         t0 = time.perf_counter()
                         frame(f)
                         torch.cuda.synchronize()
-                        tf = measure(time.perf_counter() - t0)
+                        tf = time.perf_counter() - t0
                         t = tf if t is None else min(t, tf)
                     return t
 
-                # batch size and persistence by wall time per frame, in the
-                # first member's own shape
+                # batch size and persistence by wall time per frame
                 best = None
-                set_shape(own)
                 for bmax in ((total + 1) // 2, total):
                     for pers in (0, 1, 2, 3):
                         group.set_tuning(max_batch=bmax, persistent=pers)
                         frame(0)
-                        t = frames_min((1, 2), lambda w: w)
+                        t = frames_min((1, 2))
                         if best is None or t < best[0]:
                             best = (t, bmax, pers)
-                group.set_tuning(max_batch=best[1], persistent=best[2])
-                # the slab shape by the device time of the stages it changes
-                # (y and x transforms and the gather, HIP events on the
-                # stream): frame wall times vary by more than the shapes
-                # differ
-                xy = lambda w: (lambda st: st["pme_y"] + st["pme_x"])(group.stage_times())
-                sbest = None
-                shape_ms = []
-                for si, shape in enumerate(shapes):
-                    set_shape(shape)
-                    frame(0)
-                    t = frames_min((1, 2, 3), xy)
-                    shape_ms.append(round(t, 3))
-                    if sbest is None or t < sbest[0]:
-                        sbest = (t, si)
-                set_shape(shapes[sbest[1]])
-                group_tuning = {"max_batch": best[1], "persistent": best[2],
-                                "slab_shape": "first member's own" if sbest[1] == 0 else shapes[sbest[1]],
-                                "slab_shape_xy_ms": round(sbest[0], 3),
-                                "shapes_xy_ms": [dict(shape, xy_ms=t) for shape, t in zip(shapes, shape_ms)]}
+                group_tuning = {"max_batch": best[1], "persistent": best[2]}
             else:
                 # the group tuning the warm-up timing settles on for this
                 # workload (profiling runs): one batch, both grids persistent
@@ -541,9 +504,6 @@ def main():
         B = r["tuning"][k]["max_batch"]
         n_cfg = args.steps * r["share"][k]
         n_launch = args.steps * int(np.ceil(r["share"][k] / B))
-        folded = r["tuning"][0 if grouped else k]["fold_y"]
-        if folded:
-            work.pop("pme_y")   # the inverse y transform runs inside the x slab
         for stg, (bound, wc, wl) in work.items():
             a = tot.setdefault(stg, dict(bound=bound, work=0.0, ms=0.0, cfg=0, launch=0, wl=wl))
             a["work"] += wc * n_cfg
@@ -558,7 +518,7 @@ def main():
         # pairs once (persistent) or once per solute, the rest once per solute
         nrun = sum(1 for x in r["share"] if x > 0)
         for stg, a in tot.items():
-            once = stg in ("pme_y", "pme_x") or (stg == "pme_z" and pmask & 1) or (stg == "pair" and pmask & 2)
+            once = stg == "pme_x" or (stg == "pme_z" and pmask & 1) or (stg == "pair" and pmask & 2)
             a["launch"] = args.steps * nb_group * (1 if once else nrun)
             a["work"] += a["wl"] * args.steps * nb_group
             a["ms"] = r["stage"][0].get(stg, 0.0)
@@ -589,8 +549,7 @@ def main():
                                   "matrix (FP64 MFMA) per solute; cutoff 12 A, alpha 0.35, PME 64^3 p4",
                       "frames": args.steps, "insertions_per_frame": sum(r["share"]),
                       "precision": args.precision,
-                      "tuning": [{k: t[k] for k in ("max_batch", "pme_path", "slab_planes", "group_planes",
-                                                    "slab_threads", "column_threads", "fold_y")}
+                      "tuning": [{k: t[k] for k in ("max_batch", "pme_path", "slab_planes", "column_threads")}
                                  for t in r["tuning"]],
                       "schedule": {"group": "one group on one stream: y/x transforms and gather one launch over "
                                             "the four solutes; z columns "

@@ -42,9 +42,11 @@ FP64_MFMA_PEAK = 78.6      # TFLOP/s dense FP64 MFMA
 FP64_PEAK = 78.6           # TFLOP/s dense FP64 vector
 FP32_PEAK = 157.3          # TFLOP/s dense FP32 vector
 
-STAGE_KERNELS = {"prep": "k_pose + k_solute_prep", "pme_z": "k_pme_zcol_fft",
-                 "pme_x": "k_pme_xyslab", "mol_sum": "k_mol_sum", "pair": "k_pair_tile", "self": "k_selfreal + k_u0",
+STAGE_KERNELS = {"prep": "k_pose + k_solute_prep", "pme_z": "k_pme_zcol_fft", "pme_y": "k_pme_ycol_reg",
+                 "pme_x": "k_pme_xslab", "mol_sum": "k_mol_sum", "pair": "k_pair_tile", "self": "k_selfreal + k_u0",
                  "bin": "k_bin + k_scalars + k_edens", "corr": "k_corr"}
+# FP64 at 64^3: z columns in two steps, y and x transforms and gather in one kernel
+STAGE_KERNELS64 = dict(STAGE_KERNELS, pme_z="k_pme_zcol2", pme_x="k_pme_xyslab")
 
 
 def pair_count(sy, pos, P, rc=12.0):
@@ -96,19 +98,25 @@ def stage_work(sy, T, slvmax, ermax, npair):
     ns = s.nsite(sy.solute_mol)
     nv = int(sum(s.nsite(m) for m in s.physical()))
     hk = 2 * T * H * K2 * K3                          # half spectrum of one configuration
-    return {
+    work = {
         # spread along z + z FFT + Green's function: the spectrum it writes,
         # the per-site x / y spectra and z weights it reads
         "pme_z": ("hbm", hk + ns * (2 * T * (H + K2) + (T + 4) * p + T), 0),
-        # y and x transforms + gather: the half spectrum it reads and the
-        # per-site sums it writes; solvent site data (base, charge, 3p
-        # weights, index) once per launch
-        "pme_x": ("hbm", hk + 8 * nv, nv * (8 + T * (3 * p + 1))),
+        "pme_y": ("hbm", 2 * hk, 0),                   # inverse y transform in place
+        # x transform + gather: the potential grid (T K^3) and the per-site
+        # sums it writes; solvent site data (base, charge, 3p weights, index)
+        # once per launch
+        "pme_x": ("hbm", T * K1 * K2 * K3 + 8 * nv, nv * (8 + T * (3 * p + 1))),
         "mol_sum": ("hbm", 8 * nv + 8 * (slvmax + 1), 16 * slvmax),
         "pair": ("valu", 40.0 * npair, 0),
         "bin": ("hbm", 8 * (slvmax + 1) + 8 * ermax, 4 * slvmax),
         "corr": ("mfma", 2.0 * ermax * ermax, 0),
     }
+    if T == 8:
+        # y and x transforms + gather read the half spectrum
+        del work["pme_y"]
+        work["pme_x"] = ("hbm", hk + 8 * nv, work["pme_x"][2])
+    return work
 
 
 def measure_peaks(torch, dev):
@@ -167,7 +175,7 @@ def roofline_of(stage, bound, work_cfg, work_launch, ms_total, n_cfg, n_launch, 
     per_launch = total / max(n_launch, 1)
     avg_ms = ms_total / max(n_launch, 1)
     ach = per_launch / (avg_ms * 1e-3) / (1e9 if unit == "GB/s" else 1e12)
-    out = {"kernel": STAGE_KERNELS.get(stage, stage), "stage": stage, "bound": bound, "achieved": ach,
+    out = {"kernel": (STAGE_KERNELS if T == 4 else STAGE_KERNELS64).get(stage, stage), "stage": stage, "bound": bound, "achieved": ach,
            "peak": peak, "unit": unit, "frac": ach / peak, "avg_launch_ms": avg_ms,
            ("bytes_per_launch" if unit == "GB/s" else "flops_per_launch"): per_launch,
            "configs_per_launch": n_cfg / max(n_launch, 1), "launches": n_launch}
@@ -212,7 +220,8 @@ def mixed_setup(torch, dev, nframes):
 
 # the shape the autotuner settles on for the mixed-solvent workload, used
 # when it is skipped (profiling runs)
-FIXED_TUNING = dict(max_batch=1024, pme_path="register", slab_planes=6, column_threads=256)
+FIXED_TUNING = dict(max_batch=1024, pme_path="register", slab_planes=6, group_planes=9, slab_threads=512,
+                    column_threads=256, fold_y=True)
 
 
 def run_mixed(torch, syss, dpos, prec, steps, warmup, per_frame, tune=True, schedule="group", graph_steps=0):
@@ -259,28 +268,63 @@ def run_mixed(torch, syss, dpos, prec, steps, warmup, per_frame, tune=True, sche
             group = ErmGroup(engines)
             total = sum(share)
             if tune:
-                def frames_min(fs):
-                    # the smallest wall time of a few frames
+                # the group's y/x transforms and gather run in the slab shape
+                # of its first member, autotuned alone on a quarter of the
+                # insertions: the shapes of the fixed tuning compete with it
+                t0m = engines[0].tuning()
+                own = dict(slab_planes=t0m["slab_cap"], group_planes=t0m["group_cap"],
+                           slab_threads=t0m["slab_threads"], fold_y=t0m["fold_y"])
+                # (slab_planes caps the slab depth: 16 gives 8-plane slabs of
+                # 16 sites per thread on this workload, 8 gives 4-plane slabs)
+                shapes = [own] + [dict(slab_planes=sp, group_planes=gp, slab_threads=512, fold_y=fy)
+                                  for sp, gp, fy in ((16, 8, True), (16, 8, False), (8, 8, True), (6, 9, True))]
+
+                def set_shape(shape):
+                    engines[0].set_tuning(max_batch=0, pme_path=t0m["pme_path"], use_graph=False, **shape)
+
+                def frames_min(fs, measure):
+                    # the smallest of a few frames' measures
                     t = None
                     for f in fs:
                         torch.cuda.synchronize()
                         t0 = time.perf_counter()
                         frame(f)
                         torch.cuda.synchronize()
-                        tf = time.perf_counter() - t0
+                        tf = measure(time.perf_counter() - t0)
                         t = tf if t is None else min(t, tf)
                     return t
 
-                # batch size and persistence by wall time per frame
+                # batch size and persistence by wall time per frame, in the
+                # first member's own shape
                 best = None
+                set_shape(own)
                 for bmax in ((total + 1) // 2, total):
                     for pers in (0, 1, 2, 3):
                         group.set_tuning(max_batch=bmax, persistent=pers)
                         frame(0)
-                        t = frames_min((1, 2))
+                        t = frames_min((1, 2), lambda w: w)
                         if best is None or t < best[0]:
                             best = (t, bmax, pers)
-                group_tuning = {"max_batch": best[1], "persistent": best[2]}
+                group.set_tuning(max_batch=best[1], persistent=best[2])
+                # the slab shape by the device time of the stages it changes
+                # (y and x transforms and the gather, HIP events on the
+                # stream): frame wall times vary by more than the shapes
+                # differ
+                xy = lambda w: (lambda st: st["pme_y"] + st["pme_x"])(group.stage_times())
+                sbest = None
+                shape_ms = []
+                for si, shape in enumerate(shapes):
+                    set_shape(shape)
+                    frame(0)
+                    t = frames_min((1, 2, 3), xy)
+                    shape_ms.append(round(t, 3))
+                    if sbest is None or t < sbest[0]:
+                        sbest = (t, si)
+                set_shape(shapes[sbest[1]])
+                group_tuning = {"max_batch": best[1], "persistent": best[2],
+                                "slab_shape": "first member's own" if sbest[1] == 0 else shapes[sbest[1]],
+                                "slab_shape_xy_ms": round(sbest[0], 3),
+                                "shapes_xy_ms": [dict(shape, xy_ms=t) for shape, t in zip(shapes, shape_ms)]}
             else:
                 # the group tuning the warm-up timing settles on for this
                 # workload (profiling runs): one batch, both grids persistent
@@ -504,6 +548,9 @@ def main():
         B = r["tuning"][k]["max_batch"]
         n_cfg = args.steps * r["share"][k]
         n_launch = args.steps * int(np.ceil(r["share"][k] / B))
+        folded = r["tuning"][0 if grouped else k]["fold_y"]
+        if folded:
+            work.pop("pme_y", None)   # the inverse y transform runs inside the x slab
         for stg, (bound, wc, wl) in work.items():
             a = tot.setdefault(stg, dict(bound=bound, work=0.0, ms=0.0, cfg=0, launch=0, wl=wl))
             a["work"] += wc * n_cfg
@@ -518,7 +565,7 @@ def main():
         # pairs once (persistent) or once per solute, the rest once per solute
         nrun = sum(1 for x in r["share"] if x > 0)
         for stg, a in tot.items():
-            once = stg == "pme_x" or (stg == "pme_z" and pmask & 1) or (stg == "pair" and pmask & 2)
+            once = stg in ("pme_y", "pme_x") or (stg == "pme_z" and pmask & 1) or (stg == "pair" and pmask & 2)
             a["launch"] = args.steps * nb_group * (1 if once else nrun)
             a["work"] += a["wl"] * args.steps * nb_group
             a["ms"] = r["stage"][0].get(stg, 0.0)
@@ -529,7 +576,7 @@ def main():
             continue
         stage_rows[stg] = roofline_of(stg, a["bound"], a["work"] / a["cfg"], 0.0, a["ms"], a["cfg"], a["launch"], T)
         stage_rows[stg]["ms_total"] = round(a["ms"], 3)
-        if (stg == "pme_z" and pmask & 1) or (stg == "pair" and pmask & 2):
+        if (stg == "pme_z" and pmask & 1 and T == 4) or (stg == "pair" and pmask & 2):
             stage_rows[stg]["kernel"] += "_runs"
     dom = max(stage_rows, key=lambda k: stage_rows[k]["ms_total"])
     roof = dict(stage_rows[dom])
@@ -549,7 +596,8 @@ def main():
                                   "matrix (FP64 MFMA) per solute; cutoff 12 A, alpha 0.35, PME 64^3 p4",
                       "frames": args.steps, "insertions_per_frame": sum(r["share"]),
                       "precision": args.precision,
-                      "tuning": [{k: t[k] for k in ("max_batch", "pme_path", "slab_planes", "column_threads")}
+                      "tuning": [{k: t[k] for k in ("max_batch", "pme_path", "slab_planes", "group_planes",
+                                                    "slab_threads", "column_threads", "fold_y")}
                                  for t in r["tuning"]],
                       "schedule": {"group": "one group on one stream: y/x transforms and gather one launch over "
                                             "the four solutes; z columns "

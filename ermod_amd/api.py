@@ -590,8 +590,10 @@ class ErmGPU:
 
     def set_tuning(self, max_batch=0, pme_path="auto", use_graph=False, slab_planes=0, group_planes=0,
                    slab_threads=0, column_threads=0, fold_y=None):
-        """group_planes, slab_threads and fold_y (None keeps it) are kept and
-        returned by tuning(); the y/x transform kernel chooses its shape."""
+        """fold_y: True / False moves the inverse y transform into the x slab
+        or not; None keeps the current setting.  In FP64 group_planes,
+        slab_threads and fold_y are kept and returned by tuning() alone: the
+        y/x transform kernel chooses its shape."""
         pp = {"auto": 0, "fused": 1, "unfused": 2, "register": 3}[pme_path]
         fy = -1 if fold_y is None else int(bool(fold_y))
         self._check(lib().erm_set_tuning(self.h, int(max_batch), pp, int(bool(use_graph)), int(slab_planes),

@@ -665,6 +665,38 @@ template <typename T> int launch_xyslab(erm_ctx *c, const Params &k, int n) {
   return launch_check(c, "k_pme_xyslab");
 }
 
+// The y and x transforms and the gather of n configurations into d_esite,
+// with stage marks 3 and 4.  FP64 and the two-step lengths take
+// k_pme_xyslab.  The register lengths in FP32 keep whole transforms in a
+// lane (y columns in memory or in the slab, then k_pme_xslab): an energy
+// within its FP32 rounding of a bin's edge counts in the one bin or the
+// other, so another order of the transform's steps moves counts, and a
+// correlation matrix of a few hundred insertions by more than FP32's rounding
+// (with k_pme_xyslab by up to 3e-5 of its norm).  k_pme_xyslab's
+// order cost 0.29 instead of 0.75 ms per 1000 configurations of 48^3.
+template <typename T> int launch_yx(erm_ctx *c, const Params &k, int n, bool regp) {
+  TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
+  if constexpr (sizeof(T) == 4) {
+    if (regp) {
+      int rc = ERM_OK;
+      if (!xslab_folds_y(c)) {
+        rc = ERM_E_UNSUPPORTED;
+        ERM_KSWITCH(k.K2, (rc = launch_ycol_reg<T, KK>(c, k, n)));
+        TRY(rc);
+      }
+      TRY(mark(c, 3));
+      const size_t lx = 2 * sizeof(T) * (size_t)c->xslab_Q * k.H * k.K2;
+      rc = ERM_E_UNSUPPORTED;
+      ERM_KSWITCH(k.K1, (rc = launch_xslab<T, KK>(c, k, n, lx)));
+      TRY(rc);
+      return mark(c, 4);
+    }
+  }
+  TRY(mark(c, 3));
+  TRY(launch_xyslab<T>(c, k, n));
+  return mark(c, 4);
+}
+
 // Slab shape of the fused PME kernels from the frame's z-sorted site counts:
 // the deepest slab (at most tune_S planes) whose busiest slab fits the
 // per-thread site registers (R = 16 or 32), with at most 3x halo planes;
@@ -757,7 +789,8 @@ template <typename T> int frame_prep(erm_ctx *c) {
   const int KB = (K3 * ncls <= ZBUCKET_MAX) ? ncls : 1, nbk = K3 * KB;
   // values of a real row in LDS, in the kernel the grid will take
   Fft2 f2;
-  const bool xy = (c->P.pme_path == 0 || c->P.pme_path == 3) && fft2_split<T>(k.K1, f2) && fft2_split<T>(k.K2, f2);
+  const bool xy = (c->P.pme_path == 0 || c->P.pme_path == 3) && !(c->fp32 && reg_path_ok<T>(c)) &&
+                  fft2_split<T>(k.K1, f2) && fft2_split<T>(k.K2, f2);
   const int rowp = 2 * (xy ? xy2_row(k.K1, k.p) : k.H);
   if (zsort) TRY(ensure(c, c->d_zcount, sizeof(int) * (nbk + 1)));
   const int nclr = std::max(ncell + 1, zsort ? nbk + 1 : 0);
@@ -891,6 +924,17 @@ int stage_configs(erm_ctx *c, const Batch &bt, const Params &k) {
 int prep_sites(int n, int ns) {
   const int nblk = std::max(1, std::min((ns + 7) / 8, 512 / std::max(n, 1)));
   return (ns + nblk - 1) / nblk;
+}
+
+// Order in which k_solute_prep writes a configuration's sites: sorted by z
+// plane within runs of so many sites (1: as given).  The z kernels that spread
+// from plane buckets want it sorted within their chunks.  In FP64 the whole
+// solute is one run; FP32 sums keep the order that they always had
+// (launch_yx), which is the solute's own order but for the register
+// columns.
+template <typename T> int prep_run(const erm_ctx *c, ZKernel zk) {
+  if (!c->fp32 || zk == Z_TWO) return std::max(1, c->ns);
+  return (zk == Z_FFT || zk == Z_FFT256) ? zfft_sch<T> : 1;
 }
 
 // workgroups per configuration of the tiled pair kernel: nchunk chunks of 64
@@ -1063,7 +1107,7 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
   TRY(stage_configs(c, bt, k));
   const int spb = prep_sites(n, ns);
   hipLaunchKernelGGL(k_solute_prep<T>, dim3(n, (ns + spb - 1) / spb), dim3(PREP_THR), sizeof(int) * ns, c->st, k, spb,
-                     dp<double>(c->d_spos),
+                     prep_run<T>(c, zk), dp<double>(c->d_spos),
                      dp<double>(c->d_qslt), dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<V>(c->d_tw3),
                      dp<double>(c->d_sref), dp<int>(c->d_sg3), dp<T>(c->d_sw3), dp<T>(c->d_sqv),
                      dp<V>(c->d_w1h), dp<V>(c->d_w2h), zspec ? dp<V>(c->d_w3h) : (V *)nullptr);
@@ -1083,10 +1127,7 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
     TRY(rz);
     TRY(launch_check(c, "z columns"));
     TRY(mark(c, 2));
-    TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
-    TRY(mark(c, 3));
-    TRY(launch_xyslab<T>(c, k, n));
-    TRY(mark(c, 4));
+    TRY(launch_yx<T>(c, k, n, regp));
     Params kg = k;
     if (!(flags & DO_RESIDUAL)) kg.solute_charge = 0.0;
     TRY(launch_mol_sum(c, kg, n, dp<double>(c->d_esite), dp<int>(c->d_sltj), dp<double>(c->d_uv)));
@@ -1571,7 +1612,7 @@ template <typename T> int gradient_batch(erm_ctx *c, const Batch &bt, const Grad
   TRY(stage_configs(c, bt, k));
   const int spb = prep_sites(n, ns);
   hipLaunchKernelGGL(k_solute_prep<T>, dim3(n, (ns + spb - 1) / spb), dim3(PREP_THR), sizeof(int) * ns, c->st, k, spb,
-                     dp<double>(c->d_spos),
+                     1, dp<double>(c->d_spos),
                      dp<double>(c->d_qslt), dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<V>(c->d_tw3),
                      dp<double>(c->d_sref), dp<int>(c->d_sg3), dp<T>(c->d_sw3), dp<T>(c->d_sqv),
                      dp<V>(c->d_w1h), dp<V>(c->d_w2h), (V *)nullptr);
@@ -1727,6 +1768,7 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
   int Emax = 0;
   for (int r = 0; r < nrun; ++r) sites += (size_t)R[r].ncfg * R[r].ns;
   for (erm_ctx *m : g->ctx) Emax = std::max(Emax, m->ermax);
+  const ZKernel zk = z_kernel(c, true);
   const int nzg = zcol_groups(c, true, (int)sizeof(V));
   TRY(ensure(c, c->d_spos, sizeof(double) * sites * 3));
   TRY(ensure(c, c->d_sref, sizeof(double) * 4 * n));
@@ -1762,7 +1804,7 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
     TRY(launch_check(c, "k_pose"));
     const int spb = prep_sites(R[r].ncfg, m->ns);
     hipLaunchKernelGGL(k_solute_prep<T>, dim3(R[r].ncfg, (m->ns + spb - 1) / spb), dim3(PREP_THR), sizeof(int) * m->ns,
-                       c->st, km, spb, dp<double>(c->d_spos) + so * 3,
+                       c->st, km, spb, prep_run<T>(m, zk), dp<double>(c->d_spos) + so * 3,
                        dp<double>(m->d_qslt), dp<V>(c->d_tw1), dp<V>(c->d_tw2), dp<V>(c->d_tw3),
                        dp<double>(c->d_sref) + 4 * (size_t)R[r].cfg0, dp<int>(c->d_sg3) + so, dp<T>(c->d_sw3) + so * p,
                        dp<T>(c->d_sqv) + so, dp<V>(c->d_w1h) + so * H, dp<V>(c->d_w2h) + so * K2, (V *)nullptr);
@@ -1773,7 +1815,6 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
   hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(32), 0, c->st, dp<int>(g->d_counter), (size_t)4, 0);
   TRY(launch_check(c, "k_fill"));
   // z columns over every run: one persistent launch, or one launch per run
-  const ZKernel zk = z_kernel(c, true);
   if (zk == Z_FFT && (g->persistent & 1)) {
     int rz = ERM_E_UNSUPPORTED;
     ERM_KSWITCH(K3, (rz = launch_zcol_fft_runs<T, KK>(c, k, nzg, d_runs, nrun, nitem_z, dp<int>(g->d_counter))));
@@ -1794,9 +1835,7 @@ template <typename T> int group_batch(erm_group *g, const GRun *R, int nrun, con
     }
   }
   TRY(mark(c, 2));
-  TRY(mark(c, 3));
-  TRY(launch_xyslab<T>(c, k, n));
-  TRY(mark(c, 4));
+  TRY(launch_yx<T>(c, k, n, true));
   for (int r = 0; r < nrun; ++r) {
     erm_ctx *m = g->ctx[R[r].member];
     Params kg = k;
@@ -3163,49 +3202,61 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
   if (c->slab_S) paths.push_back(1);
   paths.push_back(2);
   double best = 1e300;
-  int bestB = c->Bmax, bestP = c->P.pme_path, bestS = c->tune_S, bestZ = 0;
+  int bestB = c->Bmax, bestP = c->P.pme_path, bestS = c->tune_S, bestQ = c->tune_Q, bestT = c->xslab_T, bestZ = 0;
   auto timed = [&](double *ms) -> int {
     Batch bt{n_trial, 0, nullptr, nullptr, nullptr, true, seed, 0};
     TRY(process(c, bt, flags, nullptr));  // warm-up (allocations, first launches)
-    HIPCHK(c, hipEventRecord(c->ev[0], c->st));
-    TRY(process(c, bt, flags, nullptr));
-    HIPCHK(c, hipEventRecord(c->ev[7], c->st));
-    TRY(sync(c));
-    float f = 0;
-    HIPCHK(c, hipEventElapsedTime(&f, c->ev[0], c->ev[7]));
-    *ms = f;
+    *ms = 1e300;
+    for (int rep = 0; rep < 3; ++rep) {
+      auto t0 = std::chrono::steady_clock::now();
+      TRY(process(c, bt, flags, nullptr));
+      const double dt = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+      *ms = std::min(*ms, dt);
+    }
     return ERM_OK;
   };
   c->use_graph = false;
-  auto apply = [&](int B, int pp, int Sc) -> int {
+  auto apply = [&](int B, int pp, int Sc, int Qc, int Tc) -> int {
     c->Bmax = B;
     c->P.pme_path = pp;
     c->tune_S = Sc;
+    c->tune_Q = Qc;
+    c->xslab_T = Tc;
     return c->fp32 ? choose_slab<float>(c) : choose_slab<double>(c);
   };
-  const int S0 = c->tune_S;
+  const int S0 = c->tune_S, Q0 = c->tune_Q, T0 = c->xslab_T;
   for (int B : {128, 256, 512, 1024}) {
     if (B > 4 * n_trial && B > 128) break;
     for (int pp : paths) {
+      // the slab depth shapes the fused LDS path and the FP32 x slab, the
+      // planes per group and the workgroup size the latter alone
+      const bool xs = pp == 3 && c->fp32, deep = pp == 1 || xs;
       for (int Sc : {16, 8, 6, 5, 4, 3}) {
-        // the slab depth shapes the fused LDS path alone
-        if (pp != 1 && Sc != 16) continue;
-        if (apply(B, pp, pp == 1 ? Sc : S0) != ERM_OK) {
-          c->err.clear();
-          continue;
-        }
-        double ms;
-        TRY(timed(&ms));
-        if (ms < best) {
-          best = ms;
-          bestB = B;
-          bestP = pp;
-          bestS = pp == 1 ? Sc : S0;
+        for (int Qc : {16, 9, 8, 5, 4, 3}) {
+          for (int Tc : {256, 512}) {
+            if (!deep && Sc != 16) continue;
+            if (!xs && (Qc != 8 || Tc != 256)) continue;
+            const int S1 = deep ? Sc : S0, Q1 = xs ? Qc : Q0, T1 = xs ? Tc : T0;
+            if (apply(B, pp, S1, Q1, T1) != ERM_OK) {
+              c->err.clear();
+              continue;
+            }
+            double ms;
+            TRY(timed(&ms));
+            if (ms < best) {
+              best = ms;
+              bestB = B;
+              bestP = pp;
+              bestS = S1;
+              bestQ = Q1;
+              bestT = T1;
+            }
+          }
         }
       }
     }
   }
-  TRY(apply(bestB, bestP, bestS));
+  TRY(apply(bestB, bestP, bestS, bestQ, bestT));
   c->batch_set = true;
   if (bestP == 3) {  // z-column workgroup size for the chosen shape
     const int z0 = c->zcol_T;
@@ -3219,6 +3270,20 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
       }
     }
     c->zcol_T = bestZ ? bestZ : z0;
+    // inverse y transform inside the x slab, or its own kernel
+    if (c->fp32 && c->xslab_T == 512 && c->kp.K2 == c->kp.K1) {
+      const bool y0 = c->xslab_yf;
+      int besty = -1;
+      for (int yf : {0, 1}) {
+        c->xslab_yf = (yf == 1);
+        TRY(timed(&ms));
+        if (ms < best) {
+          best = ms;
+          besty = yf;
+        }
+      }
+      c->xslab_yf = (besty >= 0) ? (besty == 1) : y0;
+    }
   }
   // real-space kernel: compacted tiles or one thread per candidate molecule
   {

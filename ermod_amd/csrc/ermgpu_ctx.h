@@ -262,6 +262,9 @@ int launch_zcol_fft(erm_ctx *c, const Params &k, int n, int nblk, size_t site0 =
 template <typename T, int K> int launch_zcol_fft256(erm_ctx *c, const Params &k, int n, int nblk);
 template <typename T, int K>
 int launch_zcol_fft_runs(erm_ctx *c, const Params &k, int nblk, const GRun *runs, int nrun, int nitem, int *counter);
+// FP32 alone (FP64: k_pme_xyslab)
+template <typename T, int K> int launch_ycol_reg(erm_ctx *c, const Params &k, int n);
+template <typename T, int K> int launch_xslab(erm_ctx *c, const Params &k, int n, size_t lds);
 template <typename T, int K> void launch_xr2c(erm_ctx *c, const Params &k);
 template <typename T, int K> void launch_xc2r(erm_ctx *c, const Params &k);
 template <typename T, int K, int SIGN> void launch_ydense(erm_ctx *c, const Params &k);

@@ -292,7 +292,23 @@ template <typename V> __host__ __device__ __forceinline__ V cadd_h(V a, V b) {
   return r;
 }
 
-// R-point DFT, R = 2, 3, 4, 5
+// output q of an R-point DFT: sum_s v[s] w_R^(s q)
+template <int R, int SIGN, int Q, typename V, int... S>
+__host__ __device__ __forceinline__ V dft_out(const V (&v)[R], std::integer_sequence<int, S...>) {
+  V acc = v[0];
+  ((acc = (S == 0) ? acc : cadd_h(acc, rot<SIGN, (S * Q) % R, R>(v[S]))), ...);
+  return acc;
+}
+
+template <int R, int SIGN, typename V, int... Q>
+__host__ __device__ __forceinline__ void dft_outs(const V (&v)[R], V (&o)[R], std::integer_sequence<int, Q...>) {
+  ((o[Q] = dft_out<R, SIGN, Q>(v, std::make_integer_sequence<int, R>{})), ...);
+}
+
+// R-point DFT, R = 2, 3, 4, 5.  Radix 3 and 5 in FP32 sum their terms one by
+// one: the symmetric forms that FP64 takes (half the products) round
+// otherwise, and an FP32 energy beside a bin's edge then counts in another bin
+// than it did.
 template <int R, int SIGN, typename V> __host__ __device__ __forceinline__ void small_dft(const V (&v)[R], V (&o)[R]) {
   if constexpr (R == 4) {
     const V s0 = cadd_h(v[0], v[2]), s1 = cadd_h(v[1], v[3]);
@@ -312,6 +328,8 @@ template <int R, int SIGN, typename V> __host__ __device__ __forceinline__ void 
     o[0] = cadd_h(v[0], v[1]);
     o[1].x = v[0].x - v[1].x;
     o[1].y = v[0].y - v[1].y;
+  } else if constexpr (sizeof(v[0].x) == 4) {
+    dft_outs<R, SIGN>(v, o, std::make_integer_sequence<int, R>{});
   } else if constexpr (R == 3) {
     // v1 w + v2 w^2 = -(v1 + v2) / 2 + SIGN i sin(2 pi / 3) (v1 - v2)
     using S = decltype(v[0].x);
@@ -408,6 +426,38 @@ template <int N, int SIGN, typename V> __host__ __device__ __forceinline__ void 
   static_assert(Fact<N>::valid(), "FFT length must factor into 2, 3, 4, 5");
   dif<N, N, 0, SIGN>(x);
   dif_unscramble<N>(x, std::make_integer_sequence<int, N>{});
+}
+
+// Inverse real transform of one Hermitian row through a half-length complex
+// FFT: for k < M = N/2 with X[0] and X[M] taken as real,
+//   E[k] = X[k] + conj X[M-k],  O[k] = (X[k] - conj X[M-k]) e^{+2 pi i k/N},
+//   z = IFFT_M(E + i O)  gives  x[2m] = Re z[m], x[2m+1] = Im z[m]
+// (unnormalised, e^{+i}), i.e. x[n] = sum_{k<N} X[k] e^{2 pi i k n / N}.
+template <typename V> __host__ __device__ __forceinline__ V c2r_one(V a, V b, V w) {
+  V e, d, z;
+  e.x = a.x + b.x;
+  e.y = a.y - b.y;
+  d.x = a.x - b.x;
+  d.y = a.y + b.y;
+  const V o = cmul_h(d, w);
+  z.x = e.x - o.y;
+  z.y = e.y + o.x;
+  return z;
+}
+
+template <int N, typename V, int... K>
+__host__ __device__ __forceinline__ void c2r_pack(const V *__restrict__ X, V (&Z)[N / 2],
+                                                  std::integer_sequence<int, K...>) {
+  constexpr int M = N / 2;
+  V x0 = X[0], xm = X[M];
+  x0.y = 0;
+  xm.y = 0;
+  ((Z[K] = c2r_one(K == 0 ? x0 : X[K], K == 0 ? xm : X[M - K], root_v<V, +1, K, N>())), ...);
+}
+
+template <int N, typename V> __host__ __device__ __forceinline__ void c2r_half(const V *__restrict__ X, V (&Z)[N / 2]) {
+  c2r_pack<N>(X, Z, std::make_integer_sequence<int, N / 2>{});
+  reg_fft<N / 2, +1>(Z);
 }
 
 // the same with the (unused) twiddle table of the axis, for the kernels that

@@ -460,10 +460,10 @@ static __global__ __launch_bounds__(64) void k_pose(Params P, int n, const uint6
 
 // Solute configurations for the PME kernels: the reference point (sref), and
 // per site its z plane, z weights, charge and the spectra of its weights
-// along x and y (z too when w3h is given).  The sites are written in the order
-// of (z plane, index), which is how the z-column kernels read them: they
-// ranked every chunk again in each of their workgroups before (5000 FP32
-// configurations of 5 to 150 sites at 64^3: z columns 2.93 -> 2.37 ms).
+// along x and y (z too when w3h is given).  Each run of `run` sites is written
+// in the order of (z plane, index), which is how the z-column kernels read
+// them: they ranked every chunk again in each of their workgroups before (5000
+// FP32 configurations of 5 to 150 sites at 64^3: z columns 2.93 -> 2.37 ms).
 // Grid (configuration, block of spb sites): one block per configuration of a
 // full batch, up to one per 8 sites where a few configurations would leave
 // the chip idle (one solute of 300 sites, 96^3: 0.34 -> 0.03 ms).  Bound by the spectra
@@ -471,7 +471,7 @@ static __global__ __launch_bounds__(64) void k_pose(Params P, int n, const uint6
 constexpr int PREP_THR = 128;
 constexpr int PREP_SITES = 64;  // sites per chunk through LDS
 template <typename T>
-__global__ __launch_bounds__(PREP_THR) void k_solute_prep(Params P, int spb, const double *__restrict__ spos,
+__global__ __launch_bounds__(PREP_THR) void k_solute_prep(Params P, int spb, int run, const double *__restrict__ spos,
                                                      const double *__restrict__ qsolute,
                                                      const typename C2<T>::type *__restrict__ tw1,
                                                      const typename C2<T>::type *__restrict__ tw2,
@@ -551,11 +551,11 @@ __global__ __launch_bounds__(PREP_THR) void k_solute_prep(Params P, int spb, con
         wsh[((t / 3) * 3 + d) * MAXP + k] = spline_value_dev(P.coeff, p, factor - (double)(rci - k));
       gsh[(t / 3) * 3 + d] = rci % Ks[d];
     }
-    // the site's place in the order of (plane, index)
+    // the site's place: its run's sites in the order of (plane, index)
     for (int t = threadIdx.x; t < nc; t += PREP_THR) {
-      const int s = s0c + t, g = prep_g3[s];
-      int r = 0;
-      for (int u = 0; u < ns; ++u) {
+      const int s = s0c + t, g = prep_g3[s], u0 = s - s % run, u1 = min(ns, u0 + run);
+      int r = u0;
+      for (int u = u0; u < u1; ++u) {
         const int gu = prep_g3[u];
         r += (gu < g || (gu == g && u < s)) ? 1 : 0;
       }
@@ -866,8 +866,11 @@ __global__ __launch_bounds__(NTHR) void k_pme_slab(Params P, int S, int nsites,
 //                  self energy (recpcal.F90:377-398), inverse z FFT -> Hk
 //  k_pme_zcol_fft  the same from the z spread and a forward z FFT (spline
 //                  orders 4 and 6)
-// The y and x transforms and the gather follow in k_pme_xyslab
-// (ermgpu_fft2.h).
+// The y and x transforms and the gather follow in k_pme_xyslab (FP64,
+// ermgpu_fft2.h), or in FP32 in
+//  k_pme_ycol_reg  column (z, m1): y FFT in place in Hk (inverse by default)
+//  k_pme_xslab     slab of z planes: x c2r of row pairs into an LDS ring of
+//                  planes, then the gather into per-site FP64 sums
 // --------------------------------------------------------------------------
 constexpr int ZREG_SCH = 16;  // solute sites per LDS chunk of k_pme_zcol_reg
 
@@ -1389,7 +1392,7 @@ __global__ __launch_bounds__(XT) void k_pme_zcol_fft_runs(Params P, const T *__r
 }
 
 // y transform of the columns (z, m1) of a half spectrum in place, one lane
-// per column (the adjoint's solvent grid)
+// per column (FP32 configurations and the adjoint's solvent grid)
 template <typename T, int K2, int SIGN = +1>
 __global__ __launch_bounds__(NTHR) void k_pme_ycol_reg(Params P, const typename C2<T>::type *__restrict__ tw2,
                                                        typename C2<T>::type *Hk) {
@@ -1405,6 +1408,288 @@ __global__ __launch_bounds__(NTHR) void k_pme_ycol_reg(Params P, const typename 
   reg_fft<K2, SIGN>(X, tw2);
 #pragma unroll
   for (int y = 0; y < K2; ++y) col[(size_t)y * H] = X[y];
+}
+
+// Slab of z planes [zb, zb + S) of configuration b.  The planes a site
+// touches, [g3 - p + 1, g3], are processed Q at a time: the Q complex planes
+// Hk[b][z][y][m1] are copied into LDS with coalesced loads; thread (q, y)
+// holds row y of plane q in registers and inverts it through a half-length
+// complex FFT (c2r_half), then writes the real row in place over its own
+// complex row as (x[2m], x[2m+1]) pairs with a row stride of K1 + 2 values
+// (consecutive lanes on distinct LDS banks; each real row fills exactly its
+// complex row's bytes), and repeats x[0], x[1] in the row's two spare values
+// K1, K1 + 1.  Each thread then adds the planes' contributions to its MAXR
+// owned sites (FP64 sums).
+// gather of one group of nq real planes (first plane zz0, rows of K1 + 2)
+// into the per-site sums acc[] of the sites a thread owns.  PP: the spline
+// order at compile time (weights, row offsets and the p^3 products in
+// registers, loads independent); PP = 0 takes it from P.p.
+template <typename T, int K1, int MAXR, int PP, int XT>
+__device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int zz0, int nq, int s_beg,
+                                             const int *gz, const int *__restrict__ zg, const T *__restrict__ zq,
+                                             const T *__restrict__ zw, double *acc) {
+  constexpr int K1P = K1 + 2;
+  const int K2 = P.K2, p = PP ? PP : P.p;
+  const size_t plane = (size_t)K2 * (K1 / 2 + 1) * 2;  // reals per plane
+#pragma unroll
+  for (int r = 0; r < MAXR; ++r) {
+    const int g3 = gz[r];
+    const int clo = max(0, g3 - (zz0 + nq - 1)), chi = min(p - 1, g3 - zz0);
+    if (clo > chi) continue;
+    int idx = s_beg + r * XT + (int)threadIdx.x;
+    // formed here, not hoisted out of the caller's plane-group loop (which
+    // would hold the load addresses of every site in registers across the
+    // transforms)
+    asm volatile("" : "+v"(idx));
+    const int gp = zg[idx];
+    const int g1 = gp & 1023, g2 = (gp >> 10) & 1023;
+    const T qv = zq[idx];
+    const T *wz = zw + (size_t)idx * 3 * p;  // the site's weights [3][p]
+    if constexpr (PP > 0) {
+      T w1[PP], w2[PP];
+      int xo[PP], yo[PP];
+#pragma unroll
+      for (int k = 0; k < PP; ++k) {
+        w1[k] = wz[k];
+        w2[k] = wz[PP + k];
+        int x = g1 - k, y = g2 - k;
+        xo[k] = x + ((x < 0) ? K1 : 0);
+        yo[k] = (y + ((y < 0) ? K2 : 0)) * K1P;
+      }
+      for (int c3 = clo; c3 <= chi; ++c3) {
+        const T *ph = real + (size_t)(g3 - c3 - zz0) * plane;
+        T sum = 0;
+#pragma unroll
+        for (int c2 = 0; c2 < PP; ++c2) {
+          const T *row = ph + yo[c2];
+          T rs = 0;
+#pragma unroll
+          for (int c1 = 0; c1 < PP; ++c1) rs += w1[c1] * row[xo[c1]];
+          sum += w2[c2] * rs;
+        }
+        acc[r] += (double)(qv * wz[2 * PP + c3] * sum);
+      }
+    } else {
+      T w1[MAXP], w2[MAXP];
+      for (int k = 0; k < p; ++k) {
+        w1[k] = wz[k];
+        w2[k] = wz[p + k];
+      }
+      for (int c3 = clo; c3 <= chi; ++c3) {
+        const T *ph = real + (size_t)(g3 - c3 - zz0) * plane;
+        T sum = 0;
+        for (int c2 = 0; c2 < p; ++c2) {
+          int y = g2 - c2;
+          y += (y < 0) ? K2 : 0;
+          const T *row = ph + (size_t)y * K1P;
+          T rs = 0;
+          for (int c1 = 0; c1 < p; ++c1) {
+            int xx = g1 - c1;
+            xx += (xx < 0) ? K1 : 0;
+            rs += w1[c1] * row[xx];
+          }
+          sum += w2[c2] * rs;
+        }
+        acc[r] += (double)(qv * wz[2 * p + c3] * sum);
+      }
+    }
+  }
+}
+
+// The gather for spline order 4.  The weights of the owned sites that touch
+// the group are loaded four sites at a time (each site's twelve weights are
+// one 16-byte-aligned record: three 16-byte loads in FP32), so their loads
+// are in flight together (one wait per four sites rather than one per
+// site).  The four x values g1 - 3 .. g1 of a row are two pairs of adjacent
+// values, (xa, xa + 1) and (xb, xb + 1), each one two-value LDS read: with
+// x[0], x[1] repeated at K1, K1 + 1 every wrap of the stencil over the row's
+// end is such a pair (g1 = 0: (K1-3, K1-2), (K1-1, K1); g1 = 1: (K1-2, K1-1),
+// (0, 1); g1 = 2: (K1-1, K1), (1, 2)).  Products and sums are formed in the
+// order of xslab_gather, so both give the same values.
+template <typename T, int K1, int MAXR, int XT>
+__device__ __forceinline__ void xslab_gather4(const Params &P, const T *real, int zz0, int nq, int s_beg,
+                                              size_t np, const int *gz, const int *__restrict__ zg,
+                                              const T *__restrict__ zq, const T *__restrict__ zw, double *acc) {
+  constexpr int K1P = K1 + 2;
+  const int K2 = P.K2;
+  const ptrdiff_t plane = (ptrdiff_t)K2 * (K1 / 2 + 1) * 2;  // reals per plane
+  constexpr int RB = MAXR < 4 ? MAXR : 4;  // sites whose loads fly together
+#pragma unroll
+  for (int r0 = 0; r0 < MAXR; r0 += RB) {
+    int gp[RB];
+    T qv[RB], w[RB][12];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      // site r meets the group's planes [zz0, zz0 + nq) when
+      // g3 - 3 <= zz0 + nq - 1 and g3 >= zz0 (none for the padding, g3 < 0)
+      const int g3 = gz[r0 + i];
+      const bool need = g3 >= zz0 && g3 <= zz0 + nq + 2;
+      gp[i] = 0;
+      qv[i] = 0;
+#pragma unroll
+      for (int k = 0; k < 12; ++k) w[i][k] = 0;
+      if (__builtin_amdgcn_ballot_w64(need)) {  // uniform: some lane's site r
+        int idx = min(s_beg + (r0 + i) * XT + (int)threadIdx.x, (int)np - 1);
+        asm volatile("" : "+v"(idx));  // not hoisted out of the plane-group loop
+        gp[i] = zg[idx];
+        qv[i] = zq[idx];
+        const T *wz = static_cast<const T *>(__builtin_assume_aligned(zw + (size_t)idx * 12, 16));
+#pragma unroll
+        for (int k = 0; k < 12; ++k) w[i][k] = wz[k];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const int r = r0 + i;
+      const int g3 = gz[r];
+      const int clo = max(0, g3 - (zz0 + nq - 1)), chi = min(3, g3 - zz0);
+      if (clo > chi) continue;
+      const int g1 = gp[i] & 1023, g2 = (gp[i] >> 10) & 1023;
+      const int xa = g1 - 3 + ((g1 < 3) ? K1 : 0);
+      const int xb = g1 - 1 + ((g1 < 1) ? K1 : 0);
+      int ra[4], rb[4];  // the row's two pairs, offsets within a plane
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int y = g2 - k;
+        const int ro = (y + ((y < 0) ? K2 : 0)) * K1P;
+        ra[k] = ro + xa;
+        rb[k] = ro + xb;
+      }
+      const T *ph0 = real + (ptrdiff_t)(g3 - zz0) * plane;  // plane of c3 = 0
+#pragma unroll
+      for (int c3 = 0; c3 < 4; ++c3) {
+        if (c3 < clo || c3 > chi) continue;
+        const T *ph = ph0 - (ptrdiff_t)c3 * plane;
+        T sum = 0;
+#pragma unroll
+        for (int c2 = 0; c2 < 4; ++c2) {
+          const T *a = ph + ra[c2], *bb = ph + rb[c2];
+          const T a0 = a[0], a1 = a[1], b0 = bb[0], b1 = bb[1];
+          T rs = 0;
+          rs += w[i][0] * b1;
+          rs += w[i][1] * b0;
+          rs += w[i][2] * a1;
+          rs += w[i][3] * a0;
+          sum += w[i][4 + c2] * rs;
+        }
+        acc[r] += (double)(qv[i] * w[i][8 + c3] * sum);
+      }
+    }
+  }
+}
+
+// Planes [zz0, zz0 + nq) (periodic in K3) of configuration b's spectrum
+// Hk[b][z][m2][m1] into LDS and transformed there: (with YF the inverse y
+// transform per (plane, m1) column, then) the inverse x transform of every
+// row, each real row written over its own complex row with x[0], x[1]
+// repeated at K1, K1 + 1.  Returns the real planes [nq][K2][K1 + 2]; every
+// thread of the workgroup takes part, and the last barrier has been passed.
+template <typename T, int K1, bool YF>
+__device__ __forceinline__ T *xslab_stage(const typename C2<T>::type *__restrict__ Hk,
+                                          typename C2<T>::type *stage, int b, int zz0, int nq, int K2,
+                                          int K3) {
+  using V = typename C2<T>::type;
+  constexpr int H = K1 / 2 + 1;
+  constexpr int K1P = K1 + 2;
+  const int cplane = K2 * H;
+  // the nq complex planes straight into LDS: 16-byte global-to-LDS loads,
+  // one 1 KiB run per wave instruction, all in flight until the wait
+  {
+    const int ln = threadIdx.x & 63, nch = cplane * (int)sizeof(V) / 16;
+    for (int q = 0; q < nq; ++q) {
+      const int z = (((zz0 + q) % K3) + K3) % K3;
+      const uint4 *src = reinterpret_cast<const uint4 *>(Hk + ((size_t)b * K3 + z) * cplane);
+      uint4 *dst = reinterpret_cast<uint4 *>(stage + (size_t)q * cplane);
+      for (int e0 = (int)(threadIdx.x & ~63u); e0 < nch; e0 += blockDim.x)
+        if (e0 + ln < nch)
+          __builtin_amdgcn_global_load_lds(src + e0 + ln, (__attribute__((address_space(3))) void *)(dst + e0), 16,
+                                           0, 0);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+  }
+  __syncthreads();
+  if constexpr (YF) {
+    // inverse y transform of column (q, m1), in place (consecutive lanes
+    // take consecutive m1: distinct banks)
+    for (int t = threadIdx.x; t < nq * H; t += blockDim.x) {
+      const int q = t / H, m1 = t - q * H;
+      V *col = stage + (size_t)q * cplane + m1;
+      V X[K1];
+#pragma unroll
+      for (int m2 = 0; m2 < K1; ++m2) X[m2] = col[(size_t)m2 * H];
+      reg_fft<K1, +1>(X);
+#pragma unroll
+      for (int y = 0; y < K1; ++y) col[(size_t)y * H] = X[y];
+    }
+    __syncthreads();
+  }
+  // the real row (q, y) occupies exactly the bytes of the complex row
+  // (q, y) (K1P = 2H), which only this thread reads: no barrier between
+  // the transform and its write, any number of rows per thread
+  T *real = reinterpret_cast<T *>(stage);
+  for (int t = threadIdx.x; t < nq * K2; t += blockDim.x) {
+    const int q = t / K2, y = t - q * K2;
+    V Z[K1 / 2];
+    c2r_half<K1>(stage + (size_t)q * cplane + (size_t)y * H, Z);
+    V *d = reinterpret_cast<V *>(real + (size_t)q * cplane * 2 + (size_t)y * K1P);
+#pragma unroll
+    for (int m = 0; m < K1 / 2; ++m) d[m] = Z[m];
+    d[K1 / 2] = Z[0];  // x[0], x[1] again at K1, K1 + 1 (the gather's wrap)
+  }
+  __syncthreads();
+  return real;
+}
+
+// YF: the planes arrive before the inverse y transform, which is done here
+// per (plane, m1) column in LDS (K2 = K1), so k_pme_ycol_reg is skipped
+template <typename T, int K1, int MAXR, int XT = NTHR, bool YF = false>
+__global__ __launch_bounds__(XT) void k_pme_xslab(Params P, int S, int Q, int nsites,
+                                                    const typename C2<T>::type *__restrict__ Hk,
+                                                    const typename C2<T>::type *__restrict__ tw1,
+                                                    const int *__restrict__ z_start, const int *__restrict__ zg,
+                                                    const T *__restrict__ zq, const T *__restrict__ zw,
+                                                    const int *__restrict__ zsite, double *e_site) {
+  using V = typename C2<T>::type;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int K2 = P.K2, K3 = P.K3, p = P.p;
+  V *stage = reinterpret_cast<V *>(lds_raw);  // [Q][K2][H] complex, then [Q][K2][K1 + 2] real in place
+  // XCD-aware order: workgroups go to the 8 XCDs round-robin by linear
+  // index, so XCD x is given the x-th contiguous share of the (configuration,
+  // slab) items; consecutive slabs of a configuration then run on one XCD
+  // and find their p - 1 shared halo planes in its L2
+  const int nwg = gridDim.x * gridDim.y;
+  int L = blockIdx.y * gridDim.x + blockIdx.x;
+  if (nwg % 8 == 0) L = (L % 8) * (nwg / 8) + L / 8;
+  const int b = L / gridDim.x;
+  const int zb = (L - b * gridDim.x) * S, ze = min(zb + S, K3);
+  const int s_beg = z_start[zb], s_end = z_start[ze];
+  double acc[MAXR];
+  int gz[MAXR];
+#pragma unroll
+  for (int r = 0; r < MAXR; ++r) {
+    int idx = s_beg + r * (int)blockDim.x + (int)threadIdx.x;
+    acc[r] = 0.0;
+    gz[r] = (idx < s_end) ? ((zg[idx] >> 20) & 1023) : -(1 << 20);
+  }
+  const size_t np = (size_t)nsites;
+  for (int zz0 = zb - p + 1; zz0 < ze; zz0 += Q) {
+    const int nq = min(Q, ze - zz0);
+    T *real = xslab_stage<T, K1, YF>(Hk, stage, b, zz0, nq, K2, K3);
+    // gather: owned sites whose support g3 - c3 meets planes [zz0, zz0 + nq);
+    // the common spline orders get fully unrolled register code
+    if (p == 4)
+      xslab_gather4<T, K1, MAXR, XT>(P, real, zz0, nq, s_beg, np, gz, zg, zq, zw, acc);
+    else if (p == 6)
+      xslab_gather<T, K1, MAXR, 6, XT>(P, real, zz0, nq, s_beg, gz, zg, zq, zw, acc);
+    else
+      xslab_gather<T, K1, MAXR, 0, XT>(P, real, zz0, nq, s_beg, gz, zg, zq, zw, acc);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < MAXR; ++r) {
+    int idx = s_beg + r * (int)blockDim.x + (int)threadIdx.x;
+    if (idx < s_end) e_site[(size_t)b * np + idx] = acc[r];
+  }
 }
 
 // per-molecule reciprocal energy from the per-site sums (stored in the

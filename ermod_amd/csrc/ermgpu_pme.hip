@@ -1,8 +1,9 @@
 // ermgpu_pme.hip -- the register-FFT kernels of one precision and grid
-// length: z columns and the adjoint's solvent-potential transforms.  Compiled
-// once per (ERM_T, ERM_K), or per (ERM_T, list ERM_ZLENS of lengths whose z
-// columns alone are wanted), so that the instantiations build in parallel;
-// ermgpu.hip dispatches on the grid length at run time.
+// length: z columns, in FP32 the y columns and the x slab with the gather, and
+// the adjoint's solvent-potential transforms.  Compiled once per (ERM_T,
+// ERM_K), or per (ERM_T, list ERM_ZLENS of lengths whose z columns alone are
+// wanted), so that the instantiations build in parallel; ermgpu.hip dispatches
+// on the grid length at run time.
 #include <algorithm>
 
 #include "ermgpu_ctx.h"
@@ -85,6 +86,47 @@ int launch_zcol_fft_runs(erm_ctx *c, const Params &k, int nblk, const GRun *runs
   if (c->zcol_T == 512) return launch_zcol_runs_t<T, K, 6, 512>(c, k, nblk, runs, nrun, nitem, counter);
   return launch_zcol_runs_t<T, K, 6, NTHR>(c, k, nblk, runs, nrun, nitem, counter);
 }
+// inverse y columns, one lane per column
+template <typename T, int K> int launch_ycol_reg(erm_ctx *c, const Params &k, int n) {
+  if constexpr (sizeof(T) == 4) {
+    using V = typename C2<T>::type;
+    int nblk = (k.K3 * k.H + NTHR - 1) / NTHR;
+    hipLaunchKernelGGL((k_pme_ycol_reg<T, K>), dim3(nblk, n), dim3(NTHR), 0, c->st, k, dp<V>(c->d_tw2),
+                       dp<V>(c->d_Hk));
+    return launch_check(c, "k_pme_ycol_reg");
+  }
+  return fail(c, ERM_E_ENG_BUG, "y columns in FP64");
+}
+template <typename T, int K, int R, int XT = NTHR, bool YF = false>
+int launch_xslab_r(erm_ctx *c, const Params &k, int n, size_t lds) {
+  using V = typename C2<T>::type;
+  TRY(set_lds(c, (const void *)k_pme_xslab<T, K, R, XT, YF>, lds, "k_pme_xslab"));
+  const int nslab = (k.K3 + c->slab_S - 1) / c->slab_S;
+  hipLaunchKernelGGL((k_pme_xslab<T, K, R, XT, YF>), dim3(nslab, n), dim3(XT), lds, c->st, k, c->slab_S, c->xslab_Q,
+                     c->nsites, dp<V>(c->d_Hk), dp<V>(c->d_tw1), dp<int>(c->d_zstart), dp<int>(c->d_zg),
+                     dp<T>(c->d_zq), dp<T>(c->d_zw), dp<int>(c->d_zsite), dp<double>(c->d_esite));
+  return launch_check(c, "k_pme_xslab");
+}
+// slab_R counts sites per thread of a 256-thread workgroup; a 512-thread
+// workgroup owns the same sites with half as many per thread
+template <typename T, int K> int launch_xslab(erm_ctx *c, const Params &k, int n, size_t lds) {
+  if constexpr (sizeof(T) == 4) {
+    if (xslab_folds_y(c)) {
+      if (c->slab_R == 8) return launch_xslab_r<T, K, 4, 512, true>(c, k, n, lds);
+      if (c->slab_R == 16) return launch_xslab_r<T, K, 8, 512, true>(c, k, n, lds);
+      return launch_xslab_r<T, K, 16, 512, true>(c, k, n, lds);
+    }
+    if (c->xslab_T == 512) {
+      if (c->slab_R == 8) return launch_xslab_r<T, K, 4, 512>(c, k, n, lds);
+      if (c->slab_R == 16) return launch_xslab_r<T, K, 8, 512>(c, k, n, lds);
+      return launch_xslab_r<T, K, 16, 512>(c, k, n, lds);
+    }
+    if (c->slab_R == 8) return launch_xslab_r<T, K, 8>(c, k, n, lds);
+    if (c->slab_R == 16) return launch_xslab_r<T, K, 16>(c, k, n, lds);
+    return launch_xslab_r<T, K, 32>(c, k, n, lds);
+  }
+  return fail(c, ERM_E_ENG_BUG, "x slab in FP64");
+}
 template <typename T, int K> void launch_xr2c(erm_ctx *c, const Params &k) {
   using V = typename C2<T>::type;
   const int nt = k.K3 * ((k.K2 + 1) / 2);
@@ -117,6 +159,8 @@ ERM_ZLENS
 template int launch_zcol_reg<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int);
 template int launch_zcol_fft<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int, size_t, size_t);
 template int launch_zcol_fft_runs<ERM_T, ERM_K>(erm_ctx *, const Params &, int, const GRun *, int, int, int *);
+template int launch_ycol_reg<ERM_T, ERM_K>(erm_ctx *, const Params &, int);
+template int launch_xslab<ERM_T, ERM_K>(erm_ctx *, const Params &, int, size_t);
 template void launch_xr2c<ERM_T, ERM_K>(erm_ctx *, const Params &);
 template void launch_xc2r<ERM_T, ERM_K>(erm_ctx *, const Params &);
 template void launch_ydense<ERM_T, ERM_K, -1>(erm_ctx *, const Params &);

@@ -71,7 +71,7 @@ typedef struct erm_params {
   int32_t device;         /* HIP device ordinal */
   int32_t pme_path;       /* reciprocal-space kernels: 0 auto, 1 fused slab with
                              LDS FFTs, 2 separate plane and gather kernels,
-                             3 register-column z FFTs + fused y/x/gather slab */
+                             3 register-column FFTs + fused x/gather slab */
   int32_t cltype;         /* electrostatics, the reference's numbering
                              (engmain.F90:314): ERM_EL_COULOMB bare 1/r
                              (realcal_bare), ERM_EL_PME, ERM_EL_PPPM; Ewald (1)
@@ -376,20 +376,22 @@ int32_t erm_stage_times(const erm_ctx *ctx, double *ms10);
  * pme_path as in erm_params; use_graph = 1 replays erm_insert_random calls
  * without uvengy from a captured HIP graph (the first call of a given shape
  * runs eagerly and captures; a change of frame geometry, batch shape or
- * buffers re-captures); slab_planes (1..16) caps the z planes of one slab of
- * the fused LDS path (pme_path 1); column_threads (256 or 512) is the
- * workgroup size of the register path's z columns (0 keeps either).
- * group_planes, slab_threads and fold_y are kept and returned by
- * erm_get_tuning: the y and x transforms of the register and two-step paths
- * run as one kernel that chooses its own shape (fold_y = -1 keeps the
- * setting). */
+ * buffers re-captures); slab_planes (1..16) caps the z planes of one fused
+ * PME slab (paths 1 and 3) and group_planes (1..16) the planes the FP32
+ * register path transforms per group, slab_threads and column_threads (256 or
+ * 512) the workgroup sizes of its x slab and of the z columns (0 keeps any of
+ * them); fold_y = 1 moves the inverse y transform into 512-thread x slabs of a
+ * grid with K2 = K1, 0 keeps it in its own kernel, -1 keeps the setting.  In
+ * FP64 group_planes, slab_threads and fold_y are kept and returned by
+ * erm_get_tuning: there, as for the grid lengths without a register kernel,
+ * the y and x transforms run as one kernel that chooses its own shape. */
 int32_t erm_set_tuning(erm_ctx *ctx, int32_t max_batch, int32_t pme_path, int32_t use_graph,
                        int32_t slab_planes, int32_t group_planes, int32_t slab_threads,
                        int32_t column_threads, int32_t fold_y);
-/* out10 = {max_batch, pme_path, use_graph, slab_threads (256 / 512), planes
- * of a slab of pme_path 1, group planes under its cap, slab cap, group cap,
- * z-column threads (256 / 512), fold_y with 512 slab_threads and K2 = K1
- * (0 / 1)} */
+/* out10 = {max_batch, pme_path, use_graph, slab threads (256 / 512), slab
+ * planes in use, group planes in use, slab cap, group cap, z-column
+ * threads (256 / 512), y transform inside the x slab (0 / 1; in FP64 the
+ * setting alone)} */
 int32_t erm_get_tuning(const erm_ctx *ctx, int32_t *out10);
 /* Real-space kernel (no counterpart in the reference): 0 (default) walks the
  * candidates in tiles of 64 solvent sites and evaluates the pairs inside the
@@ -399,7 +401,7 @@ int32_t erm_get_tuning(const erm_ctx *ctx, int32_t *out10);
 int32_t erm_set_pair_path(erm_ctx *ctx, int32_t path);
 int32_t erm_get_pair_path(const erm_ctx *ctx);
 /* Times n_trial random insertions (seed) on the current frame for batch
- * sizes 128..1024, every applicable PME path (and slab depth), the
+ * sizes 128..1024, every applicable PME path and slab / group shapes, the
  * real-space kernel, then graph replay against eager launches, and keeps
  * the fastest; accumulators
  * are untouched.  best_ms (optional) receives the chosen time. */

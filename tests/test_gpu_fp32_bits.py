@@ -1,0 +1,68 @@
+"""FP32 energies are the same in every version of the kernels.
+
+A run's histograms count energies in bins, and an energy that differs in its
+FP32 rounding may count in the neighbouring bin: one such count moves a bin of
+a single configuration, or a row of a short run's correlation matrix, by far
+more than the rounding itself.  The energies of golden/fp32_energies.npz (made
+by golden/make_fp32_energies.py) hold what the transforms gave when every
+register length ran them as radix 4, 2, 3, 5 steps within one lane and every
+other length as such steps through LDS.  Only the order of sums in FP64 is
+free, which the tolerance allows for: 1e-10 kcal/mol + 1e-12 relative, where
+FP32 rounds at 1e-7.
+"""
+import dataclasses
+import os
+
+import numpy as np
+import pytest
+
+import oracle as O
+from ermod_amd import synth
+from ermod_amd.api import ErmGPU
+
+pytestmark = pytest.mark.gpu
+
+GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "fp32_energies.npz")
+#: name: (sites, grid, spline order, configurations)
+REGISTER = {
+    "48_order4": (20, (48, 48, 48), 4, 3),
+    "64_order6": (20, (64, 64, 64), 6, 2),
+    "64_sites150": (150, (64, 64, 64), 4, 2),        # two chunks of z columns
+    "mixed_order4": (5, (16, 96, 24), 4, 3),
+    "mixed_order6": (140, (96, 32, 16), 6, 2),
+    "long_z": (12, (24, 16, 96), 4, 2),
+    "order5": (12, (32, 24, 48), 5, 2),              # z columns from the sites' spectra
+}
+OTHER = {
+    "18_20_25": (5, (18, 20, 25), 4, 2),
+    "25_27_30": (70, (25, 27, 30), 6, 2),            # several chunks of sites
+    "36_40_45": (33, (36, 40, 45), 4, 3),
+    "45_50_54": (12, (45, 50, 54), 5, 2),
+    "60_64_80": (12, (60, 64, 80), 4, 2),
+    "25_32_50": (17, (25, 32, 50), 6, 2),
+    "81_90_100": (130, (81, 90, 100), 4, 1),
+    "90_36_108": (12, (90, 36, 108), 4, 1),
+    "96_32_120": (12, (96, 32, 120), 3, 1),
+    "16_24_128": (12, (16, 24, 128), 4, 1),
+    "100_20_75": (12, (100, 20, 75), 4, 1),
+    "30_72_27": (12, (30, 72, 27), 8, 2),
+}
+
+
+def energies(case, index):
+    sites, grid, order, n = case
+    sy = synth.refs20(nwater=220, L=25.0, K=16, nsite=sites)
+    s = sy.system = dataclasses.replace(sy.system, ms=grid, splodr=order)
+    places = [O.place_solute(s.bfcoord, s.solute_mass(sy.solute_mol), sy.cell, *O.random_pose(40 + index, i))
+              for i in range(n)]
+    with ErmGPU(s, "fp32") as g:
+        g.set_frame(sy.frame(0), sy.cell)
+        return g.get_uv_energy(sy.solute_mol, np.array(places))
+
+
+@pytest.mark.parametrize("name", list(REGISTER))
+def test_register_lengths(name):
+    print(f"\n[gpu case] FP32 rounding, register lengths {name} {REGISTER[name]}", flush=True)
+    want = np.load(GOLDEN)[name]
+    got = energies(REGISTER[name], list(REGISTER).index(name))
+    np.testing.assert_allclose(got, want, rtol=1e-12, atol=1e-10)

@@ -516,50 +516,23 @@ template <typename T> bool reg_path_ok(const erm_ctx *c) {
   return reg_len<T>(k.K1) && reg_len<T>(k.K2) && reg_len<T>(k.K3) && (k.K1 % 2 == 0);
 }
 
-// FP32 grid lengths compiled for their z columns alone
-#define ERM_ZSWITCH(K, CALL)                   \
-  switch (K) {                                 \
-    case 18: { constexpr int KK = 18; CALL; } break; \
-    case 20: { constexpr int KK = 20; CALL; } break; \
-    case 25: { constexpr int KK = 25; CALL; } break; \
-    case 27: { constexpr int KK = 27; CALL; } break; \
-    case 30: { constexpr int KK = 30; CALL; } break; \
-    case 36: { constexpr int KK = 36; CALL; } break; \
-    case 40: { constexpr int KK = 40; CALL; } break; \
-    case 45: { constexpr int KK = 45; CALL; } break; \
-    case 50: { constexpr int KK = 50; CALL; } break; \
-    case 54: { constexpr int KK = 54; CALL; } break; \
-    case 60: { constexpr int KK = 60; CALL; } break; \
-    case 72: { constexpr int KK = 72; CALL; } break; \
-    case 75: { constexpr int KK = 75; CALL; } break; \
-    case 80: { constexpr int KK = 80; CALL; } break; \
-    case 81: { constexpr int KK = 81; CALL; } break; \
-    case 90: { constexpr int KK = 90; CALL; } break; \
-    case 100: { constexpr int KK = 100; CALL; } break; \
-    default: break;                            \
-  }
-
 // Kernel of the z columns.  Z_SPEC sums the solute's z spectra (register
-// lengths, spline orders without a z FFT kernel), Z_FFT and Z_FFT256 spread
-// and transform a column in registers (orders 4 and 6; the tuned workgroup
-// size, or 256 threads for the lengths with z columns alone), Z_TWO is the
-// two-step kernel, Z_LDS the general one.  The registers win where a column
-// leaves room for two waves per SIMD: 1000 FP32 configurations of 48^3 0.138
-// against 0.250 ms in two steps, FP64 0.335 against 0.416; a 64-point FP64
-// column does not (500 configurations of 64^3, order 6: 0.751 against 0.475).
-// 701 FP32 configurations of 45 x 60 x 75: 0.236 in registers, 0.618 in two
-// steps.
-enum ZKernel { Z_SPEC, Z_FFT, Z_FFT256, Z_TWO, Z_LDS };
+// lengths, spline orders without a z FFT kernel), Z_FFT spreads and transforms
+// a column in registers (orders 4 and 6), Z_TWO is the two-step kernel, Z_LDS
+// the general one.  In FP64 the registers win where a column leaves room for two
+// waves per SIMD: 1000 configurations of 48^3 0.335 against 0.416 ms in two
+// steps; a 64-point column does not (500 configurations of 64^3, order 6: 0.751
+// against 0.475).  FP32 takes registers where the whole grid has register
+// lengths and two steps elsewhere, the order of whose sums each had before
+// (launch_yx).
+enum ZKernel { Z_SPEC, Z_FFT, Z_TWO, Z_LDS };
 ZKernel z_kernel(const erm_ctx *c, bool regp) {
   const int K3 = c->kp.K3;
   const bool p46 = c->kp.p == 4 || c->kp.p == 6;
-  const bool reg = p46 && (c->fp32 ? reg_len<float>(K3) : reg_len<double>(K3) && K3 < 64);
+  const bool reg = p46 && (c->fp32 ? regp : reg_len<double>(K3) && K3 < 64);
   if (regp) return !p46 ? Z_SPEC : reg ? Z_FFT : Z_TWO;
   if (!c->two_step) return Z_LDS;
-  if (reg) return Z_FFT;
-  bool z32 = false;
-  if (c->fp32 && p46) ERM_ZSWITCH(K3, z32 = KK > 0)
-  return z32 ? Z_FFT256 : Z_TWO;
+  return reg ? Z_FFT : Z_TWO;
 }
 // z-column workgroups per configuration
 int zcol_groups(const erm_ctx *c, bool regp, int vb) {
@@ -570,7 +543,7 @@ int zcol_groups(const erm_ctx *c, bool regp, int vb) {
     const int w = zcol_width(c->kp.K3, vb);
     return (ncol + w - 1) / w;
   }
-  const int zt = (c->zcol_T == 512 && zk != Z_FFT256) ? 512 : NTHR;
+  const int zt = (c->zcol_T == 512) ? 512 : NTHR;
   // lanes per column: the spectral form one, the spread-and-FFT form
   // zfft_lanes (vb = 2 sizeof(T))
   const int L = zk == Z_SPEC ? 1 : zfft_lanes(vb / 2, c->kp.K3);
@@ -643,10 +616,16 @@ int launch_zcol2(erm_ctx *c, const Params &k, int n, int nblk, size_t site0 = 0,
   using V = typename C2<T>::type;
   Fft2 f;
   if (!fft2_split<T>(k.K3, f)) return fail(c, ERM_E_ENG_BUG, "two-step z length");
-  const size_t lds = z2_lds<T>(k.K3, k.p);
-  auto *kz = f.B <= 10 ? k_pme_zcol2<T, 10> : k_pme_zcol2<T, fft2_bmax<T>>;
+  const size_t lds = z2_lds_of<T>(k.K3, k.p);
+  auto *kz = [&] {
+    if constexpr (sizeof(T) == 4)
+      return k_pme_zcol2_f32;
+    else
+      return f.B <= 10 ? k_pme_zcol2<T, 10> : k_pme_zcol2<T, 12>;
+  }();
+  const int thr = sizeof(T) == 4 ? z2_threads32(f.A, f.B) : z2_threads(f.B);
   TRY(set_lds(c, (const void *)kz, lds, "k_pme_zcol2"));
-  hipLaunchKernelGGL(kz, dim3(nblk, n), dim3(z2_threads(f.B)), lds, c->st, k, f.A, f.B, dp<T>(c->d_engfac),
+  hipLaunchKernelGGL(kz, dim3(nblk, n), dim3(thr), lds, c->st, k, f.A, f.B, dp<T>(c->d_engfac),
                      dp<int>(c->d_sg3) + site0, dp<T>(c->d_sw3) + site0 * k.p, dp<T>(c->d_sqv) + site0,
                      dp<V>(c->d_w1h) + site0 * k.H, dp<V>(c->d_w2h) + site0 * k.K2, dp<V>(c->d_tw3),
                      dp<V>(c->d_Hk) + cfg0 * k.K3 * (size_t)k.K2 * k.H, dp<double>(c->d_selfp) + cfg0 * nblk);
@@ -672,8 +651,9 @@ template <typename T> int launch_xyslab(erm_ctx *c, const Params &k, int n) {
 // within its FP32 rounding of a bin's edge counts in the one bin or the
 // other, so another order of the transform's steps moves counts, and a
 // correlation matrix of a few hundred insertions by more than FP32's rounding
-// (with k_pme_xyslab by up to 3e-5 of its norm).  k_pme_xyslab's
-// order cost 0.29 instead of 0.75 ms per 1000 configurations of 48^3.
+// (up to 3e-5 of its norm, where the steps were an A-point and a B-point
+// transform).  The two-step lengths' steps in FP32 are those of lds_fft for the
+// same reason.
 template <typename T> int launch_yx(erm_ctx *c, const Params &k, int n, bool regp) {
   TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
   if constexpr (sizeof(T) == 4) {
@@ -736,7 +716,7 @@ template <typename T> int choose_slab(erm_ctx *c) {
     return fail(c, ERM_E_UNSUPPORTED, "register-column PME path does not support this grid");
   Fft2 f;
   c->two_step = c->P.pme_path == 0 && !c->xslab_Q && fft2_split<T>(k.K1, f) && fft2_split<T>(k.K2, f) &&
-                fft2_split<T>(K3, f) && z2_lds<T>(K3, k.p) <= c->lds_cap && xy2_shape<T>(c, 1).S > 0;
+                fft2_split<T>(K3, f) && z2_lds_of<T>(K3, k.p) <= c->lds_cap && xy2_shape<T>(c, 1).S > 0;
   return ERM_OK;
 }
 
@@ -933,8 +913,8 @@ int prep_sites(int n, int ns) {
 // (launch_yx), which is the solute's own order but for the register
 // columns.
 template <typename T> int prep_run(const erm_ctx *c, ZKernel zk) {
-  if (!c->fp32 || zk == Z_TWO) return std::max(1, c->ns);
-  return (zk == Z_FFT || zk == Z_FFT256) ? zfft_sch<T> : 1;
+  if (!c->fp32) return std::max(1, c->ns);
+  return zk == Z_FFT ? zfft_sch<T> : 1;
 }
 
 // workgroups per configuration of the tiled pair kernel: nchunk chunks of 64
@@ -1119,10 +1099,8 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
       rz = launch_zcol2<T>(c, k, n, nzg);
     } else if (zk == Z_SPEC) {
       ERM_KSWITCH(K3, (rz = launch_zcol_reg<T, KK>(c, k, n, nzg)));
-    } else if (zk == Z_FFT) {
+    } else {
       ERM_KSWITCH(K3, (rz = launch_zcol_fft<T, KK>(c, k, n, nzg)));
-    } else if constexpr (sizeof(T) == 4) {
-      ERM_ZSWITCH(K3, (rz = launch_zcol_fft256<T, KK>(c, k, n, nzg)));
     }
     TRY(rz);
     TRY(launch_check(c, "z columns"));

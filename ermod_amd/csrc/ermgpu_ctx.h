@@ -259,7 +259,6 @@ template <typename T, int K> int launch_zcol_reg(erm_ctx *c, const Params &k, in
 // table with a persistent grid)
 template <typename T, int K>
 int launch_zcol_fft(erm_ctx *c, const Params &k, int n, int nblk, size_t site0 = 0, size_t cfg0 = 0);
-template <typename T, int K> int launch_zcol_fft256(erm_ctx *c, const Params &k, int n, int nblk);
 template <typename T, int K>
 int launch_zcol_fft_runs(erm_ctx *c, const Params &k, int nblk, const GRun *runs, int nrun, int nitem, int *counter);
 // FP32 alone (FP64: k_pme_xyslab)

@@ -1,6 +1,6 @@
 // ermgpu_fft2.h -- PME kernels for grid lengths K = A B transformed in two
 // steps: an A-point DFT of x[n1 + B n2] over n2, the twiddle w_K^(n1 k2), a
-// B-point DFT over n1.  Both steps run in registers (A, B <= 16 values) with
+// B-point DFT over n1.  Both steps run in registers (A, B <= 20 values) with
 // one exchange through LDS between them, so a length needs no kernel of its
 // own: the radices are launch arguments.  fft2_split() lists the lengths.
 #pragma once
@@ -13,51 +13,145 @@ struct Fft2 {
   int A, B;
 };
 
-// the largest B: in FP64 12, where a step's values still fit 128 registers
-// beside their addresses
-template <typename T> constexpr int fft2_bmax = sizeof(T) == 4 ? 16 : 12;
-
-// K = A B with A <= B, both with a case in ERM_RADIX_A / _B below (B <= BMAX,
-// a constant in scope)
+// K = A B with cases in the radix switches below.  FP64: A <= B <= 12, where a
+// step's values still fit 128 registers beside their addresses.  FP32: A is a
+// product of the first radices of K in the order 4, 2, 3, 5 and B of the
+// others, so that the two steps are the radix steps of lds_fft (dit_steps).
 template <typename T> inline bool fft2_split(int K, Fft2 &f) {
-  static const int tab[][3] = {{16, 4, 4},  {18, 3, 6},  {20, 4, 5},   {24, 4, 6},   {25, 5, 5},   {27, 3, 9},
-                               {30, 5, 6},  {32, 4, 8},  {36, 6, 6},   {40, 5, 8},   {45, 5, 9},   {48, 6, 8},
-                               {50, 5, 10}, {54, 6, 9},  {60, 6, 10},  {64, 8, 8},   {72, 8, 9},   {75, 5, 15},
-                               {80, 8, 10}, {81, 9, 9},  {90, 9, 10},  {96, 8, 12},  {100, 10, 10}, {108, 9, 12},
-                               {120, 10, 12}, {128, 8, 16}};
-  for (const auto &t : tab)
-    if (t[0] == K && t[2] <= fft2_bmax<T>) {
-      f.A = t[1];
-      f.B = t[2];
-      return true;
-    }
-  return false;
+  static const int t64[][3] = {{16, 4, 4},   {18, 3, 6},  {20, 4, 5},  {24, 4, 6},  {25, 5, 5},  {27, 3, 9},
+                               {30, 5, 6},   {32, 4, 8},  {36, 6, 6},  {40, 5, 8},  {45, 5, 9},  {48, 6, 8},
+                               {50, 5, 10},  {54, 6, 9},  {60, 6, 10}, {64, 8, 8},  {72, 8, 9},  {80, 8, 10},
+                               {81, 9, 9},   {90, 9, 10}, {96, 8, 12}, {100, 10, 10}, {108, 9, 12}, {120, 10, 12}};
+  static const int t32[][3] = {{16, 4, 4},   {18, 6, 3},  {20, 4, 5},  {24, 4, 6},  {25, 5, 5},  {27, 9, 3},
+                               {30, 6, 5},   {32, 4, 8},  {36, 4, 9},  {40, 8, 5},  {45, 9, 5},  {48, 4, 12},
+                               {50, 10, 5},  {54, 6, 9},  {60, 12, 5}, {64, 16, 4}, {72, 8, 9},  {75, 15, 5},
+                               {80, 16, 5},  {81, 9, 9},  {90, 6, 15}, {96, 16, 6}, {100, 20, 5}, {108, 12, 9},
+                               {120, 8, 15}, {128, 16, 8}};
+  auto find = [&](const auto &tab) {
+    for (const auto &t : tab)
+      if (t[0] == K) {
+        f.A = t[1];
+        f.B = t[2];
+        return true;
+      }
+    return false;
+  };
+  return sizeof(T) == 4 ? find(t32) : find(t64);
 }
 
-#define ERM_RADIX_A(A, CALL)                          \
-  switch (A) {                                        \
-    case 3: { constexpr int RR = 3; CALL; } break;    \
-    case 4: { constexpr int RR = 4; CALL; } break;    \
-    case 5: { constexpr int RR = 5; CALL; } break;    \
-    case 6: { constexpr int RR = 6; CALL; } break;    \
-    case 8: { constexpr int RR = 8; CALL; } break;    \
-    case 9: { constexpr int RR = 9; CALL; } break;    \
-    case 10: { constexpr int RR = 10; CALL; } break;  \
-    default: break;                                   \
+#define ERM_RADIX(R, CALL) \
+  case R: { constexpr int RR = R; CALL; } break;
+// FP64
+#define ERM_RADIX_A(A, CALL)                                                                                \
+  switch (A) {                                                                                              \
+    ERM_RADIX(3, CALL) ERM_RADIX(4, CALL) ERM_RADIX(5, CALL) ERM_RADIX(6, CALL) ERM_RADIX(8, CALL)          \
+    ERM_RADIX(9, CALL) ERM_RADIX(10, CALL)                                                                  \
+    default: break;                                                                                         \
   }
-#define ERM_RADIX_B(B, CALL)                          \
-  switch (B) {                                        \
-    case 4: { constexpr int RR = 4; CALL; } break;    \
-    case 5: { constexpr int RR = 5; CALL; } break;    \
-    case 6: { constexpr int RR = 6; CALL; } break;    \
-    case 8: { constexpr int RR = 8; CALL; } break;    \
-    case 9: { constexpr int RR = 9; CALL; } break;    \
-    case 10: { constexpr int RR = 10; CALL; } break;  \
-    case 12: if constexpr (BMAX >= 12) { constexpr int RR = 12; CALL; } break; \
-    case 15: if constexpr (BMAX >= 15) { constexpr int RR = 15; CALL; } break; \
-    case 16: if constexpr (BMAX >= 16) { constexpr int RR = 16; CALL; } break; \
-    default: break;                                   \
+#define ERM_RADIX_B(B, CALL)                                                                                \
+  switch (B) {                                                                                              \
+    ERM_RADIX(4, CALL) ERM_RADIX(5, CALL) ERM_RADIX(6, CALL) ERM_RADIX(8, CALL) ERM_RADIX(9, CALL)          \
+    ERM_RADIX(10, CALL)                                                                                     \
+    case 12: if constexpr (BMAX >= 12) { constexpr int RR = 12; CALL; } break;                              \
+    default: break;                                                                                         \
   }
+// FP32
+#define ERM_RADIX_A32(A, CALL)                                                                              \
+  switch (A) {                                                                                              \
+    ERM_RADIX(4, CALL) ERM_RADIX(5, CALL) ERM_RADIX(6, CALL) ERM_RADIX(8, CALL) ERM_RADIX(9, CALL)          \
+    ERM_RADIX(10, CALL) ERM_RADIX(12, CALL) ERM_RADIX(15, CALL) ERM_RADIX(16, CALL) ERM_RADIX(20, CALL)     \
+    default: break;                                                                                         \
+  }
+#define ERM_RADIX_B32(B, CALL)                                                                              \
+  switch (B) {                                                                                              \
+    ERM_RADIX(3, CALL) ERM_RADIX(4, CALL) ERM_RADIX(5, CALL) ERM_RADIX(6, CALL) ERM_RADIX(8, CALL)          \
+    ERM_RADIX(9, CALL) ERM_RADIX(12, CALL) ERM_RADIX(15, CALL)                                              \
+    default: break;                                                                                         \
+  }
+
+// --------------------------------------------------------------------------
+// The FP32 steps.  They give bit for bit what lds_fft gives with one radix
+// step per trip through LDS, since the bins' counts of an FP32 run move with
+// the transforms' rounding (launch_yx): the same radices in the same order,
+// each input times its table twiddle before the butterfly, products and sums
+// fused where that code's are, which is written out here (explicit fmaf,
+// nothing else contracted).
+// --------------------------------------------------------------------------
+// a times w of a table e^{-2 pi i j / K} (SIGN < 0), or its conjugate.  Of the
+// imaginary part's products lds_fft rounds a.x w.y for a step's twiddles and
+// a.y w.x for a root within a butterfly (ROOT); the same with the conjugate.
+template <int SIGN, bool ROOT = false> __device__ __forceinline__ float2 tmul(float2 a, float2 w) {
+#pragma clang fp contract(off)
+  float2 r;
+  if constexpr (SIGN < 0) {
+    r.x = fmaf(a.x, w.x, -(a.y * w.y));
+    r.y = ROOT ? fmaf(a.x, w.y, a.y * w.x) : fmaf(a.y, w.x, a.x * w.y);
+  } else {
+    r.x = fmaf(a.x, w.x, a.y * w.y);
+    r.y = fmaf(a.y, w.x, -(a.x * w.y));
+  }
+  return r;
+}
+// R-point DFT; tw, str: w_R^j = tw[str j]
+template <int R, int SIGN>
+__device__ __forceinline__ void dit_dft(float2 (&x)[R], const float2 *__restrict__ tw, int str) {
+#pragma clang fp contract(off)
+  if constexpr (R == 4) {
+    const float2 s0 = cadd(x[0], x[2]), d0 = csub(x[0], x[2]), s1 = cadd(x[1], x[3]), d1 = csub(x[1], x[3]);
+    const float2 j = make_float2(-SIGN * d1.y, SIGN * d1.x);
+    x[0] = cadd(s0, s1);
+    x[1] = cadd(d0, j);
+    x[2] = csub(s0, s1);
+    x[3] = csub(d0, j);
+  } else if constexpr (R == 2) {
+    const float2 a = x[0];
+    x[0] = cadd(a, x[1]);
+    x[1] = csub(a, x[1]);
+  } else {
+    float2 y[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      y[q] = x[0];
+#pragma unroll
+      for (int s = 1; s < R; ++s)
+        y[q] = cadd(y[q], (s * q) % R ? tmul<SIGN, true>(x[s], tw[(s * q) % R * str]) : x[s]);
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) x[q] = y[q];
+  }
+}
+// The radix steps of an N-point block of a K-point transform, those before it
+// (with product A) giving its place k: x[n1] in, frequency k + A kk out at
+// x[kk].  tw is the table in memory (read at uniform places), lt the same in
+// LDS (read at the lane's own); A = 1 for the first block (FIRST).
+template <int N, int PP, int SIGN, bool FIRST>
+__device__ __forceinline__ void dit_steps(float2 (&x)[N], int K, int A, int k, const float2 *__restrict__ tw,
+                                          const float2 *lt) {
+  constexpr int R = first_radix(N / PP), M = N / (PP * R);
+  asm volatile("" : "+s"(K));  // the table's values stay out of the registers of other steps
+  float2 y[N];
+#pragma unroll
+  for (int r = 0; r < M; ++r)
+#pragma unroll
+    for (int kk = 0; kk < PP; ++kk) {
+      float2 v[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        v[q] = x[kk + PP * (r + q * M)];
+        if constexpr (FIRST) {
+          if (q && kk) v[q] = tmul<SIGN>(v[q], tw[q * kk * (K / (PP * R))]);
+        } else {
+          if (q) v[q] = tmul<SIGN>(v[q], lt[q * (k + A * kk) * M]);
+        }
+      }
+      dit_dft<R, SIGN>(v, tw, K / R);
+#pragma unroll
+      for (int q = 0; q < R; ++q) y[kk + PP * (q + R * r)] = v[q];
+    }
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = y[i];
+  if constexpr (PP * R < N) dit_steps<N, PP * R, SIGN, FIRST>(x, K, A, k, tw, lt);
+}
 
 // a times the conjugate of w (the twiddle tables hold e^{-2 pi i j / K})
 template <typename V> __device__ __forceinline__ V cmulc(V a, V w) {
@@ -222,6 +316,7 @@ __device__ __forceinline__ void z2_last(const typename C2<T>::type *col, int B, 
   for (int i = 0; i < A; ++i) out[(size_t)(n1 + B * i) * ostr] = x[i];
 }
 
+// (FP64; BMAX bounds the registers)
 template <typename T, int BMAX>
 __global__ __launch_bounds__(Z2_MAXT) void k_pme_zcol2(Params P, int A, int B, const T *__restrict__ engfac,
                                                        const int *__restrict__ sg3, const T *__restrict__ sw3,
@@ -275,6 +370,188 @@ __global__ __launch_bounds__(Z2_MAXT) void k_pme_zcol2(Params P, int A, int B, c
   }
 }
 
+// The FP32 z columns: the same division of work, with the sums and steps in
+// lds_fft's order.  The chunk's sites are added to a plane in the solute's own
+// order (a bit mask per plane holds the sites that reach it), and the inverse
+// transform starts with an A-point step as the forward one does, so a column
+// makes one trip through LDS more.  701 configurations of 45 x 60 x 75 with 33
+// solute sites: 0.66 ms (k_pme_zcol 6.08); 500 of 60^3, order 6: 0.43 (3.37).
+constexpr int Z2_MAXT32 = 320;  // 16 columns x 20 values of n1 or k2
+inline int z2_threads32(int A, int B) { return (Z2_COLS * (A > B ? A : B) + 63) & ~63; }
+__host__ __device__ inline size_t z2_lds32(int K3, int p) {
+  const size_t buf = sizeof(float2) * (size_t)K3 * Z2_COLS;
+  const size_t chunk = sizeof(float2) * (size_t)Z2_SCH * Z2_COLS + sizeof(unsigned long long) * K3 +
+                       (sizeof(float) * p + sizeof(int)) * (size_t)Z2_SCH;
+  return (((buf > chunk ? buf : chunk) + 15) & ~(size_t)15) + sizeof(float2) * K3 + sizeof(double) * (Z2_MAXT32 / 64);
+}
+template <typename T> __host__ __device__ inline size_t z2_lds_of(int K3, int p) {
+  return sizeof(T) == 4 ? z2_lds32(K3, p) : z2_lds<T>(K3, p);
+}
+
+// spread and first forward step of (n1 = sub, column)
+template <int A>
+__device__ __forceinline__ void z2_front32(const Z2Args &q, int B, unsigned char *lds, const float2 *__restrict__ tw,
+                                           const int *__restrict__ sg3, const float *__restrict__ sw3,
+                                           const float *__restrict__ sqv, const float2 *__restrict__ w1h,
+                                           const float2 *__restrict__ w2h) {
+  constexpr int C = Z2_COLS;
+  const int p = q.p, K3 = q.K3;
+  float2 *amp = reinterpret_cast<float2 *>(lds);  // [Z2_SCH][C] q what1 what2 of the chunk's sites
+  unsigned long long *mask = reinterpret_cast<unsigned long long *>(amp + (size_t)Z2_SCH * C);  // [K3]
+  float *wz = reinterpret_cast<float *>(mask + K3);            // [Z2_SCH][p] z weights
+  int *gz = reinterpret_cast<int *>(wz + (size_t)Z2_SCH * p);  // [Z2_SCH] planes g3
+  static_assert(Z2_SCH <= 64, "a bit per site");
+  float2 x[A];
+#pragma unroll
+  for (int i = 0; i < A; ++i) x[i] = make_float2(0.0f, 0.0f);
+  for (int s0 = 0; s0 < q.ns; s0 += Z2_SCH) {
+    const int nc = min(Z2_SCH, q.ns - s0);
+    if (s0) __syncthreads();  // the previous chunk's sites are used up
+    for (int z = threadIdx.x; z < K3; z += blockDim.x) mask[z] = 0ull;
+    for (int t = threadIdx.x; t < nc * p; t += blockDim.x) wz[t] = sw3[(size_t)s0 * p + t];
+    for (int j = q.sub; j < nc; j += q.nsub) {
+      const size_t s = (size_t)s0 + j;
+      float2 a = tmul<-1>(w1h[s * q.H + q.m1], w2h[s * q.K2 + q.m2]);
+      const float c = q.on ? sqv[s] : 0.0f;
+      a.x *= c;
+      a.y *= c;
+      amp[j * C + q.cl] = a;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < nc * p; t += blockDim.x) {
+      const int j = t / p, k = t - j * p, g = sg3[s0 + j], z = g - k + (g < k ? K3 : 0);
+      if (k == 0) gz[j] = g;
+      atomicOr(mask + z, 1ull << j);
+    }
+    __syncthreads();
+    if (q.sub < B) {
+#pragma unroll
+      for (int i = 0; i < A; ++i) {
+        int z = q.sub + B * i;
+        asm volatile("" : "+v"(z));  // the planes' addresses are formed one plane at a time
+        for (unsigned long long m = mask[z]; m; m &= m - 1) {
+          const int j = __ffsll((long long)m) - 1;
+          const int d = gz[j] - z;
+          const float2 a = amp[j * C + q.cl];
+          const float w = wz[j * p + d + (d < 0 ? K3 : 0)];
+          x[i].x = fmaf(a.x, w, x[i].x);
+          x[i].y = fmaf(a.y, w, x[i].y);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  if (q.sub < B) {
+    float2 *col = reinterpret_cast<float2 *>(lds) + q.cl;
+    dit_steps<A, 1, -1, true>(x, K3, 1, 0, tw, tw);
+#pragma unroll
+    for (int k = 0; k < A; ++k) col[(q.sub + B * k) * C] = x[k];
+  }
+}
+
+// second forward step of (k2 < A, column) and the Green's function, the
+// spectrum in the place of the first step's values; returns the column's share
+// of the self energy (weight 1).  Every thread calls it.
+template <int B>
+__device__ __forceinline__ double z2_mid32(float2 *col, int K3, int A, int k2, const float *__restrict__ g,
+                                           size_t gstr, const float2 *__restrict__ tw, const float2 *lt) {
+#pragma clang fp contract(off)
+  float2 x[B];
+  double self = 0.0;
+  if (k2 < A) {
+    float gv[B];
+#pragma unroll
+    for (int k = 0; k < B; ++k) gv[k] = g[(size_t)(k2 + A * k) * gstr];
+#pragma unroll
+    for (int n = 0; n < B; ++n) x[n] = col[(B * k2 + n) * Z2_COLS];
+    dit_steps<B, 1, -1, false>(x, K3, A, k2, tw, lt);
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+      self += (double)gv[k] * ((double)x[k].x * (double)x[k].x + (double)x[k].y * (double)x[k].y);
+      x[k].x *= gv[k];
+      x[k].y *= gv[k];
+    }
+  }
+  __syncthreads();
+  if (k2 < A) {
+#pragma unroll
+    for (int k = 0; k < B; ++k) col[(k2 + A * k) * Z2_COLS] = x[k];
+  }
+  return self;
+}
+
+// first inverse step of (n1, column), in place
+template <int A>
+__device__ __forceinline__ void z2_back32(float2 *col, int K3, int B, int n1, const float2 *__restrict__ tw) {
+  float2 x[A];
+#pragma unroll
+  for (int i = 0; i < A; ++i) x[i] = col[(n1 + B * i) * Z2_COLS];
+  dit_steps<A, 1, +1, true>(x, K3, 1, 0, tw, tw);
+#pragma unroll
+  for (int k = 0; k < A; ++k) col[(n1 + B * k) * Z2_COLS] = x[k];
+}
+
+// last inverse step of (k2, column), into Hk
+template <int B>
+__device__ __forceinline__ void z2_last32(const float2 *col, int K3, int A, int k2, const float2 *__restrict__ tw,
+                                          const float2 *lt, float2 *out, size_t ostr) {
+  float2 x[B];
+#pragma unroll
+  for (int n = 0; n < B; ++n) x[n] = col[(B * k2 + n) * Z2_COLS];
+  dit_steps<B, 1, +1, false>(x, K3, A, k2, tw, lt);
+#pragma unroll
+  for (int k = 0; k < B; ++k) out[(size_t)(k2 + A * k) * ostr] = x[k];
+}
+
+static __global__ __launch_bounds__(Z2_MAXT32) void k_pme_zcol2_f32(
+    Params P, int A, int B, const float *__restrict__ engfac, const int *__restrict__ sg3,
+    const float *__restrict__ sw3, const float *__restrict__ sqv, const float2 *__restrict__ w1h,
+    const float2 *__restrict__ w2h, const float2 *__restrict__ tw3, float2 *Hk, double *selfp) {
+  constexpr int C = Z2_COLS;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int b = blockIdx.y, K3 = P.K3;
+  float2 *buf = reinterpret_cast<float2 *>(lds_raw);  // [K3][C], after the last chunk
+  double *red = reinterpret_cast<double *>(lds_raw + z2_lds32(K3, P.p) - sizeof(double) * (Z2_MAXT32 / 64));
+  float2 *lt = reinterpret_cast<float2 *>(red) - K3;  // [K3] twiddles
+  Z2Args q;
+  q.ns = P.ns;
+  q.p = P.p;
+  q.K2 = P.K2;
+  q.K3 = K3;
+  q.H = P.H;
+  q.cl = threadIdx.x % C;
+  q.sub = threadIdx.x / C;
+  q.nsub = blockDim.x / C;
+  const int ncol = P.H * P.K2, c = blockIdx.x * C + q.cl;
+  q.on = c < ncol;
+  q.m2 = q.on ? c / P.H : 0;
+  q.m1 = q.on ? c - q.m2 * P.H : 0;
+  for (int t = threadIdx.x; t < K3; t += blockDim.x) lt[t] = tw3[t];
+  const size_t bs = (size_t)b * q.ns;
+  ERM_RADIX_A32(A, (z2_front32<RR>(q, B, lds_raw, tw3, sg3 + bs, sw3 + bs * q.p, sqv + bs, w1h + bs * q.H,
+                                   w2h + bs * q.K2)))
+  __syncthreads();
+  float2 *col = buf + q.cl;
+  double self = 0.0;
+  const float *g = engfac + (size_t)q.m2 * q.H + q.m1;
+  ERM_RADIX_B32(B, (self = z2_mid32<RR>(col, K3, A, q.sub, g, (size_t)ncol, tw3, lt)))
+  self = q.on ? ((q.m1 == 0 || 2 * q.m1 == P.K1) ? 0.5 : 1.0) * self : 0.0;
+  for (int o = 32; o > 0; o >>= 1) self += __shfl_xor(self, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = self;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double sum = red[0];
+    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) sum += red[w];
+    selfp[(size_t)b * gridDim.x + blockIdx.x] = sum;
+  }
+  if (q.sub < B) ERM_RADIX_A32(A, (z2_back32<RR>(col, K3, B, q.sub, tw3)))
+  __syncthreads();
+  if (q.on && q.sub < A) {
+    float2 *out = Hk + (size_t)b * K3 * ncol + c;
+    ERM_RADIX_B32(B, (z2_last32<RR>(col, K3, A, q.sub, tw3, lt, out, (size_t)ncol)))
+  }
+}
+
 // --------------------------------------------------------------------------
 // y and x transforms of a slab of z planes, and the gather (the owned planes
 // [zb, zb + S) and their p - 1 halo planes, Q planes in LDS at a time; the
@@ -285,42 +562,49 @@ __global__ __launch_bounds__(Z2_MAXT) void k_pme_zcol2(Params P, int A, int B, c
 // three barriers.  The y transform's first step reads Hk straight into
 // registers; the x transform takes two Hermitian rows as one complex row of
 // length K1 (even or odd), and its real rows end in natural order behind
-// a copy of their last p - 1 values for the gather.  Bound in FP32 by VALU issue
-// (66% busy at 48^3) and LDS (59%) in turn, in FP64 by LDS (65%), a group's phases
+// a copy of their last p - 1 values for the gather.  Bound in FP64 by LDS (65%
+// busy at 48^3), in FP32 by VALU issue and LDS in turn, a group's phases
 // overlapping with the other workgroup of the CU; the gather is 40 to 60% of the
 // time, and half its LDS cycles are bank conflicts between sites of a plane's
 // largest class.  Measured: 500 FP64
 // configurations of 40 x 40 x 80, 12000 sites, 0.29 ms (k_pme_slab 2.71); 701
-// FP32 ones of 45 x 60 x 75, 18000 sites, 0.52 ms (3.62).  Against a register
+// FP32 ones of 45 x 60 x 75, 18000 sites, 0.61 ms (3.61).  Against a register
 // FFT per row with the planes staged in LDS and y columns transformed in HBM
-// (the register lengths until then): 1000 configurations of 48^3, 12000 sites,
-// FP64 1.24 -> 0.49 ms, FP32 0.75 -> 0.29; 500 of 64^3, order 6, 21000 sites,
-// FP64 2.23 -> 0.86; 5000 of 64^3, 29200 sites, FP32 with the y columns in
-// LDS, 4.03 -> 3.23 ms.
+// (FP64's register lengths until then): 1000 configurations of 48^3, 12000
+// sites, 1.24 -> 0.49 ms; 500 of 64^3, order 6, 21000 sites, 2.23 -> 0.86.
 // --------------------------------------------------------------------------
 // (off lanes, on = false, read where they may and write nothing)
 template <typename T, int A>
 __device__ __forceinline__ void xy2_yfirst(bool on, const typename C2<T>::type *__restrict__ src, unsigned off,
-                                           unsigned sstr, typename C2<T>::type *dst, int dstr, int n1,
+                                           unsigned sstr, typename C2<T>::type *dst, int dstr, int n1, int K,
+                                           const typename C2<T>::type *__restrict__ gtw,
                                            const typename C2<T>::type *tw) {
   using V = typename C2<T>::type;
   V x[A];
 #pragma unroll
   for (int i = 0; i < A; ++i) x[i] = src[off + i * sstr];
-  reg_fft<A, +1>(x);
+  if constexpr (sizeof(T) == 4)
+    dit_steps<A, 1, +1, true>(x, K, 1, 0, gtw, gtw);
+  else
+    reg_fft<A, +1>(x);
   if (!on) return;
   dst[0] = x[0];
 #pragma unroll
-  for (int k = 1; k < A; ++k) dst[k * dstr] = cmulc(x[k], tw[n1 * k]);
+  for (int k = 1; k < A; ++k) dst[k * dstr] = sizeof(T) == 4 ? x[k] : cmulc(x[k], tw[n1 * k]);
 }
 template <typename T, int B>
-__device__ __forceinline__ void xy2_ysecond(bool on, typename C2<T>::type *col, int rs, int A, int k2) {
+__device__ __forceinline__ void xy2_ysecond(bool on, typename C2<T>::type *col, int rs, int A, int k2, int K,
+                                            const typename C2<T>::type *__restrict__ gtw,
+                                            const typename C2<T>::type *tw) {
   using V = typename C2<T>::type;
   V x[B];
 #pragma unroll
   for (int n = 0; n < B; ++n) x[n] = col[(k2 * B + n) * rs];
   wave_lds_sync();
-  reg_fft<B, +1>(x);
+  if constexpr (sizeof(T) == 4)
+    dit_steps<B, 1, +1, false>(x, K, A, k2, gtw, tw);
+  else
+    reg_fft<B, +1>(x);
   if (!on) return;
 #pragma unroll
   for (int k = 0; k < B; ++k) col[(k2 + A * k) * rs] = x[k];
@@ -339,7 +623,9 @@ __device__ __forceinline__ int xy2_blk(int k, int B, int pad) { return B * k + (
 // not read, i = 0 and i = A / 2 again.
 template <typename T, int A>
 __device__ __forceinline__ void xy2_xfirst(bool on, int o2, typename C2<T>::type *pr, int K1, int B, int pad, int n1,
+                                           const typename C2<T>::type *__restrict__ gtw,
                                            const typename C2<T>::type *tw) {
+#pragma clang fp contract(off)
   using V = typename C2<T>::type;
   V x[A];
 #pragma unroll
@@ -366,27 +652,38 @@ __device__ __forceinline__ void xy2_xfirst(bool on, int o2, typename C2<T>::type
       a.y = sg * a.y;
       c.y = sg * c.y;
     }
+    if constexpr (sizeof(T) == 4) {  // no partner: a row of zeros, which rounds as itself
+      c.x = o2 ? c.x : (T)0;
+      c.y = o2 ? c.y : (T)0;
+    }
     x[i].x = a.x - c.y;
     x[i].y = a.y + c.x;
   }
   wave_lds_sync();
-  reg_fft<A, +1>(x);
+  if constexpr (sizeof(T) == 4)
+    dit_steps<A, 1, +1, true>(x, K1, 1, 0, gtw, gtw);
+  else
+    reg_fft<A, +1>(x);
   if (!on) return;
   pr[n1] = x[0];
 #pragma unroll
-  for (int k = 1; k < A; ++k) pr[xy2_blk(k, B, pad) + n1] = cmulc(x[k], tw[n1 * k]);
+  for (int k = 1; k < A; ++k) pr[xy2_blk(k, B, pad) + n1] = sizeof(T) == 4 ? x[k] : cmulc(x[k], tw[n1 * k]);
 }
 // the real rows, x[n] at n + h, with x[K1 - h + i] again at i < h (the
 // gather's wrap, h = p - 1)
 template <typename T, int B>
 __device__ __forceinline__ void xy2_xsecond(bool on, bool two, typename C2<T>::type *pr, int rs, int K1, int A, int h,
-                                            int pad, int k2) {
+                                            int pad, int k2, const typename C2<T>::type *__restrict__ gtw,
+                                            const typename C2<T>::type *tw) {
   using V = typename C2<T>::type;
   V x[B];
 #pragma unroll
   for (int n = 0; n < B; ++n) x[n] = pr[xy2_blk(k2, B, pad) + n];
   wave_lds_sync();
-  reg_fft<B, +1>(x);
+  if constexpr (sizeof(T) == 4)
+    dit_steps<B, 1, +1, false>(x, K1, A, k2, gtw, tw);
+  else
+    reg_fft<B, +1>(x);
   if (!on) return;
   T *r0 = reinterpret_cast<T *>(pr) + h + k2, *r1 = r0 + 2 * rs;
 #pragma unroll
@@ -491,6 +788,10 @@ __device__ __forceinline__ void xy2_gather(const Params &P, const T *real, const
   }
 }
 
+#define ERM_XY_A(A, CALL)                                                                    \
+  if constexpr (sizeof(T) == 4) { ERM_RADIX_A32(A, CALL) } else { ERM_RADIX_A(A, CALL) }
+#define ERM_XY_B(B, CALL)                                                                    \
+  if constexpr (sizeof(T) == 4) { ERM_RADIX_B32(B, CALL) } else { ERM_RADIX_B(B, CALL) }
 template <typename T>
 __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) void k_pme_xyslab(Params P, int S, int Q, Fft2 fy, Fft2 fx, int nsites,
                                                         const typename C2<T>::type *__restrict__ Hk,
@@ -503,7 +804,7 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int K1 = P.K1, K2 = P.K2, K3 = P.K3, H = P.H, p = P.p;
   const int rs = xy2_row(K1, p), plane = xy2_plane(K2, rs);
-  constexpr int BMAX = fft2_bmax<T>;
+  [[maybe_unused]] constexpr int BMAX = 12;
   V *stage = reinterpret_cast<V *>(lds_raw);   // [Q][plane]
   V *twy = stage + (size_t)Q * plane;          // [K2]
   V *twx = twy + K2;                           // [K1]
@@ -519,11 +820,18 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
   const int zb = (L - b * gridDim.x) * S, ze = min(zb + S, K3);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   constexpr int NW = XY2_THR / 64;
-  // columns of a wave's round: lane = n1 Gy + column in the first step,
-  // k2 Gy + column in the second
-  const int Gy = 64 / fy.B, ly0 = lane / Gy, lg = lane - ly0 * Gy;
-  // row pairs of a round: lane = pair B + n1, then pair A + k2
-  const int Gx = 64 / fx.B;
+  // A wave's round: Cy columns, dealt over its lanes by n1 (lane = n1 Gya +
+  // column) in the first step and by k2 in the second, and Cx row pairs (lane =
+  // pair B + n1, then pair A + k2).  FP64 has A <= B < 2 A and takes a round's
+  // columns in one part each; the FP32 radices are as unlike as 4 and 12, so
+  // there the step with fewer lanes per column sets the round and the
+  // other takes it in parts.
+  constexpr bool F32 = sizeof(T) == 4;
+  const int Gya = 64 / fy.B, Gyb = F32 ? 64 / fy.A : Gya;
+  const int Gxa = 64 / fx.B, Gxb = F32 ? 64 / fx.A : Gxa;
+  auto round = [](int a, int b) { return min(a, b) * (max(a, b) / min(a, b)); };
+  const int Cy = round(Gya, Gyb), Cx = round(Gxa, Gxb);
+  const int lya = lane / Gya, lga = lane - lya * Gya, lyb = lane / Gyb, lgb = lane - lyb * Gyb;
   const int xg1 = lane / fx.B, xn0 = lane - xg1 * fx.B, xg2 = lane / fx.A, xk0 = lane - xg2 * fx.A;
   const int npair = (K2 + 1) / 2;
   const int pad = (fx.B & 3) ? 0 : min((2 * rs - K1) * 256 / (fx.A - 1), 256);
@@ -533,38 +841,49 @@ __global__ __launch_bounds__(XY2_THR) __attribute__((amdgpu_waves_per_eu(4))) vo
   __syncthreads();
   for (int zz0 = zb - p + 1; zz0 < ze; zz0 += Q) {
     const int nq = min(Q, ze - zz0), ncol = nq * H;
-    for (int c0 = wv * Gy; c0 < ncol; c0 += NW * Gy) {
-      int ly = ly0;
-      asm volatile("" : "+v"(ly));  // no radix's addresses are hoisted out of the loop
-      const bool in = lg < Gy && c0 + lg < ncol;  // lanes past B Gy have ly >= B
-      const int cid = in ? c0 + lg : c0, q = div_by(cid, fH), m1 = cid - q * H;
-      const int z = zz0 + q + ((zz0 + q < 0) ? K3 : 0);
-      V *col = stage + q * plane + m1;
-      const int l1 = min(ly, fy.B - 1), l2 = min(ly, fy.A - 1);
-      ERM_RADIX_A(fy.A, (xy2_yfirst<T, RR>(in && ly < fy.B, src, (unsigned)((z * K2 + l1) * H + m1),
-                                           (unsigned)(fy.B * H), col + l1 * rs, fy.B * rs, l1, twy)))
+    for (int c0 = wv * Cy; c0 < ncol; c0 += NW * Cy) {
+      const int c1 = min(c0 + Cy, ncol);
+      for (int g = c0; g < c1; g += Gya) {
+        int ly = lya;
+        asm volatile("" : "+v"(ly));  // no radix's addresses are hoisted out of the loop
+        const bool in = lga < Gya && g + lga < c1;  // lanes past B Gya have ly >= B
+        const int cid = in ? g + lga : c0, q = div_by(cid, fH), m1 = cid - q * H;
+        const int z = zz0 + q + ((zz0 + q < 0) ? K3 : 0);
+        V *col = stage + q * plane + m1;
+        const int l1 = min(ly, fy.B - 1);
+        ERM_XY_A(fy.A, (xy2_yfirst<T, RR>(in && ly < fy.B, src, (unsigned)((z * K2 + l1) * H + m1),
+                                          (unsigned)(fy.B * H), col + l1 * rs, fy.B * rs, l1, K2, tw2, twy)))
+      }
       wave_lds_sync();
-      ERM_RADIX_B(fy.B, (xy2_ysecond<T, RR>(in && ly < fy.A, col, rs, fy.A, l2)))
+      for (int g = c0; g < c1; g += Gyb) {
+        int ly = lyb;
+        asm volatile("" : "+v"(ly));
+        const bool in = lgb < Gyb && g + lgb < c1;
+        const int cid = in ? g + lgb : c0, q = div_by(cid, fH), m1 = cid - q * H;
+        V *col = stage + q * plane + m1;
+        ERM_XY_B(fy.B, (xy2_ysecond<T, RR>(in && ly < fy.A, col, rs, fy.A, min(ly, fy.A - 1), K2, tw2, twy)))
+      }
     }
     __syncthreads();
     const int nrow = nq * npair;
-    for (int p0 = wv * Gx; p0 < nrow; p0 += NW * Gx) {
-      {
+    for (int p0 = wv * Cx; p0 < nrow; p0 += NW * Cx) {
+      const int p1 = min(p0 + Cx, nrow);
+      for (int g = p0; g < p1; g += Gxa) {
         int xn1 = xn0;
         asm volatile("" : "+v"(xn1));
-        const bool in = xg1 < Gx && p0 + xg1 < nrow;
-        const int pid = in ? p0 + xg1 : p0, q = div_by(pid, fpair), pr = pid - q * npair;
+        const bool in = xg1 < Gxa && g + xg1 < p1;
+        const int pid = in ? g + xg1 : p0, q = div_by(pid, fpair), pr = pid - q * npair;
         V *row = stage + q * plane + 2 * pr * rs;
-        ERM_RADIX_A(fx.A, (xy2_xfirst<T, RR>(in, (2 * pr + 1 < K2) ? rs : 0, row, K1, fx.B, pad, xn1, twx)))
+        ERM_XY_A(fx.A, (xy2_xfirst<T, RR>(in, (2 * pr + 1 < K2) ? rs : 0, row, K1, fx.B, pad, xn1, tw1, twx)))
       }
       wave_lds_sync();
-      {
+      for (int g = p0; g < p1; g += Gxb) {
         int xk2 = xk0;
         asm volatile("" : "+v"(xk2));
-        const bool in = xg2 < Gx && p0 + xg2 < nrow;
-        const int pid = in ? p0 + xg2 : p0, q = div_by(pid, fpair), pr = pid - q * npair;
+        const bool in = xg2 < Gxb && g + xg2 < p1;
+        const int pid = in ? g + xg2 : p0, q = div_by(pid, fpair), pr = pid - q * npair;
         V *row = stage + q * plane + 2 * pr * rs;
-        ERM_RADIX_B(fx.B, (xy2_xsecond<T, RR>(in, 2 * pr + 1 < K2, row, rs, K1, fx.A, p - 1, pad, xk2)))
+        ERM_XY_B(fx.B, (xy2_xsecond<T, RR>(in, 2 * pr + 1 < K2, row, rs, K1, fx.A, p - 1, pad, xk2, tw1, twx)))
       }
       wave_lds_sync();
     }

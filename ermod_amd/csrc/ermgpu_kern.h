@@ -1044,12 +1044,11 @@ __device__ __forceinline__ void zspread_half(V (&Y)[K3 / 2], const V a, const T 
 // (128 in FP32: the 150-site solutes take two chunks, and three
 // 256-thread workgroups still fit a CU's LDS)
 template <typename T> constexpr int zfft_sch = sizeof(T) == 4 ? 128 : 64;
-constexpr int ZFFT_KMAX = 100;  // largest z grid length of the register kernels
+constexpr int ZFFT_KMAX = 96;  // largest z grid length of the register kernels
 
-// lanes per z column in k_pme_zcol_fft: one in FP32 up to K3 = 81 (the
-// whole column, 2 K3 floats, in one lane's registers; 238 of them at 81), else
-// a lane pair
-__host__ __device__ constexpr int zfft_lanes(int tbytes, int K3) { return (tbytes == 4 && K3 <= 81) ? 1 : 2; }
+// lanes per z column in k_pme_zcol_fft: one in FP32 up to K3 = 64 (the
+// whole column, 2 K3 floats, in one lane's registers), else a lane pair
+__host__ __device__ constexpr int zfft_lanes(int tbytes, int K3) { return (tbytes == 4 && K3 <= 64) ? 1 : 2; }
 
 // m2 rows a workgroup of XT threads (XT / L columns, m1 fastest) touches
 __host__ __device__ inline int zcol_fft_rows(int H, int K2, int XT, int L = 2) {
@@ -1099,7 +1098,7 @@ __device__ __forceinline__ void zcol_stage_chunk(int s0, int nc, int K3, int H, 
   __syncthreads();
 }
 
-// One lane per column (m1, m2) (FP32, K3 <= 81): the same spread, Green's
+// One lane per column (m1, m2) (FP32, K3 <= 64): the same spread, Green's
 // function and transforms as the lane-pair form below, with the whole column
 // in one lane's registers in plane order.  Every site adds to its PP planes
 // directly (no lane masks), the forward and inverse z FFTs are one K3-point

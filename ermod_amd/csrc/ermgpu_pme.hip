@@ -1,8 +1,7 @@
 // ermgpu_pme.hip -- the register-FFT kernels of one precision and grid
 // length: z columns, in FP32 the y columns and the x slab with the gather, and
 // the adjoint's solvent-potential transforms.  Compiled once per (ERM_T,
-// ERM_K), or per (ERM_T, list ERM_ZLENS of lengths whose z columns alone are
-// wanted), so that the instantiations build in parallel; ermgpu.hip dispatches
+// ERM_K) so that the instantiations build in parallel; ermgpu.hip dispatches
 // on the grid length at run time.
 #include <algorithm>
 
@@ -10,7 +9,7 @@
 #include "ermgpu_grad.h"
 
 #ifndef ERM_T
-#error "ERM_T (float or double) and ERM_K (grid length) or ERM_ZLENS select the instantiations"
+#error "ERM_T (float or double) and ERM_K (grid length) select the instantiation"
 #endif
 
 namespace ermh {
@@ -51,11 +50,6 @@ int launch_zcol_fft(erm_ctx *c, const Params &k, int n, int nblk, size_t site0, 
   }
   if (c->zcol_T == 512) return launch_zcol_fft_t<T, K, 6, 512>(c, k, n, nblk, site0, cfg0);
   return launch_zcol_fft_t<T, K, 6, NTHR>(c, k, n, nblk, site0, cfg0);
-}
-// the same with 256 threads (lengths compiled for their z columns alone)
-template <typename T, int K> int launch_zcol_fft256(erm_ctx *c, const Params &k, int n, int nblk) {
-  if (k.p == 4) return launch_zcol_fft_t<T, K, 4, NTHR>(c, k, n, nblk, 0, 0);
-  return launch_zcol_fft_t<T, K, 6, NTHR>(c, k, n, nblk, 0, 0);
 }
 // z columns of a heterogeneous batch (run table in device memory): a
 // persistent grid (as many workgroups as fit the device at once) pulling
@@ -152,10 +146,6 @@ template <typename T, int K> void launch_zgreen(erm_ctx *c, const Params &k) {
                      dp<T>(c->d_engfac), dp<V>(c->d_tw3), dp<V>(c->d_gHk));
 }
 
-#ifdef ERM_ZLENS
-#define ERM_Z(K) template int launch_zcol_fft256<ERM_T, K>(erm_ctx *, const Params &, int, int);
-ERM_ZLENS
-#else
 template int launch_zcol_reg<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int);
 template int launch_zcol_fft<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int, size_t, size_t);
 template int launch_zcol_fft_runs<ERM_T, ERM_K>(erm_ctx *, const Params &, int, const GRun *, int, int, int *);
@@ -166,6 +156,5 @@ template void launch_xc2r<ERM_T, ERM_K>(erm_ctx *, const Params &);
 template void launch_ydense<ERM_T, ERM_K, -1>(erm_ctx *, const Params &);
 template void launch_ydense<ERM_T, ERM_K, +1>(erm_ctx *, const Params &);
 template void launch_zgreen<ERM_T, ERM_K>(erm_ctx *, const Params &);
-#endif
 
 }  // namespace ermh

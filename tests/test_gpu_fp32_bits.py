@@ -66,3 +66,36 @@ def test_register_lengths(name):
     want = np.load(GOLDEN)[name]
     got = energies(REGISTER[name], list(REGISTER).index(name))
     np.testing.assert_allclose(got, want, rtol=1e-12, atol=1e-10)
+
+
+@pytest.mark.parametrize("name", list(OTHER))
+def test_other_lengths(name):
+    print(f"\n[gpu case] FP32 rounding, lengths {name} {OTHER[name]}", flush=True)
+    want = np.load(GOLDEN)[name]
+    got = energies(OTHER[name], list(OTHER).index(name))
+    np.testing.assert_allclose(got, want, rtol=1e-12, atol=1e-10)
+
+
+#: every length that the two-step kernels take
+LENGTHS = (16, 18, 20, 24, 25, 27, 30, 32, 36, 40, 45, 48, 50, 54, 60, 64, 72, 75, 80, 81, 90, 96, 100, 108, 120, 128)
+
+
+@pytest.mark.parametrize("i", range(len(LENGTHS)), ids=lambda i: str(LENGTHS[i]))
+def test_two_step_against_one_radix_at_a_time(i):
+    """Every length on every axis, solutes of one to three chunks of sites,
+    spline orders with and without a gather of their own, one configuration
+    and several: the same energies, the self energy among them, as from the
+    kernels with a trip through LDS per radix."""
+    grid = (LENGTHS[i], LENGTHS[(i + 1) % 26], LENGTHS[(i + 9) % 26])
+    sites, order, n = ((64, 4, 1), (65, 5, 2), (130, 6, 3), (12, 3, 5))[i % 4]
+    print(f"\n[gpu case] two steps against single radices, {grid} order {order} {sites} sites {n}", flush=True)
+    sy = synth.refs20(nwater=220, L=25.0, K=16, nsite=sites)
+    s = sy.system = dataclasses.replace(sy.system, ms=grid, splodr=order)
+    places = np.array([O.place_solute(s.bfcoord, s.solute_mass(sy.solute_mol), sy.cell, *O.random_pose(90 + i, j))
+                       for j in range(n)])
+    got = {}
+    for path in ("auto", "fused"):
+        with ErmGPU(s, "fp32", pme_path=path) as g:
+            g.set_frame(sy.frame(0), sy.cell)
+            got[path] = g.get_uv_energy(sy.solute_mol, places)
+    np.testing.assert_allclose(got["auto"], got["fused"], rtol=1e-12, atol=1e-10)

@@ -644,6 +644,54 @@ template <typename T> int launch_xyslab(erm_ctx *c, const Params &k, int n) {
   return launch_check(c, "k_pme_xyslab");
 }
 
+// Shape of the FP32 x slab for n configurations: the tuned one where
+// erm_set_tuning or the autotuner chose it, else 512 threads, the y transform in
+// the slab where K1 = K2 < 64 (there it rounds as in its own kernel, at 64 the
+// compiler fuses other products) and the planes of the least estimated time:
+// rounds of lanes over y columns (K2 log K2 each) and rows (half of K1 log K1), a
+// constant per group of planes, all for the busiest CU.  Against 256 threads,
+// 16 planes in groups of 8 and y columns transformed in memory, y and x: 1000
+// configurations on 48^3 0.753 -> 0.346 ms (12 planes in one group of 15), 500
+// on 64^3 0.619 -> 0.506, order 6 1.656 -> 1.066 (11 in groups of 8).
+XsShape xslab_shape(const erm_ctx *c, int n) {
+  const Params &k = c->kp;
+  XsShape s;
+  if (c->xslab_set) {
+    s.S = c->slab_S;
+    s.Q = c->xslab_Q;
+    s.R = c->slab_R;
+    s.T = c->xslab_T;
+    s.fold = xslab_folds_y(c);
+    return s;
+  }
+  s.T = 512;
+  s.fold = k.K1 == k.K2 && k.K1 < 64;
+  const size_t plane = sizeof(float2) * (size_t)k.H * k.K2, cu = c->lds_cap + 10 * 1024;
+  const int qmax = (int)std::min<size_t>(16, c->lds_cap / plane);
+  const double ty = s.fold ? k.K2 * std::log2(k.K2) : 0.0, tx = 0.5 * k.K1 * std::log2(k.K1);
+  double best = 0.0;
+  for (int S = 1; S <= std::min(16, k.K3); ++S) {
+    const int nslab = (k.K3 + S - 1) / S, planes = S + k.p - 1;
+    // 32: twice the registers, where nothing less holds the sites of a plane
+    if (!c->xslab_R[S] || (c->xslab_R[S] == 32 && c->xslab_R[1] < 32)) continue;
+    for (int Q = 1; Q <= std::min(qmax, planes); ++Q) {
+      double t = 0.0;
+      for (int left = planes; left > 0; left -= Q) {
+        const int q = std::min(Q, left);
+        t += ty * ((q * k.H + s.T - 1) / s.T) + tx * ((q * k.K2 + s.T - 1) / s.T) + 200.0;
+      }
+      t *= std::max(1.0, (double)n * nslab / (c->ncu * (2 * Q * plane <= cu ? 1.1 : 1.0)));
+      if (!s.S || t < best) {
+        best = t;
+        s.S = S;
+        s.Q = Q;
+        s.R = c->xslab_R[S];
+      }
+    }
+  }
+  return s;
+}
+
 // The y and x transforms and the gather of n configurations into d_esite,
 // with stage marks 3 and 4.  FP64 and the two-step lengths take
 // k_pme_xyslab.  The register lengths in FP32 keep whole transforms in a
@@ -658,16 +706,17 @@ template <typename T> int launch_yx(erm_ctx *c, const Params &k, int n, bool reg
   TRY(ensure(c, c->d_esite, sizeof(double) * (size_t)n * c->nsites));
   if constexpr (sizeof(T) == 4) {
     if (regp) {
+      const XsShape s = xslab_shape(c, n);
+      if (!s.S) return fail(c, ERM_E_ENG_BUG, "x slab shape");
       int rc = ERM_OK;
-      if (!xslab_folds_y(c)) {
+      if (!s.fold) {
         rc = ERM_E_UNSUPPORTED;
         ERM_KSWITCH(k.K2, (rc = launch_ycol_reg<T, KK>(c, k, n)));
         TRY(rc);
       }
       TRY(mark(c, 3));
-      const size_t lx = 2 * sizeof(T) * (size_t)c->xslab_Q * k.H * k.K2;
       rc = ERM_E_UNSUPPORTED;
-      ERM_KSWITCH(k.K1, (rc = launch_xslab<T, KK>(c, k, n, lx)));
+      ERM_KSWITCH(k.K1, (rc = launch_xslab<T, KK>(c, k, n, s)));
       TRY(rc);
       return mark(c, 4);
     }
@@ -686,6 +735,11 @@ template <typename T> int choose_slab(erm_ctx *c) {
   const Params &k = c->kp;
   const int K3 = k.K3;
   const std::vector<int> &zst = c->zst;
+  for (int S = 1; S <= 16; ++S) {
+    int mx = 0;
+    for (int zb = 0; zb < K3; zb += S) mx = std::max(mx, zst[std::min(zb + S, K3)] - zst[zb]);
+    c->xslab_R[S] = mx <= 8 * NTHR ? 8 : mx <= 16 * NTHR ? 16 : mx <= 32 * NTHR ? 32 : 0;
+  }
   c->slab_S = 0;
   c->slab_R = 0;
   // R = 8 only for the register path with shallow slabs (fewer live registers)
@@ -1403,6 +1457,14 @@ int process(erm_ctx *c, const Batch &all, int flags, double *uv_out) {
   return stage_times(c, nb, (flags & DO_HIST) != 0);
 }
 
+// the part of a captured launch's shape that comes from the frame's site
+// counts or the x slab's settings
+std::string slab_key(const erm_ctx *c) {
+  std::string k = "|" + std::to_string((int)c->xslab_set) + (c->xslab_yf ? "y" : "n");
+  for (int S = 1; S <= 16; ++S) k += "|" + std::to_string(c->xslab_R[S]);
+  return k;
+}
+
 // identity of a captured call: everything its kernels take by value or by
 // device address
 std::string graph_key(erm_ctx *c, const Batch &all, int flags) {
@@ -1411,7 +1473,7 @@ std::string graph_key(erm_ctx *c, const Batch &all, int flags) {
   snprintf(buf, sizeof buf, "|%d|%d|%d|%d|%d|%d|%d|%d|%d|%d|%d|%llu|%d", all.n, c->Bmax, flags, c->P.pme_path,
            c->slab_S, c->slab_R, c->xslab_Q, c->xslab_T, c->zcol_T, (int)c->have_usreal, c->wsol_ones,
            (unsigned long long)c->alloc_gen, (int)all.random);
-  return k + buf;
+  return k + buf + slab_key(c);
 }
 
 // random insertions replayed from a captured graph: the first call with a
@@ -2835,6 +2897,7 @@ int32_t erm_group_insert_random(erm_group *g, const int32_t *n, const uint64_t *
     snprintf(buf, sizeof buf, "|%d|%d|%d|%d|%d|%d|%d|%d|%d", nb, g->persistent, c->slab_S, c->slab_R, c->xslab_Q,
              c->xslab_T, c->zcol_T, (int)c->xslab_yf, c->wsol_ones);
     kk += buf;
+    kk += slab_key(c);
     for (erm_ctx *m : g->ctx) {
       kk.append(reinterpret_cast<const char *>(&m->kp), sizeof(Params));
       snprintf(buf, sizeof buf, "|%llu|%d|%d", (unsigned long long)m->alloc_gen, (int)m->have_usreal, m->ns);
@@ -3128,6 +3191,7 @@ int32_t erm_set_tuning(erm_ctx *c, int32_t max_batch, int32_t pme_path, int32_t 
       (column_threads != 0 && column_threads != 256 && column_threads != 512))
     return fail(c, ERM_E_ARG, "tuning out of range");
   if (column_threads > 0) c->zcol_T = column_threads;
+  if (slab_planes > 0 || group_planes > 0 || slab_threads > 0 || fold_y >= 0) c->xslab_set = true;
   if (max_batch > 0) {
     c->Bmax = max_batch;
     c->batch_set = true;
@@ -3194,6 +3258,7 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
     return ERM_OK;
   };
   c->use_graph = false;
+  c->xslab_set = true;
   auto apply = [&](int B, int pp, int Sc, int Qc, int Tc) -> int {
     c->Bmax = B;
     c->P.pme_path = pp;

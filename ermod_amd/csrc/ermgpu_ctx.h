@@ -104,6 +104,8 @@ struct erm_ctx {
   int xslab_T = erm::NTHR;           // threads per x-slab workgroup, 256 or 512 (autotuned)
   int zcol_T = erm::NTHR;            // threads per z-column workgroup, 256 or 512 (autotuned)
   bool xslab_yf = false;        // inverse y transform inside the x slab (autotuned)
+  bool xslab_set = false;       // these four chosen by erm_set_tuning or the autotuner
+  int xslab_R[17] = {};         // the frame's sites per slab of 1..16 planes as XsShape::R, 0: too many
   int pair_path = 0;            // 0 tiled pair kernel, 1 one thread per candidate molecule
   int ncu = 256;                // compute units of the device (persistent grids)
   double slt_radius = 8.0;      // test particle's largest site distance from its centroid
@@ -263,7 +265,13 @@ template <typename T, int K>
 int launch_zcol_fft_runs(erm_ctx *c, const Params &k, int nblk, const GRun *runs, int nrun, int nitem, int *counter);
 // FP32 alone (FP64: k_pme_xyslab)
 template <typename T, int K> int launch_ycol_reg(erm_ctx *c, const Params &k, int n);
-template <typename T, int K> int launch_xslab(erm_ctx *c, const Params &k, int n, size_t lds);
+struct XsShape {
+  int S = 0, Q = 0;   // owned planes per workgroup, planes in LDS at a time
+  int R = 0;          // most sites of a slab, in 256s: 8, 16 or 32
+  int T = NTHR;       // threads, 256 or 512
+  bool fold = false;  // inverse y transform in the slab (512 threads, K1 = K2)
+};
+template <typename T, int K> int launch_xslab(erm_ctx *c, const Params &k, int n, const XsShape &s);
 template <typename T, int K> void launch_xr2c(erm_ctx *c, const Params &k);
 template <typename T, int K> void launch_xc2r(erm_ctx *c, const Params &k);
 template <typename T, int K, int SIGN> void launch_ydense(erm_ctx *c, const Params &k);

@@ -92,32 +92,33 @@ template <typename T, int K> int launch_ycol_reg(erm_ctx *c, const Params &k, in
   return fail(c, ERM_E_ENG_BUG, "y columns in FP64");
 }
 template <typename T, int K, int R, int XT = NTHR, bool YF = false>
-int launch_xslab_r(erm_ctx *c, const Params &k, int n, size_t lds) {
+int launch_xslab_r(erm_ctx *c, const Params &k, int n, const XsShape &s) {
   using V = typename C2<T>::type;
+  const size_t lds = sizeof(V) * (size_t)s.Q * k.H * k.K2;
   TRY(set_lds(c, (const void *)k_pme_xslab<T, K, R, XT, YF>, lds, "k_pme_xslab"));
-  const int nslab = (k.K3 + c->slab_S - 1) / c->slab_S;
-  hipLaunchKernelGGL((k_pme_xslab<T, K, R, XT, YF>), dim3(nslab, n), dim3(XT), lds, c->st, k, c->slab_S, c->xslab_Q,
-                     c->nsites, dp<V>(c->d_Hk), dp<V>(c->d_tw1), dp<int>(c->d_zstart), dp<int>(c->d_zg),
-                     dp<T>(c->d_zq), dp<T>(c->d_zw), dp<int>(c->d_zsite), dp<double>(c->d_esite));
+  const int nslab = (k.K3 + s.S - 1) / s.S;
+  hipLaunchKernelGGL((k_pme_xslab<T, K, R, XT, YF>), dim3(nslab, n), dim3(XT), lds, c->st, k, s.S, s.Q, c->nsites,
+                     dp<V>(c->d_Hk), dp<V>(c->d_tw1), dp<int>(c->d_zstart), dp<int>(c->d_zg), dp<T>(c->d_zq),
+                     dp<T>(c->d_zw), dp<int>(c->d_zsite), dp<double>(c->d_esite));
   return launch_check(c, "k_pme_xslab");
 }
-// slab_R counts sites per thread of a 256-thread workgroup; a 512-thread
-// workgroup owns the same sites with half as many per thread
-template <typename T, int K> int launch_xslab(erm_ctx *c, const Params &k, int n, size_t lds) {
+// a 512-thread workgroup owns the same sites as one of 256 with half as many
+// per thread
+template <typename T, int K> int launch_xslab(erm_ctx *c, const Params &k, int n, const XsShape &s) {
   if constexpr (sizeof(T) == 4) {
-    if (xslab_folds_y(c)) {
-      if (c->slab_R == 8) return launch_xslab_r<T, K, 4, 512, true>(c, k, n, lds);
-      if (c->slab_R == 16) return launch_xslab_r<T, K, 8, 512, true>(c, k, n, lds);
-      return launch_xslab_r<T, K, 16, 512, true>(c, k, n, lds);
+    if (s.fold) {
+      if (s.R == 8) return launch_xslab_r<T, K, 4, 512, true>(c, k, n, s);
+      if (s.R == 16) return launch_xslab_r<T, K, 8, 512, true>(c, k, n, s);
+      return launch_xslab_r<T, K, 16, 512, true>(c, k, n, s);
     }
-    if (c->xslab_T == 512) {
-      if (c->slab_R == 8) return launch_xslab_r<T, K, 4, 512>(c, k, n, lds);
-      if (c->slab_R == 16) return launch_xslab_r<T, K, 8, 512>(c, k, n, lds);
-      return launch_xslab_r<T, K, 16, 512>(c, k, n, lds);
+    if (s.T == 512) {
+      if (s.R == 8) return launch_xslab_r<T, K, 4, 512>(c, k, n, s);
+      if (s.R == 16) return launch_xslab_r<T, K, 8, 512>(c, k, n, s);
+      return launch_xslab_r<T, K, 16, 512>(c, k, n, s);
     }
-    if (c->slab_R == 8) return launch_xslab_r<T, K, 8>(c, k, n, lds);
-    if (c->slab_R == 16) return launch_xslab_r<T, K, 16>(c, k, n, lds);
-    return launch_xslab_r<T, K, 32>(c, k, n, lds);
+    if (s.R == 8) return launch_xslab_r<T, K, 8>(c, k, n, s);
+    if (s.R == 16) return launch_xslab_r<T, K, 16>(c, k, n, s);
+    return launch_xslab_r<T, K, 32>(c, k, n, s);
   }
   return fail(c, ERM_E_ENG_BUG, "x slab in FP64");
 }
@@ -150,7 +151,7 @@ template int launch_zcol_reg<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int);
 template int launch_zcol_fft<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int, size_t, size_t);
 template int launch_zcol_fft_runs<ERM_T, ERM_K>(erm_ctx *, const Params &, int, const GRun *, int, int, int *);
 template int launch_ycol_reg<ERM_T, ERM_K>(erm_ctx *, const Params &, int);
-template int launch_xslab<ERM_T, ERM_K>(erm_ctx *, const Params &, int, size_t);
+template int launch_xslab<ERM_T, ERM_K>(erm_ctx *, const Params &, int, const XsShape &);
 template void launch_xr2c<ERM_T, ERM_K>(erm_ctx *, const Params &);
 template void launch_xc2r<ERM_T, ERM_K>(erm_ctx *, const Params &);
 template void launch_ydense<ERM_T, ERM_K, -1>(erm_ctx *, const Params &);

@@ -381,7 +381,9 @@ int32_t erm_stage_times(const erm_ctx *ctx, double *ms10);
  * register path transforms per group, slab_threads and column_threads (256 or
  * 512) the workgroup sizes of its x slab and of the z columns (0 keeps any of
  * them); fold_y = 1 moves the inverse y transform into 512-thread x slabs of a
- * grid with K2 = K1, 0 keeps it in its own kernel, -1 keeps the setting.  In
+ * grid with K2 = K1, 0 keeps it in its own kernel, -1 keeps the setting.
+ * Until one of these is given, or the autotuner has run, the FP32 register
+ * path chooses them for each launch (erm_get_tuning returns the settings).  In
  * FP64 group_planes, slab_threads and fold_y are kept and returned by
  * erm_get_tuning: there, as for the grid lengths without a register kernel,
  * the y and x transforms run as one kernel that chooses its own shape. */

@@ -68,6 +68,44 @@ def test_register_lengths(name):
     np.testing.assert_allclose(got, want, rtol=1e-12, atol=1e-10)
 
 
+@pytest.mark.parametrize("K,n", [(16, 3), (24, 3), (32, 3), (48, 40), (64, 3)])
+def test_slab_shapes_round_alike(K, n):
+    """The slab shape that a launch chooses against 256 threads with the y
+    columns in a kernel of their own."""
+    print(f"\n[gpu case] FP32 slab shapes, {K}^3, {n} configurations", flush=True)
+    sy = synth.refs20(nwater=220, L=25.0, K=16, nsite=12)
+    s = sy.system = dataclasses.replace(sy.system, ms=(K, K, K))
+    places = np.array([O.place_solute(s.bfcoord, s.solute_mass(sy.solute_mol), sy.cell, *O.random_pose(70 + K, j))
+                       for j in range(n)])
+    got = []
+    with ErmGPU(s, "fp32") as g:
+        g.set_frame(sy.frame(0), sy.cell)
+        got.append(g.get_uv_energy(sy.solute_mol, places))
+        g.set_tuning(slab_planes=16, group_planes=8, slab_threads=256, fold_y=False)
+        got.append(g.get_uv_energy(sy.solute_mol, places))
+    np.testing.assert_allclose(got[0], got[1], rtol=1e-12, atol=1e-10)
+
+
+def test_graph_follows_the_slab_shape():
+    """A captured call is not replayed on a frame whose sites per slab want
+    another kernel: the second frame's molecules lie in 0.4 of the box."""
+    print("\n[gpu case] FP32 slab shape of a captured call", flush=True)
+    sy = synth.refs20()
+    s = sy.system
+    wide = sy.frame(0)
+    dense = wide.copy()
+    for m in range(s.nmol):
+        b, e = int(s.mol_begin[m]), int(s.mol_begin[m + 1])
+        dense[b:e, 2] -= 0.6 * wide[b, 2]
+    with ErmGPU(s, "fp32") as eager, ErmGPU(s, "fp32") as graph:
+        graph.set_tuning(use_graph=True)
+        for k, frame in enumerate((wide, wide, dense, dense, wide)):
+            for g in (eager, graph):
+                g.set_frame(frame, sy.cell)
+                g.insert_random(30, 5, first_index=30 * k)
+            np.testing.assert_array_equal(eager.fetch()["ecorr"], graph.fetch()["ecorr"], err_msg=str(k))
+
+
 @pytest.mark.parametrize("name", list(OTHER))
 def test_other_lengths(name):
     print(f"\n[gpu case] FP32 rounding, lengths {name} {OTHER[name]}", flush=True)

@@ -442,22 +442,6 @@ int upload_real(erm_ctx *c, DBuf &b, const std::vector<double> &v) {
   return upload(c, b, v.data(), v.size());
 }
 
-// Configurations per batch when the caller leaves the choice (max_batch = 0):
-// 1024 where the half spectra, per-site sums and energies of so many stay
-// within 4 GiB, else 256.  A launch of the light kernels (poses, solute
-// splines, binning, weights, edens, the correlation matrix) costs 5-30 us
-// however few configurations it holds, and the heavy ones fill the chip's last
-// wave of workgroups once a batch.  Measured, 256 against 1024: 4 frames of
-// 1000 insertions of 20 sites among 4000 waters, 48^3, 11.08 -> 9.60 ms in
-// FP64, 7.97 -> 6.61 ms in FP32 (binning 450 -> 196, poses 304 -> 95, solute
-// splines 264 -> 92 us); 500 insertions at 64^3, order 6, 4.12 -> 3.93 ms.
-int default_batch(const erm_ctx *c) {
-  const size_t vb = c->fp32 ? sizeof(float2) : sizeof(double2);
-  const size_t hk = c->P.cltype == ERM_EL_COULOMB ? 0 : vb * c->kp.H * c->kp.K2 * c->kp.K3;
-  const size_t one = hk + sizeof(double) * ((size_t)c->nsites + c->slvmax + 1);
-  return 1024 * one <= ((size_t)4 << 30) ? 1024 : 256;
-}
-
 // per-solute-type tables: charges and LJ rows against the solvent types
 int solute_tables(erm_ctx *c) {
   int m = c->slt_template;
@@ -514,6 +498,37 @@ template <typename T> bool reg_len(int K) {
 template <typename T> bool reg_path_ok(const erm_ctx *c) {
   const Params &k = c->kp;
   return reg_len<T>(k.K1) && reg_len<T>(k.K2) && reg_len<T>(k.K3) && (k.K1 % 2 == 0);
+}
+
+// Configurations per batch when the caller leaves the choice (max_batch = 0):
+// 1024 where the buffers of so many stay within 4 GiB, else 256.  Counted is
+// what grows with the grid or with a molecule count: half spectra, the sites'
+// spectra along the axes, real grids where they go through memory, per-site sums
+// and energies; a site's own few values and a configuration's bins are not.  A
+// launch of the light kernels (poses, solute
+// splines, binning, weights, edens, the correlation matrix) costs 5-30 us
+// however few configurations it holds, and the heavy ones fill the chip's last
+// wave of workgroups once a batch.  Measured, 256 against 1024: 4 frames of
+// 1000 insertions of 20 sites among 4000 waters, 48^3, 11.08 -> 9.60 ms in
+// FP64, 7.97 -> 6.61 ms in FP32 (binning 450 -> 196, poses 304 -> 95, solute
+// splines 264 -> 92 us); 500 insertions at 64^3, order 6, 4.12 -> 3.93 ms.
+template <typename T> int default_batch(const erm_ctx *c) {
+  using V = typename C2<T>::type;
+  const Params &k = c->kp;
+  size_t one = sizeof(double) * ((size_t)c->nsites + c->slvmax + 1);
+  if (c->P.cltype != ERM_EL_COULOMB) {
+    const size_t H = k.H, K1 = k.K1, K2 = k.K2, K3 = k.K3, ns = c->ns;
+    one += sizeof(V) * (H * K2 * K3 + ns * (H + K2));
+    const bool reg = reg_path_ok<T>(c);
+    Fft2 f;
+    if (reg && k.p != 4 && k.p != 6) one += sizeof(V) * ns * K3;
+    if (c->P.pme_path == 2 || !(reg || (fft2_split<T>(k.K1, f) && fft2_split<T>(k.K2, f) && fft2_split<T>(k.K3, f))))
+      one += sizeof(T) * K1 * K2 * K3;
+  }
+  return 1024 * one <= ((size_t)4 << 30) ? 1024 : 256;
+}
+void set_default_batch(erm_ctx *c) {
+  if (c->P.max_batch <= 0 && !c->batch_set) c->Bmax = c->fp32 ? default_batch<float>(c) : default_batch<double>(c);
 }
 
 // Kernel of the z columns.  Z_SPEC sums the solute's z spectra (register
@@ -2265,7 +2280,7 @@ int32_t erm_set_topology(erm_ctx *c, int32_t natom, int32_t nmol, const int32_t 
       site_a.push_back(a);
     }
   c->nsites = (int)site_k.size();
-  if (c->P.max_batch <= 0 && !c->batch_set) c->Bmax = default_batch(c);
+  set_default_batch(c);
   c->nvt = (int)c->vtypes.size();
   size_t tbytes = c->fp32 ? 4 : 8;
   if ((size_t)2 * c->ns * c->nvt * tbytes + 4 * (size_t)c->ns * tbytes > 100 * 1024)
@@ -3200,6 +3215,7 @@ int32_t erm_set_tuning(erm_ctx *c, int32_t max_batch, int32_t pme_path, int32_t 
   if (group_planes > 0) c->tune_Q = group_planes;
   if (slab_threads > 0) c->xslab_T = slab_threads;
   c->P.pme_path = pme_path;
+  if (c->have_topo) set_default_batch(c);
   c->use_graph = use_graph != 0;
   if (c->have_frame) TRY(c->fp32 ? choose_slab<float>(c) : choose_slab<double>(c));
   return ERM_OK;

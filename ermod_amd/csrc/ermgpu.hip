@@ -1023,11 +1023,12 @@ struct PairShape {
 // Enough waves to fill the chip come first.  Every wave would take
 // PAIR_CHUNKS_PER_WAVE chunks of 64 molecules (the set-up of a workgroup is
 // shared); with fewer than PAIR_WAVES waves in all it takes less, down to
-// PAIR_MIN_MOLS molecules (48 water sites of a tile of 64), and a solute of
-// more than PAIR_PART sites whose configurations still leave half the chip
-// idle goes over in parts of at least PAIR_PART sites.  A rigid test particle
-// stays whole: a group's members sum its sites in one order whatever the
-// batch, and so does the context alone.  PAIR_WAVES = 1024 (4 per CU): with
+// PAIR_MIN_MOLS molecules (48 water sites of a tile of 64).  A molecule's sum
+// does not depend on that.  A large solute in solution, one configuration of
+// which would leave half the chip idle, goes over in parts of at least
+// PAIR_PART sites: always, since the parts' sums are added up and a
+// configuration gives the same bits in any batch.  A test particle has batches
+// to fill the chip with and stays whole.  PAIR_WAVES = 1024 (4 per CU): with
 // 4096, 256 configurations of a 20-site solute took four workgroups each and
 // their set-up cost more than it gave (12000 sites: division 11.35 against
 // 11.08 ms).  Measured per launch against 4 chunks per wave throughout: one
@@ -1042,10 +1043,7 @@ PairShape pair_shape(int n, double cand, int ns, int nwave, bool whole) {
   s.cm = std::min(64, (int)std::ceil(mpw / 16.0) * 16);
   const int per = s.cm * std::max(1, (int)std::ceil(mpw / s.cm)) * nwave;
   s.nsplit = std::max(1, (int)std::ceil(cand / per));
-  s.parts = 1;
-  const long waves = (long)n * s.nsplit * nwave;
-  if (!whole && ns > PAIR_PART && waves < PAIR_WAVES)
-    s.parts = std::min({PAIR_MAX_PARTS, ns / PAIR_PART, (int)((2 * PAIR_WAVES + waves - 1) / waves)});
+  s.parts = whole ? 1 : std::max(1, std::min(PAIR_MAX_PARTS, ns / PAIR_PART));
   s.nss = (ns + s.parts - 1) / s.parts;
   s.nss = (s.nss + PT_GRP - 1) / PT_GRP * PT_GRP;
   s.parts = (ns + s.nss - 1) / s.nss;
@@ -1064,7 +1062,7 @@ template <typename T> int launch_pair(erm_ctx *c, const Params &k, int n, bool b
   const int nwave = NTHR / 64;
   const size_t lt = pair_tile_lds<T>(ns, c->nvt, segcap, nwave);
   if (c->pair_path == 0 && lt <= c->lds_cap) {
-    const PairShape ps = pair_shape(n, frac * S, ns, nwave, c->P.slttype == 2);
+    const PairShape ps = pair_shape(n, frac * S, ns, nwave, c->P.slttype != 1);
     const size_t nuv = (size_t)n * (S + 1);
     double *out = dp<double>(c->d_uv);
     if (ps.parts > 1) {

@@ -1419,10 +1419,12 @@ __global__ __launch_bounds__(NTHR) void k_pme_ycol_reg(Params P, const typename 
 // complex row's bytes), and repeats x[0], x[1] in the row's two spare values
 // K1, K1 + 1.  Each thread then adds the planes' contributions to its MAXR
 // owned sites (FP64 sums).
-// gather of one group of nq real planes (first plane zz0, rows of K1 + 2)
-// into the per-site sums acc[] of the sites a thread owns.  PP: the spline
-// order at compile time (weights, row offsets and the p^3 products in
-// registers, loads independent); PP = 0 takes it from P.p.
+//
+// Gather of one group of nq real planes (first plane zz0, rows of K1 + 2)
+// into the per-site sums acc[] of the sites a thread owns, the planes in
+// ascending order as the groups are, so that a sum does not depend on the
+// slab's shape.  PP: the spline order at compile time (weights, row offsets and
+// the p^3 products in registers, loads independent); PP = 0 takes it from P.p.
 template <typename T, int K1, int MAXR, int PP, int XT>
 __device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int zz0, int nq, int s_beg,
                                              const int *gz, const int *__restrict__ zg, const T *__restrict__ zq,
@@ -1455,7 +1457,7 @@ __device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int
         xo[k] = x + ((x < 0) ? K1 : 0);
         yo[k] = (y + ((y < 0) ? K2 : 0)) * K1P;
       }
-      for (int c3 = clo; c3 <= chi; ++c3) {
+      for (int c3 = chi; c3 >= clo; --c3) {
         const T *ph = real + (size_t)(g3 - c3 - zz0) * plane;
         T sum = 0;
 #pragma unroll
@@ -1474,7 +1476,7 @@ __device__ __forceinline__ void xslab_gather(const Params &P, const T *real, int
         w1[k] = wz[k];
         w2[k] = wz[p + k];
       }
-      for (int c3 = clo; c3 <= chi; ++c3) {
+      for (int c3 = chi; c3 >= clo; --c3) {
         const T *ph = real + (size_t)(g3 - c3 - zz0) * plane;
         T sum = 0;
         for (int c2 = 0; c2 < p; ++c2) {
@@ -1556,7 +1558,7 @@ __device__ __forceinline__ void xslab_gather4(const Params &P, const T *real, in
       }
       const T *ph0 = real + (ptrdiff_t)(g3 - zz0) * plane;  // plane of c3 = 0
 #pragma unroll
-      for (int c3 = 0; c3 < 4; ++c3) {
+      for (int c3 = 3; c3 >= 0; --c3) {
         if (c3 < clo || c3 > chi) continue;
         const T *ph = ph0 - (ptrdiff_t)c3 * plane;
         T sum = 0;

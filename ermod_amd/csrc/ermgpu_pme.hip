@@ -41,15 +41,19 @@ int launch_zcol_fft_t(erm_ctx *c, const Params &k, int n, int nblk, size_t site0
                      dp<double>(c->d_selfp) + cfg0 * nblk);
   return ERM_OK;
 }
-// z columns spread and transformed along z (spline orders 4 and 6)
+// z columns spread and transformed along z (spline orders 4 and 6; not FP64
+// columns of 64, which z_kernel gives to the two-step kernel)
 template <typename T, int K>
 int launch_zcol_fft(erm_ctx *c, const Params &k, int n, int nblk, size_t site0, size_t cfg0) {
-  if (k.p == 4) {
-    if (c->zcol_T == 512) return launch_zcol_fft_t<T, K, 4, 512>(c, k, n, nblk, site0, cfg0);
-    return launch_zcol_fft_t<T, K, 4, NTHR>(c, k, n, nblk, site0, cfg0);
+  if constexpr (sizeof(T) == 4 || K < 64) {
+    if (k.p == 4) {
+      if (c->zcol_T == 512) return launch_zcol_fft_t<T, K, 4, 512>(c, k, n, nblk, site0, cfg0);
+      return launch_zcol_fft_t<T, K, 4, NTHR>(c, k, n, nblk, site0, cfg0);
+    }
+    if (c->zcol_T == 512) return launch_zcol_fft_t<T, K, 6, 512>(c, k, n, nblk, site0, cfg0);
+    return launch_zcol_fft_t<T, K, 6, NTHR>(c, k, n, nblk, site0, cfg0);
   }
-  if (c->zcol_T == 512) return launch_zcol_fft_t<T, K, 6, 512>(c, k, n, nblk, site0, cfg0);
-  return launch_zcol_fft_t<T, K, 6, NTHR>(c, k, n, nblk, site0, cfg0);
+  return fail(c, ERM_E_ENG_BUG, "register z columns of 64 in FP64");
 }
 // z columns of a heterogeneous batch (run table in device memory): a
 // persistent grid (as many workgroups as fit the device at once) pulling
@@ -73,12 +77,15 @@ int launch_zcol_runs_t(erm_ctx *c, const Params &k, int nblk, const GRun *runs, 
 }
 template <typename T, int K>
 int launch_zcol_fft_runs(erm_ctx *c, const Params &k, int nblk, const GRun *runs, int nrun, int nitem, int *counter) {
-  if (k.p == 4) {
-    if (c->zcol_T == 512) return launch_zcol_runs_t<T, K, 4, 512>(c, k, nblk, runs, nrun, nitem, counter);
-    return launch_zcol_runs_t<T, K, 4, NTHR>(c, k, nblk, runs, nrun, nitem, counter);
+  if constexpr (sizeof(T) == 4 || K < 64) {
+    if (k.p == 4) {
+      if (c->zcol_T == 512) return launch_zcol_runs_t<T, K, 4, 512>(c, k, nblk, runs, nrun, nitem, counter);
+      return launch_zcol_runs_t<T, K, 4, NTHR>(c, k, nblk, runs, nrun, nitem, counter);
+    }
+    if (c->zcol_T == 512) return launch_zcol_runs_t<T, K, 6, 512>(c, k, nblk, runs, nrun, nitem, counter);
+    return launch_zcol_runs_t<T, K, 6, NTHR>(c, k, nblk, runs, nrun, nitem, counter);
   }
-  if (c->zcol_T == 512) return launch_zcol_runs_t<T, K, 6, 512>(c, k, nblk, runs, nrun, nitem, counter);
-  return launch_zcol_runs_t<T, K, 6, NTHR>(c, k, nblk, runs, nrun, nitem, counter);
+  return fail(c, ERM_E_ENG_BUG, "register z columns of 64 in FP64");
 }
 // inverse y columns, one lane per column
 template <typename T, int K> int launch_ycol_reg(erm_ctx *c, const Params &k, int n) {

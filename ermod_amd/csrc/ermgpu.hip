@@ -995,7 +995,8 @@ inline int pair_splits(int nchunk, int nwave) {
 }
 
 // Waves per workgroup of the persistent pair grid: the fewest (4, 8 or 12)
-// with which the CU holds the most waves, up to the 12 their registers allow.
+// with which the CU holds the most waves, up to 12 (three per SIMD, see
+// k_pair_tile).
 // The solute's sites and LJ rows are in LDS once per workgroup, so a large
 // solute's grid wants many waves in one workgroup (150 sites against 14
 // solvent types: 28 KB, with 4 waves 8 per CU, with 12 in one
@@ -1108,10 +1109,8 @@ template <typename T> int launch_pair(erm_ctx *c, const Params &k, int n, bool b
   return launch_check(c, "k_pair");
 }
 
-// realcal_self of n configurations of k.ns sites into out[n].  A workgroup
-// per configuration: 1024 threads from 64 sites on (2016 pairs, two or more
-// per thread), where a configuration's pairs are the longest chain of the
-// launch, 256 below it.
+// realcal_self of n configurations of k.ns sites into out[n][self_parts(k.ns)],
+// a workgroup of 256 threads each; k_u0 or the host adds a configuration's parts
 void launch_selfreal(erm_ctx *c, const Params &k, int n, const double *spos, const double *q, double *out) {
   hipLaunchKernelGGL(k_selfreal, dim3(n, self_parts(k.ns)), dim3(NTHR), 0, c->st, k, spos, q, out);
 }
@@ -3272,8 +3271,9 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
     return ERM_OK;
   };
   c->use_graph = false;
-  c->xslab_set = true;
-  auto apply = [&](int B, int pp, int Sc, int Qc, int Tc) -> int {
+  bool bestX = c->xslab_set;
+  auto apply = [&](int B, int pp, int Sc, int Qc, int Tc, bool set) -> int {
+    c->xslab_set = set;
     c->Bmax = B;
     c->P.pme_path = pp;
     c->tune_S = Sc;
@@ -3282,19 +3282,22 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
     return c->fp32 ? choose_slab<float>(c) : choose_slab<double>(c);
   };
   const int S0 = c->tune_S, Q0 = c->tune_Q, T0 = c->xslab_T;
+  const bool X0 = c->xslab_set;
   for (int B : {128, 256, 512, 1024}) {
     if (B > 4 * n_trial && B > 128) break;
     for (int pp : paths) {
       // the slab depth shapes the fused LDS path and the FP32 x slab, the
-      // planes per group and the workgroup size the latter alone
+      // planes per group and the workgroup size the latter alone, which also
+      // has the shape that it chooses itself (Sc = 0)
       const bool xs = pp == 3 && c->fp32, deep = pp == 1 || xs;
-      for (int Sc : {16, 8, 6, 5, 4, 3}) {
+      for (int Sc : {0, 16, 8, 6, 5, 4, 3}) {
         for (int Qc : {16, 9, 8, 5, 4, 3}) {
           for (int Tc : {256, 512}) {
-            if (!deep && Sc != 16) continue;
-            if (!xs && (Qc != 8 || Tc != 256)) continue;
-            const int S1 = deep ? Sc : S0, Q1 = xs ? Qc : Q0, T1 = xs ? Tc : T0;
-            if (apply(B, pp, S1, Q1, T1) != ERM_OK) {
+            if (deep ? Sc == 0 && !xs : Sc != 16) continue;
+            if ((!xs || Sc == 0) && (Qc != 8 || Tc != 256)) continue;
+            const bool set = xs ? Sc != 0 : X0;
+            const int S1 = deep && Sc ? Sc : S0, Q1 = xs && Sc ? Qc : Q0, T1 = xs && Sc ? Tc : T0;
+            if (apply(B, pp, S1, Q1, T1, set) != ERM_OK) {
               c->err.clear();
               continue;
             }
@@ -3307,13 +3310,14 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
               bestS = S1;
               bestQ = Q1;
               bestT = T1;
+              bestX = set;
             }
           }
         }
       }
     }
   }
-  TRY(apply(bestB, bestP, bestS, bestQ, bestT));
+  TRY(apply(bestB, bestP, bestS, bestQ, bestT, bestX));
   c->batch_set = true;
   if (bestP == 3) {  // z-column workgroup size for the chosen shape
     const int z0 = c->zcol_T;
@@ -3328,7 +3332,7 @@ int32_t erm_autotune(erm_ctx *c, int32_t n_trial, uint64_t seed, double *best_ms
     }
     c->zcol_T = bestZ ? bestZ : z0;
     // inverse y transform inside the x slab, or its own kernel
-    if (c->fp32 && c->xslab_T == 512 && c->kp.K2 == c->kp.K1) {
+    if (c->fp32 && bestX && c->xslab_T == 512 && c->kp.K2 == c->kp.K1) {
       const bool y0 = c->xslab_yf;
       int besty = -1;
       for (int yf : {0, 1}) {

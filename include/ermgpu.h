@@ -377,8 +377,10 @@ int32_t erm_stage_times(const erm_ctx *ctx, double *ms10);
  * without uvengy from a captured HIP graph (the first call of a given shape
  * runs eagerly and captures; a change of frame geometry, batch shape or
  * buffers re-captures); slab_planes (1..16) caps the z planes of one fused
- * PME slab (paths 1 and 3) and group_planes (1..16) the planes the FP32
- * register path transforms per group, slab_threads and column_threads (256 or
+ * PME slab (paths 1 and 3, which with groups need a slab of at most two thirds
+ * halo, planes + order - 1 <= 3 planes, in either precision) and group_planes
+ * (1..16) the planes the FP32 register path transforms per group, slab_threads
+ * and column_threads (256 or
  * 512) the workgroup sizes of its x slab and of the z columns (0 keeps any of
  * them); fold_y = 1 moves the inverse y transform into 512-thread x slabs of a
  * grid with K2 = K1, 0 keeps it in its own kernel, -1 keeps the setting.

@@ -21,6 +21,8 @@ PEAK = os.path.join(HERE, "csrc", "ermpeak.hip")
 # register-FFT grid lengths per precision (the run-time dispatch in
 # ermgpu.hip covers exactly these)
 PME_UNITS = [("double", k) for k in (16, 24, 32, 48, 64)] + [("float", k) for k in (16, 24, 32, 48, 64, 96)]
+# FP32 lengths of the z columns with all radix steps in registers, several per unit
+Z_UNITS = [(16, 18, 20, 24, 25, 27, 30), (32, 36, 40, 45), (48, 50, 54), (60, 64), (72, 75), (80, 81), (90, 96), (100,)]
 HEADERS = [os.path.join(HERE, "csrc", f) for f in ("ermgpu_dev.h", "ermgpu_kern.h", "ermgpu_fft2.h", "ermgpu_grad.h", "ermgpu_erfc.h",
                                                          "ermgpu_traj.h", "ermgpu_ctx.h")] + [
     os.path.join(ROOT, "include", "ermgpu.h")]
@@ -48,6 +50,9 @@ def build_lib(verbose: bool = False, jobs: int = 0) -> str:
     units = [([MAIN], os.path.join(BUILD_DIR, "ermgpu.o"))]
     for t, k in PME_UNITS:
         units.append(([f"-DERM_T={t}", f"-DERM_K={k}", PME], os.path.join(BUILD_DIR, f"pme_{t[0]}{k}.o")))
+    for i, ks in enumerate(Z_UNITS):
+        lens = " ".join(f"ERM_Z({k})" for k in ks)
+        units.append((["-DERM_T=float", f"-DERM_ZLENS={lens}", PME], os.path.join(BUILD_DIR, f"z_f{i}.o")))
     jobs = jobs or min(len(units) + 1, max(1, os.cpu_count() or 1), 16)
     cmds = [[HIPCC, *FLAGS, "-c", *src, "-o", obj] for src, obj in units]
     peak = os.path.join(HERE, "libermpeak.so")

@@ -500,6 +500,35 @@ template <typename T> bool reg_path_ok(const erm_ctx *c) {
   return reg_len<T>(k.K1) && reg_len<T>(k.K2) && reg_len<T>(k.K3) && (k.K1 % 2 == 0);
 }
 
+// FP32 z lengths with k_pme_zcol_dit
+#define ERM_ZSWITCH(K, CALL)                   \
+  switch (K) {                                 \
+    case 16: { constexpr int KK = 16; CALL; } break; \
+    case 18: { constexpr int KK = 18; CALL; } break; \
+    case 20: { constexpr int KK = 20; CALL; } break; \
+    case 24: { constexpr int KK = 24; CALL; } break; \
+    case 25: { constexpr int KK = 25; CALL; } break; \
+    case 27: { constexpr int KK = 27; CALL; } break; \
+    case 30: { constexpr int KK = 30; CALL; } break; \
+    case 32: { constexpr int KK = 32; CALL; } break; \
+    case 36: { constexpr int KK = 36; CALL; } break; \
+    case 40: { constexpr int KK = 40; CALL; } break; \
+    case 45: { constexpr int KK = 45; CALL; } break; \
+    case 48: { constexpr int KK = 48; CALL; } break; \
+    case 50: { constexpr int KK = 50; CALL; } break; \
+    case 54: { constexpr int KK = 54; CALL; } break; \
+    case 60: { constexpr int KK = 60; CALL; } break; \
+    case 64: { constexpr int KK = 64; CALL; } break; \
+    case 72: { constexpr int KK = 72; CALL; } break; \
+    case 75: { constexpr int KK = 75; CALL; } break; \
+    case 80: { constexpr int KK = 80; CALL; } break; \
+    case 81: { constexpr int KK = 81; CALL; } break; \
+    case 90: { constexpr int KK = 90; CALL; } break; \
+    case 96: { constexpr int KK = 96; CALL; } break; \
+    case 100: { constexpr int KK = 100; CALL; } break; \
+    default: break;                            \
+  }
+
 // Configurations per batch when the caller leaves the choice (max_batch = 0):
 // 1024 where the buffers of so many stay within 4 GiB, else 256.  Counted is
 // what grows with the grid or with a molecule count: half spectra, the sites'
@@ -537,17 +566,21 @@ void set_default_batch(erm_ctx *c) {
 // the general one.  In FP64 the registers win where a column leaves room for two
 // waves per SIMD: 1000 configurations of 48^3 0.335 against 0.416 ms in two
 // steps; a 64-point column does not (500 configurations of 64^3, order 6: 0.751
-// against 0.475).  FP32 takes registers where the whole grid has register
-// lengths and two steps elsewhere, the order of whose sums each had before
-// (launch_yx).
-enum ZKernel { Z_SPEC, Z_FFT, Z_TWO, Z_LDS };
+// against 0.475).  FP32 takes them where the whole grid has register lengths;
+// elsewhere Z_DIT, which has a column in registers too and the order of sums of
+// Z_LDS, up to 100 points, and two steps in that order beyond and for other
+// spline orders (launch_yx).
+enum ZKernel { Z_SPEC, Z_FFT, Z_DIT, Z_TWO, Z_LDS };
 ZKernel z_kernel(const erm_ctx *c, bool regp) {
   const int K3 = c->kp.K3;
   const bool p46 = c->kp.p == 4 || c->kp.p == 6;
   const bool reg = p46 && (c->fp32 ? regp : reg_len<double>(K3) && K3 < 64);
   if (regp) return !p46 ? Z_SPEC : reg ? Z_FFT : Z_TWO;
   if (!c->two_step) return Z_LDS;
-  return reg ? Z_FFT : Z_TWO;
+  if (reg) return Z_FFT;
+  bool dit = false;
+  if (c->fp32 && p46) ERM_ZSWITCH(K3, dit = KK > 0)
+  return dit ? Z_DIT : Z_TWO;
 }
 // z-column workgroups per configuration
 int zcol_groups(const erm_ctx *c, bool regp, int vb) {
@@ -558,10 +591,10 @@ int zcol_groups(const erm_ctx *c, bool regp, int vb) {
     const int w = zcol_width(c->kp.K3, vb);
     return (ncol + w - 1) / w;
   }
-  const int zt = (c->zcol_T == 512) ? 512 : NTHR;
+  const int zt = (c->zcol_T == 512 && zk != Z_DIT) ? 512 : NTHR;
   // lanes per column: the spectral form one, the spread-and-FFT form
   // zfft_lanes (vb = 2 sizeof(T))
-  const int L = zk == Z_SPEC ? 1 : zfft_lanes(vb / 2, c->kp.K3);
+  const int L = (zk == Z_SPEC || zk == Z_DIT) ? 1 : zfft_lanes(vb / 2, c->kp.K3);
   return (L * ncol + zt - 1) / zt;
 }
 
@@ -1165,8 +1198,10 @@ template <typename T> int run_energies(erm_ctx *c, const Batch &bt, int flags) {
       rz = launch_zcol2<T>(c, k, n, nzg);
     } else if (zk == Z_SPEC) {
       ERM_KSWITCH(K3, (rz = launch_zcol_reg<T, KK>(c, k, n, nzg)));
-    } else {
+    } else if (zk == Z_FFT) {
       ERM_KSWITCH(K3, (rz = launch_zcol_fft<T, KK>(c, k, n, nzg)));
+    } else if constexpr (sizeof(T) == 4) {
+      ERM_ZSWITCH(K3, (rz = launch_zcol_dit<KK>(c, k, n, nzg)));
     }
     TRY(rz);
     TRY(launch_check(c, "z columns"));

@@ -263,6 +263,8 @@ template <typename T, int K>
 int launch_zcol_fft(erm_ctx *c, const Params &k, int n, int nblk, size_t site0 = 0, size_t cfg0 = 0);
 template <typename T, int K>
 int launch_zcol_fft_runs(erm_ctx *c, const Params &k, int nblk, const GRun *runs, int nrun, int nitem, int *counter);
+// FP32 alone
+template <int K> int launch_zcol_dit(erm_ctx *c, const Params &k, int n, int nblk);
 // FP32 alone (FP64: k_pme_xyslab)
 template <typename T, int K> int launch_ycol_reg(erm_ctx *c, const Params &k, int n);
 struct XsShape {

@@ -92,9 +92,17 @@ template <int SIGN, bool ROOT = false> __device__ __forceinline__ float2 tmul(fl
   }
   return r;
 }
+// an axis' table at places that are the same in every lane: through the
+// constant address space it comes by scalar loads, also behind barriers
+struct UTab {
+  const __attribute__((address_space(4))) float *t;
+  __device__ __forceinline__ explicit UTab(const float2 *tw)
+      : t((const __attribute__((address_space(4))) float *)(uintptr_t)tw) {}
+  __device__ __forceinline__ float2 operator[](int i) const { return make_float2(t[2 * i], t[2 * i + 1]); }
+};
 // R-point DFT; tw, str: w_R^j = tw[str j]
 template <int R, int SIGN>
-__device__ __forceinline__ void dit_dft(float2 (&x)[R], const float2 *__restrict__ tw, int str) {
+__device__ __forceinline__ void dit_dft(float2 (&x)[R], UTab tw, int str) {
 #pragma clang fp contract(off)
   if constexpr (R == 4) {
     const float2 s0 = cadd(x[0], x[2]), d0 = csub(x[0], x[2]), s1 = cadd(x[1], x[3]), d1 = csub(x[1], x[3]);
@@ -123,12 +131,15 @@ __device__ __forceinline__ void dit_dft(float2 (&x)[R], const float2 *__restrict
 // The radix steps of an N-point block of a K-point transform, those before it
 // (with product A) giving its place k: x[n1] in, frequency k + A kk out at
 // x[kk].  tw is the table in memory (read at uniform places), lt the same in
-// LDS (read at the lane's own); A = 1 for the first block (FIRST).
-template <int N, int PP, int SIGN, bool FIRST>
-__device__ __forceinline__ void dit_steps(float2 (&x)[N], int K, int A, int k, const float2 *__restrict__ tw,
-                                          const float2 *lt) {
+// LDS (read at the lane's own); A = 1 for the first block (FIRST), N = K where
+// that is the whole transform.
+template <int N, int PP, int SIGN, bool FIRST, bool WHOLE = false>
+__device__ __forceinline__ void dit_steps(float2 (&x)[N], int K, int A, int k, UTab tw, const float2 *lt) {
   constexpr int R = first_radix(N / PP), M = N / (PP * R);
-  asm volatile("" : "+s"(K));  // the table's values stay out of the registers of other steps
+  if constexpr (WHOLE)
+    K = N;
+  else
+    asm volatile("" : "+s"(K));  // the table's values stay out of the registers of other steps
   float2 y[N];
 #pragma unroll
   for (int r = 0; r < M; ++r)
@@ -146,11 +157,16 @@ __device__ __forceinline__ void dit_steps(float2 (&x)[N], int K, int A, int k, c
       }
       dit_dft<R, SIGN>(v, tw, K / R);
 #pragma unroll
-      for (int q = 0; q < R; ++q) y[kk + PP * (q + R * r)] = v[q];
+      for (int q = 0; q < R; ++q) {
+        // a whole transform's butterflies stay in this order and in this place:
+        // mixed or moved to where their results are used they take twice the registers
+        if constexpr (WHOLE) asm volatile("" : "+v"(v[q].x), "+v"(v[q].y));
+        y[kk + PP * (q + R * r)] = v[q];
+      }
     }
 #pragma unroll
   for (int i = 0; i < N; ++i) x[i] = y[i];
-  if constexpr (PP * R < N) dit_steps<N, PP * R, SIGN, FIRST>(x, K, A, k, tw, lt);
+  if constexpr (PP * R < N) dit_steps<N, PP * R, SIGN, FIRST, WHOLE>(x, K, A, k, tw, lt);
 }
 
 // a times the conjugate of w (the twiddle tables hold e^{-2 pi i j / K})
@@ -443,10 +459,16 @@ __device__ __forceinline__ void z2_front32(const Z2Args &q, int B, unsigned char
   __syncthreads();
   if (q.sub < B) {
     float2 *col = reinterpret_cast<float2 *>(lds) + q.cl;
-    dit_steps<A, 1, -1, true>(x, K3, 1, 0, tw, tw);
+    dit_steps<A, 1, -1, true>(x, K3, 1, 0, UTab(tw), tw);
 #pragma unroll
     for (int k = 0; k < A; ++k) col[(q.sub + B * k) * C] = x[k];
   }
+}
+
+// a product that no sum after it is fused with
+__device__ __forceinline__ float2 zscale(float2 a, float g) {
+#pragma clang fp contract(off)
+  return make_float2(a.x * g, a.y * g);
 }
 
 // second forward step of (k2 < A, column) and the Green's function, the
@@ -464,7 +486,7 @@ __device__ __forceinline__ double z2_mid32(float2 *col, int K3, int A, int k2, c
     for (int k = 0; k < B; ++k) gv[k] = g[(size_t)(k2 + A * k) * gstr];
 #pragma unroll
     for (int n = 0; n < B; ++n) x[n] = col[(B * k2 + n) * Z2_COLS];
-    dit_steps<B, 1, -1, false>(x, K3, A, k2, tw, lt);
+    dit_steps<B, 1, -1, false>(x, K3, A, k2, UTab(tw), lt);
 #pragma unroll
     for (int k = 0; k < B; ++k) {
       self += (double)gv[k] * ((double)x[k].x * (double)x[k].x + (double)x[k].y * (double)x[k].y);
@@ -486,7 +508,7 @@ __device__ __forceinline__ void z2_back32(float2 *col, int K3, int B, int n1, co
   float2 x[A];
 #pragma unroll
   for (int i = 0; i < A; ++i) x[i] = col[(n1 + B * i) * Z2_COLS];
-  dit_steps<A, 1, +1, true>(x, K3, 1, 0, tw, tw);
+  dit_steps<A, 1, +1, true>(x, K3, 1, 0, UTab(tw), tw);
 #pragma unroll
   for (int k = 0; k < A; ++k) col[(n1 + B * k) * Z2_COLS] = x[k];
 }
@@ -498,7 +520,7 @@ __device__ __forceinline__ void z2_last32(const float2 *col, int K3, int A, int 
   float2 x[B];
 #pragma unroll
   for (int n = 0; n < B; ++n) x[n] = col[(B * k2 + n) * Z2_COLS];
-  dit_steps<B, 1, +1, false>(x, K3, A, k2, tw, lt);
+  dit_steps<B, 1, +1, false>(x, K3, A, k2, UTab(tw), lt);
 #pragma unroll
   for (int k = 0; k < B; ++k) out[(size_t)(k2 + A * k) * ostr] = x[k];
 }
@@ -552,6 +574,156 @@ static __global__ __launch_bounds__(Z2_MAXT32) void k_pme_zcol2_f32(
   }
 }
 
+// FP32 z columns of up to 100 points and spline orders 4 and 6 with one lane per
+// column (m1, m2), the whole column in its registers: spread plane by plane
+// from a list of each plane's sites in the solute's order, transformed by all
+// radix steps at once.  The same values as k_pme_zcol2_f32 without its trips
+// through LDS: 701 configurations of 45 x 60 x 75 with 33 solute sites 0.66 ->
+// 0.42 ms, 500 of 60^3, order 6, 0.43 -> 0.27, 40 of 90^3 with 300 sites 0.33 ->
+// 0.29.  Bound by issue in the transforms (two waves per SIMD) and by latency in
+// the spread, whose reads run one entry ahead.
+constexpr int ZD_SCH = 64;  // solute sites per chunk, a bit each
+constexpr int ZD_KMAX = 127;
+__host__ __device__ inline size_t zdit_lds(int H, int K2, int K3, int p) {
+  return sizeof(int4) * ((size_t)ZD_SCH * p + 2) + sizeof(unsigned long long) * K3 + sizeof(double) * (NTHR / 64) +
+         sizeof(float2) * (size_t)ZD_SCH * (H + zcol_fft_rows(H, K2, NTHR, 1)) + sizeof(float) * ZD_SCH +
+         sizeof(int) * (K3 + 1);
+}
+template <int K3, int PP>
+__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2))) void k_pme_zcol_dit(
+    Params P, const float *__restrict__ engfac, const int *__restrict__ sg3, const float *__restrict__ sw3,
+    const float *__restrict__ sqv, const float2 *__restrict__ w1h, const float2 *__restrict__ w2h,
+    const float2 *__restrict__ tw3, float2 *Hk, double *selfp) {
+  static_assert(K3 <= ZD_KMAX, "two planes per lane of the scan");
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int b = blockIdx.y, ns = P.ns, H = P.H, K2 = P.K2, ncol = H * K2;
+  const int c = blockIdx.x * NTHR + (int)threadIdx.x;
+  const bool on = c < ncol;
+  const int m2 = on ? c / H : 0, m1 = on ? c - m2 * H : 0;
+  const int m2lo = blockIdx.x * NTHR / H, nm2 = min((int)(blockIdx.x + 1) * NTHR - 1, ncol - 1) / H - m2lo + 1;
+  // [ZD_SCH PP + 2] the planes' sites in order: places in l1 and l2, z weight, charge
+  int4 *ent = reinterpret_cast<int4 *>(lds_raw);
+  unsigned long long *mask = reinterpret_cast<unsigned long long *>(ent + ZD_SCH * PP + 2);  // [K3] sites of a plane
+  double *red = reinterpret_cast<double *>(mask + K3);
+  float2 *l1 = reinterpret_cast<float2 *>(red + NTHR / 64);  // [ZD_SCH][H] spectra along x
+  float2 *l2 = l1 + ZD_SCH * H;                              // [ZD_SCH][nm2] the block's rows of those along y
+  float *lq = reinterpret_cast<float *>(l2 + ZD_SCH * zcol_fft_rows(H, K2, NTHR, 1));  // [ZD_SCH] charges
+  int *st = reinterpret_cast<int *>(lq + ZD_SCH);            // [K3 + 1] first entry of a plane
+  float2 x[K3];
+#pragma unroll
+  for (int z = 0; z < K3; ++z) x[z] = make_float2(0.0f, 0.0f);
+  const size_t bs = (size_t)b * ns;
+  const int row = on ? m2 - m2lo : 0;
+  for (int s0 = 0; s0 < ns; s0 += ZD_SCH) {
+    const int nc = min(ZD_SCH, ns - s0);
+    const size_t o = bs + s0;
+    __syncthreads();  // the previous chunk is used up
+    for (int z = threadIdx.x; z < K3; z += NTHR) mask[z] = 0ull;
+    for (int t = threadIdx.x; t < nc * H; t += NTHR) l1[t] = w1h[o * H + t];
+    for (int t = threadIdx.x; t < nc * nm2; t += NTHR) {
+      const int j = t / nm2;
+      l2[t] = w2h[(o + j) * K2 + m2lo + (t - j * nm2)];
+    }
+    for (int t = threadIdx.x; t < nc; t += NTHR) lq[t] = sqv[o + t];
+    __syncthreads();
+    auto plane = [&](int t, int &j) {
+      j = t / PP;
+      const int k = t - j * PP, g = sg3[o + j];
+      return g - k + (g < k ? K3 : 0);
+    };
+    for (int t = threadIdx.x; t < nc * PP; t += NTHR) {
+      int j;
+      const int z = plane(t, j);
+      atomicOr(mask + z, 1ull << j);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {  // first entries: a scan over the planes, two per lane
+      const int z = 2 * threadIdx.x;
+      const int n0 = z < K3 ? __popcll(mask[z]) : 0, n1 = z + 1 < K3 ? __popcll(mask[z + 1]) : 0;
+      int inc = n0 + n1;
+      for (int d = 1; d < 64; d <<= 1) {
+        const int u = __shfl_up(inc, d, 64);
+        if ((int)threadIdx.x >= d) inc += u;
+      }
+      if (z <= K3) st[z] = inc - n0 - n1;
+      if (z + 1 <= K3) st[z + 1] = inc - n1;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < nc * PP; t += NTHR) {
+      int j;
+      const int z = plane(t, j), e = st[z] + __popcll(mask[z] & ((1ull << j) - 1));
+      ent[e] = make_int4(j * H, j * nm2, __float_as_int(sw3[o * PP + t]), __float_as_int(lq[j]));
+    }
+    if (threadIdx.x < 2) ent[nc * PP + threadIdx.x] = make_int4(0, 0, 0, 0);  // read ahead, not used
+    __syncthreads();
+    // one entry after another, its spectra loaded one entry ahead and its place two
+    int e = 0;
+    int4 h = ent[0], h1 = ent[1];
+    float2 u = l1[h.x + m1], v = l2[h.y + row];
+#pragma unroll
+    for (int z = 0; z < K3; ++z) {
+      const int e1 = __builtin_amdgcn_readfirstlane(st[z + 1]);
+      while (e < e1) {
+        const int4 h2 = ent[e + 2];
+        const float2 u1 = l1[h1.x + m1], v1 = l2[h1.y + row];
+        float2 a = tmul<-1>(u, v);
+        const float w = __int_as_float(h.z), q = __int_as_float(h.w);
+        a.x *= q;
+        a.y *= q;
+        x[z].x = fmaf(a.x, w, x[z].x);
+        x[z].y = fmaf(a.y, w, x[z].y);
+        h = h1;
+        h1 = h2;
+        u = u1;
+        v = v1;
+        ++e;
+      }
+    }
+  }
+  dit_steps<K3, 1, -1, true, true>(x, K3, 1, 0, UTab(tw3), tw3);
+  // the Green's function in groups of 8 values, loaded a group ahead
+  constexpr int GL = 8, NG = (K3 + GL - 1) / GL;
+  int gi = on ? c : 0;
+  float gv[2][GL];
+  auto load = [&](float (&v)[GL], int m0) {
+    asm volatile("" : "+v"(gi));  // not before the transform, nor all at once
+#pragma unroll
+    for (int i = 0; i < GL; ++i)
+      if (m0 + i < K3) v[i] = engfac[gi + (size_t)i * ncol];
+    gi += GL * ncol;
+  };
+  load(gv[0], 0);
+  double self = 0.0;
+#pragma unroll
+  for (int q = 0; q < NG; ++q) {
+    if (q + 1 < NG) load(gv[(q + 1) & 1], (q + 1) * GL);
+#pragma unroll
+    for (int i = 0; i < GL; ++i)
+      if (q * GL + i < K3) {
+        float2 &v = x[q * GL + i];
+        const float g = gv[q & 1][i];
+        self += (double)g * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
+        v = zscale(v, g);
+      }
+    asm volatile("" : "+v"(self));  // here, not after the inverse transform
+  }
+  dit_steps<K3, 1, +1, true, true>(x, K3, 1, 0, UTab(tw3), tw3);
+  if (on) {
+    float2 *out = Hk + (size_t)b * K3 * ncol + c;
+#pragma unroll
+    for (int z = 0; z < K3; ++z) out[(size_t)z * ncol] = x[z];
+  }
+  self = on ? ((m1 == 0 || 2 * m1 == P.K1) ? 0.5 : 1.0) * self : 0.0;
+  for (int d = 32; d > 0; d >>= 1) self += __shfl_xor(self, d, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = self;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double sum = red[0];
+    for (int w = 1; w < NTHR / 64; ++w) sum += red[w];
+    selfp[(size_t)b * gridDim.x + blockIdx.x] = sum;
+  }
+}
+
 // --------------------------------------------------------------------------
 // y and x transforms of a slab of z planes, and the gather (the owned planes
 // [zb, zb + S) and their p - 1 halo planes, Q planes in LDS at a time; the
@@ -584,7 +756,7 @@ __device__ __forceinline__ void xy2_yfirst(bool on, const typename C2<T>::type *
 #pragma unroll
   for (int i = 0; i < A; ++i) x[i] = src[off + i * sstr];
   if constexpr (sizeof(T) == 4)
-    dit_steps<A, 1, +1, true>(x, K, 1, 0, gtw, gtw);
+    dit_steps<A, 1, +1, true>(x, K, 1, 0, UTab(gtw), gtw);
   else
     reg_fft<A, +1>(x);
   if (!on) return;
@@ -602,7 +774,7 @@ __device__ __forceinline__ void xy2_ysecond(bool on, typename C2<T>::type *col, 
   for (int n = 0; n < B; ++n) x[n] = col[(k2 * B + n) * rs];
   wave_lds_sync();
   if constexpr (sizeof(T) == 4)
-    dit_steps<B, 1, +1, false>(x, K, A, k2, gtw, tw);
+    dit_steps<B, 1, +1, false>(x, K, A, k2, UTab(gtw), tw);
   else
     reg_fft<B, +1>(x);
   if (!on) return;
@@ -661,7 +833,7 @@ __device__ __forceinline__ void xy2_xfirst(bool on, int o2, typename C2<T>::type
   }
   wave_lds_sync();
   if constexpr (sizeof(T) == 4)
-    dit_steps<A, 1, +1, true>(x, K1, 1, 0, gtw, gtw);
+    dit_steps<A, 1, +1, true>(x, K1, 1, 0, UTab(gtw), gtw);
   else
     reg_fft<A, +1>(x);
   if (!on) return;
@@ -681,7 +853,7 @@ __device__ __forceinline__ void xy2_xsecond(bool on, bool two, typename C2<T>::t
   for (int n = 0; n < B; ++n) x[n] = pr[xy2_blk(k2, B, pad) + n];
   wave_lds_sync();
   if constexpr (sizeof(T) == 4)
-    dit_steps<B, 1, +1, false>(x, K1, A, k2, gtw, tw);
+    dit_steps<B, 1, +1, false>(x, K1, A, k2, UTab(gtw), tw);
   else
     reg_fft<B, +1>(x);
   if (!on) return;

@@ -1,15 +1,17 @@
 // ermgpu_pme.hip -- the register-FFT kernels of one precision and grid
 // length: z columns, in FP32 the y columns and the x slab with the gather, and
 // the adjoint's solvent-potential transforms.  Compiled once per (ERM_T,
-// ERM_K) so that the instantiations build in parallel; ermgpu.hip dispatches
-// on the grid length at run time.
+// ERM_K), or per list ERM_ZLENS of FP32 lengths of k_pme_zcol_dit, so that the
+// instantiations build in parallel; ermgpu.hip dispatches on the grid length at
+// run time.
 #include <algorithm>
 
 #include "ermgpu_ctx.h"
+#include "ermgpu_fft2.h"
 #include "ermgpu_grad.h"
 
 #ifndef ERM_T
-#error "ERM_T (float or double) and ERM_K (grid length) select the instantiation"
+#error "ERM_T (float or double) and ERM_K (grid length), or ERM_ZLENS, select the instantiations"
 #endif
 
 namespace ermh {
@@ -154,6 +156,21 @@ template <typename T, int K> void launch_zgreen(erm_ctx *c, const Params &k) {
                      dp<T>(c->d_engfac), dp<V>(c->d_tw3), dp<V>(c->d_gHk));
 }
 
+#ifdef ERM_ZLENS
+template <int K, int PP> int launch_zcol_dit_t(erm_ctx *c, const Params &k, int n, int nblk) {
+  const size_t lds = zdit_lds(k.H, k.K2, K, PP);
+  TRY(set_lds(c, (const void *)k_pme_zcol_dit<K, PP>, lds, "k_pme_zcol_dit"));
+  hipLaunchKernelGGL((k_pme_zcol_dit<K, PP>), dim3(nblk, n), dim3(NTHR), lds, c->st, k, dp<float>(c->d_engfac),
+                     dp<int>(c->d_sg3), dp<float>(c->d_sw3), dp<float>(c->d_sqv), dp<float2>(c->d_w1h),
+                     dp<float2>(c->d_w2h), dp<float2>(c->d_tw3), dp<float2>(c->d_Hk), dp<double>(c->d_selfp));
+  return launch_check(c, "k_pme_zcol_dit");
+}
+template <int K> int launch_zcol_dit(erm_ctx *c, const Params &k, int n, int nblk) {
+  return k.p == 4 ? launch_zcol_dit_t<K, 4>(c, k, n, nblk) : launch_zcol_dit_t<K, 6>(c, k, n, nblk);
+}
+#define ERM_Z(K) template int launch_zcol_dit<K>(erm_ctx *, const Params &, int, int);
+ERM_ZLENS
+#else
 template int launch_zcol_reg<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int);
 template int launch_zcol_fft<ERM_T, ERM_K>(erm_ctx *, const Params &, int, int, size_t, size_t);
 template int launch_zcol_fft_runs<ERM_T, ERM_K>(erm_ctx *, const Params &, int, const GRun *, int, int, int *);
@@ -164,5 +181,6 @@ template void launch_xc2r<ERM_T, ERM_K>(erm_ctx *, const Params &);
 template void launch_ydense<ERM_T, ERM_K, -1>(erm_ctx *, const Params &);
 template void launch_ydense<ERM_T, ERM_K, +1>(erm_ctx *, const Params &);
 template void launch_zgreen<ERM_T, ERM_K>(erm_ctx *, const Params &);
+#endif
 
 }  // namespace ermh

@@ -68,13 +68,14 @@ def test_register_lengths(name):
     np.testing.assert_allclose(got, want, rtol=1e-12, atol=1e-10)
 
 
-@pytest.mark.parametrize("K,n", [(16, 3), (24, 3), (32, 3), (48, 40), (64, 3)])
-def test_slab_shapes_round_alike(K, n):
+@pytest.mark.parametrize("K,order,n", [(16, 4, 3), (24, 4, 3), (32, 4, 3), (48, 4, 40), (64, 4, 3), (16, 6, 3),
+                                       (24, 5, 3), (32, 6, 40), (48, 6, 3), (48, 5, 3), (96, 4, 2)])
+def test_slab_shapes_round_alike(K, order, n):
     """The slab shape that a launch chooses against 256 threads with the y
     columns in a kernel of their own."""
-    print(f"\n[gpu case] FP32 slab shapes, {K}^3, {n} configurations", flush=True)
+    print(f"\n[gpu case] FP32 slab shapes, {K}^3 order {order}, {n} configurations", flush=True)
     sy = synth.refs20(nwater=220, L=25.0, K=16, nsite=12)
-    s = sy.system = dataclasses.replace(sy.system, ms=(K, K, K))
+    s = sy.system = dataclasses.replace(sy.system, ms=(K, K, K), splodr=order)
     places = np.array([O.place_solute(s.bfcoord, s.solute_mass(sy.solute_mol), sy.cell, *O.random_pose(70 + K, j))
                        for j in range(n)])
     got = []
